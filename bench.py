@@ -666,7 +666,7 @@ def main():
                "rel_err_gpu_vs_cpu": err}
 
     achieved = main_res["kernel_tflops"]
-    kernel_name = "k_assemble" if os.environ.get("BIE_AMD_KERNEL") == "atomic" else "k_assemble_slots"
+    kernel_name = "k_assemble" if os.environ.get("BIE_AMD_KERNEL") == "atomic" else "k_stream"
     out = {
         "metric": METRIC,
         "value": main_res["entries_per_s"],

@@ -15,7 +15,7 @@ PKG = os.path.dirname(HERE)
 CSRC = os.path.join(PKG, "csrc")
 LIB_PATH = os.path.join(HERE, "libbie_amd.so")
 
-SOURCES = ["rules.cpp", "schedule.cpp", "assemble.hip", "sweep.hip", "adjoint.hip", "apply.hip",
+SOURCES = ["rules.cpp", "schedule.cpp", "assemble.hip", "stream.hip", "sweep.hip", "adjoint.hip", "apply.hip",
            "solve.hip", "sparse.hip", "near_field.cpp", "api.hip"]
 # rocSOLVER (LU) and rocBLAS (GEMV) from the ROCm install, found at run time by rpath
 ROCM_LIB = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "lib")

@@ -118,6 +118,9 @@ std::vector<int> convert_topology(const int64_t* t, int rows, int64_t E, int64_t
   return out;
 }
 
+// Flat elements with their own linear physics take the flat form of the stream kernels.
+bool flat_elements(const bie_dmesh* dm) { return dm->gkind == BIE_TRI3 && dm->pkind == BIE_TRI3; }
+
 void ensure_rules(bie_dmesh* dm, int n, int m, hipStream_t s) {
   if (dm->cn == n && dm->cm == m && dm->d_elem) return;
   RuleSet rs = build_ruleset(dm->gkind, dm->pkind, dm->beta, n, m);
@@ -125,25 +128,22 @@ void ensure_rules(bie_dmesh* dm, int n, int m, hipStream_t s) {
   dfree(dm->d_pts);
   dfree(dm->d_phi);
   dfree(dm->d_elem);
-  dm->d_pts = dm->d_phi = dm->d_elem = nullptr;
+  dfree(dm->d_stab);
+  dm->d_pts = dm->d_phi = dm->d_elem = dm->d_stab = nullptr;
   dm->cn = dm->cm = -1;
   dm->geom_valid = false;
   dm->d_pts = dalloc<double>(rs.pts.size());
-  // basis table, padded to phi_pad doubles, then the trig table of the slot kernels
-  const int nphi = rs.R * rs.Qmax * dm->pk;
-  BIE_REQUIRE((size_t)nphi == rs.phi.size(), BIE_EINVAL, "internal: basis table size mismatch");
-  std::vector<double> phi_trig((size_t)phi_pad(nphi) + kTrigDoubles, 0.0);
-  std::copy(rs.phi.begin(), rs.phi.end(), phi_trig.begin());
-  for (int j = 0; j < kTrigN; ++j) {  // (cos, sin)(j pi / 64), rounded from long double
-    const long double th = (long double)j * (3.14159265358979323846264338327950288L / 64);
-    phi_trig[phi_pad(nphi) + 2 * j] = (double)cosl(th);
-    phi_trig[phi_pad(nphi) + 2 * j + 1] = (double)sinl(th);
-  }
-  dm->d_phi = dalloc<double>(phi_trig.size());
+  BIE_REQUIRE((size_t)rs.R * rs.Qmax * dm->pk == rs.phi.size(), BIE_EINVAL,
+              "internal: basis table size mismatch");
+  dm->d_phi = dalloc<double>(rs.phi.size());
   dm->d_elem = dalloc<double>((size_t)std::max<int64_t>(dm->E, 1) * rs.Pe * 8);
+  const std::vector<double> stab = stream_tables(rs, flat_elements(dm));
+  dm->d_stab = dalloc<double>(stab.size());
+  BIE_HIP_CHECK(hipMemcpyAsync(dm->d_stab, stab.data(), stab.size() * sizeof(double),
+                               hipMemcpyHostToDevice, s));
   BIE_HIP_CHECK(hipMemcpyAsync(dm->d_pts, rs.pts.data(), rs.pts.size() * sizeof(double),
                                hipMemcpyHostToDevice, s));
-  BIE_HIP_CHECK(hipMemcpyAsync(dm->d_phi, phi_trig.data(), phi_trig.size() * sizeof(double),
+  BIE_HIP_CHECK(hipMemcpyAsync(dm->d_phi, rs.phi.data(), rs.phi.size() * sizeof(double),
                                hipMemcpyHostToDevice, s));
   BIE_HIP_CHECK(hipStreamSynchronize(s));
   dm->rs = std::move(rs);
@@ -178,54 +178,11 @@ struct Timing {
 };
 Timing g_timing;
 
-// Which assembly kernel to use: the LDS-slot kernel (default) or the all-atomics kernel
-// (BIE_AMD_KERNEL=atomic), kept for small problems and as a cross-check.
+// Which assembly kernel to use: the stream kernel (default) or the all-atomics kernel
+// (BIE_AMD_KERNEL=atomic), kept for very long rules and as a cross-check.
 bool use_atomic_kernel() {
   const char* v = std::getenv("BIE_AMD_KERNEL");
   return v && std::strcmp(v, "atomic") == 0;
-}
-
-// LDS slots per workgroup of the single-k slot kernel: as many as fit beside the basis
-// and trig tables, the staged table rows and the mid-edge queue (one workgroup per CU);
-// BIE_AMD_SLOTS=<n> asks for fewer.
-int slot_occupancy() {
-  const char* v = std::getenv("BIE_AMD_OCC");
-  return (v && std::atoi(v) == 2) ? 2 : 1;
-}
-
-// Elements each wave takes per step of the single-k slot kernel (1 or 2).
-int slot_elems_per_wave() {
-  const char* v = std::getenv("BIE_AMD_V");
-  return (v && std::atoi(v) == 2) ? 2 : 1;
-}
-
-int slot_split() {
-  const char* v = std::getenv("BIE_AMD_SPLIT");
-  return (v && std::atoi(v) == 2) ? 2 : 1;
-}
-
-// Waves per workgroup of the single-k slot kernel on the real-k unrolled instances:
-// kWideWaves (three per SIMD) for three-node physics, kSlotWaves for six-node physics,
-// whose wide instance needs more registers than three waves per SIMD leave (measured
-// slower); BIE_AMD_WAVES=8 or 12 forces either.
-int slot_waves(int NP) {
-  if (const char* v = std::getenv("BIE_AMD_WAVES")) {
-    const int x = std::atoi(v);
-    if (x == kWideWaves || x == kSlotWaves) return x;
-  }
-  return NP == 3 ? kWideWaves : kSlotWaves;
-}
-
-int plain_slot_count(int nphi, int Qc, int occ = 1, int split = 1, int waves = kSlotWaves) {
-  // LDS of one workgroup when occ of them share a CU (allocation granularity left spare)
-  const long budget = occ == 2 ? kLdsBytes / 2 - 1024 : kLdsBytes;
-  const int stage = split == 2 ? split_stage_doubles(Qc, 2) : stage_doubles(Qc, waves);
-  int S = fitting_slots(phi_pad(nphi) + kTrigDoubles + stage, 1, budget);
-  if (const char* v = std::getenv("BIE_AMD_SLOTS")) {
-    const int x = std::atoi(v);
-    if (x >= 8 && x < S) S = x;
-  }
-  return S;
 }
 
 template <class T>
@@ -236,58 +193,27 @@ T* upload_vec(const std::vector<T>& v, hipStream_t s) {
   return d;
 }
 
-void free_schedule(bie_dmesh::Sched& sc) {
-  // kernels still in flight may read the schedule being replaced
-  if (sc.d_step_elems) (void)hipDeviceSynchronize();
-  for (int** p : {&sc.d_seg_step_begin, &sc.d_step_elems, &sc.d_step_slot, &sc.d_flush_begin,
-                  &sc.d_flush_node, &sc.d_flush_slot, &sc.d_zero_cols}) {
-    dfree(*p);
-    *p = nullptr;
-  }
-  dfree(sc.d_step_sel);
-  sc.d_step_sel = nullptr;
-  sc.key = -1;
-  sc.S = -1;
-}
-
-void free_schedules(bie_dmesh* dm) {
-  for (auto& sc : dm->sched) free_schedule(sc);
-}
-
-// Segment count of the single-k slot kernel's schedule: at least 8 tiles (row block x
-// segment) per CU, and among counts up to twice that, the one whose tile count fills whole
-// rounds of resident workgroups (one per CU) best, so that the last round leaves few CUs
-// idle.  (The schedule may split further where a segment's front exceeds the slots.)
-int choose_segment_count(int device, int64_t rowblocks, int64_t E, int per_cu = 1) {
+int device_cus(int device) {
+  static std::mutex mu;
   static int cus_of[16] = {0};
+  std::lock_guard<std::mutex> lk(mu);
   int& cus = cus_of[device & 15];
   if (cus == 0) {
     BIE_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
     if (cus <= 0) cus = 1;
   }
-  const int64_t round = (int64_t)cus * per_cu;  // workgroups resident at once
-  const int64_t hi_e = std::max<int64_t>(1, E);
-  const int64_t base = std::max<int64_t>(1, std::min<int64_t>(hi_e, (8LL * round + rowblocks - 1) / rowblocks));
-  int64_t best = base;
-  double best_waste = 1e300;
-  for (int64_t p = base; p <= std::min<int64_t>(hi_e, 2 * base); ++p) {
-    const int64_t tiles = rowblocks * p;
-    const double waste = (double)((tiles + round - 1) / round * round) / (double)tiles;
-    if (waste < best_waste - 1e-12) {
-      best_waste = waste;
-      best = p;
-    }
-  }
-  return (int)best;
+  return cus;
 }
 
-// Schedule `which` (0: single-k kernel, 1: sweep kernel, 2: batch kernel) for S live
-// slots and at least min_segments segments.
-bie_dmesh::Sched& ensure_schedule(bie_dmesh* dm, int which, int S, int min_segments,
-                                  hipStream_t s, int wv = kSlotWaves) {
-  bie_dmesh::Sched& out = dm->sched[which];
-  if (out.key == min_segments && out.S == S && out.wv == wv && out.d_step_elems) return out;
-  free_schedule(out);
+void free_stream(bie_dmesh::Stream& sc) {
+  if (sc.d_order) (void)hipDeviceSynchronize();  // kernels in flight may read it
+  for (void* p : {(void*)sc.d_seg_begin, (void*)sc.d_order, (void*)sc.d_ent, (void*)sc.d_psel,
+                  (void*)sc.d_flat, (void*)sc.d_zero_cols})
+    dfree(p);
+  sc = bie_dmesh::Stream{};
+}
+
+std::vector<double> element_centres(const bie_dmesh* dm) {
   std::vector<double> cent((size_t)dm->E * 3);
   for (int64_t e = 0; e < dm->E; ++e)
     for (int d = 0; d < 3; ++d) {
@@ -295,134 +221,218 @@ bie_dmesh::Sched& ensure_schedule(bie_dmesh* dm, int which, int S, int min_segme
       for (int k = 0; k < 3; ++k) acc += dm->h_coords[3 * (size_t)dm->h_topo[e * dm->gk + k] + d];
       cent[3 * e + d] = acc / 3.0;
     }
-  SlotSchedule sc = build_slot_schedule(dm->h_ptopo.data(), dm->pk, (int)dm->E, (int)dm->N,
-                                        cent.data(), wv, S, min_segments);
-  out.d_seg_step_begin = upload_vec(sc.seg_step_begin, s);
-  out.h_seg_step_begin = sc.seg_step_begin;
-  out.d_step_elems = upload_vec(sc.step_elems, s);
-  // per (step, wave) copies of the selection nodes and slots, in the order the kernel
-  // reads them
-  const size_t nsw = (size_t)sc.n_steps * wv;
-  std::vector<int> step_slot(nsw * dm->pk, 0);
-  std::vector<double> step_sel(nsw * dm->pk * 4, 0.0);
-  for (size_t t = 0; t < nsw; ++t) {
-    const int e = sc.step_elems[t];
-    if (e < 0) continue;
-    for (int k = 0; k < dm->pk; ++k) {
-      step_slot[t * dm->pk + k] = sc.slot_of[(size_t)e * dm->pk + k];
-      const int node = dm->h_ptopo[(size_t)e * dm->pk + k];
-      for (int d = 0; d < 3; ++d)
-        step_sel[(t * dm->pk + k) * 4 + d] = dm->h_sources[3 * (size_t)node + d];
+  return cent;
+}
+
+// Segments of the stream kernel's schedule (at least `least`, which the slots force), from an
+// estimate of its time in clocks of a CU: the rounds of tiles that the CUs work off, each a
+// segment's pairs plus about 2.5 us to begin, and the columns that several segments add to
+// (about 1.5 sqrt(E segments) on three-node, 3.4 sqrt(E segments) on six-node physics), which
+// cost zeros and atomics.
+int choose_stream_segments(int64_t rowblocks, int64_t E, int Q, int NP, int cus, int64_t least) {
+  const double pair = 100.0 * Q + 80.0 * NP, begin = 6000.0, border = NP >= 6 ? 3.4 : 1.5;
+  int best = (int)least;
+  double best_cost = 1e300;
+  for (int64_t p = least; p <= std::max(least, std::min<int64_t>(E / 8, 512)); ++p) {
+    const int64_t rounds = (rowblocks * p + cus - 1) / cus;
+    const double cost = (double)rounds * ((double)((E + p - 1) / p) * pair + begin) +
+                        200.0 * border * std::sqrt((double)E * p) * rowblocks / cus;
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = (int)p;
     }
   }
-  out.d_step_slot = upload_vec(step_slot, s);
-  out.d_step_sel = upload_vec(step_sel, s);
-  out.d_flush_begin = upload_vec(sc.flush_begin, s);
-  out.d_flush_node = upload_vec(sc.flush_node, s);
-  out.d_flush_slot = upload_vec(sc.flush_slot, s);
+  return best;
+}
+
+StreamSchedule stream_schedule(const bie_dmesh* dm, const std::vector<double>& cent, int S,
+                               int64_t segments) {
+  return build_stream_schedule(dm->h_ptopo.data(), dm->pk, (int)dm->E, (int)dm->N, cent.data(), S,
+                               (int)segments);
+}
+
+// Puts a schedule on the device (key: what it was chosen for).
+void upload_stream(bie_dmesh* dm, bie_dmesh::Stream& out, const StreamSchedule& sc, int S,
+                   int64_t key, hipStream_t s) {
+  free_stream(out);
+  std::vector<int4> ent(sc.ent.size());
+  std::vector<double> psel(sc.ent.size() * 3);
+  for (size_t t = 0; t < sc.ent.size(); ++t) {
+    const StreamEntry& x = sc.ent[t];
+    ent[t] = make_int4(x.slot, x.count, x.turn, x.node);
+    for (int d = 0; d < 3; ++d)
+      psel[3 * t + d] = dm->h_sources[3 * (size_t)(x.node & ~kSharedBit) + d];
+  }
+  out.d_seg_begin = upload_vec(sc.seg_begin, s);
+  out.d_order = upload_vec(sc.order, s);
+  out.d_ent = upload_vec(ent, s);
+  out.d_psel = upload_vec(psel, s);
   out.d_zero_cols = upload_vec(sc.zero_cols, s);
+  if (flat_elements(dm)) out.d_flat = dalloc<double>((size_t)dm->E * kFlatDoubles);
   BIE_HIP_CHECK(hipStreamSynchronize(s));
+  out.h_seg_begin = sc.seg_begin;
   out.segments = sc.n_segments;
   out.zero_cols = (int)sc.zero_cols.size();
-  out.max_live = sc.max_live;
-  out.key = min_segments;
+  out.key = key;
   out.S = S;
-  out.wv = wv;
+}
+
+// Segments cannot have more elements than a position within one has bits (24).
+int64_t least_segments(const bie_dmesh* dm) { return dm->E / (1 << 24) + 1; }
+
+// The schedule for S slots that suits single-mesh calls of rowblocks row blocks.
+bie_dmesh::Stream& ensure_stream(bie_dmesh* dm, int S, int64_t rowblocks, int cus,
+                                 hipStream_t s) {
+  bie_dmesh::Stream& out = dm->stream;
+  const int Q = dm->rs.len[0];
+  const int64_t key = rowblocks * 65536 + std::min(Q, 65535);
+  if (out.key == key && out.S == S && out.d_order) return out;
+  const std::vector<double> cent = element_centres(dm);
+  const int64_t least = least_segments(dm);
+  int want = choose_stream_segments(rowblocks, dm->E, Q, dm->pk, cus, least);
+  StreamSchedule sc = stream_schedule(dm, cent, S, want);
+  if (sc.n_segments != want) {  // the slots force more: fill the rounds of those
+    want = choose_stream_segments(rowblocks, dm->E, Q, dm->pk, cus, sc.n_segments);
+    StreamSchedule other = stream_schedule(dm, cent, S, want);
+    if (std::abs(other.n_segments - want) <= 1 || other.n_segments < sc.n_segments)
+      sc = std::move(other);
+  }
+  upload_stream(dm, out, sc, S, key, s);
   return out;
 }
 
-SlotArgs slot_args(bie_dmesh* dm, const bie_dmesh::Sched& sc, int64_t rowblocks) {
-  SlotArgs sa{};
-  sa.W = sc.wv;
-  sa.S = sc.S;
-  sa.n_segments = sc.segments;
-  sa.n_rowblocks = (int)rowblocks;
-  sa.n_tiles = rowblocks * sc.segments;
-  const char* ord = std::getenv("BIE_AMD_TILE_ORDER");
-  sa.seg_major = (ord && std::strcmp(ord, "rowblock") == 0) ? 0 : 1;
-  sa.phi_in_lds = 1;
-  sa.seg_step_begin = sc.d_seg_step_begin;
-  sa.step_elems = sc.d_step_elems;
-  sa.step_slot = sc.d_step_slot;
-  sa.step_sel = sc.d_step_sel;
-  sa.flush_begin = sc.d_flush_begin;
-  sa.flush_node = sc.d_flush_node;
-  sa.flush_slot = sc.d_flush_slot;
-  sa.mid_count = dm->d_mid_count;
-  sa.mid_queue = dm->d_mid_queue;
-  sa.mid_cap = dm->mid_cap;
-  sa.push_mid = 1;
-  return sa;
+// The schedule of dm in a batch: S slots, at least `segments` segments.  The records of flat
+// elements are written here, once (a single-mesh call writes its own each time).
+bie_dmesh::Stream& ensure_batch_stream(bie_dmesh* dm, int S, int64_t segments, hipStream_t s) {
+  bie_dmesh::Stream& out = dm->bstream;
+  if (out.key == segments && out.S == S && out.d_order) return out;
+  upload_stream(dm, out,
+                stream_schedule(dm, element_centres(dm), S,
+                                std::max(segments, least_segments(dm))),
+                S, segments, s);
+  if (out.d_flat) {
+    StreamPrep p{};
+    p.E = (int)dm->E;
+    p.coords = dm->d_coords;
+    p.sources = dm->d_sources;
+    p.topo = dm->d_topo;
+    p.ptopo = dm->d_ptopo;
+    p.order = out.d_order;
+    p.flat = out.d_flat;
+    launch_stream_flat(p, s);
+    // another stream's batch may read them before an event of this one is recorded
+    BIE_HIP_CHECK(hipStreamSynchronize(s));
+  }
+  return out;
 }
 
-void ensure_mid_queue(bie_dmesh* dm, int64_t cap) {
-  if (!dm->d_mid_count) dm->d_mid_count = dalloc<unsigned>(1);
-  if (dm->mid_cap >= cap && dm->d_mid_queue) return;
-  dfree(dm->d_mid_queue);
-  dm->d_mid_queue = nullptr;
-  dm->mid_cap = 0;
-  dm->d_mid_queue = dalloc<int2>((size_t)cap);
-  dm->mid_cap = cap;
-}
-
-// Records the collocation mid-edge pairs that the slot kernel queued: the pairs sorted by
-// (element, target), and the distinct (column, row) entries of F and G they add to, sorted
-// by (column, row), each with the list of (pair, node) contributions.  Releases the queue.
-// Host work once per mesh; synchronises the stream.
-void record_mid_pairs(bie_dmesh* dm, hipStream_t s) {
-  unsigned count = 0;
-  BIE_HIP_CHECK(hipMemcpyAsync(&count, dm->d_mid_count, sizeof(unsigned), hipMemcpyDeviceToHost, s));
-  BIE_HIP_CHECK(hipStreamSynchronize(s));
-  const int64_t n = std::min<int64_t>((int64_t)count, dm->mid_cap);
-  BIE_REQUIRE(n < (int64_t)1 << 28, BIE_EINVAL, "too many mid-edge pairs to record");
-  std::vector<int2> q((size_t)n);
-  if (n)
-    BIE_HIP_CHECK(hipMemcpy(q.data(), dm->d_mid_queue, sizeof(int2) * n, hipMemcpyDeviceToHost));
-  std::vector<unsigned long long> keys((size_t)n);
-  for (int64_t p = 0; p < n; ++p)
-    keys[p] = ((unsigned long long)(q[p].y & 0x0fffffff) << 34) |
-              ((unsigned long long)(unsigned)q[p].x << 2) | (unsigned long long)(q[p].y >> 28);
-  std::sort(keys.begin(), keys.end());
-  std::vector<std::pair<unsigned long long, int>> con((size_t)n * 6);
-  for (int64_t p = 0; p < n; ++p) {
-    const int e = (int)(keys[p] >> 34);
-    const unsigned row = (unsigned)((keys[p] >> 2) & 0xffffffffull);
-    for (int k = 0; k < 6; ++k) {
-      const unsigned col = (unsigned)dm->h_ptopo[(size_t)e * 6 + k];
-      con[(size_t)p * 6 + k] = {((unsigned long long)col << 32) | row, (int)(p * 6 + k)};
-    }
-  }
-  std::sort(con.begin(), con.end());
-  std::vector<unsigned long long> entries;
-  std::vector<int> off, refs(con.size());
-  for (size_t t = 0; t < con.size(); ++t) {
-    if (t == 0 || con[t].first != con[t - 1].first) {
-      entries.push_back(con[t].first);
-      off.push_back((int)t);
-    }
-    refs[t] = con[t].second;
-  }
-  off.push_back((int)con.size());
-  auto up = [&](auto& v) { return upload_vec(v, s); };
-  unsigned long long* d_keys = up(keys);
-  unsigned long long* d_entries = up(entries);
-  int* d_off = up(off);
-  int* d_refs = up(refs);
-  double* d_vals = dalloc<double>((size_t)std::max<int64_t>(n, 1) * 24);
-  BIE_HIP_CHECK(hipStreamSynchronize(s));
-  for (void* p : {(void*)dm->d_mid_keys, (void*)dm->d_mid_entries, (void*)dm->d_mid_off,
-                  (void*)dm->d_mid_refs, (void*)dm->d_mid_vals})
+void free_lists(StreamLists& l) {
+  for (void* p : {(void*)l.counters, (void*)l.mid_queue, (void*)l.mid_tiles, (void*)l.slow})
     dfree(p);
-  dm->d_mid_keys = d_keys;
-  dm->d_mid_entries = d_entries;
-  dm->d_mid_off = d_off;
-  dm->d_mid_refs = d_refs;
-  dm->d_mid_vals = d_vals;
-  dm->n_mid_keys = n;
-  dm->n_mid_entries = (int64_t)entries.size();
-  dfree(dm->d_mid_queue);  // the M x E queue is no longer needed for collocation
-  dm->d_mid_queue = nullptr;
-  dm->mid_cap = 0;
+  l = StreamLists{};
+}
+
+// Room in a call's lists.  mids: for the mid-edge pairs of M targets and E elements, a
+// sixteenth of all pairs (a sphere has one in a hundred), and for every tile of one matrix
+// block should that not do; slow_tiles: for so many slow tiles.
+void ensure_lists(StreamLists& l, bool mids, int64_t M, int64_t E, int segments,
+                  int64_t slow_tiles) {
+  if (!l.counters) l.counters = dalloc<unsigned>(kStreamCounters);
+  const int64_t pairs = M * E;
+  const int64_t cap =
+      std::min<int64_t>(std::min<int64_t>(pairs, pairs / 16 + (1 << 18)), 1LL << 30);
+  const int64_t tiles = (M + 63) / 64 * segments;
+  if (mids && (l.mid_cap < cap || l.mid_tiles_cap < tiles)) {
+    if (l.mid_queue) (void)hipDeviceSynchronize();  // a launch may still use them
+    dfree(l.mid_queue);
+    dfree(l.mid_tiles);
+    l.mid_queue = l.mid_tiles = nullptr;
+    l.mid_cap = l.mid_tiles_cap = 0;
+    l.mid_queue = dalloc<int2>((size_t)cap);
+    l.mid_tiles = dalloc<int2>((size_t)tiles);
+    l.mid_cap = cap;
+    l.mid_tiles_cap = tiles;
+  }
+  if (l.slow_cap < slow_tiles) {
+    if (l.slow) (void)hipDeviceSynchronize();
+    dfree(l.slow);
+    l.slow = nullptr;
+    l.slow_cap = 0;
+    l.slow = dalloc<int>((size_t)slow_tiles);
+    l.slow_cap = slow_tiles;
+  }
+}
+
+StreamInst stream_inst(const bie_dmesh* dm, const AssemblyArgs& a, const bie_dmesh::Stream& sc,
+                       const StreamLists& l, int64_t rowblocks) {
+  StreamInst in{};
+  in.coords = dm->d_coords;
+  in.topo = dm->d_topo;
+  in.own_basis = dm->pkind == dm->gkind ? 1 : 0;
+  in.mid_off = stream_mid_offset(dm->rs, flat_elements(dm));
+  in.a = a;
+  in.seg_begin = sc.d_seg_begin;
+  in.order = sc.d_order;
+  in.ent = sc.d_ent;
+  in.psel = sc.d_psel;
+  in.flat = sc.d_flat;
+  in.n_segments = sc.segments;
+  in.n_rowblocks = (int)rowblocks;
+  in.mid_count = l.counters + kMidCount;
+  in.mid_queue = l.mid_queue;
+  in.mid_tiles = l.mid_tiles;
+  in.mid_cap = (unsigned)l.mid_cap;
+  for (int d = 0; d < 3; ++d) in.center[d] = dm->center[d];
+  in.reach = 4.0 * dm->coord_radius;
+  return in;
+}
+
+// The preparation of a call on the stream kernels for nk matrices: geometry (flat records, or
+// element tables where points are tabulated), zeros and counters.
+StreamPrep stream_prep(bie_dmesh* dm, const AssemblyArgs& a, const bie_dmesh::Stream& sc,
+                       const StreamLists& l, int nk, int64_t stride) {
+  StreamPrep p{};
+  p.M = a.M;
+  p.E = a.E;
+  p.Pe = a.Pe;
+  p.Pv = std::min(a.R, 3) * a.len[0];
+  p.gk = dm->gk;
+  p.flags = a.flags;
+  p.F = a.F;
+  p.G = a.G;
+  p.C = a.C;
+  p.zero_cols = sc.d_zero_cols;
+  p.n_zero = sc.zero_cols;
+  // (a disabled output of a sweep may be NULL)
+  p.n_whole = (!(a.flags & BIE_F) && a.F) || (!(a.flags & BIE_G) && a.G) ? (int)a.N : 0;
+  p.nk = nk;
+  p.stride = stride;
+  p.counters = l.counters;
+  p.mid_cap = (unsigned)l.mid_cap;
+  p.coords = dm->d_coords;
+  p.sources = dm->d_sources;
+  p.pts = dm->d_pts;
+  p.topo = dm->d_topo;
+  p.ptopo = dm->d_ptopo;
+  p.order = sc.d_order;
+  p.flat = sc.d_flat;
+  p.elem = sc.d_flat ? nullptr : dm->d_elem;
+  return p;
+}
+
+// The sweep kernel's schedule: S slots and at least min_segments segments (0: as suits the
+// collocation rows).  It does not depend on a call's targets or matrices: a graph keeps it.
+bie_dmesh::Stream& ensure_sweep_stream(bie_dmesh* dm, int S, int64_t min_segments, int cus,
+                                       hipStream_t s) {
+  bie_dmesh::Stream& out = dm->sstream;
+  const int64_t key = min_segments * 65536 + std::min(dm->rs.len[0], 65535);
+  if (out.key == key && out.S == S && out.d_order) return out;
+  int64_t want = std::max(min_segments, least_segments(dm));
+  if (min_segments == 0)
+    want = choose_stream_segments((dm->N + 63) / 64, dm->E, dm->rs.len[0], dm->pk, cus,
+                                  least_segments(dm));
+  upload_stream(dm, out, stream_schedule(dm, element_centres(dm), S, want), S, key, s);
+  return out;
 }
 
 AssemblyArgs make_args(bie_dmesh* dm, const double* d_targets, int64_t M, double kr,
@@ -492,8 +502,8 @@ double radius_about(const double* c, const double* x, int64_t n) {
 // at most |x - c| + |y - c| for a target x and an element point y, and y = sum N_k X_k with
 // sum |N_k| <= 2 on linear and quadratic triangles, so |y - c| <= 2 coord_radius (taken
 // twice again for margin).  target_radius < 0: unknown (device targets), never fast.
-bool fast_trig_ok(const bie_dmesh* dm, double kr, double ki, double target_radius) {
-  if (ki != 0.0 || !(target_radius >= 0.0)) return false;
+bool fast_trig_ok(const bie_dmesh* dm, double kr, double target_radius) {
+  if (!(target_radius >= 0.0)) return false;
   const double reach = target_radius + 4.0 * dm->coord_radius;
   return std::isfinite(reach) && std::fabs(kr) * reach < 0.5 * kTabFastMaxArg;
 }
@@ -525,81 +535,33 @@ void assemble_device_impl(bie_dmesh* dm, double kr, double ki, const double* d_t
     }
   }
   if (timed) BIE_HIP_CHECK(hipEventRecord(ev[0], s));
-  const bool atomic_path = use_atomic_kernel() || M == 0 || dm->E == 0 ||
-                           sizeof(double) * (size_t)dm->rs.R * dm->rs.Qmax * dm->pk > 24 * 1024;
-  if (atomic_path || !(flags & BIE_F)) launch_fill_zero(dF, 2 * M * dm->N, s);
-  if (atomic_path || !(flags & BIE_G)) launch_fill_zero(dG, 2 * M * dm->N, s);
-  launch_fill_zero(dC, 2 * M, s);
+  const StreamPlan plan = stream_plan(dm->rs, flat_elements(dm), (flags & BIE_G) != 0);
+  const bool atomic_path =
+      use_atomic_kernel() || sizeof(double) * (size_t)dm->rs.R * dm->rs.Qmax * dm->pk > 24 * 1024;
+  if (M == 0 || dm->E == 0 || atomic_path) {
+    launch_fill_zero(dF, 2 * M * dm->N, s);
+    launch_fill_zero(dG, 2 * M * dm->N, s);
+    launch_fill_zero(dC, 2 * M, s);
+  }
   if (M > 0 && dm->E > 0) {
-    refresh_geometry(dm, s);
     AssemblyArgs a = make_args(dm, d_targets, M, kr, ki, flags, dF, dG, dC);
-    const bool phi_fits = sizeof(double) * (size_t)a.R * a.Qmax * a.NP <= 24 * 1024;
-    if (use_atomic_kernel() || !phi_fits) {
+    if (atomic_path) {
+      refresh_geometry(dm, s);
       if (timed) BIE_HIP_CHECK(hipEventRecord(ev[1], s));
       launch_assemble(a, s);
       if (timed) BIE_HIP_CHECK(hipEventRecord(ev[2], s));
     } else {
       const int64_t rowblocks = (M + 63) / 64;
-      const bool fast = fast_trig_ok(dm, kr, ki, target_radius);
-      const bool qc_inst = fast && (a.len[0] == 4 || a.len[0] == 6 || a.len[0] == 16);
-      // the occupancy, split and two-element variants exist for three- and six-node physics
-      const bool tuned = qc_inst && (dm->pk == 3 || dm->pk == 6);
-      const int occ = tuned ? slot_occupancy() : 1;
-      const int split = tuned && occ == 1 ? slot_split() : 1;
-      const int waves = tuned && occ == 1 && split == 1 ? slot_waves(dm->pk) : kSlotWaves;
-      const int vpw =
-          tuned && occ == 1 && split == 1 && waves == kSlotWaves ? slot_elems_per_wave() : 1;
-      const int min_segments = choose_segment_count(dm->device, rowblocks, dm->E, occ);
-      const bie_dmesh::Sched& sc = ensure_schedule(
-          dm, 0, plain_slot_count(a.R * a.Qmax * a.NP, a.len[0], occ, split, waves),
-          min_segments, s, waves * vpw);
-      // collocation on quadratic physics: after the first call the mid-edge pairs come
-      // from the recorded sorted list instead of the slot kernel's queue
-      const bool colloc = d_targets == dm->d_sources && M == dm->N;
-      const bool mids = uses_mid_rules(dm->gk, dm->pk);
-      const bool recorded = mids && colloc && dm->n_mid_keys >= 0;
-      if (mids && !recorded) {
-        ensure_mid_queue(dm, M * dm->E);
-        launch_fill_zero_u32(dm->d_mid_count, s);
-      } else if (!dm->d_mid_count) {
-        dm->d_mid_count = dalloc<unsigned>(1);
-      }
-      SlotArgs sa = slot_args(dm, sc, rowblocks);
-      sa.push_mid = recorded ? 0 : 1;
-      sa.occupancy = occ;
-      sa.split = split;
-      // The slot kernel stores owned columns once; only shared/untouched columns need
-      // zeros (a disabled output is zeroed whole above and never written).
-      if (flags & BIE_F) launch_zero_columns(dF, M, sc.d_zero_cols, sc.zero_cols, s);
-      if (flags & BIE_G) launch_zero_columns(dG, M, sc.d_zero_cols, sc.zero_cols, s);
-      // recorded mid-edge pairs: their values do not depend on the slot kernel, so they are
-      // computed on the handle's side stream while it runs (in a captured graph: in order)
-      const bool side = recorded && dm->n_mid_keys > 0 && !capturing(s);
-      if (side) {
-        if (!dm->side) {
-          BIE_HIP_CHECK(hipStreamCreateWithFlags(&dm->side, hipStreamNonBlocking));
-          BIE_HIP_CHECK(hipEventCreateWithFlags(&dm->side_fork, hipEventDisableTiming));
-          BIE_HIP_CHECK(hipEventCreateWithFlags(&dm->side_join, hipEventDisableTiming));
-        }
-        BIE_HIP_CHECK(hipEventRecord(dm->side_fork, s));  // after the zero fills and geometry
-        BIE_HIP_CHECK(hipStreamWaitEvent(dm->side, dm->side_fork, 0));
-        launch_mid_compute(a, dm->d_mid_keys, dm->n_mid_keys, dm->d_mid_vals, dm->side);
-        BIE_HIP_CHECK(hipEventRecord(dm->side_join, dm->side));
-      }
+      const bool fast = fast_trig_ok(dm, kr, target_radius);
+      const int cus = device_cus(dm->device);
+      bie_dmesh::Stream& sc = ensure_stream(dm, plan.S, rowblocks, cus, s);
+      StreamLists& l = dm->lists;
+      ensure_lists(l, plan.mids, M, dm->E, sc.segments, fast ? 0 : rowblocks * sc.segments);
+      launch_stream_prep(stream_prep(dm, a, sc, l, 1, 0), s);
       if (timed) BIE_HIP_CHECK(hipEventRecord(ev[1], s));
-      launch_assemble_slots(a, sa, fast, s);
+      launch_stream(stream_inst(dm, a, sc, l, rowblocks), plan, dm->d_stab, l.counters, l.slow,
+                    cus, fast, s);
       if (timed) BIE_HIP_CHECK(hipEventRecord(ev[2], s));
-      if (side) {
-        BIE_HIP_CHECK(hipStreamWaitEvent(s, dm->side_join, 0));
-        launch_mid_scatter(a, dm->n_mid_keys, dm->d_mid_vals, dm->d_mid_entries, dm->d_mid_off,
-                           dm->d_mid_refs, dm->n_mid_entries, s);
-      } else if (recorded) {
-        launch_mid_recorded(a, dm->d_mid_keys, dm->n_mid_keys, dm->d_mid_vals, dm->d_mid_entries,
-                            dm->d_mid_off, dm->d_mid_refs, dm->n_mid_entries, s);
-      } else {
-        launch_assemble_mid(a, sa, s);
-        if (mids && colloc) record_mid_pairs(dm, s);
-      }
     }
   } else if (timed) {
     BIE_HIP_CHECK(hipEventRecord(ev[1], s));
@@ -615,12 +577,13 @@ void assemble_device_impl(bie_dmesh* dm, double kr, double ki, const double* d_t
 
 // Batched sweep over nk real wavenumbers (d_k on the device), or with taylor the k
 // derivatives of orders 0..nk-1 at k_re + i k_im (d_k unused).  prepare_only builds every
-// cache (rules, schedule, queues) without launching, so that a later call can be
-// captured into a graph.
+// cache (rules, schedule, lists) without launching, so that a later call can be captured
+// into a graph; lists are the graph's own then.
 void sweep_device_impl(bie_dmesh* dm, const double* d_k, int nk, const double* d_targets,
                        int64_t M, int n, int m, uint32_t flags, double* dF, double* dG,
-                       int64_t stride, double* dC, hipStream_t s, bool prepare_only,
-                       bool taylor = false, double k_re = 0.0, double k_im = 0.0) {
+                       int64_t stride, double* dC, hipStream_t s, StreamLists& lists,
+                       bool prepare_only, bool taylor = false, double k_re = 0.0,
+                       double k_im = 0.0) {
   BIE_REQUIRE(dm != nullptr, BIE_EINVAL, "dmesh is NULL");
   BIE_REQUIRE(!kind_is_quad(dm->gkind), BIE_EUNSUPPORTED,
               "sweeps and k-derivatives: triangular meshes only");
@@ -633,89 +596,97 @@ void sweep_device_impl(bie_dmesh* dm, const double* d_k, int nk, const double* d
   BIE_REQUIRE(((flags & BIE_F) == 0 || dF) && ((flags & BIE_G) == 0 || dG) && dC, BIE_EINVAL,
               "output pointer is NULL");
   BIE_REQUIRE(stride >= M * dm->N, BIE_EINVAL, "stride smaller than M * N");
+  double target_radius = -1.0;
   if (d_targets == nullptr) {
     d_targets = dm->d_sources;
     BIE_REQUIRE(M == dm->N, BIE_EINVAL, "collocation (NULL targets) needs n_targets == n_sources");
+    target_radius = dm->source_radius;
   }
   BIE_HIP_CHECK(hipSetDevice(dm->device));
   ensure_rules(dm, n, m, s);
-  const int KB = sweep_kb(dm->pk);
   BIE_REQUIRE(sizeof(double) * (size_t)dm->rs.R * dm->rs.Qmax * dm->pk <= 24 * 1024,
               BIE_EUNSUPPORTED, "sweep supports quadrature orders up to n*m' = 36");
-  const int fit = fitting_slots(sweep_fixed_doubles(dm->rs.R * dm->rs.Qmax * dm->pk), KB);
-  const int S = dm->sweep_slots ? std::min(dm->sweep_slots, fit) : fit;
-  const int min_seg = dm->sweep_elems_per_tile
-                          ? (int)std::max<int64_t>(1, (dm->E + dm->sweep_elems_per_tile - 1) /
-                                                          dm->sweep_elems_per_tile)
-                          : 1;
-  const bie_dmesh::Sched& sc = ensure_schedule(dm, 1, S, min_seg, s);
-  if (!dm->d_mid_count) dm->d_mid_count = dalloc<unsigned>(1);
-  if (uses_mid_rules(dm->gk, dm->pk)) ensure_mid_queue(dm, std::max<int64_t>(1, M * dm->E));
-  const int KBk = sweep_block_size(dm->pk, (flags & BIE_G) != 0);
-  const int nkb = (nk + KBk - 1) / KBk;
-  if (dm->block_uniform_cap < std::max(nkb, 1)) {
-    dfree(dm->d_block_uniform);
-    dm->d_block_uniform = nullptr;
-    dm->block_uniform_cap = 0;
-    dm->d_block_uniform = dalloc<int>((size_t)std::max(nkb, 1));
-    dm->block_uniform_cap = std::max(nkb, 1);
-  }
-  if (prepare_only) return;
-  order_after_previous(dm, s);
-  launch_fill_zero(dC, 2 * M, s);
-  launch_fill_zero_u32(dm->d_mid_count, s);
-  for (int which = 0; which < 2; ++which) {
-    double* X = which == 0 ? dF : dG;
-    const bool on = (flags & (which == 0 ? BIE_F : BIE_G)) != 0;
-    if (on)
-      launch_zero_columns_multi(X, stride, nk, M, sc.d_zero_cols, sc.zero_cols, s);
-    else if (X)
-      for (int q = 0; q < nk; ++q) launch_fill_zero(X + 2 * (size_t)q * stride, 2 * M * dm->N, s);
-  }
-  if (M == 0 || dm->E == 0 || nk == 0) {
-    mark_done(dm, s);
-    return;
-  }
-  refresh_geometry(dm, s);
-  if (!taylor) launch_block_uniform(d_k, nk, KBk, dm->d_block_uniform, s);
+  const int cus = device_cus(dm->device);
+  const StreamPlan plan = sweep_plan(dm->rs, flat_elements(dm), dm->sweep_slots);
+  const int64_t min_seg =
+      dm->sweep_elems_per_tile
+          ? std::max<int64_t>(1, (dm->E + dm->sweep_elems_per_tile - 1) / dm->sweep_elems_per_tile)
+          : 0;
+  const bie_dmesh::Stream& sc = ensure_sweep_stream(dm, plan.S, min_seg, cus, s);
+  // the wavenumbers of a sweep are on the device: its tiles decide there
+  const bool fast = taylor && fast_trig_ok(dm, k_re, target_radius);
   const int64_t rowblocks = (M + 63) / 64;
+  const int KB = sweep_block_size(dm->pk, (flags & BIE_G) != 0);
+  ensure_lists(lists, plan.mids, M, dm->E, sc.segments,
+               fast ? 0 : (int64_t)((nk + KB - 1) / KB) * rowblocks * sc.segments);
   AssemblyArgs a = make_args(dm, d_targets, M, 0.0, 0.0, flags, dF, dG, dC);
-  SlotArgs sa = slot_args(dm, sc, rowblocks);
-  SweepArgs sw{};
-  sw.k = taylor ? nullptr : d_k;
-  sw.nk = nk;
-  sw.block_uniform = taylor ? nullptr : dm->d_block_uniform;
-  sw.stride = stride;
-  sw.n_tiles = (int64_t)nkb * sc.segments * rowblocks;
-  sw.taylor = taylor ? 1 : 0;
-  sw.k_re = k_re;
-  sw.k_im = k_im;
-  launch_sweep(a, sa, sw, s);
-  mark_done(dm, s);
+  const bool any = M > 0 && dm->E > 0 && nk > 0;
+  if (!prepare_only) {
+    order_after_previous(dm, s);
+    launch_stream_prep(stream_prep(dm, a, sc, lists, nk, stride), s);
+  }
+  if (any) {
+    SweepArgs sw{};
+    sw.k = taylor ? nullptr : d_k;
+    sw.nk = nk;
+    sw.stride = stride;
+    sw.taylor = taylor ? 1 : 0;
+    sw.k_re = k_re;
+    sw.k_im = k_im;
+    launch_sweep(stream_inst(dm, a, sc, lists, rowblocks), sw, plan, dm->d_stab, lists.counters,
+                 lists.slow, cus, fast, prepare_only, s);
+  }
+  if (!prepare_only) mark_done(dm, s);
 }
-
 
 // ---- uneven batch -------------------------------------------------------------------
 
+// Elements per segment of a batch whose schedule was not configured, from the single-mesh
+// estimate (choose_stream_segments): all tiles share the CUs, longest first, so the time is
+// their mean load or the longest tile, and the last tiles to end are half a small one late.
+int64_t fitted_elems_per_tile(const std::vector<bie_dmesh*>& meshes, int Q, int NP, int cus) {
+  const double pair = 100.0 * Q + 80.0 * NP, begin = 6000.0, border = NP >= 6 ? 3.4 : 1.5;
+  int64_t largest = 1, best = 1;
+  for (const bie_dmesh* dm : meshes) largest = std::max(largest, dm->E);
+  double best_cost = 1e300;
+  for (double t = 16.0; t < 2.0 * largest; t *= 1.25) {
+    const int64_t T = std::min<int64_t>((int64_t)t, largest);
+    double sum = 0.0, longest = 0.0, least = 1e300;
+    for (const bie_dmesh* dm : meshes) {
+      if (dm->N == 0 || dm->E == 0) continue;
+      const double rb = (double)((dm->N + 63) / 64), p = (double)((dm->E + T - 1) / T);
+      const double tile = (double)dm->E / p * pair + begin;
+      sum += rb * (p * tile + 200.0 * border * std::sqrt((double)dm->E * p));
+      longest = std::max(longest, tile);
+      least = std::min(least, tile);
+    }
+    const double cost = std::max(sum / cus + 0.5 * least, longest);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = T;
+    }
+  }
+  return best;
+}
+
 // Tile list of the batch for its current configuration: every (instance, row block,
-// segment), costed by the segment's step count, ordered longest-first (order 0; ties in
+// segment), costed by the segment's elements, ordered longest-first (order 0; ties in
 // instance, segment, row block order) or interleaved across instances (order 1).
-void batch_configure(bie_batch* b, hipStream_t s) {
-  const int key = b->elems_per_tile * 1000 + b->slots * 10 + b->order;
+void batch_configure(bie_batch* b, const StreamPlan& pl, int cus, hipStream_t s) {
   bie_dmesh* d0 = b->meshes[0];
-  // slots = 32 or 64 asks for that many, capped at what fits beside the tables and staging
-  const int fit = fitting_slots(
-      phi_pad(d0->rs.R * d0->rs.Qmax * d0->pk) + kTrigDoubles + stage_doubles(d0->rs.len[0]), 1);
-  const int S = b->slots ? std::min(b->slots, fit) : fit;
+  const int64_t per_tile =
+      b->fitted ? fitted_elems_per_tile(b->meshes, d0->rs.len[0], b->pk, cus) : b->elems_per_tile;
+  const int64_t key = per_tile * 2 + b->order;
+  const int S = pl.S;
   bool current = b->configured_key == key && b->d_tiles != nullptr && b->slots_used == S;
   // a mesh's batch schedule may have been rebuilt by another batch that shares it
   for (size_t ii = 0; current && ii < b->meshes.size(); ++ii) {
-    const bie_dmesh::Sched& sc = b->meshes[ii]->sched[2];
-    current = sc.d_step_elems != nullptr && sc.S == S && sc.key == b->min_segments[ii];
+    const bie_dmesh::Stream& sc = b->meshes[ii]->bstream;
+    current = sc.d_order != nullptr && sc.S == S && sc.key == b->min_segments[ii];
   }
   if (current) return;
   struct Tile {
-    int steps, inst, rb, seg;
+    int elems, inst, rb, seg;
     int64_t rank;
   };
   std::vector<Tile> tiles;
@@ -727,20 +698,20 @@ void batch_configure(bie_batch* b, hipStream_t s) {
     bie_dmesh* dm = b->meshes[ii];
     const int64_t rbs = (dm->N + 63) / 64;
     b->rowblocks[ii] = rbs;
-    const int min_seg = (int)std::max<int64_t>(1, (dm->E + b->elems_per_tile - 1) / b->elems_per_tile);
+    const int64_t min_seg = std::max<int64_t>(1, (dm->E + per_tile - 1) / per_tile);
     b->min_segments[ii] = min_seg;
-    const bie_dmesh::Sched& sc = ensure_schedule(dm, 2, S, min_seg, s);
-    if (dm->N == 0) continue;
+    const bie_dmesh::Stream& sc = ensure_batch_stream(dm, S, min_seg, s);
+    if (dm->N == 0 || dm->E == 0) continue;
     int64_t rank = 0;
     for (int g = 0; g < sc.segments; ++g) {
-      const int steps = sc.h_seg_step_begin[g + 1] - sc.h_seg_step_begin[g];
-      for (int64_t rb = 0; rb < rbs; ++rb) tiles.push_back(Tile{steps, ii, (int)rb, g, rank++});
+      const int elems = sc.h_seg_begin[g + 1] - sc.h_seg_begin[g];
+      for (int64_t rb = 0; rb < rbs; ++rb) tiles.push_back(Tile{elems, ii, (int)rb, g, rank++});
     }
   }
   BIE_REQUIRE(tiles.size() < (size_t)INT32_MAX, BIE_EINVAL, "batch has too many tiles");
   if (b->order == 0)
     std::stable_sort(tiles.begin(), tiles.end(),
-                     [](const Tile& x, const Tile& y) { return x.steps > y.steps; });
+                     [](const Tile& x, const Tile& y) { return x.elems > y.elems; });
   else
     std::stable_sort(tiles.begin(), tiles.end(),
                      [](const Tile& x, const Tile& y) { return x.rank < y.rank; });
@@ -749,8 +720,11 @@ void batch_configure(bie_batch* b, hipStream_t s) {
     h[t] = make_int4(tiles[t].inst, tiles[t].rb, tiles[t].seg, 0);
   if (b->d_tiles) (void)hipDeviceSynchronize();  // a previous launch may still read it
   dfree(b->d_tiles);
+  dfree(b->d_slow);
   b->d_tiles = nullptr;
+  b->d_slow = nullptr;
   b->n_tiles = 0;
+  b->d_slow = dalloc<int>(std::max<size_t>(h.size(), 1));
   b->d_tiles = upload_vec(h, s);
   BIE_HIP_CHECK(hipStreamSynchronize(s));
   b->n_tiles = (int)h.size();
@@ -785,14 +759,12 @@ void batch_validate(bie_batch* b, const double* k_re, const double* k_im, uint32
 
 // What the batch's kernels need besides the instance table.
 struct BatchPlan {
+  StreamPlan pl;
+  int cus = 1;
   bool cplx = false;
-  bool fast = true;  // every instance: real k with |k| r below the fast sincos bound
+  bool fast = true;  // every instance: |k| r below the fast sincos bound
   bool gon = true;
-  int64_t max_work = 1;
-  // compile-time rule length of the fast kernel instance (0: the generic instance)
-  int qc(int len0) const {
-    return fast && !cplx && (len0 == 4 || len0 == 6 || len0 == 16) ? len0 : 0;
-  }
+  int64_t max_cols = 1;  // columns to zero per output, at most
 };
 
 // Host half of a batched assembly (under the batch and mesh locks): every per-mesh cache,
@@ -801,57 +773,48 @@ struct BatchPlan {
 BatchPlan batch_fill(bie_batch* b, const double* k_re, const double* k_im, uint32_t flags,
                      double* const* dF, double* const* dG, double* const* dC, hipStream_t s) {
   const int n_inst = (int)b->meshes.size();
+  bie_dmesh* d0 = b->meshes[0];
+  const bool flat = flat_elements(d0);
   for (bie_dmesh* dm : b->meshes) {
     ensure_rules(dm, b->n, b->m, s);
-    if (!dm->geom_valid) refresh_geometry(dm, s);
-    if (uses_mid_rules(dm->gk, dm->pk))
-      ensure_mid_queue(dm, std::max<int64_t>(1, dm->N * dm->E));
-    else if (!dm->d_mid_count)
-      dm->d_mid_count = dalloc<unsigned>(1);
+    if (!flat && !dm->geom_valid) refresh_geometry(dm, s);
   }
-  batch_configure(b, s);
-  BIE_HIP_CHECK(hipEventSynchronize(b->staged));  // the previous upload has left h_inst
   BatchPlan plan;
   plan.gon = (flags & BIE_G) != 0;
+  plan.pl = stream_plan(d0->rs, flat, true, b->fitted ? 0 : b->slots);
+  plan.cus = device_cus(b->device);
+  batch_configure(b, plan.pl, plan.cus, s);
+  BIE_HIP_CHECK(hipEventSynchronize(b->staged));  // the previous upload has left h_inst
   for (int ii = 0; ii < n_inst; ++ii) {
     bie_dmesh* dm = b->meshes[ii];
     const double ki = k_im ? k_im[ii] : 0.0;
     plan.cplx = plan.cplx || ki != 0.0;
-    plan.fast = plan.fast && fast_trig_ok(dm, k_re[ii], ki, dm->source_radius);
-    const bie_dmesh::Sched& sc = dm->sched[2];
+    plan.fast = plan.fast && fast_trig_ok(dm, k_re[ii], dm->source_radius);
+    bie_dmesh::Stream& sc = dm->bstream;
+    ensure_lists(dm->blists, plan.pl.mids, dm->N, dm->E, sc.segments, 0);
     BatchInst& bi = b->h_inst[ii];
-    bi.a = make_args(dm, dm->d_sources, dm->N, k_re[ii], ki, flags, dF[ii], dG[ii], dC[ii]);
-    bi.sa = slot_args(dm, sc, b->rowblocks[ii]);
+    bi.s = stream_inst(
+        dm, make_args(dm, dm->d_sources, dm->N, k_re[ii], ki, flags, dF[ii], dG[ii], dC[ii]), sc,
+        dm->blists, b->rowblocks[ii]);
     bi.zero_cols = sc.d_zero_cols;
     bi.n_zero = sc.zero_cols;
     bi.pad = 0;
-    plan.max_work = std::max<int64_t>(plan.max_work, sc.zero_cols);  // columns to zero per output
+    plan.max_cols = std::max<int64_t>(plan.max_cols, sc.zero_cols);
     if ((!(flags & BIE_F) && dF[ii]) || (!(flags & BIE_G) && dG[ii]))
-      plan.max_work = std::max<int64_t>(plan.max_work, dm->N);
+      plan.max_cols = std::max<int64_t>(plan.max_cols, dm->N);
   }
   return plan;
 }
 
 // Device half: zero fills, the persistent assembly over the tile list, the mid-edge pairs.
 // Kernels only (no memset, no host synchronisation), so it can be captured.
-void batch_kernels(bie_batch* b, const BatchInst* d_inst, const int4* d_tiles,
+void batch_kernels(bie_batch* b, const BatchInst* d_inst, const int4* d_tiles, int* d_slow,
                    unsigned* d_counter, const BatchPlan& plan, hipStream_t s) {
-  const int n_inst = (int)b->meshes.size();
-  launch_batch_prep(d_inst, n_inst, plan.max_work, s);
-  if (b->n_tiles > 0) {
-    bie_dmesh* d0 = b->meshes[0];
-    const int nphi = d0->rs.R * d0->rs.Qmax * d0->pk;
-    int cus = 0;
-    BIE_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device));
-    const int nstage = stage_doubles(d0->rs.len[0]);
-    const int qc = plan.qc(d0->rs.len[0]);
-    const int per_cu =
-        batch_blocks_per_cu(b->pk, plan.cplx, plan.gon, qc, b->slots_used, nphi, nstage);
-    const int grid = (int)std::min<int64_t>((int64_t)std::max(cus, 1) * per_cu, b->n_tiles);
-    launch_assemble_batch(d_inst, d_tiles, b->n_tiles, d_counter, d0->d_phi, nphi, nstage,
-                          b->slots_used, b->pk, plan.cplx, plan.gon, qc, grid, s);
-  }
-  if (uses_mid_rules(b->gk, b->pk)) launch_assemble_mid_batch(d_inst, n_inst, plan.cplx, s);
+  const bie_dmesh* d0 = b->meshes[0];
+  launch_stream_batch(d_inst, (int)b->meshes.size(), plan.max_cols, d_tiles, b->n_tiles, plan.pl,
+                      b->pk, plan.cplx, plan.gon, plan.fast, d0->d_stab,
+                      stream_mid_offset(d0->rs, flat_elements(d0)), d_counter, d_slow, plan.cus,
+                      s);
 }
 
 void batch_assemble_impl(bie_batch* b, const double* k_re, const double* k_im, uint32_t flags,
@@ -867,7 +830,7 @@ void batch_assemble_impl(bie_batch* b, const double* k_re, const double* k_im, u
   BIE_HIP_CHECK(hipMemcpyAsync(b->d_inst, b->h_inst, sizeof(BatchInst) * n_inst,
                                hipMemcpyHostToDevice, s));
   BIE_HIP_CHECK(hipEventRecord(b->staged, s));
-  batch_kernels(b, b->d_inst, b->d_tiles, b->d_counter, plan, s);
+  batch_kernels(b, b->d_inst, b->d_tiles, b->d_slow, b->d_counter, plan, s);
   for (bie_dmesh* dm : b->meshes) mark_done(dm, s);
 }
 
@@ -953,6 +916,7 @@ void batch_destroy_impl(bie_batch* b) {
   if (b->h_inst) (void)hipHostFree(b->h_inst);
   dfree(b->d_inst);
   dfree(b->d_tiles);
+  dfree(b->d_slow);
   dfree(b->d_counter);
   delete b;
 }
@@ -1047,12 +1011,6 @@ int bie_dmesh_destroy(bie_dmesh* dm) {
     (void)hipEventSynchronize(dm->done);
     (void)hipEventDestroy(dm->done);
   }
-  if (dm->side) {
-    (void)hipStreamSynchronize(dm->side);
-    (void)hipStreamDestroy(dm->side);
-    (void)hipEventDestroy(dm->side_fork);
-    (void)hipEventDestroy(dm->side_join);
-  }
   dfree(dm->d_coords);
   dfree(dm->d_topo);
   dfree(dm->d_sources);
@@ -1061,15 +1019,13 @@ int bie_dmesh_destroy(bie_dmesh* dm) {
   dfree(dm->d_pts);
   dfree(dm->d_phi);
   dfree(dm->d_elem);
-  free_schedules(dm);
-  dfree(dm->d_block_uniform);
-  dfree(dm->d_mid_count);
-  dfree(dm->d_mid_queue);
-  dfree(dm->d_mid_keys);
-  dfree(dm->d_mid_vals);
-  dfree(dm->d_mid_entries);
-  dfree(dm->d_mid_off);
-  dfree(dm->d_mid_refs);
+  dfree(dm->d_stab);
+  free_stream(dm->stream);
+  free_stream(dm->bstream);
+  free_stream(dm->sstream);
+  free_lists(dm->lists);
+  free_lists(dm->blists);
+  free_lists(dm->slists);
   delete dm;
   return BIE_OK;
 }
@@ -1328,12 +1284,6 @@ int bie_assemble(const bie_mesh* mesh, double k_re, double k_im, const double* t
       copy_to_host(G, dG, fg * sizeof(double));
     }
     if (M) BIE_HIP_CHECK(hipMemcpy(C, dC, 16 * M, hipMemcpyDeviceToHost));
-    if (targets) {  // the M x E pair queue of explicit targets is not kept in the cache
-      std::lock_guard<std::mutex> lk(dm->mu);
-      dfree(dm->d_mid_queue);
-      dm->d_mid_queue = nullptr;
-      dm->mid_cap = 0;
-    }
   });
   dfree(dT);
   dfree(dF);
@@ -1856,7 +1806,7 @@ int bie_host_cache_info(int64_t* hits, int64_t* builds, int64_t* n_sources,
       *queue_entries = 0;
       if (c.dm) {
         std::lock_guard<std::mutex> dl(c.dm->mu);
-        *queue_entries = c.dm->d_mid_queue ? c.dm->mid_cap : 0;
+        *queue_entries = std::max(c.dm->lists.mid_cap, c.dm->slists.mid_cap);
       }
     }
   });
@@ -1910,11 +1860,14 @@ int bie_schedule_check(const bie_mesh* mesh, int32_t min_segments, int64_t* stat
                                           (int)mesh->n_sources, cent.data(), kSlotWaves,
                                           kSlotCount, min_segments);
     validate_slot_schedule(sc, ptopo.data(), np, (int)E, (int)mesh->n_sources);
-    // the schedule of two elements per wave and step as well
-    SlotSchedule sc2 = build_slot_schedule(ptopo.data(), np, (int)E,
-                                           (int)mesh->n_sources, cent.data(), 2 * kSlotWaves,
-                                           kSlotCount, min_segments);
-    validate_slot_schedule(sc2, ptopo.data(), np, (int)E, (int)mesh->n_sources);
+    // the schedules of the kernels as well: few slots and many
+    for (int S : {17, 34, kSlotCount}) {
+      if (S < 2 * np) continue;
+      const StreamSchedule st = build_stream_schedule(ptopo.data(), np, (int)E,
+                                                      (int)mesh->n_sources, cent.data(), S,
+                                                      min_segments);
+      validate_stream_schedule(st, ptopo.data(), np, (int)E, (int)mesh->n_sources);
+    }
     if (stats) {
       stats[0] = sc.n_segments;
       stats[1] = sc.n_steps;
@@ -2060,7 +2013,7 @@ int bie_assemble_sweep_device(bie_dmesh* dm, const double* d_k, int32_t nk,
     BIE_REQUIRE(dm != nullptr, BIE_EINVAL, "dmesh is NULL");
     std::lock_guard<std::mutex> lk(dm->mu);
     sweep_device_impl(dm, d_k, nk, d_targets, n_targets, n, m, flags, dF, dG, stride, dC,
-                      static_cast<hipStream_t>(stream), false);
+                      static_cast<hipStream_t>(stream), dm->slists, false);
   });
 }
 
@@ -2090,10 +2043,10 @@ int bie_sweep_tune(bie_dmesh* dm, const double* d_k, int32_t nk, const double* d
           dm->sweep_slots = cs;
           // builds the schedule and warms up, then one timed sweep
           sweep_device_impl(dm, d_k, nk, d_targets, n_targets, n, m, flags, dF, dG, stride, dC,
-                            s, false);
+                            s, dm->slists, false);
           BIE_HIP_CHECK(hipEventRecord(e0, s));
           sweep_device_impl(dm, d_k, nk, d_targets, n_targets, n, m, flags, dF, dG, stride, dC,
-                            s, false);
+                            s, dm->slists, false);
           BIE_HIP_CHECK(hipEventRecord(e1, s));
           BIE_HIP_CHECK(hipEventSynchronize(e1));
           float ms = 0.f;
@@ -2131,7 +2084,7 @@ int bie_assemble_taylor_device(bie_dmesh* dm, double k_re, double k_im, int32_t 
                 "n_orders must be in 0..64");
     std::lock_guard<std::mutex> lk(dm->mu);
     sweep_device_impl(dm, nullptr, n_orders, d_targets, n_targets, n, m, flags, dF, dG, stride,
-                      dC, static_cast<hipStream_t>(stream), false, true, k_re, k_im);
+                      dC, static_cast<hipStream_t>(stream), dm->slists, false, true, k_re, k_im);
   });
 }
 
@@ -2162,17 +2115,16 @@ int bie_sweep_graph_create(bie_dmesh* dm, const double* d_k, int32_t nk,
     BIE_HIP_CHECK(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
     std::unique_ptr<bie_graph> g(new bie_graph);
     g->device = dm->device;
+    StreamLists lists;  // the graph's own
     try {
       // build every cache and set kernel attributes outside the capture
       sweep_device_impl(dm, d_k, nk, d_targets, n_targets, n, m, flags, dF, dG, stride, dC, cs,
-                        true);
-      sweep_prepare_attributes(dm->pk, dm->rs.R * dm->rs.Qmax * dm->pk, false,
-                               (flags & BIE_G) != 0);
+                        lists, true);
       BIE_HIP_CHECK(hipStreamSynchronize(cs));
       BIE_HIP_CHECK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
       try {
         sweep_device_impl(dm, d_k, nk, d_targets, n_targets, n, m, flags, dF, dG, stride, dC,
-                          cs, false);
+                          cs, lists, false);
       } catch (...) {
         hipGraph_t dead = nullptr;
         (void)hipStreamEndCapture(cs, &dead);
@@ -2185,8 +2137,10 @@ int bie_sweep_graph_create(bie_dmesh* dm, const double* d_k, int32_t nk,
       (void)hipStreamDestroy(cs);
       if (g->exec) (void)hipGraphExecDestroy(g->exec);
       if (g->graph) (void)hipGraphDestroy(g->graph);
+      free_lists(lists);
       throw;
     }
+    g->owned = {lists.counters, lists.mid_queue, lists.mid_tiles, lists.slow};
     (void)hipStreamDestroy(cs);
     *out = g.release();
   });
@@ -2231,38 +2185,38 @@ int bie_batch_graph_create(bie_batch* b, const double* k_re, const double* k_im,
       // gets its own copies of the table, the tile list and the tile counter
       for (bie_dmesh* dm : b->meshes) order_after_previous(dm, cs);
       const BatchPlan plan = batch_fill(b, k_re, k_im, flags, dF, dG, dC, cs);
-      // quadratic instances queue their mid-edge pairs: into queues of the graph's own (a
-      // mesh's queue is released once its collocation pairs are recorded, and regrown by
-      // calls with more targets)
+      // quadratic instances list their mid-edge pairs: in lists of the graph's own (a mesh's
+      // are emptied by every batch call)
       for (int ii = 0; ii < n_inst; ++ii) {
         bie_dmesh* dm = b->meshes[ii];
-        if (!uses_mid_rules(dm->gk, dm->pk)) continue;
-        const int64_t cap = std::max<int64_t>(1, dm->N * dm->E);
-        int2* q = dalloc<int2>((size_t)cap);
-        g->owned.push_back(q);
-        unsigned* cnt = dalloc<unsigned>(1);
-        g->owned.push_back(cnt);
-        b->h_inst[ii].sa.mid_queue = q;
-        b->h_inst[ii].sa.mid_count = cnt;
-        b->h_inst[ii].sa.mid_cap = cap;
+        if (!plan.pl.mids) continue;
+        StreamInst& in = b->h_inst[ii].s;
+        in.mid_queue = dalloc<int2>((size_t)std::max<int64_t>(1, in.mid_cap));
+        g->owned.push_back(in.mid_queue);
+        in.mid_tiles = dalloc<int2>((size_t)std::max<int64_t>(1, dm->blists.mid_tiles_cap));
+        g->owned.push_back(in.mid_tiles);
+        in.mid_count = dalloc<unsigned>(kStreamCounters - kMidCount);
+        g->owned.push_back(in.mid_count);
       }
       BatchInst* g_inst = dalloc<BatchInst>(std::max(n_inst, 1));
       g->owned.push_back(g_inst);
       int4* g_tiles = dalloc<int4>(std::max(b->n_tiles, 1));
       g->owned.push_back(g_tiles);
-      unsigned* g_counter = dalloc<unsigned>(kXcds);
+      unsigned* g_counter = dalloc<unsigned>(kMidCount);
       g->owned.push_back(g_counter);
+      int* g_slow = dalloc<int>(std::max(b->n_tiles, 1));
+      g->owned.push_back(g_slow);
       BIE_HIP_CHECK(hipMemcpyAsync(g_inst, b->h_inst, sizeof(BatchInst) * n_inst,
                                    hipMemcpyHostToDevice, cs));
       if (b->n_tiles > 0)
         BIE_HIP_CHECK(hipMemcpyAsync(g_tiles, b->d_tiles, sizeof(int4) * b->n_tiles,
                                      hipMemcpyDeviceToDevice, cs));
       // one eager run sets the kernels' attributes (LDS sizes) outside the capture
-      batch_kernels(b, g_inst, g_tiles, g_counter, plan, cs);
+      batch_kernels(b, g_inst, g_tiles, g_slow, g_counter, plan, cs);
       BIE_HIP_CHECK(hipStreamSynchronize(cs));
       BIE_HIP_CHECK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
       try {
-        batch_kernels(b, g_inst, g_tiles, g_counter, plan, cs);
+        batch_kernels(b, g_inst, g_tiles, g_slow, g_counter, plan, cs);
       } catch (...) {
         hipGraph_t dead = nullptr;
         (void)hipStreamEndCapture(cs, &dead);
@@ -2329,7 +2283,7 @@ int bie_batch_create(bie_dmesh* const* meshes, int32_t n_inst, int32_t n, int32_
       BIE_HIP_CHECK(hipHostMalloc(&h, sizeof(BatchInst) * n_inst, hipHostMallocDefault));
       b->h_inst = static_cast<BatchInst*>(h);
       b->d_inst = dalloc<BatchInst>(n_inst);
-      b->d_counter = dalloc<unsigned>(kXcds);
+      b->d_counter = dalloc<unsigned>(kMidCount);
       BIE_HIP_CHECK(hipEventCreateWithFlags(&b->staged, hipEventDisableTiming));
       BIE_HIP_CHECK(hipEventRecord(b->staged, nullptr));
     } catch (...) {
@@ -2355,6 +2309,7 @@ int bie_batch_configure(bie_batch* b, int32_t elems_per_tile, int32_t slots, int
                 "slots must be 32, 64 or 0 (as many as fit)");
     BIE_REQUIRE(order == 0 || order == 1, BIE_EINVAL, "order must be 0 or 1");
     std::lock_guard<std::mutex> bl(b->mu);
+    b->fitted = false;
     b->elems_per_tile = elems_per_tile;
     b->slots = slots;
     b->order = order;
@@ -2411,6 +2366,7 @@ int bie_batch_tune(bie_batch* b, const double* k_re, const double* k_im, uint32_
       for (const Cand& c : cands) {
         {
           std::lock_guard<std::mutex> bl(b->mu);
+          b->fitted = false;
           b->elems_per_tile = c.T;
           b->slots = c.S;
           b->order = c.order;

@@ -106,96 +106,127 @@ struct AssemblyArgs {
   double* C;
 };
 
-// Device view of a slot schedule plus the mid-edge pair queue.
-constexpr int kSlotWaves = 8;   // waves per workgroup of the slot kernel
+constexpr int kSlotWaves = 8;   // elements per step of the schedule check
 constexpr int kSlotCount = 64;  // LDS slots of the schedule check (64 rows x 4 doubles each)
-constexpr int kMidLds = 512;    // per-workgroup LDS queue of mid-edge pairs
-constexpr int kXcds = 8;        // XCDs of an MI355X; workgroup b is dispatched to XCD b mod 8
-constexpr int kLdsBytes = 160 * 1024;  // LDS per CU (one slot-kernel workgroup per CU)
+constexpr int kLdsBytes = 160 * 1024;  // LDS per CU (one workgroup of the slot kernels)
 
 constexpr int kStageMaxQ = 16;  // vertex rules up to this length are staged in LDS per wave
-// Waves of the wide single-k slot kernel (three per SIMD, one workgroup per CU), an option
-// beside kSlotWaves for real k on rules of 4, 6 or 16 points.
-constexpr int kWideWaves = 12;
 
 // Table of (cos, sin)(j pi / 64), j < kTrigN, for the table-driven sincos of the slot
-// kernels.  It follows the basis table in the same device buffer (at phi_pad(nphi)
-// doubles) and in LDS.
+// kernels.
 constexpr int kTrigN = 128;
 constexpr int kTrigDoubles = 2 * kTrigN;
 
-// LDS layout of the slot kernels, in doubles: S slots of 4 x 64 accumulators, the basis
-// table (padded to 4 doubles), the trig table (kTrigDoubles), then the per-wave staging
-// (when Qc <= kStageMaxQ) of the element's three vertex rules' table rows (3 Qc points x
-// 8 doubles) and its selection nodes (kStageSel doubles), then the mid-edge queue.
-constexpr int kStageSel = 24;  // NP x 4 doubles of selection-node data, NP <= 6
-__host__ __device__ inline int phi_pad(int nphi) { return (nphi + 3) & ~3; }
-__host__ __device__ inline int stage_wave_doubles(int Qc) { return 3 * Qc * 8 + kStageSel; }
-// The sweep kernel's fixed LDS (doubles): basis and trig tables, no staging.
-__host__ __device__ inline int sweep_fixed_doubles(int nphi) {
-  return phi_pad(nphi) + kTrigDoubles;
-}
-__host__ __device__ inline int stage_doubles(int Qc, int waves = kSlotWaves) {
-  return Qc <= kStageMaxQ ? waves * stage_wave_doubles(Qc) : 0;
-}
-// Split form of the slot kernel: `split` waves share each element of a step, wave h taking
-// the rule points h Qc/split .. (h+1) Qc/split - 1; each stages the rows of its points of
-// the three vertex rules and the selection nodes.
-__host__ __device__ inline int split_stage_wave_doubles(int Qh) { return 3 * Qh * 8 + kStageSel; }
-__host__ __device__ inline int split_stage_doubles(int Qc, int split) {
-  return kSlotWaves * split * split_stage_wave_doubles(Qc / split);
-}
+// Stream kernel (stream.hip): dense assembly of one mesh or of a batch.
+constexpr int kExpN = 64;         // entries of its table 2^(j / 64)
+constexpr int kStreamMid = 2048;  // mid-edge pairs a tile may queue in LDS (4 bytes each)
+// Counters of a call: tiles drawn, slow tiles listed and drawn, then StreamInst::mid_count:
+// mid-edge pairs listed, tiles without room for theirs, end of the list.
+enum { kSlowCount = 1, kSlowNext = 2, kMidCount = 3, kMidEnd = 5, kStreamCounters = 6 };
+constexpr int kFlatDoubles = 24;  // record of a flat element
+// Waves of its workgroup (one per CU): four per SIMD with 128 VGPRs each; eight- and nine-node
+// physics keep 32 and 36 sums per lane and take two per SIMD.
+constexpr int stream_waves(int NP) { return NP >= 8 ? 8 : 16; }
 
-// LDS slots that fit beside `fixed_doubles` (padded basis table + staging) and the
-// mid-edge queue when each slot holds `per_slot` accumulators of 64 rows x 4 doubles.
-inline int fitting_slots(int fixed_doubles, int per_slot, long lds_bytes = kLdsBytes) {
-  const long fixed = (long)sizeof(double) * fixed_doubles + 8L * kMidLds + 16;
-  const long S = (lds_bytes - fixed) / (256L * (long)sizeof(double) * per_slot);
-  return (int)(S < 120 ? S : 120);
-}
-
-struct SlotArgs {
-  int W, S;
-  int n_segments;
-  int n_rowblocks;
-  int seg_major;
-  int64_t n_tiles;
-  int phi_in_lds;
-  const int* seg_step_begin;
-  const int* step_elems;
-  const int* step_slot;    // (step, wave, node) slot, schedule order
-  const double* step_sel;  // (step, wave, node) selection node xyz_, schedule order
-  const int* flush_begin;
-  const int* flush_node;
-  const int* flush_slot;
-  unsigned* mid_count;
-  int2* mid_queue;
-  int64_t mid_cap;
-  int push_mid;            // 1: queue mid-edge pairs; 0: they come from a cached sorted list
-  int occupancy;           // slot-kernel workgroups per CU the schedule's LDS size allows
-  int split;               // waves per element of a step (1, or 2 for the split kernel)
+struct StreamInst {
+  AssemblyArgs a;
+  const int* seg_begin;     // n_segments + 1
+  const int* order;         // element at each position
+  const int4* ent;          // E x NP schedule entries (StreamEntry), by position
+  const double* psel;       // E x NP x 3 selection nodes, by position
+  const double* flat;       // E x kFlatDoubles records of flat elements, by position
+  const double* coords;     // geometry nodes and topology (mid-edge pairs)
+  const int* topo;
+  unsigned* mid_count;      // mid-edge pairs listed, tiles without room, end of the list
+  int2* mid_queue;          // (row, element | (rule - 4) << 28)
+  int2* mid_tiles;          // (row block, segment) of tiles whose pairs are not listed
+  unsigned mid_cap;
+  int own_basis;            // the physics basis is the geometry basis
+  int mid_off;              // of the mid-edge points in the tables
+  int n_segments, n_rowblocks;
+  double center[3], reach;  // every element point is within reach of the centre
 };
 
-// One instance of an uneven batch (assemble.hip, k_assemble_batch): its assembly and
-// slot-schedule arguments, and the columns its shared-column atomics need zeroed.
+// Device lists of a call: tile counters, mid-edge pairs (quadratic physics) and the tiles they
+// have no room for, tiles left to the launch for large arguments.
+struct StreamLists {
+  unsigned* counters = nullptr;  // kStreamCounters
+  int2* mid_queue = nullptr;
+  int2* mid_tiles = nullptr;
+  int64_t mid_cap = 0, mid_tiles_cap = 0;
+  int* slow = nullptr;
+  int64_t slow_cap = 0;
+};
+
+struct StreamRun {
+  const double* tab;        // stream_tables
+  unsigned* counters;       // kStreamCounters
+  int* slow;                // tiles left to the second launch
+  int tab_doubles, S, row_doubles, mids;
+};
+
+struct StreamPlan {
+  bool flat = false, mids = false;
+  int waves = 16, S = 0, tab_doubles = 0, row_doubles = 0;
+  size_t shmem = 0;
+};
+
+struct StreamPrep {
+  int64_t M;
+  int E, Pe, Pv, gk;        // Pv: points of the vertex rules
+  unsigned flags;
+  double *F, *G, *C;
+  const int* zero_cols;     // columns of enabled outputs to zero
+  int n_zero, n_whole;      // n_whole: columns of disabled outputs to zero (N or 0)
+  int nk;                   // matrices of F and G, `stride` complex entries apart
+  int64_t stride;
+  int col_blocks;
+  unsigned* counters;       // kStreamCounters
+  unsigned mid_cap;
+  const double *coords, *sources, *pts;
+  const int *topo, *ptopo, *order;
+  double* flat;             // records to write, or NULL
+  double* elem;             // element tables to write, or NULL
+};
+
+std::vector<double> stream_tables(const RuleSet& rs, bool flat);
+int stream_tab_doubles(const RuleSet& rs, bool flat);
+int stream_mid_offset(const RuleSet& rs, bool flat);
+// slots: at most so many LDS slots (0: as many as fit)
+StreamPlan stream_plan(const RuleSet& rs, bool flat, bool gon, int slots = 0);
+void launch_stream_prep(const StreamPrep& p, hipStream_t s);
+void launch_stream(const StreamInst& in, const StreamPlan& pl, const double* d_tab,
+                   unsigned* d_counters, int* d_slow, int cus, bool fast, hipStream_t s);
+
+// One instance of an uneven batch: its assembly and schedule, and the columns to zero.
 struct BatchInst {
-  AssemblyArgs a;
-  SlotArgs sa;
+  StreamInst s;
   const int* zero_cols;
   int n_zero;
   int pad;
 };
+void launch_stream_flat(const StreamPrep& p, hipStream_t s);
+// n_tiles tiles (instance, row block, segment); d_counters: kMidCount of them
+void launch_stream_batch(const BatchInst* d_inst, int n_inst, int64_t max_cols,
+                         const int4* d_tiles, int n_tiles, const StreamPlan& pl, int NP,
+                         bool cplx, bool gon, bool fast, const double* d_tab, int mid_off,
+                         unsigned* d_counters, int* d_slow, int cus, hipStream_t s);
 
-// Batched frequency sweep (sweep.hip).
+// Batched frequency sweep and k-derivatives (sweep.hip).
 struct SweepArgs {
   const double* k;           // nk real wavenumbers (device)
-  int nk;
-  const int* block_uniform;  // per k block: 1 when its k are uniformly spaced
   int64_t stride;            // complex elements between consecutive F_k (and G_k)
-  int64_t n_tiles;           // k blocks x segments x row blocks
-  int taylor;                // 1: the nk matrices are d^q/dk^q, q = 0..nk-1, at k_re + i k_im
   double k_re, k_im;
+  int nk;
+  int taylor;                // 1: the nk matrices are d^q/dk^q, q = 0..nk-1, at k_re + i k_im
 };
+int sweep_block_size(int NP, bool gon);  // matrices per block of the kernel
+// slots: at most so many LDS slots (0: as many as fit)
+StreamPlan sweep_plan(const RuleSet& rs, bool flat, int slots);
+// prepare_only: sets the kernels' attributes, launches nothing
+void launch_sweep(const StreamInst& in, const SweepArgs& sw, const StreamPlan& pl,
+                  const double* d_tab, unsigned* d_counters, int* d_slow, int cus, bool fast,
+                  bool prepare_only, hipStream_t s);
 
 // Vector-Jacobian product of the assembly (adjoint.hip).
 struct AdjointArgs {
@@ -303,29 +334,6 @@ void launch_geometry(const double* coords, const int* topo, int gk, int E,
 void launch_gather_selnodes(const double* sources, const int* ptopo, int NP, int E,
                             double* selnodes, hipStream_t s);
 void launch_assemble(const AssemblyArgs& a, hipStream_t s);
-// fast: every |k| r of the launch is below kTabFastMaxArg (kernels_math.hpp), so real-k
-// launches may use the branch-free sincos
-void launch_assemble_slots(const AssemblyArgs& a, const SlotArgs& sa, bool fast, hipStream_t s);
-void launch_assemble_mid(const AssemblyArgs& a, const SlotArgs& sa, hipStream_t s);
-void launch_zero_columns(double* X, int64_t M, const int* cols, int ncols, hipStream_t s);
-void launch_batch_prep(const BatchInst* d_inst, int n_inst, int64_t max_cols, hipStream_t s);
-size_t batch_shmem(int S, int nphi, int nstage);
-void launch_assemble_batch(const BatchInst* d_inst, const int4* d_tiles, int n_tiles,
-                           unsigned* d_counter, const double* d_phi, int nphi, int nstage,
-                           int S, int NP, bool cplx, bool gon, int qc, int grid,
-                           hipStream_t s);
-void launch_assemble_mid_batch(const BatchInst* d_inst, int n_inst, bool cplx, hipStream_t s);
-void launch_mid_recorded(const AssemblyArgs& a, const unsigned long long* keys, int64_t n_pairs,
-                         double* vals, const unsigned long long* entries, const int* off,
-                         const int* refs, int64_t n_entries, hipStream_t s);
-// The two halves of launch_mid_recorded: the pairs' values (reads the element tables, adds
-// C), then their addition into F and G (after the slot kernel's column writes).
-void launch_mid_compute(const AssemblyArgs& a, const unsigned long long* keys, int64_t n_pairs,
-                        double* vals, hipStream_t s);
-void launch_mid_scatter(const AssemblyArgs& a, int64_t n_pairs, const double* vals,
-                        const unsigned long long* entries, const int* off, const int* refs,
-                        int64_t n_entries, hipStream_t s);
-int batch_blocks_per_cu(int NP, bool cplx, bool gon, int qc, int S, int nphi, int nstage);
 void zgemv_batched_device(int64_t M, int64_t K, const double* dA, int64_t strideA, int64_t lda,
                           const double* dX, int64_t ldx, double* dY, int64_t ldy,
                           const int32_t* d_idx, int32_t n_idx, hipStream_t s);
@@ -343,15 +351,6 @@ constexpr int64_t kApplyScratchComplex = int64_t(1) << 20;
 void zgemm_device_noalloc(int64_t M, int64_t nrhs, int64_t K, const double* dA, int64_t lda,
                           const double* dX, int64_t ldx, double* dY, int64_t ldy,
                           hipStream_t s);
-void launch_zero_columns_multi(double* X, int64_t stride, int nk, int64_t M, const int* cols,
-                               int ncols, hipStream_t s);
-int sweep_kb(int NP);  // slot groups (wavenumbers) per k block of the sweep kernel
-// k (or derivative-order) matrices per block: twice sweep_kb without G
-int sweep_block_size(int NP, bool gon);
-void launch_sweep(const AssemblyArgs& a, const SlotArgs& sa, const SweepArgs& sw,
-                  hipStream_t s);
-void sweep_prepare_attributes(int NP, int nphi, bool taylor, bool gon);
-void launch_block_uniform(const double* k, int nk, int KB, int* out, hipStream_t s);
 void launch_adjoint(const AdjointArgs& a, int gk, int pk, bool cplx, hipStream_t s);
 // tiles: (instance, 256-row block, chunk of ech elements)
 void launch_dfdk_batch(const DfdkInst* d_inst, const int4* d_tiles, int n_tiles, int ech, int NP,
@@ -399,48 +398,32 @@ struct bie_dmesh {
   // host copies for scheduling
   std::vector<double> h_coords, h_sources;
   std::vector<int> h_topo, h_ptopo;
-  // slot schedules (mesh-only): [0] single-k kernel, [1] sweep kernel, [2] batch kernel
-  struct Sched {
-    int S = -1, key = -1, wv = 0;  // wv: elements per step
-    int segments = 0, zero_cols = 0, max_live = 0;
-    int* d_seg_step_begin = nullptr;
-    int* d_step_elems = nullptr;
-    int* d_step_slot = nullptr;
-    double* d_step_sel = nullptr;
-    int* d_flush_begin = nullptr;
-    int* d_flush_node = nullptr;
-    int* d_flush_slot = nullptr;
+  // stream schedule of the dense kernel (stream.hip) and what goes with it
+  struct Stream {
+    int S = -1;                  // slots it was built for
+    int64_t key = -1;            // and what the segments were chosen for
+    int segments = 0, zero_cols = 0;
+    int* d_seg_begin = nullptr;
+    int* d_order = nullptr;
+    int4* d_ent = nullptr;
+    double* d_psel = nullptr;    // selection nodes by position
+    double* d_flat = nullptr;    // records of flat elements by position
     int* d_zero_cols = nullptr;
-    std::vector<int> h_seg_step_begin;  // host copy (tile costs of the batch kernel)
-  } sched[3];
-  int* d_block_uniform = nullptr;
-  int block_uniform_cap = 0;
+    std::vector<int> h_seg_begin;  // (batch) host copy, for the tile list
+  };
+  // of single-mesh calls, of batches, of sweeps and k-derivatives
+  Stream stream, bstream, sstream;
+  bie::StreamLists lists, blists, slists;
+  double* d_stab = nullptr;      // its tables for the cached rule set (stream_tables)
   // tile shape of the frequency sweep (bie_sweep_tune): elements per tile (0: one segment per
   // row block) and LDS slots (0: as many as fit)
   int sweep_elems_per_tile = 0;
   int sweep_slots = 0;
-  // mid-edge pair queue
-  unsigned* d_mid_count = nullptr;
-  int2* d_mid_queue = nullptr;
-  int64_t mid_cap = 0;
-  // mid-edge pairs of collocation (targets = sources): they depend on the geometry only,
-  // so the first collocation assembly records them, sorted by (element, target), with the
-  // distinct (column, row) entries they add to (CSR over pair * 6 + node)
-  unsigned long long* d_mid_keys = nullptr;
-  int64_t n_mid_keys = -1;  // -1: not recorded yet
-  double* d_mid_vals = nullptr;  // 24 per pair
-  unsigned long long* d_mid_entries = nullptr;
-  int* d_mid_off = nullptr;
-  int* d_mid_refs = nullptr;
-  int64_t n_mid_entries = 0;
   // calls on the handle share the scratch above: each call's work waits for the previous
   // call's (recorded in `done` on `done_stream`) when it runs on another stream
   hipEvent_t done = nullptr;
   hipStream_t done_stream = nullptr;
   bool done_valid = false;
-  // side stream of the recorded mid-edge pairs' values, computed while the slot kernel runs
-  hipStream_t side = nullptr;
-  hipEvent_t side_fork = nullptr, side_join = nullptr;
   std::mutex mu;
 };
 
@@ -453,19 +436,21 @@ struct bie_batch {
   double beta = 0.0;
   std::vector<bie_dmesh*> meshes;
   // schedule configuration (chosen by bie_batch_tune)
-  int elems_per_tile = 64;   // target elements per segment
+  bool fitted = true;        // segments chosen from the batch's work (not configured)
+  int elems_per_tile = 64;   // else: target elements per segment
   int slots = 64;            // LDS slots per workgroup (0: as many as fit)
   int slots_used = 64;       // the slot count the tile list was built with
   int order = 0;             // 0: longest tiles first, 1: instances interleaved
-  int configured_key = -1;   // configuration the tile list was built for
+  int64_t configured_key = -1;  // configuration the tile list was built for
   // device state
   bie::BatchInst* d_inst = nullptr;
   bie::BatchInst* h_inst = nullptr;  // pinned staging for the per-call table
   hipEvent_t staged = nullptr;       // the last upload of h_inst has completed
   int4* d_tiles = nullptr;
   int n_tiles = 0;
+  int* d_slow = nullptr;             // tiles left to the launch for large arguments
   unsigned* d_counter = nullptr;
   std::vector<int64_t> rowblocks;
-  std::vector<int> min_segments;     // per instance: the schedule the tile list indexes
+  std::vector<int64_t> min_segments; // per instance: the schedule the tile list indexes
   std::mutex mu;
 };

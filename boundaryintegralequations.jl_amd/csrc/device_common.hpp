@@ -35,7 +35,7 @@ typedef double d2v __attribute__((ext_vector_type(2)));
 
 // Julia Base n-ary hypot for Float64 (maxabs * sqrt(sum((x_i/maxabs)^2)), left to
 // right), with no fused multiply-add so that the result is bit-identical to the CPU.
-__device__ __noinline__ double julia_hypot3(double x, double y, double z) {
+__device__ __forceinline__ double julia_hypot3_inline(double x, double y, double z) {
 #pragma clang fp contract(off)
   const double ax = fabs(x), ay = fabs(y), az = fabs(z);
   if (isinf(ax) || isinf(ay) || isinf(az)) return INFINITY;
@@ -50,12 +50,16 @@ __device__ __noinline__ double julia_hypot3(double x, double y, double z) {
   return mx * sqrt(s);
 }
 
+__device__ __noinline__ double julia_hypot3(double x, double y, double z) {
+  return julia_hypot3_inline(x, y, z);
+}
+
 // The n-ary hypot that later Julia releases use for IEEE floats: the arguments scaled by
 // 2^-E with E the exponent of maxabs (clamped to the normal range), squared and summed left
 // to right, square-rooted and scaled back by 2^E.  The scalings are exact, so away from overflow and underflow this is
 // sqrt((x^2 + y^2) + z^2) with every operation rounded once; no fused multiply-add, so the
 // result is bit-identical to the CPU.
-__device__ __noinline__ double scaled_hypot3(double x, double y, double z) {
+__device__ __forceinline__ double scaled_hypot3_inline(double x, double y, double z) {
 #pragma clang fp contract(off)
   const double ax = fabs(x), ay = fabs(y), az = fabs(z);
   if (isinf(ax) || isinf(ay) || isinf(az)) return INFINITY;
@@ -72,6 +76,10 @@ __device__ __noinline__ double scaled_hypot3(double x, double y, double z) {
   s = s + b * b;
   s = s + c * c;
   return scale * sqrt(s);
+}
+
+__device__ __noinline__ double scaled_hypot3(double x, double y, double z) {
+  return scaled_hypot3_inline(x, y, z);
 }
 
 // 1-based rule index of the node nearest to x (first strict minimum of the Julia hypot
@@ -165,43 +173,6 @@ __device__ __forceinline__ void stage_store(double* rows, int nchunk, double* se
   for (int t = 0; t < 3; ++t) {
     const int j = lane + 64 * t;
     if (j < nchunk) reinterpret_cast<double2*>(rows)[j] = v[t];
-  }
-  if (lane < nsel) reinterpret_cast<double2*>(sel_rows)[lane] = vs;
-}
-
-// Split-kernel staging: a wave takes the rows of points half*QH .. half*QH + QH - 1 of
-// each of the element's three vertex rules (Qc points each, 64 bytes per row): 12 QH chunks
-// of 16 bytes, chunk t from rule t / (4 QH), row chunk t % (4 QH), at the element's
-// table chunk rule * 4 Qc + half * 4 QH + t % (4 QH).  Bounds-checked buffer loads as in
-// stage_load (lanes past 12 QH read zeros), plus the nsel selection-node chunks.
-template <int QC, int QH, int NV>
-__device__ __forceinline__ void stage_load_half(const double* __restrict__ elem_e, int half,
-                                                const double* __restrict__ sel, int nsel,
-                                                int lane, double2 (&v)[NV], double2& vs) {
-  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
-  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<double*>(elem_e), (short)0, 12 * QC * 16, 0x00020000);
-#pragma unroll
-  for (int u = 0; u < NV; ++u) {
-    const int t = lane + 64 * u;
-    const int c = t / (4 * QH);
-    const int src = c * 4 * QC + half * 4 * QH + (t - c * 4 * QH);
-    const int off = t < 12 * QH ? src * 16 : 12 * QC * 16;
-    v[u] = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
-  }
-  const __amdgpu_buffer_rsrc_t rsel = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<double*>(sel), (short)0, nsel * 16, 0x00020000);
-  vs = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(rsel, lane * 16, 0, 0));
-}
-
-template <int QH, int NV>
-__device__ __forceinline__ void stage_store_half(double* rows, double* sel_rows, int nsel,
-                                                 int lane, const double2 (&v)[NV],
-                                                 const double2& vs) {
-#pragma unroll
-  for (int u = 0; u < NV; ++u) {
-    const int t = lane + 64 * u;
-    if (t < 12 * QH) reinterpret_cast<double2*>(rows)[t] = v[u];
   }
   if (lane < nsel) reinterpret_cast<double2*>(sel_rows)[lane] = vs;
 }

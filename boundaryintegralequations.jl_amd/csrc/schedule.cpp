@@ -18,6 +18,7 @@
 // further until their front fits the slot budget.
 #include <algorithm>
 #include <cmath>
+#include <deque>
 #include <numeric>
 
 #include "schedule.hpp"
@@ -83,14 +84,14 @@ int front_width(const std::vector<int>& idx, const int* ptopo, int NP, int W,
 // Splits idx into `parts` segments of nearly equal size along longest axes (halves of
 // the part count at every level, so any count is reachable), then splits further any
 // segment whose front exceeds S slots.
-void split(std::vector<int> idx, int parts, const double* cent, const int* ptopo, int NP, int W,
-           int S, std::vector<int>& first, std::vector<int>& last, std::vector<int>& touched,
+template <class Fits>
+void split(std::vector<int> idx, int parts, const double* cent, const Fits& fits,
            std::vector<SegOrder>& out) {
   const int ax = longest_axis(idx, cent);
   sort_along(idx, cent, ax);
   if ((int)idx.size() < parts) parts = std::max(1, (int)idx.size());
   if (parts <= 1) {
-    if (idx.size() <= 1 || front_width(idx, ptopo, NP, W, first, last, touched) <= S) {
+    if (idx.size() <= 1 || fits(idx)) {
       out.push_back(SegOrder{std::move(idx)});
       return;
     }
@@ -99,8 +100,8 @@ void split(std::vector<int> idx, int parts, const double* cent, const int* ptopo
   const int pa = parts / 2, pb = parts - pa;
   const size_t h = idx.size() * (size_t)pa / (size_t)parts;
   std::vector<int> a(idx.begin(), idx.begin() + h), b(idx.begin() + h, idx.end());
-  split(std::move(a), pa, cent, ptopo, NP, W, S, first, last, touched, out);
-  split(std::move(b), pb, cent, ptopo, NP, W, S, first, last, touched, out);
+  split(std::move(a), pa, cent, fits, out);
+  split(std::move(b), pb, cent, fits, out);
 }
 
 }  // namespace
@@ -116,8 +117,10 @@ SlotSchedule build_slot_schedule(const int* ptopo, int NP, int E, int N, const d
   if (E > 0) {
     std::vector<int> all(E);
     std::iota(all.begin(), all.end(), 0);
-    split(std::move(all), std::max(1, min_segments), cent, ptopo, NP, W, S, first, last, touched,
-          segs);
+    auto fits = [&](const std::vector<int>& idx) {
+      return front_width(idx, ptopo, NP, W, first, last, touched) <= S;
+    };
+    split(std::move(all), std::max(1, min_segments), cent, fits, segs);
   }
   sc.n_segments = (int)segs.size();
   // how many segments touch each node
@@ -268,6 +271,165 @@ void validate_slot_schedule(const SlotSchedule& sc, const int* ptopo, int NP, in
     const bool shared = (sc.flush_slot[f] & kSharedBit) != 0;
     if (shared != (nseg[sc.flush_node[f]] > 1)) fail("shared flag wrong");
   }
+}
+
+namespace {
+
+// Nodes of a segment in stream order: first and last position and number of contributions.
+struct StreamNodes {
+  std::vector<int> first, last, count, touched;
+  explicit StreamNodes(int N) : first(N, -1), last(N, -1), count(N, 0) {}
+  void sweep(const std::vector<int>& idx, const int* ptopo, int NP) {
+    for (int node : touched) first[node] = -1, count[node] = 0;
+    touched.clear();
+    for (size_t t = 0; t < idx.size(); ++t)
+      for (int s = 0; s < NP; ++s) {
+        const int node = ptopo[(size_t)idx[t] * NP + s];
+        if (first[node] < 0) {
+          first[node] = (int)t;
+          touched.push_back(node);
+        }
+        last[node] = (int)t;
+        ++count[node];
+      }
+  }
+  // the largest number of slots held at once: a node holds one from its first position to
+  // kStreamLag past its last; a node with a single contribution needs none
+  int front(size_t n) const {
+    std::vector<int> delta(n + kStreamLag + 2, 0);
+    for (int node : touched)
+      if (count[node] > 1) {
+        ++delta[first[node]];
+        --delta[last[node] + kStreamLag];
+      }
+    int live = 0, best = 0;
+    for (size_t t = 0; t < n; ++t) best = std::max(best, live += delta[t]);
+    return best;
+  }
+};
+
+}  // namespace
+
+StreamSchedule build_stream_schedule(const int* ptopo, int NP, int E, int N, const double* cent,
+                                     int S, int min_segments) {
+  StreamSchedule sc;
+  sc.S = S;
+  sc.NP = NP;
+  StreamNodes nd(N);
+  std::vector<SegOrder> segs;
+  if (E > 0) {
+    std::vector<int> all(E);
+    std::iota(all.begin(), all.end(), 0);
+    auto fits = [&](const std::vector<int>& idx) {
+      nd.sweep(idx, ptopo, NP);
+      return nd.front(idx.size()) <= S;
+    };
+    split(std::move(all), std::max(1, min_segments), cent, fits, segs);
+  }
+  sc.n_segments = (int)segs.size();
+  std::vector<int> nseg(N, 0), mark(N, -1);
+  for (int g = 0; g < sc.n_segments; ++g)
+    for (int e : segs[g].elems)
+      for (int s = 0; s < NP; ++s) {
+        const int node = ptopo[(size_t)e * NP + s];
+        if (mark[node] != g) {
+          mark[node] = g;
+          ++nseg[node];
+        }
+      }
+  for (int j = 0; j < N; ++j) {
+    if (nseg[j] != 1) sc.zero_cols.push_back(j);
+    sc.n_shared += nseg[j] > 1;
+  }
+  sc.order.reserve(E);
+  sc.ent.reserve((size_t)E * NP);
+  sc.seg_begin.push_back(0);
+  std::vector<int> slot(N, -1), turn_of(N, 0), turns(S);
+  for (const SegOrder& seg : segs) {
+    const std::vector<int>& el = seg.elems;
+    nd.sweep(el, ptopo, NP);
+    std::fill(turns.begin(), turns.end(), 0);
+    std::vector<std::vector<int>> release(el.size() + kStreamLag + 1);  // slots by position
+    // slots change hands in the order they were given back: the longest possible distance
+    // between a node's last contribution and its slot's next node
+    std::deque<int> freelist;
+    for (int q = 0; q < S; ++q) freelist.push_back(q);
+    for (size_t t = 0; t < el.size(); ++t) {
+      for (int q : release[t]) freelist.push_back(q);
+      for (int s = 0; s < NP; ++s) {
+        const int node = ptopo[(size_t)el[t] * NP + s];
+        if (nd.first[node] == (int)t && nd.count[node] > 1 && slot[node] < 0) {
+          if (freelist.empty()) throw Error{BIE_EINVAL, "stream schedule overflow"};
+          slot[node] = freelist.front();
+          freelist.pop_front();
+          turn_of[node] = turns[slot[node]]++;
+          release[nd.last[node] + kStreamLag].push_back(slot[node]);
+        }
+        sc.ent.push_back(StreamEntry{slot[node], nd.count[node], turn_of[node],
+                                     node | (nseg[node] > 1 ? kSharedBit : 0)});
+      }
+      sc.max_live = std::max(sc.max_live, S - (int)freelist.size());
+      sc.order.push_back(el[t]);
+    }
+    for (int node : nd.touched) slot[node] = -1, turn_of[node] = 0;
+    sc.seg_begin.push_back((int)sc.order.size());
+  }
+  return sc;
+}
+
+// Replays a stream schedule: every element once; a node keeps one slot within a segment,
+// its entries agree on count and turn; a slot changes hands only after all contributions of
+// the node before, at least kStreamLag positions later, with the turn counted up by one.
+void validate_stream_schedule(const StreamSchedule& sc, const int* ptopo, int NP, int E, int N) {
+  auto fail = [](const std::string& m) { throw Error{BIE_EINVAL, "stream schedule: " + m}; };
+  if ((int)sc.order.size() != E || sc.ent.size() != (size_t)E * NP) fail("sizes");
+  if ((int)sc.seg_begin.size() != sc.n_segments + 1 || sc.seg_begin[sc.n_segments] != E)
+    fail("segment bounds");
+  std::vector<int> seen(E, 0), nseg(N, 0), mark(N, -1);
+  struct Hold {
+    int node = -1, got = 0, count = 0, turn = -1, freed = 0;
+  };
+  for (int g = 0; g < sc.n_segments; ++g) {
+    std::vector<Hold> hold(sc.S);
+    for (int t = sc.seg_begin[g]; t < sc.seg_begin[g + 1]; ++t) {
+      const int e = sc.order[t];
+      if (e < 0 || e >= E || seen[e]++) fail("element swept twice or out of range");
+      for (int s = 0; s < NP; ++s) {
+        const StreamEntry& x = sc.ent[(size_t)t * NP + s];
+        const int node = ptopo[(size_t)e * NP + s];
+        if ((x.node & ~kSharedBit) != node) fail("entry of another node");
+        if (mark[node] != g) {
+          mark[node] = g;
+          ++nseg[node];
+        } else if (x.slot < 0) {
+          fail("direct node with several contributions");
+        }
+        if (x.slot < 0) {
+          if (x.count != 1) fail("direct node with several contributions");
+          continue;
+        }
+        if (x.slot >= sc.S || x.count < 2) fail("slot out of range");
+        Hold& h = hold[x.slot];
+        if (h.node != node) {
+          if (h.got != h.count) fail("slot handed on before its node is complete");
+          if (h.node >= 0 && t < h.freed) fail("slot handed on too early");
+          if (x.turn != h.turn + 1) fail("turn");
+          h = Hold{node, 0, x.count, x.turn, 0};
+        }
+        if (x.count != h.count || x.turn != h.turn) fail("entries of a node disagree");
+        if (++h.got > h.count) fail("more contributions than counted");
+        if (h.got == h.count) h.freed = t + kStreamLag;
+      }
+    }
+    for (const Hold& h : hold)
+      if (h.got != h.count) fail("node incomplete at the segment's end");
+  }
+  std::vector<char> zero(N, 0);
+  for (int j : sc.zero_cols) zero[j] = 1;
+  for (int j = 0; j < N; ++j)
+    if ((nseg[j] != 1) != (zero[j] != 0)) fail("zero_cols disagrees with segment counts");
+  for (const StreamEntry& x : sc.ent)
+    if (((x.node & kSharedBit) != 0) != (nseg[x.node & ~kSharedBit] > 1)) fail("shared flag");
 }
 
 }  // namespace bie

@@ -33,6 +33,30 @@ struct SlotSchedule {
 SlotSchedule build_slot_schedule(const int* ptopo, int NP, int E, int N, const double* cent,
                                  int W, int S, int min_segments);
 
+// Stream schedule of the barrier-free slot kernels (stream.hip): every segment is an ordered
+// list of elements that the waves of a workgroup take one at a time; a node's contributions
+// meet in an LDS slot, which the wave that brings the last one writes out.
+struct StreamEntry {  // one per (position, element node): an int4 on the device
+  int slot;           // LDS slot, or -1: the node's only element of the segment is this one
+  int count;          // contributions the node receives in the segment
+  int turn;           // how many nodes held the slot before (it must have been freed so often)
+  int node;           // column | kSharedBit when other segments add to it as well
+};
+struct StreamSchedule {
+  int S = 0, NP = 0, n_segments = 0, n_shared = 0, max_live = 0;
+  std::vector<int> seg_begin;      // n_segments + 1 positions
+  std::vector<int> order;          // element at each position
+  std::vector<StreamEntry> ent;    // E * NP, by position
+  std::vector<int> zero_cols;      // columns the kernel adds to, or does not touch at all
+};
+// A slot is handed to a new node kStreamLag positions after its last contribution at the
+// earliest (any positive distance is correct; a few positions keep the waves, which run
+// that far apart, from waiting for each other).
+constexpr int kStreamLag = 6;
+StreamSchedule build_stream_schedule(const int* ptopo, int NP, int E, int N, const double* cent,
+                                     int S, int min_segments);
+void validate_stream_schedule(const StreamSchedule& sc, const int* ptopo, int NP, int E, int N);
+
 void validate_slot_schedule(const SlotSchedule& sc, const int* ptopo, int NP, int E, int N);
 
 }  // namespace bie

@@ -1,574 +1,727 @@
 // Batched frequency sweep: dense F_k, G_k for a list of real wavenumbers k_0..k_{nk-1}
-// on one mesh, in one launch per kernel (graph-capturable: no host synchronisation, no
-// memset nodes).
+// on one mesh, and the k-derivatives of F and G at one wavenumber (taylor_assemble!,
+// src/3d/rosebem.jl:56-157), in one launch per kernel (graph-capturable: no host
+// synchronisation, no memset nodes).  The reference has no batched path: it calls
+// assemble_parallel! once per k.
 //
-// Each wave carries KB wavenumbers at once.  Everything that does not depend on k is
-// shared between them: rule selection (find_closest_corner,
-// src/3d/assembly_collocation.jl:102-115), the table loads, d = y - x, 1/r, n.d, the
-// C integrand (C is k-independent, kernels.jl:48-55, and is formed once by the first
-// k block).  For a block of uniformly spaced k, e^{i k_b r} = e^{i k_0 r} (e^{i dk r})^b
-// replaces KB sincos evaluations by two plus KB-1 complex products; other blocks evaluate
-// each e^{i k_b r} directly, so any list of k is exact.  Accumulation uses the LDS-slot
-// schedule of the single-k kernel with KB accumulators per slot (the schedule is built
-// for as many slots of KB accumulators as fit in LDS).  The reference has no batched path: it calls
-// assemble_parallel! once per k (e.g. the Taylor sweep of src/3d/rosebem.jl:56-157
-// shares geometry across derivative orders in the same way).
+// The kernel is the stream kernel (stream.hip) with KB matrices at once: tiles are (block of
+// KB wavenumbers or orders, segment, 64 rows), an LDS slot holds KB node sums of 64 rows.
+// What does not depend on the matrix is formed once per pair or point: rule selection, y - x,
+// 1/r, the C integrand (first block only).  Four matrices of F and G (eight of F alone, two
+// and four with six-node physics) are 96 registers of sums; eight waves per CU (two per SIMD,
+// 256 VGPRs) hold them (with twelve, 168 VGPRs, they spilled: 11.9 ms and 10.9 ms where eight
+// take 11.8 and 5.7 for 16 wavenumbers and 26 orders on 4002 nodes).  A slot of 8 KB leaves 17
+// of them, which the surface's segments have to fit (44 for 8000 elements).
+//   * Uniformly spaced k: e^{i k_b r} = e^{i k_0 r} (e^{i dk r})^b, two sincos per point and
+//     one complex product per further k; other blocks form each e^{i k_b r}.  The kernel
+//     finds out for every block, so any list of k is exact.
+//   * k-derivatives: G_m = (i r)^m G, F_m = (i k r - 1 + m) (n.d / r^2) G_m.  On a flat
+//     element n.d is a constant of the pair, and with A_j = sum N (i r)^j e^{ikr} J w / 4 pi r
+//     F_m = -(n.d) [k A_{m-1} + (m - 1) A_{m-2}], G_m = A_m:
+//     one sequence of sums (two products and six multiply-adds per point and order) gives
+//     both.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "bie_common.hpp"
-#include "device_common.hpp"
-#include "kernels_math.hpp"
-#include "schedule.hpp"
+#include "stream_device.hpp"
 
 namespace bie {
 namespace {
 
-// With TAB, e^{ikr} comes from the LDS trig table trig (sincos_tab), else from sincos_f64.
-template <int NP, int KB, bool TAB>
-__device__ __forceinline__ void sweep_point(double x0, double x1, double x2, const double4 A,
-                                            const double4 B, const double* __restrict__ p,
-                                            const double* kv, double dk, bool rec, bool doG,
-                                            double (&fr)[KB][NP], double (&fi)[KB][NP],
-                                            double (&gr)[KB][NP], double (&gi)[KB][NP],
-                                            double& csum, const double2* trig) {
-  const double dx = A.x - x0, dy = A.y - x1, dz = A.z - x2;
+constexpr int kSweepWaves = 8;
+
+// Matrices of a block.
+__host__ __device__ constexpr int sweep_block(int NP, bool gon) {
+  return (NP == 6 ? 2 : 4) * (gon ? 1 : 2);
+}
+constexpr int sweep_slot_doubles(int NP) { return sweep_block(NP, true) * 256; }
+
+typedef const __attribute__((address_space(4))) SweepArgs* SweepPtr;
+
+template <int NP, int KB, bool GON>
+struct Multi {  // an element's node sums of one row, KB matrices
+  double fr[KB][NP], fi[KB][NP], gr[GON ? KB : 1][GON ? NP : 1], gi[GON ? KB : 1][GON ? NP : 1];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int b = 0; b < KB; ++b)
+#pragma unroll
+      for (int s = 0; s < NP; ++s) {
+        fr[b][s] = fi[b][s] = 0.0;
+        if constexpr (GON) gr[b][s] = gi[b][s] = 0.0;
+      }
+  }
+  template <class Fn>
+  __device__ __forceinline__ void each(Fn fn) {
+#pragma unroll
+    for (int b = 0; b < KB; ++b)
+#pragma unroll
+      for (int s = 0; s < NP; ++s) {
+        fn(b, fr[b][s], fi[b][s]);
+        if constexpr (GON) fn(b, gr[b][s], gi[b][s]);
+      }
+  }
+};
+
+template <bool FIRST>
+__device__ __forceinline__ void plus(double& x, double v, double w) {
+  x = FIRST ? v * w : fma(v, w, x);
+}
+
+// x + iy times i^m.
+__device__ __forceinline__ void rotate(int m, double& x, double& y) {
+  if (m & 1) {
+    const double t = -y;
+    y = x;
+    x = t;
+  }
+  if (m & 2) {
+    x = -x;
+    y = -y;
+  }
+}
+
+// A block's wavenumbers.
+template <int KB>
+struct Block {
+  double k[KB], dk;
+};
+
+// One point of a flat element: K <= KB wavenumbers; the sums leave out J (of G) and n.d J (of
+// F).  H = G / r^2 runs through the wavenumbers.
+template <int KB, int K, bool GON, bool FAST, bool REC, bool FIRST>
+__device__ __forceinline__ void sweep_point_flat(const double (&d0)[3], const double (&a)[3],
+                                                 const double (&b)[3], double (&n)[4],
+                                                 const double* next, const Block<KB>& kv,
+                                                 const Trig& tr, Multi<3, KB, GON>& v,
+                                                 double& c3) {
+  const double m[4] = {n[0], n[1], n[2], n[3]};
+#pragma unroll
+  for (int s = 0; s < 4; ++s) n[s] = next[s];
+  __builtin_amdgcn_sched_barrier(0);
+  const double dx = fma(m[2], b[0], fma(m[1], a[0], d0[0]));
+  const double dy = fma(m[2], b[1], fma(m[1], a[1], d0[1]));
+  const double dz = fma(m[2], b[2], fma(m[1], a[2], d0[2]));
   const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
   const double rinv = rsqrt_nr(r2);
   const double r = r2 * rinv;
-  const double nd = fma(A.w, dx, fma(B.x, dy, B.y * dz));
-  const double g = B.z * rinv;          // J w / (4 pi r)
-  const double t = nd * rinv * rinv;     // (n.d) / r^2: f = t (ikr - 1) g e^{ikr}
-  csum -= t * g;
-  // the recurrence runs on g e^{ik_b r} (= G_b): one complex product per further k
-  double sn, cs, zs = 0.0, zc = 1.0;
-  if (TAB) {
-    sincos_tab(kv[0] * r, trig, &sn, &cs);
-    if (rec) sincos_tab(dk * r, trig, &zs, &zc);
-  } else {
-    sincos_f64(kv[0] * r, &sn, &cs);
-    if (rec) sincos_f64(dk * r, &zs, &zc);
+  Phase<false, FAST> e0, e1;
+  e0.begin(kv.k[0] * r, 0.0, tr);
+  if (REC) e1.begin(kv.dk * r, 0.0, tr);
+  const double h = (m[3] * rinv) * (rinv * rinv);
+  c3 = FIRST ? h : c3 + h;
+  double w[3];
+  if constexpr (GON) {
+#pragma unroll
+    for (int s = 0; s < 3; ++s) w[s] = m[s] * r2;
   }
-  double Gr = g * cs, Gi = g * sn;
-  double ps[NP];
+  double sn, cs, zs = 0.0, zc = 0.0, damp;
+  e0.end(tr, sn, cs, damp);
+  if (REC) e1.end(tr, zs, zc, damp);
+  double Hr = h * cs, Hi = h * sn;
 #pragma unroll
-  for (int s = 0; s < NP; ++s) ps[s] = p[s];
-#pragma unroll
-  for (int b = 0; b < KB; ++b) {
-    if (b > 0) {
-      if (rec) {
-        const double c2 = fma(Gr, zc, -Gi * zs);
-        Gi = fma(Gr, zs, Gi * zc);
-        Gr = c2;
+  for (int q = 0; q < K; ++q) {
+    if (q > 0) {
+      if (REC) {
+        const double c2 = fma(Hr, zc, -(Hi * zs));
+        Hi = fma(Hr, zs, Hi * zc);
+        Hr = c2;
       } else {
-        if (TAB)
-          sincos_tab(kv[b] * r, trig, &sn, &cs);
-        else
-          sincos_f64(kv[b] * r, &sn, &cs);
-        Gr = g * cs;
-        Gi = g * sn;
+        Phase<false, FAST> e;
+        e.begin(kv.k[q] * r, 0.0, tr);
+        e.end(tr, sn, cs, damp);
+        Hr = h * cs;
+        Hi = h * sn;
       }
     }
-    const double krr = kv[b] * r;
-    const double Fr = -t * fma(krr, Gi, Gr);
-    const double Fi = t * fma(krr, Gr, -Gi);
+    const double krr = kv.k[q] * r;
+    const double Fr = fma(-krr, Hi, -Hr), Fi = fma(krr, Hr, -Hi);
 #pragma unroll
-    for (int s = 0; s < NP; ++s) {
-      fr[b][s] = fma(Fr, ps[s], fr[b][s]);
-      fi[b][s] = fma(Fi, ps[s], fi[b][s]);
-    }
-    if (doG) {  // the same for every lane: F-only sweeps (gOn = false) skip this work
-#pragma unroll
-      for (int s = 0; s < NP; ++s) {
-        gr[b][s] = fma(Gr, ps[s], gr[b][s]);
-        gi[b][s] = fma(Gi, ps[s], gi[b][s]);
+    for (int s = 0; s < 3; ++s) {
+      plus<FIRST>(v.fr[q][s], Fr, m[s]);
+      plus<FIRST>(v.fi[q][s], Fi, m[s]);
+      if constexpr (GON) {
+        plus<FIRST>(v.gr[q][s], Hr, w[s]);
+        plus<FIRST>(v.gi[q][s], Hi, w[s]);
       }
     }
   }
 }
 
-// k-derivatives of orders m0 .. m0+KB-1 at one complex k = kr + i ki (taylor_greens3d!,
-// taylor_freens3d!, src/3d/kernels.jl:94-118, as taylor_assemble! integrates them,
-// src/3d/rosebem.jl:7-44):
-//   G_m = (i r)^m e^{ikr} J w / (4 pi r),   F_m = (i k r - 1 + m) (n.d / r^2) G_m,
-// so one e^{ikr} serves every order and each further order is one product by i r.
-template <int NP, int KB, bool TAB>
-__device__ __forceinline__ void taylor_point(double x0, double x1, double x2, const double4 A,
-                                             const double4 B, const double* __restrict__ p,
-                                             double kr, double ki, int m0, bool doG,
-                                             double (&fr)[KB][NP], double (&fi)[KB][NP],
-                                             double (&gr)[KB][NP], double (&gi)[KB][NP],
-                                             double& csum, const double2* trig) {
-  const double dx = A.x - x0, dy = A.y - x1, dz = A.z - x2;
+template <int KB, int K, bool GON, bool FAST, bool REC>
+__device__ __forceinline__ void sweep_pair_flat(const double (&d0)[3], const double (&a)[3],
+                                                const double (&b)[3], const double* tab, int Q,
+                                                const Block<KB>& kv, const Trig& tr,
+                                                Multi<3, KB, GON>& v, double& c3) {
+  double n[4] = {tab[0], tab[1], tab[2], tab[3]};
+  sweep_point_flat<KB, K, GON, FAST, REC, true>(d0, a, b, n, tab += 4, kv, tr, v, c3);
+#pragma unroll 1
+  for (int q = 1; q < Q; ++q)
+    sweep_point_flat<KB, K, GON, FAST, REC, false>(d0, a, b, n, tab += 4, kv, tr, v, c3);
+}
+
+// One point of a flat element for the derivative orders m0 .. m0 + K - 1 (m0 a multiple of
+// four): sums of N r^j e^{ikr} w / (4 pi r), j = m0 - 2 .., without the factors i^j.
+template <int NA, bool CPLX, bool FAST, bool FIRST>
+__device__ __forceinline__ void taylor_point_flat(const double (&d0)[3], const double (&a)[3],
+                                                  const double (&b)[3], double (&n)[4],
+                                                  const double* next, double kr, double ki,
+                                                  int m0, const Trig& tr, double (&ac)[NA][3],
+                                                  double (&as)[NA][3], double& c3) {
+  const double m[4] = {n[0], n[1], n[2], n[3]};
+#pragma unroll
+  for (int s = 0; s < 4; ++s) n[s] = next[s];
+  __builtin_amdgcn_sched_barrier(0);
+  const double dx = fma(m[2], b[0], fma(m[1], a[0], d0[0]));
+  const double dy = fma(m[2], b[1], fma(m[1], a[1], d0[1]));
+  const double dz = fma(m[2], b[2], fma(m[1], a[2], d0[2]));
   const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
   const double rinv = rsqrt_nr(r2);
   const double r = r2 * rinv;
-  const double nd = fma(A.w, dx, fma(B.x, dy, B.y * dz));
-  const double g = B.z * rinv;       // J w / (4 pi r)
-  const double t = nd * rinv * rinv;  // (n.d) / r^2
-  csum -= t * g;
-  double sn, cs;
-  if (TAB)
-    sincos_tab(kr * r, trig, &sn, &cs);
-  else
-    sincos_f64(kr * r, &sn, &cs);
-  double gm = g;
-  if (ki != 0.0) gm *= exp(-ki * r);
-  // r^m0 by binary powering (m0 is the same for the whole wave, m0 < 64)
-  double rb = r;
-  for (int e = m0; e != 0; e >>= 1) {
-    if (e & 1) gm *= rb;
-    rb *= rb;
-  }
-  double Gr = gm * cs, Gi = gm * sn;
-  if (m0 & 1) {  // times i^m0
-    const double t2 = -Gi;
-    Gi = Gr;
-    Gr = t2;
-  }
-  if (m0 & 2) {
-    Gr = -Gr;
-    Gi = -Gi;
-  }
-  const double krr = kr * r;
-  const double a0 = (double)(m0 - 1) - ki * r;  // Re(i k r - 1 + m0)
-  double ps[NP];
-#pragma unroll
-  for (int s = 0; s < NP; ++s) ps[s] = p[s];
-#pragma unroll
-  for (int b = 0; b < KB; ++b) {
-    if (b > 0) {  // G_{m+1} = i r G_m
-      const double t2 = -r * Gi;
-      Gi = r * Gr;
-      Gr = t2;
+  Phase<CPLX, FAST> e;
+  e.begin(kr * r, CPLX ? ki * r : 0.0, tr);
+  double q = m[3] * rinv;
+  if (m0 == 0) {
+    q *= rinv * rinv;
+    c3 = FIRST ? q : c3 + q;
+  } else {  // r^(m0 - 2): even, by binary powering
+    double p = r2;
+    for (int x = (m0 - 2) >> 1; x != 0; x >>= 1) {
+      if (x & 1) q *= p;
+      p *= p;
     }
-    const double am = a0 + (double)b;
-    const double Fr = t * fma(am, Gr, -krr * Gi);
-    const double Fi = t * fma(am, Gi, krr * Gr);
+  }
+  double sn, cs, damp;
+  e.end(tr, sn, cs, damp);
+  if (CPLX) q *= damp;
+  double C = q * cs, S = q * sn;
 #pragma unroll
-    for (int s = 0; s < NP; ++s) {
-      fr[b][s] = fma(Fr, ps[s], fr[b][s]);
-      fi[b][s] = fma(Fi, ps[s], fi[b][s]);
+  for (int j = 0; j < NA; ++j) {
+    if (j > 0) {
+      C *= r;
+      S *= r;
     }
-    if (doG) {  // the same for every lane: F-only stacks (gOn = false) skip this work
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      plus<FIRST>(ac[j][s], C, m[s]);
+      plus<FIRST>(as[j][s], S, m[s]);
+    }
+  }
+}
+
+template <int KB, int K, bool CPLX, bool GON, bool FAST>
+__device__ __forceinline__ void taylor_pair_flat(const double (&d0)[3], const double (&a)[3],
+                                                 const double (&b)[3], const double* tab, int Q,
+                                                 double kr, double ki, int m0, double nd,
+                                                 double J, const Trig& tr,
+                                                 Multi<3, KB, GON>& v, double& c3) {
+  constexpr int NA = K + (GON ? 2 : 1);
+  double ac[NA][3], as[NA][3];
+  double n[4] = {tab[0], tab[1], tab[2], tab[3]};
+  taylor_point_flat<NA, CPLX, FAST, true>(d0, a, b, n, tab += 4, kr, ki, m0, tr, ac, as, c3);
+#pragma unroll 1
+  for (int q = 1; q < Q; ++q)
+    taylor_point_flat<NA, CPLX, FAST, false>(d0, a, b, n, tab += 4, kr, ki, m0, tr, ac, as, c3);
+  // F_m = (n.d) i^m [(m - 1) A'_{m-2} + i k A'_{m-1}], G_m = J i^m A'_m (A' without i^j)
+  const double kn = nd * kr, kin = CPLX ? nd * ki : 0.0;
+#pragma unroll
+  for (int q = 0; q < K; ++q) {
+    const double mn = nd * (double)(m0 + q - 1);
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      double re = fma(mn, ac[q][s], -(kn * as[q + 1][s]));
+      double im = fma(mn, as[q][s], kn * ac[q + 1][s]);
+      if constexpr (CPLX) {
+        re = fma(-kin, ac[q + 1][s], re);
+        im = fma(-kin, as[q + 1][s], im);
+      }
+      rotate(q, re, im);
+      v.fr[q][s] = re;
+      v.fi[q][s] = im;
+      if constexpr (GON) {
+        double gr = J * ac[q + 2][s], gi = J * as[q + 2][s];
+        rotate(q, gr, gi);
+        v.gr[q][s] = gr;
+        v.gi[q][s] = gi;
+      }
+    }
+  }
+}
+
+// Pair on an element with tabulated points (rows y, n, J w / (4 pi) in memory, the next one
+// always under way; basis values ph in LDS).
+template <int NP, int KB, bool TAY, bool CPLX, bool GON, bool FAST>
+__device__ __forceinline__ void multi_pair_rows(double x0, double x1, double x2,
+                                                const double* rows, const double* ph, int Q,
+                                                const Block<KB>& kv, bool rec, double ki, int m0,
+                                                const Trig& tr, Multi<NP, KB, GON>& v,
+                                                double& csum) {
+  v.clear();
+  double y[7];
+#pragma unroll
+  for (int d = 0; d < 7; ++d) y[d] = rows[d];
+#pragma unroll 1
+  for (int p = 0; p < Q; ++p, ph += NP) {
+    const double dx = y[0] - x0, dy = y[1] - x1, dz = y[2] - x2;
+    const double nd = fma(y[3], dx, fma(y[4], dy, y[5] * dz)), jw = y[6];
+    rows += p + 1 < Q ? 8 : 0;
+#pragma unroll
+    for (int d = 0; d < 7; ++d) y[d] = rows[d];
+    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+    const double rinv = rsqrt_nr(r2);
+    const double r = r2 * rinv;
+    const double g = jw * rinv;
+    const double t = nd * (rinv * rinv);
+    csum = fma(-t, g, csum);
+    double b[NP];
+#pragma unroll
+    for (int s = 0; s < NP; ++s) b[s] = ph[s];
+    double sn, cs, zs = 0.0, zc = 0.0, damp = 1.0;
+    Phase<CPLX, FAST> e;
+    e.begin(kv.k[0] * r, CPLX ? ki * r : 0.0, tr);
+    e.end(tr, sn, cs, damp);
+    double gm = g, am = 0.0;
+    if constexpr (TAY) {  // G_m without i^(m - m0), F_m = (m - 1 + i k r) t G_m
+      if (CPLX) gm *= damp;
+      double p2 = r;
+      for (int x = m0; x != 0; x >>= 1) {
+        if (x & 1) gm *= p2;
+        p2 *= p2;
+      }
+      if (m0 & 2) gm = -gm;
+      am = (double)(m0 - 1) - (CPLX ? ki * r : 0.0);
+    } else if (rec) {
+      Phase<false, FAST> z;
+      z.begin(kv.dk * r, 0.0, tr);
+      z.end(tr, zs, zc, damp);
+    }
+    double Gr = gm * cs, Gi = gm * sn;
+#pragma unroll
+    for (int q = 0; q < KB; ++q) {
+      double Fr, Fi;
+      if constexpr (TAY) {
+        if (q > 0) {
+          Gr *= r;
+          Gi *= r;
+        }
+        const double krr = kv.k[0] * r;
+        Fr = t * fma(am + (double)q, Gr, -(krr * Gi));
+        Fi = t * fma(am + (double)q, Gi, krr * Gr);
+      } else {
+        if (q > 0) {
+          if (rec) {
+            const double c2 = fma(Gr, zc, -(Gi * zs));
+            Gi = fma(Gr, zs, Gi * zc);
+            Gr = c2;
+          } else {
+            Phase<false, FAST> z;
+            z.begin(kv.k[q] * r, 0.0, tr);
+            z.end(tr, sn, cs, damp);
+            Gr = g * cs;
+            Gi = g * sn;
+          }
+        }
+        const double krr = kv.k[q] * r;
+        Fr = -t * fma(krr, Gi, Gr);
+        Fi = t * fma(krr, Gr, -Gi);
+      }
 #pragma unroll
       for (int s = 0; s < NP; ++s) {
-        gr[b][s] = fma(Gr, ps[s], gr[b][s]);
-        gi[b][s] = fma(Gi, ps[s], gi[b][s]);
-      }
-    }
-  }
-}
-
-// Flush of one step's finished nodes for the KBS slot groups of a block (see the
-// single-k kernel): slot contents to F_k, G_k columns, zeroing the slots.  With PACK a
-// group holds F of two consecutive matrices (k0 + 2 q2 at +0/+64, k0 + 2 q2 + 1 at
-// +128/+192) and no G.
-template <int KBS, int W, bool PACK>
-__device__ __forceinline__ void sweep_flush(const AssemblyArgs& a, const SlotArgs& sa,
-                                            const SweepArgs& sw, int st, int wave, int lane,
-                                            int64_t i, bool active, int k0, double* acc) {
-  const bool doF = (a.flags & BIE_F) != 0, doG = (a.flags & BIE_G) != 0;
-  const int f1 = sload(sa.flush_begin + st + 1);
-  for (int f = sload(sa.flush_begin + st) + wave; f < f1; f += W) {
-    const int node = sload(sa.flush_node + f);
-    const int ss = sload(sa.flush_slot + f);
-#pragma unroll
-    for (int q2 = 0; q2 < KBS; ++q2) {
-      double* p = acc + ((size_t)(ss & 0xffff) * KBS + q2) * 256 + lane;
-      const double vr = p[0], vi = p[64], wr = p[128], wi = p[192];
-      p[0] = 0.0;
-      p[64] = 0.0;
-      p[128] = 0.0;
-      p[192] = 0.0;
-      if constexpr (PACK) {
-        const int ka = k0 + 2 * q2;
-        if (active && doF) {
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            if (ka + h >= sw.nk) break;
-            const double xr = h ? wr : vr, xi = h ? wi : vi;
-            const size_t idx =
-                2 * ((size_t)(ka + h) * sw.stride + (size_t)i + (size_t)node * a.M);
-            if (ss & kSharedBit) {
-              unsafeAtomicAdd(a.F + idx, xr);
-              unsafeAtomicAdd(a.F + idx + 1, xi);
-            } else {
-              __builtin_nontemporal_store(d2v{xr, xi}, reinterpret_cast<d2v*>(a.F + idx));
-            }
-          }
-        }
-        continue;
-      }
-      const int kidx = k0 + q2;
-      if (active && kidx < sw.nk) {
-        const size_t idx = 2 * ((size_t)kidx * sw.stride + (size_t)i + (size_t)node * a.M);
-        if (ss & kSharedBit) {
-          if (doF) {
-            unsafeAtomicAdd(a.F + idx, vr);
-            unsafeAtomicAdd(a.F + idx + 1, vi);
-          }
-          if (doG) {
-            unsafeAtomicAdd(a.G + idx, wr);
-            unsafeAtomicAdd(a.G + idx + 1, wi);
-          }
-        } else {
-          if (doF) __builtin_nontemporal_store(d2v{vr, vi}, reinterpret_cast<d2v*>(a.F + idx));
-          if (doG) __builtin_nontemporal_store(d2v{wr, wi}, reinterpret_cast<d2v*>(a.G + idx));
+        v.fr[q][s] = fma(Fr, b[s], v.fr[q][s]);
+        v.fi[q][s] = fma(Fi, b[s], v.fi[q][s]);
+        if constexpr (GON) {
+          v.gr[q][s] = fma(Gr, b[s], v.gr[q][s]);
+          v.gi[q][s] = fma(Gi, b[s], v.gi[q][s]);
         }
       }
     }
   }
+  if constexpr (TAY) v.each([](int q, double& re, double& im) { rotate(q, re, im); });
 }
 
-// With TAY the KB accumulator sets of a block hold the k-derivative orders
-// kb*KB .. kb*KB+KB-1 at the one wavenumber sw.k_re + i sw.k_im instead of KB wavenumbers.
-// GON is whether G is formed (the BIE_G flag): F-only launches skip the G accumulation and
-// its LDS atomics in a separate instance, leaving the F-and-G code as it is.
-// Without G (PACK) the KB wavenumbers or orders of a block fill KB / 2 slot groups, two
-// matrices' F per group (see sweep_flush), so a block carries twice the matrices that the
-// slot schedule built for KB / 2 groups would otherwise allow.
-template <int NP, int KB, int W, bool TAY, bool GON>
-__global__ void __launch_bounds__(64 * W)
-k_sweep_slots(const AssemblyArgs a, const SlotArgs sa, const SweepArgs sw) {
-  constexpr bool PACK = !GON;
-  constexpr int KBS = PACK ? KB / 2 : KB;  // slot groups per slot
-  static_assert(!PACK || KB % 2 == 0, "packed blocks hold an even number of orders");
-  extern __shared__ double lds[];
-  double* acc = lds;  // [slot][group][4][64]
-  const int nphi = a.R * a.Qmax * NP;
-  double* s_phi = lds + (size_t)sa.S * KBS * 256;
-  const double2* s_trig = reinterpret_cast<const double2*>(s_phi + phi_pad(nphi));
-  int2* s_q = reinterpret_cast<int2*>(s_phi + phi_pad(nphi) + kTrigDoubles);
-  unsigned* s_qn = reinterpret_cast<unsigned*>(s_q + kMidLds);
-  const int b = blockIdx.x;
-  const int64_t per_xcd = (sw.n_tiles + 7) / 8;
-  const int64_t tile = (int64_t)(b & 7) * per_xcd + (b >> 3);
-  if ((b >> 3) >= per_xcd || tile >= sw.n_tiles) return;
-  // k block outermost, then segment, then row block
-  const int64_t per_kb = (int64_t)sa.n_segments * sa.n_rowblocks;
-  const int kb = (int)(tile / per_kb);
-  const int64_t rest = tile - (int64_t)kb * per_kb;
-  const int seg = (int)(rest / sa.n_rowblocks);
-  const int rb = (int)(rest - (int64_t)seg * sa.n_rowblocks);
+// First and middle contributions of nb matrices: into the slot (see stream.hip's give).
+template <int NP, int KB, bool GON>
+__device__ __forceinline__ void give_multi(const int4& en, const Roles& r, int lane, double* acc,
+                                           unsigned* claims, const Multi<NP, KB, GON>& v, int nb,
+                                           bool& ok) {
+  constexpr int SK = GON ? 256 : 128, SD = KB * SK;
+  const bool mine_first = lane_of_mask(r.first), mine_more = lane_of_mask(r.more);
+#pragma unroll
+  for (int s = 0; s < NP; ++s)
+    if ((r.first >> s) & 1) {
+      double* p = acc + (size_t)__builtin_amdgcn_readlane(en.x, s) * SD + lane;
+#pragma unroll
+      for (int b = 0; b < KB; ++b) {
+        if (b >= nb) break;
+        p[b * SK] = v.fr[b][s];
+        p[b * SK + 64] = v.fi[b][s];
+        if constexpr (GON) {
+          p[b * SK + 128] = v.gr[b][s];
+          p[b * SK + 192] = v.gi[b][s];
+        }
+      }
+    }
+  if (r.first) {
+    lds_wait();
+    if (mine_first) lds_count(claims + en.x, 0x10000u);
+  }
+  if (r.more) {
+    ok &= spin([&] { return !mine_more || (lds_peek(claims + en.x) >> 16) != 0; });
+#pragma unroll
+    for (int s = 0; s < NP; ++s)
+      if ((r.more >> s) & 1) {
+        double* p = acc + (size_t)__builtin_amdgcn_readlane(en.x, s) * SD + lane;
+#pragma unroll
+        for (int b = 0; b < KB; ++b) {
+          if (b >= nb) break;
+          atomicAdd(p + b * SK, v.fr[b][s]);
+          atomicAdd(p + b * SK + 64, v.fi[b][s]);
+          if constexpr (GON) {
+            atomicAdd(p + b * SK + 128, v.gr[b][s]);
+            atomicAdd(p + b * SK + 192, v.gi[b][s]);
+          }
+        }
+      }
+    lds_wait();
+    if (mine_more) lds_count(claims + en.x, 0x10000u);
+  }
+}
+
+// Last contributions: to the columns of the block's matrices (see stream.hip's finish).
+template <int NP, int KB, bool GON>
+__device__ __forceinline__ void finish_multi(InstPtr in, SweepPtr sw, const int4& en,
+                                             const Roles& r, int lane, int64_t i0, bool active,
+                                             int k0, int nb, const double* acc, unsigned* claims,
+                                             unsigned* turns, const Multi<NP, KB, GON>& v,
+                                             bool& ok) {
+  constexpr int SK = GON ? 256 : 128, SD = KB * SK;
+  const bool mine = lane_of_mask(r.last);
+  if (r.last)
+    ok &= spin([&] {
+      return !mine || (lds_peek(claims + en.x) >> 16) == (unsigned)en.y - 1u;
+    });
+  const double bad = ok ? 0.0 : NAN;
+  const InstPtr p = fresh(in);
+  const bool doF = (p->a.flags & BIE_F) != 0;
+  const int64_t M = p->a.M, stride = sw->stride;
+  double* F = p->a.F + 2 * (size_t)k0 * stride;
+  double* G = p->a.G + 2 * (size_t)k0 * stride;
+#pragma unroll
+  for (int s = 0; s < NP; ++s) {
+    const bool last = (r.last >> s) & 1;
+    if (!last && !((r.direct >> s) & 1)) continue;
+    const int nw = __builtin_amdgcn_readlane(en.w, s);
+    const bool shared = (nw & kSharedBit) != 0;
+    const double* q =
+        acc + (size_t)(last ? __builtin_amdgcn_readlane(en.x, s) : 0) * SD + lane;
+    size_t at = 2 * ((size_t)i0 + (size_t)(nw & ~kSharedBit) * (size_t)M);
+#pragma unroll
+    for (int b = 0; b < KB; ++b, at += 2 * (size_t)stride) {
+      if (b >= nb) break;
+      double f0 = v.fr[b][s] + bad, f1 = v.fi[b][s], g0 = 0.0, g1 = 0.0;
+      if constexpr (GON) {
+        g0 = v.gr[b][s] + bad;
+        g1 = v.gi[b][s];
+      }
+      if (last) {
+        f0 += q[b * SK];
+        f1 += q[b * SK + 64];
+        if constexpr (GON) {
+          g0 += q[b * SK + 128];
+          g1 += q[b * SK + 192];
+        }
+      }
+      if (active) {
+        if (doF) column_store(F + at, 16u * lane, shared, f0, f1);
+        if constexpr (GON) column_store(G + at, 16u * lane, shared, g0, g1);
+      }
+    }
+  }
+  if (mine) {
+    lds_wait();
+    lds_poke(claims + en.x, 0u);
+    lds_poke(turns + en.x, (unsigned)en.z + 1u);
+  }
+}
+
+// Elements of the tile's segment, drawn by this wave, for the matrices k0 .. of a block.
+template <int NP, bool FLAT, bool TAY, bool CPLX, bool GON, bool FAST>
+__device__ __forceinline__ void sweep_tile(InstPtr in, SweepPtr sw, int rb, int seg, int kb,
+                                           int S, int tab_doubles, double* lds, int parity) {
+  constexpr int W = kSweepWaves, KB = sweep_block(NP, GON);
+  constexpr bool kMids = NP == 6;
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int R = in->a.R;
+  const int Q = in->a.len[0];
+  const Layout L = layout_of(S, sweep_slot_doubles(NP), tab_doubles, W, 0, kMids && R == 6);
+  double* acc = lds;
+  const double* tab = lds + L.tab;
+  const Trig tr = make_trig(tab + tab_doubles);
+  unsigned* claims = reinterpret_cast<unsigned*>(lds + L.words);
+  unsigned* turns = claims + S;
+  unsigned* ctr = turns + S;
   const int64_t i = (int64_t)rb * 64 + lane;
-  const bool active = i < a.M;
-  // basis table and trig table: one buffer of phi_pad(nphi) + kTrigDoubles doubles
-  for (int t = threadIdx.x; t < phi_pad(nphi) + kTrigDoubles; t += blockDim.x) s_phi[t] = a.phi[t];
-  for (int t = threadIdx.x; t < sa.S * KBS * 256; t += blockDim.x) acc[t] = 0.0;
-  if (threadIdx.x == 0) *s_qn = 0u;
-  lds_barrier();
-  const int64_t ic = active ? i : (a.M - 1);
-  const double x0 = a.targets[3 * ic], x1 = a.targets[3 * ic + 1], x2 = a.targets[3 * ic + 2];
-  const bool first_kb = kb == 0;
-  constexpr bool doG = GON;
-  double kv[KB];
-  const int k0 = kb * KB;
-  bool rec = false;
-  double dk = 0.0;
-  if constexpr (!TAY) {
+  const int64_t M = in->a.M;
+  const bool active = i < M;
+  const double* xt = in->a.targets + 3 * (active ? i : M - 1);
+  const double x0 = xt[0], x1 = xt[1], x2 = xt[2];
+  const int k0 = kb * KB, nb = min(KB, sw->nk - k0);
+  Block<KB> kv;
+  double ki = 0.0;
+  bool rec = true;
+  if constexpr (TAY) {
+    kv.k[0] = sw->k_re;
+    ki = sw->k_im;
+  } else {
 #pragma unroll
-    for (int q = 0; q < KB; ++q) kv[q] = sw.k[min(k0 + q, sw.nk - 1)];
-    rec = sw.block_uniform[kb] != 0;
-    dk = KB > 1 ? kv[1] - kv[0] : 0.0;
+    for (int q = 0; q < KB; ++q) kv.k[q] = sload(sw->k + min(k0 + q, sw->nk - 1));
+    kv.dk = nb > 1 ? kv.k[KB > 1 ? 1 : 0] - kv.k[0] : 0.0;
+    // the recurrence forms e^{i (k0 + q dk) r}: taken where that differs from e^{i k_q r} by
+    // at most about 2 ulp of k_q r (a rounded linspace does)
+#pragma unroll
+    for (int q = 2; q < KB; ++q)
+      if (q < nb && !(fabs(kv.k[q] - (kv.k[0] + q * kv.dk)) <= 4.5e-16 * fabs(kv.k[q])))
+        rec = false;
+    rec = __builtin_amdgcn_readfirstlane(rec);
+#pragma unroll
+    for (int q = 0; q < KB; ++q) asm volatile("" : "+s"(kv.k[q]));
   }
+  const int t0 = sload(in->seg_begin + seg), t1 = sload(in->seg_begin + seg + 1);
+  const int tab_rule = FLAT ? 4 * Q + 2 : ((Q * NP + 1) & ~1) + 2;
+  auto draw = [&]() -> int { return t0 + (int)lds_draw(ctr + kTicket, 1u, lane); };
   double csum = 0.0;
-  const int st0 = sload(sa.seg_step_begin + seg), st1 = sload(sa.seg_step_begin + seg + 1);
-  int e = (st0 < st1) ? sload(sa.step_elems + (size_t)st0 * W + wave) : -1;
-  int c = 0;
-  double4 A0 = make_double4(0, 0, 0, 0), B0 = A0;
-  if (e >= 0) {
-    c = select_rule<NP>(x0, x1, x2, sa.step_sel + ((size_t)st0 * W + wave) * NP * 4, a.R,
-                        a.hyp) - 1;
-    if (!(NP == 6 && c >= 3)) {
-      const double* t0 = a.elem + ((size_t)e * a.Pe + a.off[c]) * 8;
-      A0 = *reinterpret_cast<const double4*>(t0);
-      B0 = *reinterpret_cast<const double4*>(t0 + 4);
-    }
-  }
-  for (int st = st0; st < st1; ++st) {
-    const size_t nidx = (size_t)(st + 1) * W + wave;
-    const int e_nxt =
-        (st + 1 < st1) ? sload(sa.step_elems + nidx) : -1;
-    if (e >= 0) {
-      const bool mid = NP == 6 && c >= 3;
-      if (active && !mid) {
-        double fr[KB][NP], fi[KB][NP], gr[KB][NP], gi[KB][NP];
+  int pos = draw();
+  while (pos < t1) {
+    const int nxt = draw();
+    const InstPtr u = fresh(in);
+    Multi<NP, KB, GON> v;
+    if constexpr (FLAT) {
+      const double* rec24 = u->flat + (size_t)pos * kFlatDoubles;
+      const d8 r0 = sload8(rec24), r1 = sload8(rec24 + 8), r2 = sload8(rec24 + 16);
+      const double P[3][3] = {{r0[0], r0[1], r0[2]}, {r0[3], r0[4], r0[5]},
+                              {r0[6], r0[7], r1[0]}};
+      const double ea[3] = {r1[4], r1[5], r1[6]}, eb[3] = {r1[7], r2[0], r2[1]};
+      const int c = select_rule_s<3>(x0, x1, x2, P, rec24, R, in) - 1;
+      const double d0[3] = {r1[1] - x0, r1[2] - x1, r1[3] - x2};
+      const double nd = fma(r2[2], d0[0], fma(r2[3], d0[1], r2[4] * d0[2]));  // n.d J
+      const double J = r2[5];
+      const double* tc = tab + c * tab_rule;
+      double c3 = 0.0;
+      if constexpr (TAY) {
+        if (KB > 4 && nb <= KB / 2)
+          taylor_pair_flat<KB, KB / 2, CPLX, GON, FAST>(d0, ea, eb, tc, Q, kv.k[0], ki, k0, nd,
+                                                        J, tr, v, c3);
+        else
+          taylor_pair_flat<KB, KB, CPLX, GON, FAST>(d0, ea, eb, tc, Q, kv.k[0], ki, k0, nd, J,
+                                                    tr, v, c3);
+      } else {
+        if (!rec)
+          sweep_pair_flat<KB, KB, GON, FAST, false>(d0, ea, eb, tc, Q, kv, tr, v, c3);
+        else if (KB > 4 && nb <= KB / 2)
+          sweep_pair_flat<KB, KB / 2, GON, FAST, true>(d0, ea, eb, tc, Q, kv, tr, v, c3);
+        else
+          sweep_pair_flat<KB, KB, GON, FAST, true>(d0, ea, eb, tc, Q, kv, tr, v, c3);
 #pragma unroll
         for (int q = 0; q < KB; ++q)
 #pragma unroll
-          for (int s = 0; s < NP; ++s) fr[q][s] = fi[q][s] = gr[q][s] = gi[q][s] = 0.0;
-        const double* tab = a.elem + ((size_t)e * a.Pe + a.off[c]) * 8;
-        const double* ph = s_phi + c * a.Qmax * NP;
-        const int Q = a.len[c];
-        double cs_local = 0.0;
-        // point 0 was fetched before the barrier; later rows are loaded in turn
-        if constexpr (TAY) {
-          taylor_point<NP, KB, true>(x0, x1, x2, A0, B0, ph, sw.k_re, sw.k_im, k0, doG, fr, fi,
-                                     gr, gi, cs_local, s_trig);
-          for (int q = 1; q < Q; ++q) {
-            const double4 A = *reinterpret_cast<const double4*>(tab + 8 * q);
-            const double4 B = *reinterpret_cast<const double4*>(tab + 8 * q + 4);
-            taylor_point<NP, KB, true>(x0, x1, x2, A, B, ph + q * NP, sw.k_re, sw.k_im, k0, doG,
-                                       fr, fi, gr, gi, cs_local, s_trig);
+          for (int s = 0; s < 3; ++s) {
+            v.fr[q][s] *= nd;
+            v.fi[q][s] *= nd;
+            if constexpr (GON) {
+              v.gr[q][s] *= J;
+              v.gi[q][s] *= J;
+            }
           }
-        } else {
-          sweep_point<NP, KB, true>(x0, x1, x2, A0, B0, ph, kv, dk, rec, doG, fr, fi, gr, gi,
-                                    cs_local, s_trig);
-          for (int q = 1; q < Q; ++q) {
-            const double4 A = *reinterpret_cast<const double4*>(tab + 8 * q);
-            const double4 B = *reinterpret_cast<const double4*>(tab + 8 * q + 4);
-            sweep_point<NP, KB, true>(x0, x1, x2, A, B, ph + q * NP, kv, dk, rec, doG, fr, fi,
-                                      gr, gi, cs_local, s_trig);
-          }
-        }
-        csum += cs_local;
-        const int* so = sa.step_slot + ((size_t)st * W + wave) * NP;
+      }
+      csum = fma(-nd, c3, csum);
+    } else {
+      int c = 0;
+      if (R > 1) {
+        double P[NP][3];
+        const double* ps = u->psel + (size_t)pos * NP * 3;
 #pragma unroll
         for (int s = 0; s < NP; ++s)
 #pragma unroll
-          for (int q2 = 0; q2 < KB; ++q2) {
-            if constexpr (PACK) {
-              double* p = acc + ((size_t)sload(so + s) * KBS + q2 / 2) * 256 + lane +
-                          (q2 & 1) * 128;
-              atomicAdd(p, fr[q2][s]);
-              atomicAdd(p + 64, fi[q2][s]);
-            } else {
-              double* p = acc + ((size_t)sload(so + s) * KB + q2) * 256 + lane;
-              atomicAdd(p, fr[q2][s]);
-              atomicAdd(p + 64, fi[q2][s]);
-              if (doG) {
-                atomicAdd(p + 128, gr[q2][s]);
-                atomicAdd(p + 192, gi[q2][s]);
-              }
-            }
-          }
+          for (int d = 0; d < 3; ++d) P[s][d] = sload(ps + 3 * s + d);
+        c = select_rule_s<NP>(x0, x1, x2, P, ps, R, in) - 1;
       }
-      if (NP == 6 && first_kb) {  // mid-edge pairs are queued once, for every k
-        const bool push = mid && active;
-        const unsigned long long mask = __ballot(push);
-        if (mask) {
-          const int leader = __ffsll((long long)mask) - 1;
-          unsigned base = 0;
-          if (lane == leader) base = atomicAdd(s_qn, (unsigned)__popcll(mask));
-          base = __shfl(base, leader);
-          if (push) {
-            const unsigned pos = base + (unsigned)__popcll(mask & ((1ull << lane) - 1ull));
-            const int2 entry = make_int2((int)i, e | ((c - 3) << 28));
-            if (pos < (unsigned)kMidLds) {
-              s_q[pos] = entry;
-            } else {
-              const unsigned g = atomicAdd(sa.mid_count, 1u);
-              if ((int64_t)g < sa.mid_cap) sa.mid_queue[g] = entry;
-            }
-          }
+      const bool mid = kMids && c >= 3;
+      const int cr = mid ? 0 : c;
+      double cs_pair = 0.0;
+      multi_pair_rows<NP, KB, TAY, CPLX, GON, FAST>(
+          x0, x1, x2,
+          u->a.elem + ((size_t)sload(u->order + pos) * u->a.Pe + (size_t)cr * Q) * 8,
+          tab + (size_t)cr * tab_rule, Q, kv, rec, ki, k0, tr, v, cs_pair);
+      if (kMids && R == 6 && __any(mid)) {  // those pairs leave nothing here
+        v.each([&](int, double& re, double& im) {
+          re = mid ? 0.0 : re;
+          im = mid ? 0.0 : im;
+        });
+        cs_pair = mid ? 0.0 : cs_pair;
+        const unsigned long long mask = __ballot(mid && active);
+        if (mask && kb == 0) {  // listed once, for every matrix
+          const unsigned base = lds_draw(ctr + kMidN + parity, (unsigned)__popcll(mask), lane);
+          const unsigned at =
+              base + __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                               __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+          if (mid && active && at < (unsigned)kStreamMid)  // position, rule, row of the pair
+            reinterpret_cast<unsigned*>(lds + L.queue)[parity * kStreamMid + at] =
+                ((unsigned)(pos - t0) << 8) | ((unsigned)(c - 3) << 6) | (unsigned)lane;
         }
       }
+      csum += cs_pair;
     }
-    int c_nxt = 0;
-    if (e_nxt >= 0) {
-      c_nxt = select_rule<NP>(x0, x1, x2, sa.step_sel + nidx * NP * 4, a.R, a.hyp) - 1;
-      if (!(NP == 6 && c_nxt >= 3)) {
-        const double* t0 = a.elem + ((size_t)e_nxt * a.Pe + a.off[c_nxt]) * 8;
-        A0 = *reinterpret_cast<const double4*>(t0);
-        B0 = *reinterpret_cast<const double4*>(t0 + 4);
-      }
-    }
-    // the previous step's finished nodes (their slots were complete at the last barrier)
-    if (st > st0) sweep_flush<KBS, W, PACK>(a, sa, sw, st - 1, wave, lane, i, active, k0, acc);
-    lds_barrier();
-    e = e_nxt;
-    c = c_nxt;
+    const int l = fresh_lane(lane);
+    const int4 en = fresh(in)->ent[(size_t)pos * NP + min(l, NP - 1)];
+    bool ok;
+    const Roles r = claim<NP>(en, l, claims, turns, ok);
+    give_multi<NP, KB, GON>(en, r, l, acc, claims, v, nb, ok);
+    finish_multi<NP, KB, GON>(in, sw, en, r, l, (int64_t)rb * 64, active, k0, nb, acc, claims,
+                              turns, v, ok);
+    pos = nxt;
   }
-  if (st1 > st0) {
-    sweep_flush<KBS, W, PACK>(a, sa, sw, st1 - 1, wave, lane, i, active, k0, acc);
-    lds_barrier();
-  }
-  if (NP == 6 && first_kb && wave == 0) {
-    const unsigned n = min(*s_qn, (unsigned)kMidLds);
-    if (n) {
-      unsigned base = 0;
-      if (lane == 0) base = atomicAdd(sa.mid_count, n);
-      base = __shfl(base, 0);
-      for (unsigned t = lane; t < n; t += 64)
-        if ((int64_t)(base + t) < sa.mid_cap) sa.mid_queue[base + t] = s_q[t];
-    }
-  }
-  if (first_kb && active && (a.flags & BIE_C)) unsafeAtomicAdd(a.C + 2 * i, csum);
+  if (kb == 0) atomicAdd(lds + L.csum + lane, csum);
 }
 
-// Mid-edge pairs for every k (with TAY: every derivative order): one thread per (pair, k).
-template <bool TAY>
+template <int NP, bool FLAT, bool TAY, bool CPLX, bool GON, bool FAST>
+__global__ void __launch_bounds__(64 * kSweepWaves)
+k_sweep(const StreamInst one, const SweepArgs args, int n_tiles, const StreamRun run) {
+  extern __shared__ double lds[];
+  const auto* base = (const __attribute__((address_space(4))) char*)
+      __builtin_amdgcn_kernarg_segment_ptr();
+  const InstPtr in = (InstPtr)base;
+  const SweepPtr sw = (SweepPtr)(base + ((sizeof(StreamInst) + alignof(SweepArgs) - 1) &
+                                         ~(alignof(SweepArgs) - 1)));
+  // matrix block outermost, then segment, then row block
+  const int per_kb = one.n_segments * one.n_rowblocks;
+  auto inst_of = [&](int tile, int& rb, int& seg) -> InstPtr {
+    const int t = tile % per_kb, n = in->n_rowblocks;
+    seg = t / n;
+    rb = t - seg * n;
+    return in;
+  };
+  auto kmax_of = [&](InstPtr, int tile) -> double {
+    if constexpr (TAY) {
+      return fabs(sw->k_re);
+    } else {  // of the block's wavenumbers and of their spacing
+      constexpr int KB = sweep_block(NP, GON);
+      const int k0 = tile / per_kb * KB;
+      double m = 0.0;
+      for (int q = k0; q < min(k0 + KB, sw->nk); ++q) m = fmax(m, fabs(sload(sw->k + q)));
+      return 2.0 * m;
+    }
+  };
+  stream_run<sweep_slot_doubles(NP), kSweepWaves, NP == 6, FAST>(
+      inst_of, kmax_of, [&](InstPtr, int tile) { return tile < per_kb; },
+      [&](InstPtr p, int rb, int seg, int tile, int parity) {
+        sweep_tile<NP, FLAT, TAY, CPLX, GON, FAST>(p, sw, rb, seg, tile / per_kb, run.S,
+                                                   run.tab_doubles, lds, parity);
+      },
+      n_tiles, run);
+}
+
+// The listed mid-edge pairs, for every matrix (blockIdx.y and on).
+template <bool TAY, bool CPLX, bool GON>
 __global__ void __launch_bounds__(256)
-k_sweep_mid(const AssemblyArgs a, const SlotArgs sa, const SweepArgs sw) {
-  const int64_t n = min((int64_t)*sa.mid_count, sa.mid_cap);
-  const int64_t total = n * sw.nk;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  const bool doF = (a.flags & BIE_F) != 0, doG = (a.flags & BIE_G) != 0;
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += stride) {
-    const int kidx = (int)(t / n);
-    const int2 en = sa.mid_queue[t - (int64_t)kidx * n];
-    const int64_t i = en.x;
-    const int e = en.y & 0x0fffffff;
-    const int c = 3 + (en.y >> 28);
-    const double x0 = a.targets[3 * i], x1 = a.targets[3 * i + 1], x2 = a.targets[3 * i + 2];
-    double fr[1][6], fi[1][6], gr[1][6], gi[1][6], csum = 0.0;
-#pragma unroll
-    for (int s = 0; s < 6; ++s) fr[0][s] = fi[0][s] = gr[0][s] = gi[0][s] = 0.0;
-    const double* tab = a.elem + ((size_t)e * a.Pe + a.off[c]) * 8;
-    const double* ph = a.phi + c * a.Qmax * 6;
-    const double kk = TAY ? sw.k_re : sw.k[kidx];
-    for (int q = 0; q < a.len[c]; ++q) {
-      const double4 A = *reinterpret_cast<const double4*>(tab + 8 * q);
-      const double4 B = *reinterpret_cast<const double4*>(tab + 8 * q + 4);
-      if constexpr (TAY)
-        taylor_point<6, 1, false>(x0, x1, x2, A, B, ph + q * 6, kk, sw.k_im, kidx, doG, fr, fi,
-                                  gr, gi, csum, nullptr);
-      else
-        sweep_point<6, 1, false>(x0, x1, x2, A, B, ph + q * 6, &kk, 0.0, false, doG, fr, fi,
-                                 gr, gi, csum, nullptr);
-    }
-    const int* cols = a.ptopo + (size_t)e * 6;
-#pragma unroll
-    for (int s = 0; s < 6; ++s) {
-      const size_t idx = 2 * ((size_t)kidx * sw.stride + (size_t)i + (size_t)cols[s] * a.M);
-      if (doF) {
-        unsafeAtomicAdd(a.F + idx, fr[0][s]);
-        unsafeAtomicAdd(a.F + idx + 1, fi[0][s]);
-      }
-      if (doG) {
-        unsafeAtomicAdd(a.G + idx, gr[0][s]);
-        unsafeAtomicAdd(a.G + idx + 1, gi[0][s]);
-      }
-    }
-    if (kidx == 0 && (a.flags & BIE_C)) unsafeAtomicAdd(a.C + 2 * i, csum);
+k_sweep_mid(const StreamInst one, const SweepArgs sw, const double* tab_src, int tab_doubles) {
+  extern __shared__ double lds[];
+  const InstPtr in = (InstPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  const int mid_off = in->mid_off;
+  const int ntab = tab_doubles - mid_off + kTrigDoubles + kExpN;
+  for (int t = threadIdx.x; t < ntab; t += 256) lds[t] = tab_src[mid_off + t];
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const Trig tr = make_trig(lds + tab_doubles - mid_off);
+  for (int q = blockIdx.y; q < sw.nk; q += gridDim.y) {
+    const size_t at = 2 * (size_t)q * sw.stride;
+    const MidOut o{TAY ? sw.k_re : sload(sw.k + q), TAY ? sw.k_im : 0.0, in->a.F + at,
+                   in->a.G + at, q == 0 && (in->a.flags & BIE_C), q};
+    mid_pairs<CPLX, GON, false, TAY>(in, o, lds, tr, blockIdx.x * 4 + wave, gridDim.x * 4,
+                                     threadIdx.x & 63);
   }
 }
 
-// Zero listed columns of nk column-major M x N complex matrices spaced stride apart:
-// workgroups stride over the (matrix, column) pairs, threads over the rows of a column.
-__global__ void k_zero_columns_multi(double2* __restrict__ X, int64_t stride, int nk, int64_t M,
-                                     const int* __restrict__ cols, int ncols) {
-  const double2 z = make_double2(0.0, 0.0);
-  const int64_t pairs = (int64_t)nk * ncols;
-  for (int64_t pc = blockIdx.x; pc < pairs; pc += gridDim.x) {
-    const int kq = (int)(pc / ncols);
-    const int c = (int)(pc - (int64_t)kq * ncols);
-    double2* col = X + (size_t)kq * stride + (size_t)cols[c] * M;
-    for (int64_t r = threadIdx.x; r < M; r += blockDim.x) col[r] = z;
-  }
-}
-
-}  // namespace
-
-void launch_zero_columns_multi(double* X, int64_t stride, int nk, int64_t M, const int* cols,
-                               int ncols, hipStream_t s) {
-  if (ncols <= 0 || M <= 0 || nk <= 0) return;
-  int64_t blocks = (int64_t)ncols * nk;
-  if (blocks > 65536) blocks = 65536;
-  hipLaunchKernelGGL(k_zero_columns_multi, dim3((unsigned)blocks), dim3(256), 0, s,
-                     reinterpret_cast<double2*>(X), stride, nk, M, cols, ncols);
-  BIE_HIP_CHECK(hipGetLastError());
-}
-
-int sweep_kb(int NP) { return NP == 6 ? 2 : 4; }
-
-int sweep_block_size(int NP, bool gon) { return gon ? sweep_kb(NP) : 2 * sweep_kb(NP); }
-
-namespace {
-
-__global__ void k_block_uniform(const double* __restrict__ k, int nk, int KB, int* out) {
-  const int kb = blockIdx.x * blockDim.x + threadIdx.x;
-  if (kb * KB >= nk) return;
-  const double k0 = k[kb * KB];
-  const double dk = (kb * KB + 1 < nk) ? k[kb * KB + 1] - k0 : 0.0;
-  int ok = (kb * KB + KB <= nk) ? 1 : 0;  // a partial block evaluates directly
-  for (int b = 2; b < KB && ok; ++b) {
-    const double kb_ = k[kb * KB + b];
-    // the recurrence produces e^{i (k0 + b dk) r}; accept it when it differs from
-    // e^{i k_b r} by at most ~2 ulp of k_b r (a rounded linspace passes)
-    if (fabs(kb_ - (k0 + b * dk)) > 4.5e-16 * fabs(kb_)) ok = 0;
-  }
-  out[kb] = ok;
-}
-
-size_t g_sweep_attr[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-
-template <int NP, int KB, int W>
-const void* sweep_kernel_np(bool taylor, bool gon) {
-  if (taylor)
-    return gon ? reinterpret_cast<const void*>(k_sweep_slots<NP, KB, W, true, true>)
-               : reinterpret_cast<const void*>(k_sweep_slots<NP, 2 * KB, W, true, false>);
-  return gon ? reinterpret_cast<const void*>(k_sweep_slots<NP, KB, W, false, true>)
-             : reinterpret_cast<const void*>(k_sweep_slots<NP, 2 * KB, W, false, false>);
-}
-
-template <int W>
-const void* sweep_kernel(int NP, bool taylor, bool gon) {
-  if (NP == 1) return sweep_kernel_np<1, 4, W>(taylor, gon);
-  return NP == 3 ? sweep_kernel_np<3, 4, W>(taylor, gon) : sweep_kernel_np<6, 2, W>(taylor, gon);
-}
-
-}  // namespace
-
-void launch_block_uniform(const double* k, int nk, int KB, int* out, hipStream_t s) {
-  const int nkb = (nk + KB - 1) / KB;
-  if (nkb <= 0) return;
-  hipLaunchKernelGGL(k_block_uniform, dim3((nkb + 63) / 64), dim3(64), 0, s, k, nk, KB, out);
-  BIE_HIP_CHECK(hipGetLastError());
-}
-
-size_t sweep_shmem(int NP, int nphi, int S) {
-  const int KB = sweep_kb(NP);
-  return sizeof(double) * ((size_t)S * KB * 256 + sweep_fixed_doubles(nphi)) +
-         sizeof(int2) * kMidLds + 16;
-}
-
-void sweep_prepare_attributes(int NP, int nphi, bool taylor, bool gon) {
-  const size_t shmem =
-      sweep_shmem(NP, nphi, fitting_slots(sweep_fixed_doubles(nphi), sweep_kb(NP)));
-  constexpr int W = kSlotWaves;
-  const void* kern = sweep_kernel<W>(NP, taylor, gon);
-  size_t& done = g_sweep_attr[(NP == 1 ? 0 : NP == 3 ? 1 : 2) + (taylor ? 3 : 0) + (gon ? 6 : 0)];
-  if (shmem > done) {
-    BIE_HIP_CHECK(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)std::max(shmem, (size_t)(144 * 1024))));
-    done = std::max(shmem, (size_t)(144 * 1024));
-  }
-}
-
-void launch_sweep(const AssemblyArgs& a, const SlotArgs& sa, const SweepArgs& sw,
-                  hipStream_t s) {
-  if (a.M == 0 || a.E == 0 || sw.nk == 0) return;
-  const int KB = sweep_kb(a.NP);
-  const int nphi = a.R * a.Qmax * a.NP;
-  BIE_REQUIRE(sa.W == kSlotWaves && sa.S <= fitting_slots(sweep_fixed_doubles(nphi), KB),
-              BIE_EINVAL, "sweep schedule does not match the kernel");
-  const int64_t per_xcd = (sw.n_tiles + 7) / 8;
-  BIE_REQUIRE(per_xcd * 8 <= 2147483647LL, BIE_EINVAL, "too many sweep tiles");
-  const size_t shmem = sweep_shmem(a.NP, nphi, sa.S);
-  BIE_REQUIRE(shmem <= 160 * 1024, BIE_EINVAL, "sweep kernel LDS request exceeds 160 KiB");
-  const bool tay = sw.taylor != 0;
-  const bool gon = (a.flags & BIE_G) != 0;
-  sweep_prepare_attributes(a.NP, nphi, tay, gon);
-  constexpr int W = kSlotWaves;
-  const void* kern = sweep_kernel<W>(a.NP, tay, gon);
-  AssemblyArgs a_ = a;
-  SlotArgs sa_ = sa;
-  SweepArgs sw_ = sw;
-  void* args[] = {&a_, &sa_, &sw_};
-  BIE_HIP_CHECK(hipLaunchKernel(kern, dim3((unsigned)(per_xcd * 8)), dim3(64 * W), args, shmem,
-                                s));
-  if (uses_mid_rules(a.R, a.NP)) {
-    if (tay)
-      hipLaunchKernelGGL(k_sweep_mid<true>, dim3(4096), dim3(256), 0, s, a, sa, sw);
+// Calls fn(kernel, mid-edge kernel) of (NP, flat elements, k-derivatives, complex, G, fast).
+template <class Fn>
+void with_sweep_kernel(int NP, bool flat, bool tay, bool cplx, bool gon, bool fast, Fn&& fn) {
+  using T = std::true_type;
+  using F = std::false_type;
+  auto by_fast = [&](auto np, auto fl, auto ta, auto cx, auto g) {
+    constexpr int N = decltype(np)::value;
+    constexpr bool FL = decltype(fl)::value, TA = decltype(ta)::value, CX = decltype(cx)::value,
+                   G = decltype(g)::value;
+    if (fast)
+      fn(k_sweep<N, FL, TA, CX, G, true>, k_sweep_mid<TA, CX, G>);
     else
-      hipLaunchKernelGGL(k_sweep_mid<false>, dim3(4096), dim3(256), 0, s, a, sa, sw);
-    BIE_HIP_CHECK(hipGetLastError());
-  }
+      fn(k_sweep<N, FL, TA, CX, G, false>, k_sweep_mid<TA, CX, G>);
+  };
+  auto by_g = [&](auto np, auto fl, auto ta, auto cx) {
+    gon ? by_fast(np, fl, ta, cx, T{}) : by_fast(np, fl, ta, cx, F{});
+  };
+  auto by_kind = [&](auto np, auto fl) {
+    if (!tay)
+      by_g(np, fl, F{}, F{});
+    else
+      cplx ? by_g(np, fl, T{}, T{}) : by_g(np, fl, T{}, F{});
+  };
+  if (NP == 1)
+    by_kind(std::integral_constant<int, 1>{}, F{});
+  else if (NP == 6)
+    by_kind(std::integral_constant<int, 6>{}, F{});
+  else if (flat)
+    by_kind(std::integral_constant<int, 3>{}, T{});
+  else
+    by_kind(std::integral_constant<int, 3>{}, F{});
+}
+
+}  // namespace
+
+int sweep_block_size(int NP, bool gon) { return sweep_block(NP, gon); }
+
+StreamPlan sweep_plan(const RuleSet& rs, bool flat, int slots) {
+  StreamPlan pl;
+  pl.flat = flat;
+  pl.waves = kSweepWaves;
+  pl.tab_doubles = stream_tab_doubles(rs, flat);
+  pl.mids = uses_mid_rules(rs.R, rs.pk);
+  const int sd = sweep_slot_doubles(rs.pk);
+  auto bytes = [&](int S) {
+    return layout_of(S, sd, pl.tab_doubles, kSweepWaves, 0, pl.mids).total * 8L;
+  };
+  while (pl.S < 120 && bytes(pl.S + 1) <= kLdsBytes) ++pl.S;
+  if (slots > 0) pl.S = std::min(pl.S, slots);
+  pl.shmem = (size_t)bytes(pl.S);
+  return pl;
+}
+
+void launch_sweep(const StreamInst& in, const SweepArgs& sw, const StreamPlan& pl,
+                  const double* d_tab, unsigned* d_counters, int* d_slow, int cus, bool fast,
+                  bool prepare_only, hipStream_t s) {
+  const bool gon = (in.a.flags & BIE_G) != 0, tay = sw.taylor != 0, cplx = sw.k_im != 0.0;
+  const int KB = sweep_block(in.a.NP, gon);
+  const int64_t tiles =
+      (int64_t)((sw.nk + KB - 1) / KB) * in.n_segments * (int64_t)in.n_rowblocks;
+  BIE_REQUIRE(tiles > 0 && tiles < 2147483647LL, BIE_EINVAL, "too many sweep tiles");
+  BIE_REQUIRE(pl.S > 0 && pl.shmem <= (size_t)kLdsBytes, BIE_EINVAL,
+              "internal: sweep kernel without LDS slots");
+  const StreamRun run{d_tab, d_counters, d_slow, pl.tab_doubles, pl.S, 0, pl.mids ? 1 : 0};
+  for (int pass = 0; pass < (fast ? 1 : 2); ++pass)
+    with_sweep_kernel(in.a.NP, pl.flat, tay, cplx, gon, pass == 0, [&](auto kern, auto mid) {
+      BIE_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        (int)pl.shmem));
+      if (prepare_only) return;
+      hipLaunchKernelGGL(kern, dim3((unsigned)std::min<int64_t>(tiles, cus)),
+                         dim3(64 * kSweepWaves), pl.shmem, s, in, sw, (int)tiles, run);
+      if (pl.mids && pass == (fast ? 0 : 1))
+        hipLaunchKernelGGL(mid, dim3(512, (unsigned)std::min(sw.nk, 1024)), dim3(256),
+                           sizeof(double) *
+                               (size_t)(pl.tab_doubles - in.mid_off + kTrigDoubles + kExpN),
+                           s, in, sw, d_tab, pl.tab_doubles);
+    });
+  BIE_HIP_CHECK(hipGetLastError());
 }
 
 }  // namespace bie

@@ -1,0 +1,113 @@
+"""The dense, sweep and derivative kernels where their work splits: rule lengths around the
+points taken at a time and the rows staged, odd lengths, partial blocks of wavenumbers and
+orders, spaced and scattered wavenumbers, tiles left to the launch for large arguments, and
+tiles with more mid-edge pairs than they queue."""
+import numpy as np
+import pytest
+
+import oracle
+from bie_amd import mesh as M
+from bie_amd.assembly import DeviceMesh, assemble_parallel
+from bie_amd.taylor import taylor_assemble
+from gpu_helpers import TOL, DevBuf, rel, sync
+
+pytestmark = pytest.mark.gpu
+
+
+def sweep(mesh, ks, targets, n, m, gOn=True):
+    dm = DeviceMesh(mesh)
+    N, Mt, nk = mesh.n_sources, targets.shape[1], len(ks)
+    kb, tb = DevBuf(8 * nk), DevBuf(24 * Mt)
+    kb.upload(np.asarray(ks, dtype=np.float64))
+    tb.upload(np.ascontiguousarray(targets.T))
+    F, G, C = DevBuf(16 * Mt * N * nk), DevBuf(16 * Mt * N * nk), DevBuf(16 * Mt)
+    dm.assemble_sweep(kb.ptr, nk, F.ptr, G.ptr, Mt * N, C.ptr, targets_ptr=tb.ptr, n_targets=Mt,
+                      n=n, m=m, gOn=gOn)
+    sync()
+    out = [b.download(np.empty(s, dtype=np.complex128)) for b, s in
+           ((F, (nk, N, Mt)), (G, (nk, N, Mt)), (C, (Mt,)))]
+    return out[0].transpose(0, 2, 1), out[1].transpose(0, 2, 1), out[2]
+
+
+def some_targets(mesh, count, seed=3):
+    """Mesh nodes and field points, not a multiple of a tile's rows."""
+    rng = np.random.default_rng(seed)
+    x = 1.5 * rng.standard_normal((3, count))
+    x[:, ::2] = mesh.sources[:, rng.integers(0, mesh.n_sources, x[:, ::2].shape[1])]
+    return np.asfortranarray(x)
+
+
+@pytest.mark.parametrize("kind", ["linear", "quadratic"])
+@pytest.mark.parametrize("nm", [(1, 1), (2, 1), (3, 1), (3, 3), (4, 4), (5, 5)])
+def test_rule_lengths(kind, nm):
+    mesh = M.perturb_radial(M.icosphere(3 if kind == "linear" else 2, kind), 0.02, 4)
+    n, m = nm
+    t = some_targets(mesh, 75)
+    for k in (3.0, 2.0 + 0.4j):
+        Fo, Go, Co = oracle.assemble(mesh, k, targets=t, n=n, m=m)
+        F, G, C = assemble_parallel(mesh, k, t, n=n, m=m)
+        assert rel(F, Fo) <= TOL and rel(G, Go) <= TOL and rel(C, Co) <= TOL, k
+
+
+@pytest.mark.parametrize("kind", ["linear", "quadratic"])
+@pytest.mark.parametrize("nk,spaced", [(1, True), (5, True), (7, False), (9, True), (12, False)])
+def test_sweep_blocks(kind, nk, spaced):
+    """Partial last blocks, with and without G."""
+    mesh = M.icosphere(3 if kind == "linear" else 2, kind)
+    t = some_targets(mesh, 67)
+    ks = np.linspace(0.5, 7.0, nk) if spaced else np.sort(
+        np.random.default_rng(nk).uniform(0.5, 7.0, nk))
+    F, G, C = sweep(mesh, ks, t, 3, 3)
+    Fx, _, Cx = sweep(mesh, ks, t, 3, 3, gOn=False)
+    for q, k in enumerate(ks):
+        Fo, Go, Co = oracle.assemble(mesh, k, targets=t, n=3, m=3)
+        assert rel(F[q], Fo) <= TOL and rel(G[q], Go) <= TOL and rel(Fx[q], Fo) <= TOL, q
+    assert rel(C, Co) <= TOL and rel(Cx, Co) <= TOL
+
+
+@pytest.mark.parametrize("kind", ["linear", "quadratic"])
+@pytest.mark.parametrize("orders", [1, 4, 6, 12, 13])
+def test_derivative_blocks(kind, orders):
+    """Orders in full, half and partial blocks, with and without G, real and complex k."""
+    mesh = M.icosphere(2 if kind == "linear" else 1, kind)
+    t = some_targets(mesh, 67)
+    for k in (2.5, 2.0 + 0.3j):
+        F, G, _ = taylor_assemble(mesh, k, t, M=orders - 1, n=3, m=3)
+        Fx = taylor_assemble(mesh, k, t, M=orders - 1, n=3, m=3, gOn=False)[0]
+        for q in range(orders):
+            Fo, Go = oracle.assemble_taylor(mesh, k, q, targets=t, n=3, m=3)
+            assert rel(F[:, :, q], Fo) <= TOL and rel(G[:, :, q], Go) <= TOL, q
+            assert rel(Fx[:, :, q], Fo) <= TOL, q
+
+
+@pytest.mark.parametrize("kind", ["linear", "quadratic"])
+def test_tiles_with_a_far_target(kind):
+    """One target so far off that its |k| r leaves the range of the branch-free sincos: its
+    tile's other rows come from the launch for large arguments."""
+    mesh = M.icosphere(3 if kind == "linear" else 2, kind)
+    t = some_targets(mesh, 150)
+    t[:, 70] = (0.0, 3e14, 0.0)
+    near = np.arange(150) != 70
+    Fo, Go, Co = oracle.assemble(mesh, 3.0, targets=t, n=3, m=3)
+    F, G, C = assemble_parallel(mesh, 3.0, t, n=3, m=3)
+    Fs, Gs, Cs = sweep(mesh, [3.0, 3.5], t, 3, 3)
+    for X, Xo in ((F, Fo), (Fs[0], Fo), (G, Go), (Gs[0], Go)):
+        assert rel(X[near], Xo[near]) <= TOL
+        assert np.max(np.abs(X[70])) <= np.max(np.abs(Xo[70])) * (1 + 1e-9)
+    assert rel(C[near], Co[near]) <= TOL and rel(Cs[near], Co[near]) <= TOL
+
+
+def test_more_mid_edge_pairs_than_a_tile_queues():
+    """Targets about the centre: every node is about as far, so a good part of all pairs has a
+    mid-edge rule."""
+    mesh = M.icosphere(4, "quadratic")
+    t = np.asfortranarray(1e-2 * np.random.default_rng(8).standard_normal((3, 130)))
+    for k in (2.0, 2.0 + 0.3j):
+        Fo, Go, Co = oracle.assemble(mesh, k, targets=t, n=3, m=2)
+        F, G, C = assemble_parallel(mesh, k, t, n=3, m=2)
+        assert rel(F, Fo) <= TOL and rel(G, Go) <= TOL and rel(C, Co) <= TOL
+    Fo, Go, Co = oracle.assemble(mesh, 2.0, targets=t, n=3, m=2)
+    F, G, C = sweep(mesh, [2.0, 3.0], t, 3, 2)
+    assert rel(F[0], Fo) <= TOL and rel(G[0], Go) <= TOL and rel(C, Co) <= TOL
+    F, G, C = taylor_assemble(mesh, 2.0, t, M=1, n=3, m=2)
+    assert rel(F[:, :, 0], Fo) <= TOL and rel(G[:, :, 0], Go) <= TOL

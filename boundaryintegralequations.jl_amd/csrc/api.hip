@@ -301,6 +301,22 @@ bie_dmesh::Stream& ensure_stream(bie_dmesh* dm, int S, int64_t rowblocks, int cu
   return out;
 }
 
+// Records of flat elements in element order (written once: the coordinates do not change).
+void ensure_flat(bie_dmesh* dm, hipStream_t s) {
+  if (dm->d_eflat) return;
+  double* rec = dalloc<double>((size_t)dm->E * kFlatDoubles);
+  StreamPrep p{};
+  p.E = (int)dm->E;
+  p.coords = dm->d_coords;
+  p.sources = dm->d_sources;
+  p.topo = dm->d_topo;
+  p.ptopo = dm->d_ptopo;
+  p.flat = rec;
+  launch_stream_flat(p, s);
+  BIE_HIP_CHECK(hipStreamSynchronize(s));
+  dm->d_eflat = rec;
+}
+
 // The schedule of dm in a batch: S slots, at least `segments` segments.  The records of flat
 // elements are written here, once (a single-mesh call writes its own each time).
 bie_dmesh::Stream& ensure_batch_stream(bie_dmesh* dm, int S, int64_t segments, hipStream_t s) {
@@ -850,19 +866,30 @@ void batch_dfdk_impl(bie_batch* b, const double* k_re, const double* k_im,
   std::lock_guard<std::mutex> bl(b->mu);
   MeshLocks locks(b->meshes);
   std::vector<DfdkInst> h(n_inst);
-  std::vector<int4> tiles;
-  constexpr int ech = 64;  // elements per tile
+  bie_dmesh* d0 = b->meshes[0];
+  const bool flat = flat_elements(d0);
+  const int cus = device_cus(b->device);
+  // elements per tile: some sixteen tiles for each of the 16 waves of a CU
+  int64_t work = 0;
+  for (const bie_dmesh* dm : b->meshes) work += (dm->N + 63) / 64 * dm->E;
+  const int64_t ech = std::min<int64_t>(1024, std::max<int64_t>(16, work / (256LL * cus)));
+  int64_t tiles = 0;
+  bool cplx = false, some_fast = false, some_slow = false;
   for (int ii = 0; ii < n_inst; ++ii) {
     bie_dmesh* dm = b->meshes[ii];
     order_after_previous(dm, s);
     ensure_rules(dm, b->n, b->m, s);
-    if (!dm->geom_valid) refresh_geometry(dm, s);
+    if (flat)
+      ensure_flat(dm, s);
+    else if (!dm->geom_valid)
+      refresh_geometry(dm, s);
     DfdkInst& a = h[ii];
     a = DfdkInst{};
     a.targets = dm->d_sources;
     a.M = dm->N;
     a.E = (int)dm->E;
     a.Pe = dm->rs.Pe;
+    a.flat = dm->d_eflat;
     a.elem = dm->d_elem;
     a.selnodes = dm->d_selnodes;
     a.ptopo = dm->d_ptopo;
@@ -879,31 +906,29 @@ void batch_dfdk_impl(bie_batch* b, const double* k_re, const double* k_im,
     a.alpha = reinterpret_cast<const double2*>(d_alpha[ii]);
     a.p = reinterpret_cast<const double2*>(d_p[ii]);
     a.w = d_w + 2 * (size_t)ii;
-    const int64_t rbs = (dm->N + 255) / 256, chunks = (dm->E + ech - 1) / ech;
-    for (int64_t rb = 0; rb < rbs; ++rb)
-      for (int64_t ch = 0; ch < chunks; ++ch) tiles.push_back(make_int4(ii, (int)rb, (int)ch, 0));
+    a.fast = fast_trig_ok(dm, a.kr, dm->source_radius) ? 1 : 0;
+    cplx = cplx || a.ki != 0.0;
+    (a.fast ? some_fast : some_slow) = true;
+    a.first_tile = (int)std::min<int64_t>(tiles, INT32_MAX);
+    tiles += (dm->N + 63) / 64 * ((dm->E + ech - 1) / ech);
   }
-  BIE_REQUIRE(tiles.size() < (size_t)INT32_MAX, BIE_EINVAL, "batch has too many tiles");
+  BIE_REQUIRE(tiles < INT32_MAX, BIE_EINVAL, "batch has too many tiles");
+  const int tab = stream_tab_doubles(d0->rs, flat);
   DfdkInst* d_inst = dalloc<DfdkInst>(h.size());
-  int4* d_tiles = nullptr;
   try {
-    d_tiles = dalloc<int4>(tiles.size());
     BIE_HIP_CHECK(hipMemcpyAsync(d_inst, h.data(), sizeof(DfdkInst) * h.size(),
                                  hipMemcpyHostToDevice, s));
-    if (!tiles.empty())
-      BIE_HIP_CHECK(hipMemcpyAsync(d_tiles, tiles.data(), sizeof(int4) * tiles.size(),
-                                   hipMemcpyHostToDevice, s));
     launch_fill_zero(d_w, 2 * (int64_t)n_inst, s);
-    launch_dfdk_batch(d_inst, d_tiles, (int)tiles.size(), ech, b->pk, s);
-    // the per-call tables are freed once the launch has read them
+    launch_dfdk_batch(d_inst, n_inst, (int)tiles, (int)ech, b->pk, flat, cplx, some_fast,
+                      some_slow, flat ? d0->d_stab : d0->d_phi,
+                      flat ? tab : (int)d0->rs.phi.size(), d0->d_stab + tab, cus, s);
+    // the per-call table is freed once the launch has read it
     BIE_HIP_CHECK(hipStreamSynchronize(s));
   } catch (...) {
     dfree(d_inst);
-    dfree(d_tiles);
     throw;
   }
   dfree(d_inst);
-  dfree(d_tiles);
   for (bie_dmesh* dm : b->meshes) mark_done(dm, s);
 }
 
@@ -1020,6 +1045,7 @@ int bie_dmesh_destroy(bie_dmesh* dm) {
   dfree(dm->d_phi);
   dfree(dm->d_elem);
   dfree(dm->d_stab);
+  dfree(dm->d_eflat);
   free_stream(dm->stream);
   free_stream(dm->bstream);
   free_stream(dm->sstream);
@@ -1891,8 +1917,10 @@ void assembly_vjp_impl(bie_dmesh* dm, double k, double ki, bool cplx, const doub
   BIE_REQUIRE(std::isfinite(k) && std::isfinite(ki), BIE_EINVAL, "k must be finite");
   BIE_REQUIRE(!physics_discontinuous(dm->pkind) && !kind_is_quad(dm->gkind), BIE_EUNSUPPORTED,
               "assembly adjoint: continuous physics on triangles only");
+  double target_radius = -1.0;
   if (!d_targets) {
     d_targets = dm->d_sources;
+    target_radius = dm->source_radius;
     BIE_REQUIRE(n_targets == dm->N, BIE_EINVAL, "collocation needs n_targets == n_sources");
   }
   std::lock_guard<std::mutex> lk(dm->mu);
@@ -1922,9 +1950,13 @@ void assembly_vjp_impl(bie_dmesh* dm, double k, double ki, bool cplx, const doub
   a.hyp = dm->hyp;
   a.k = k;
   a.ki = ki;
+  for (int d = 0; d < 3; ++d) a.center[d] = dm->center[d];
+  a.reach = 4.0 * dm->coord_radius;
   a.gradX = d_grad_coords;
   a.gradk = d_grad_k;
-  launch_adjoint(a, dm->gk, dm->pk, cplx, s);
+  const bool flat = flat_elements(dm);
+  launch_adjoint(a, dm->gk, dm->pk, flat, cplx, fast_trig_ok(dm, k, target_radius), dm->d_stab,
+                 stream_tab_doubles(dm->rs, flat), device_cus(dm->device), s);
   mark_done(dm, s);
 }
 

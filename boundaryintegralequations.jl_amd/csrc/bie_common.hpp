@@ -250,6 +250,7 @@ struct AdjointArgs {
   int hyp;                 // rule-selection distance (as AssemblyArgs::hyp)
   double k;               // Re k
   double ki;              // Im k (complex-k entry point; 0 for real k)
+  double center[3], reach; // every element point is within reach of the centre
   double* gradX;           // 3 x Nc, accumulated
   double* gradk;           // d/dRe k (and d/dIm k after it for complex k), accumulated, or NULL
 };
@@ -260,6 +261,9 @@ struct DfdkInst {
   int64_t M;
   int E;
   int Pe;
+  int first_tile;          // of the instance's (row block, element chunk) tiles
+  int fast;                // every |k| r is below the fast sincos bound
+  const double* flat;      // E x kFlatDoubles records of flat elements, or NULL
   const double* elem;      // element tables of the assembly (E x Pe x 8)
   const double* selnodes;  // E x NP x 4
   const int* ptopo;        // E x NP
@@ -351,9 +355,14 @@ constexpr int64_t kApplyScratchComplex = int64_t(1) << 20;
 void zgemm_device_noalloc(int64_t M, int64_t nrhs, int64_t K, const double* dA, int64_t lda,
                           const double* dX, int64_t ldx, double* dY, int64_t ldy,
                           hipStream_t s);
-void launch_adjoint(const AdjointArgs& a, int gk, int pk, bool cplx, hipStream_t s);
-// tiles: (instance, 256-row block, chunk of ech elements)
-void launch_dfdk_batch(const DfdkInst* d_inst, const int4* d_tiles, int n_tiles, int ech, int NP,
+// d_tab: stream_tables (flat elements); fast: every |k| r is below the fast sincos bound
+void launch_adjoint(const AdjointArgs& a, int gk, int pk, bool flat, bool cplx, bool fast,
+                    const double* d_tab, int tab_doubles, int cus, hipStream_t s);
+// tiles: (64-row block, chunk of ech elements) of every instance, rows fastest; d_basis: flat
+// table or basis values, d_trig: (cos, sin) and 2^(j/64) tables
+void launch_dfdk_batch(const DfdkInst* d_inst, int n_inst, int n_tiles, int ech, int NP,
+                       bool flat, bool cplx, bool some_fast, bool some_slow,
+                       const double* d_basis, int n_basis, const double* d_trig, int cus,
                        hipStream_t s);
 // Solves on the device (solve.hip)
 void lu_factor_device(int64_t n, double* dA, int64_t lda, const double* dC, int32_t* d_ipiv,
@@ -411,6 +420,7 @@ struct bie_dmesh {
     int* d_zero_cols = nullptr;
     std::vector<int> h_seg_begin;  // (batch) host copy, for the tile list
   };
+  double* d_eflat = nullptr;     // records of flat elements in element order (k-derivatives)
   // of single-mesh calls, of batches, of sweeps and k-derivatives
   Stream stream, bstream, sstream;
   bie::StreamLists lists, blists, slists;

@@ -522,10 +522,10 @@ __device__ __forceinline__ void geometry_point(const StreamPrep& p, int64_t t) {
       make_double4(-c1 / J, -c2 / J, J * P[2] * 0.079577471545947667884, 0.0);
 }
 
-// The record of one flat element at its position in the stream: selection nodes, X1, the
+// The record of one flat element at its position in the stream (order NULL: its number): selection nodes, X1, the
 // edges a, b from it, n J = -(a x b), J.
 __device__ __forceinline__ void flat_record(const StreamPrep& p, int t) {
-  const int e = p.order[t];
+  const int e = p.order ? p.order[t] : t;
   double* o = p.flat + (size_t)t * kFlatDoubles;
   double X[3][3];
 #pragma unroll

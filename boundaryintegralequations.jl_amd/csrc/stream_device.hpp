@@ -1,6 +1,7 @@
 // Device parts of the barrier-free slot kernels (stream.hip: one wavenumber, sweep.hip: many):
 // e^{ikr}, rule selection, the LDS of a workgroup, the hand-over of node sums between waves,
-// mid-edge pairs and the tile loop.  Included by those two files only.
+// mid-edge pairs and the tile loop.  The first two serve the derivative kernels (adjoint.hip)
+// as well.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -200,12 +201,12 @@ struct Sums {  // an element's node sums of one row
   }
 };
 
-// Rule of a pair as select_rule, from the element's NP selection nodes (scalar registers; at
-// Pm in memory for the exact comparison of near ties).
-template <int NP>
-__device__ __forceinline__ int select_rule_s(double x0, double x1, double x2,
-                                             const double (&P)[NP][3], const double* Pm, int R,
-                                             InstPtr in) {
+// Rule of a pair as select_rule, from the element's NP selection nodes P; node(s, d) gives a
+// coordinate for the exact comparison of near ties, hyp_of() its kind.
+template <int NP, class Node, class HypOf>
+__device__ __forceinline__ int select_rule_p(double x0, double x1, double x2,
+                                             const double (&P)[NP][3], Node node, int R,
+                                             HypOf hyp_of) {
   double d2v_[NP];
 #pragma unroll
   for (int s = 0; s < NP; ++s) {
@@ -232,11 +233,10 @@ __device__ __forceinline__ int select_rule_s(double x0, double x1, double x2,
   if (lane_of_mask(two)) {
     double best = INFINITY;
     c = 0;
-    const int hyp = fresh(in)->a.hyp;
+    const int hyp = hyp_of();
 #pragma unroll 1
     for (int s = 0; s < NP; ++s) {
-      const double dx = sload(Pm + 3 * s) - x0, dy = sload(Pm + 3 * s + 1) - x1,
-                   dz = sload(Pm + 3 * s + 2) - x2;
+      const double dx = node(s, 0) - x0, dy = node(s, 1) - x1, dz = node(s, 2) - x2;
       const double d = hyp ? scaled_hypot3_inline(dx, dy, dz) : julia_hypot3_inline(dx, dy, dz);
       if (d < best) {
         best = d;
@@ -246,6 +246,16 @@ __device__ __forceinline__ int select_rule_s(double x0, double x1, double x2,
   }
   if (c < 1 || c > R) c = R;
   return c;
+}
+
+// The same with the nodes in scalar registers and at Pm in memory.
+template <int NP>
+__device__ __forceinline__ int select_rule_s(double x0, double x1, double x2,
+                                             const double (&P)[NP][3], const double* Pm, int R,
+                                             InstPtr in) {
+  return select_rule_p<NP>(
+      x0, x1, x2, P, [&](int s, int d) { return sload(Pm + 3 * s + d); }, R,
+      [&] { return fresh(in)->a.hyp; });
 }
 
 // ---- LDS of a workgroup ------------------------------------------------------------------

@@ -111,3 +111,59 @@ def test_more_mid_edge_pairs_than_a_tile_queues():
     assert rel(F[0], Fo) <= TOL and rel(G[0], Go) <= TOL and rel(C, Co) <= TOL
     F, G, C = taylor_assemble(mesh, 2.0, t, M=1, n=3, m=2)
     assert rel(F[:, :, 0], Fo) <= TOL and rel(G[:, :, 0], Go) <= TOL
+
+
+@pytest.mark.parametrize("f,nm,k", [(2, (1, 1), 3.0), (4, (3, 1), 2.0 + 0.3j), (5, (2, 2), 4.0),
+                                    (5, (3, 3), 3.0 + 0.2j)])
+def test_flat_adjoint_sizes(f, nm, k):
+    """Elements short of a workgroup's 256 and past it, one point and odd lengths; targets
+    given as points attached to nodes, one more so far off that its row is the other
+    launch's (weight 0: finite there, nothing added)."""
+    from bie_amd.adjoint import assembly_vjp, source_nodes
+    from dual_oracle import assemble_F_C
+    mesh = M.perturb_radial(M.icosphere(f, "linear"), 0.01, 4)
+    n, m = nm
+    rng = np.random.default_rng(f)
+    N = mesh.n_sources
+    alpha, beta, p = (rng.standard_normal(N) + 1j * rng.standard_normal(N) for _ in range(3))
+    t = np.asfortranarray(np.concatenate([mesh.sources, [[0.0], [3e14], [0.0]]], axis=1))
+    node = np.append(source_nodes(mesh), -1).astype(np.int32)
+    dm = DeviceMesh(mesh)
+    g, gk = assembly_vjp(dm, k, alpha, p, beta=beta, target_node=source_nodes(mesh), n=n, m=m)
+    g2, gk2 = assembly_vjp(dm, k, np.append(alpha, 0.0), p, beta=np.append(beta, 0.0), targets=t,
+                           target_node=node, n=n, m=m)
+    assert rel(g2, g) <= 1e-12 and rel(np.atleast_1d(gk2), np.atleast_1d(gk)) <= 1e-12
+    V = rng.standard_normal(mesh.coordinates.shape)
+    rules = oracle.select(mesh, None)
+    F, C = assemble_F_C(mesh, mesh.coordinates, V, k, 0.0, rules, targets=None, n=n, m=m)
+    dd = np.real(alpha @ (F.d @ p) + beta @ C.d)
+    assert abs(float(np.sum(g * V)) - dd) <= 1e-10 * abs(dd)
+
+
+@pytest.mark.parametrize("kind", ["linear", "quadratic"])
+@pytest.mark.parametrize("nm", [(1, 1), (3, 1), (3, 3), (5, 5)])
+def test_batched_k_derivative(kind, nm):
+    """Real and complex wavenumbers side by side, and one instance whose |k| r leaves the range
+    of the branch-free sincos."""
+    from bie_amd.assembly import Batch
+    meshes = [M.icosphere(f, kind) for f in ((1, 2, 4) if kind == "linear" else (1, 2, 2))]
+    ks = [3.0, 2.0 + 0.4j, 1e14]
+    n, m = nm
+    rng = np.random.default_rng(6)
+    al, ps, w = [], [], DevBuf(16 * 3)
+    for x in meshes:
+        for out in (al, ps):
+            v = rng.standard_normal(x.n_sources) + 1j * rng.standard_normal(x.n_sources)
+            buf = DevBuf(16 * x.n_sources)
+            buf.upload(v)
+            out.append((v, buf))
+    dms = [DeviceMesh(x) for x in meshes]
+    b = Batch(dms, n=n, m=m)
+    b.dfdk(ks, [x[1].ptr for x in al], [x[1].ptr for x in ps], w.ptr)
+    got = w.download(np.empty(3, dtype=np.complex128))
+    assert np.isfinite(got).all()
+    for i in range(2):
+        D = oracle.assemble_taylor(meshes[i], ks[i], 1, n=n, m=m)[0]
+        ref = al[i][0] @ (D @ ps[i][0])
+        scale = np.abs(al[i][0]) @ (np.abs(D) @ np.abs(ps[i][0]))
+        assert abs(got[i] - ref) <= 1e-12 * scale, i

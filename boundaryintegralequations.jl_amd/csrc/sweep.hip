@@ -496,6 +496,8 @@ __device__ __forceinline__ void sweep_tile(InstPtr in, SweepPtr sw, int rb, int 
   while (pos < t1) {
     const int nxt = draw();
     const InstPtr u = fresh(in);
+    const int l = fresh_lane(lane);
+    const int4 en = u->ent[(size_t)pos * NP + min(l, NP - 1)];
     Multi<NP, KB, GON> v;
     if constexpr (FLAT) {
       const double* rec24 = u->flat + (size_t)pos * kFlatDoubles;
@@ -573,8 +575,6 @@ __device__ __forceinline__ void sweep_tile(InstPtr in, SweepPtr sw, int rb, int 
       }
       csum += cs_pair;
     }
-    const int l = fresh_lane(lane);
-    const int4 en = fresh(in)->ent[(size_t)pos * NP + min(l, NP - 1)];
     bool ok;
     const Roles r = claim<NP>(en, l, claims, turns, ok);
     give_multi<NP, KB, GON>(en, r, l, acc, claims, v, nb, ok);

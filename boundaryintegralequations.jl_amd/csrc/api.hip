@@ -1338,7 +1338,7 @@ struct bie_sparse {
   // pairs would share
   int* d_batches = nullptr;
   int64_t n_batches = 0;
-  double* d_trig = nullptr;  // the sincos table of the kernels (kTrigDoubles)
+  double* d_trig = nullptr;  // tables of the kernels (kTrigDoubles + kExpN)
   // the one rule of the partial assembly (gauss_points_triangle(partial_n)), built on demand
   double* d_partial = nullptr;
   int partial_n = -1, partial_len = 0;
@@ -1519,12 +1519,13 @@ bie_sparse* sparse_create_impl(bie_dmesh* dm, int depth, double offset, int n_ga
   sp->d_gsel = upload_vec(gsel, nullptr);
   sp->d_rules = upload_vec(rec, nullptr);
   {
-    std::vector<double> trig(kTrigDoubles);
+    std::vector<double> trig(kTrigDoubles + kExpN);
     for (int j = 0; j < kTrigN; ++j) {  // (cos, sin)(j pi / 64), rounded from long double
       const long double th = (long double)j * (3.14159265358979323846264338327950288L / 64);
       trig[2 * j] = (double)cosl(th);
       trig[2 * j + 1] = (double)sinl(th);
     }
+    for (int j = 0; j < kExpN; ++j) trig[kTrigDoubles + j] = (double)exp2l((long double)j / kExpN);
     sp->d_trig = upload_vec(trig, nullptr);
   }
   // share only where it pays: on average at least 1.5 pairs per batch (the batched kernel
@@ -1560,6 +1561,8 @@ void sparse_assemble_impl(bie_sparse* sp, double kr, double ki, const double* d_
   L.gsel = sp->d_gsel;
   L.rules = sp->d_rules;
   L.trig = sp->d_trig;
+  // (the radius of explicit sources is not known here)
+  L.fast = fast_trig_ok(dm, kr, d_sources ? -1.0 : dm->source_radius);
   L.batches = sp->d_batches;
   L.n_batches = sp->n_batches;
   for (int c = 0; c < 6; ++c) {
@@ -1626,6 +1629,8 @@ void sparse_partial_impl(bie_sparse* sp, double kr, double ki, int n_gauss,
   L.gsel = sp->d_gsel;
   L.rules = sp->d_partial;
   L.trig = sp->d_trig;
+  // (the radius of explicit sources is not known here)
+  L.fast = fast_trig_ok(dm, kr, d_sources ? -1.0 : dm->source_radius);
   for (int c = 0; c < 6; ++c) {  // whatever the selection, the one rule
     L.off[c] = 0;
     L.len[c] = sp->partial_len;

@@ -13,9 +13,14 @@
 //   greens3d!, kernels.jl:13-37) and the physics basis at the rule points; the results add
 //   into the row's entries of the element's physics nodes.
 //
-// One wave per (row, element) pair: lanes take the rule's points (a few thousand), the
-// partial sums are reduced across the wave and added into the entries with FP64 atomics
-// (a row's entries receive several elements' contributions).
+// One wave per (row, element) pair or per batch of pairs that share an element: lanes take the
+// rule's points (a few thousand), the partial sums are reduced across the wave and added into
+// the entries with FP64 atomics (a row's entries receive several elements' contributions).
+// Bound by instruction issue (VALU busy 85 % of the time): curved elements cost 290 per point
+// and pair, of which the surface with its exactly rounded normal is 200; flat ones 80.  Before
+// and after the cheaper exact divisions, the normal of flat elements taken out of the loop and
+// the branch-free sincos, 40-point rules (us): 10242 nodes, depth 1: 2350 -> 1737; depth 2,
+// quadratic 4002 nodes 5359 -> 2992, linear 1962 nodes 712 -> 622.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -27,6 +32,7 @@
 #include "bie_common.hpp"
 #include "device_common.hpp"
 #include "kernels_math.hpp"
+#include "stream_device.hpp"
 
 namespace bie {
 namespace {
@@ -44,7 +50,7 @@ struct SparseArgs {
   const int* topo;        // E x NG
   const double* gsel;     // E x NG x 4 geometry node coordinates (selection)
   const double* rules;    // point records (kSparseRec doubles)
-  const double2* trig;    // (cos, sin)(j pi / 64), j < kTrigN
+  const double* trig;     // (cos, sin)(j pi / 64), j < kTrigN, then 2^(j / 64), j < kExpN
   int off[6], len[6];
   const int* batches;     // 8 ints per batch: element, count, up to 4 pair indices
   int64_t n_batches;
@@ -135,125 +141,187 @@ __device__ __forceinline__ void sparse_phys_basis(bool disc, double beta, double
   }
 }
 
-struct SparseGeom {
-  double dx, dy, dz, nd, J;
+// A divisor's reciprocal (estimate refined by two Newton steps) and the quotient from it: the
+// residual a - b q is exact, so the correction leaves the correctly rounded a / b (Markstein's
+// theorem), the same as the division the oracle performs, at three instructions for each
+// further quotient of one divisor.  For divisors and quotients well inside the range.
+__device__ __forceinline__ double recip_for_quot(double b) {
+  double y = __builtin_amdgcn_rcp(b);
+  y = fma(fma(-b, y, 1.0), y, y);
+  return fma(fma(-b, y, 1.0), y, y);
+}
+__device__ __forceinline__ double quot(double a, double b, double y) {
+  const double q = a * y;
+  return fma(fma(-b, q, a), y, q);
+}
+// sqrt(s), correctly rounded, for s in [1, 3].
+__device__ __forceinline__ double sqrt_1_3(double s) {
+  const double y = __builtin_amdgcn_rsq(s);
+  double g = s * y, h = 0.5 * y;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  g = fma(fma(-g, g, s), h, g);
+  return fma(fma(-g, g, s), h, g);
+}
+
+// J = hypot(c) and the reference's normal n = -c / J: every operation of julia_hypot3 and of
+// the three divisions, rounded as they round (six divisions and a square root written out were
+// 80 instructions of the 370 of a point; these are 40).  Out of the middle of the range (and
+// for infinities, NaN and zero) the operations themselves.
+__device__ __forceinline__ void sparse_normal(double c0, double c1, double c2, double (&n)[3],
+                                              double& J) {
+#pragma clang fp contract(off)
+  const double ax = fabs(c0), ay = fabs(c1), az = fabs(c2);
+  double mx = ax > ay ? ax : ay;
+  mx = mx > az ? mx : az;
+  if (mx > 0x1p-300 && mx < 0x1p300) {
+    const double y = recip_for_quot(mx);
+    const double a = quot(ax, mx, y), b = quot(ay, mx, y), c = quot(az, mx, y);
+    double s = a * a;
+    s = s + b * b;
+    s = s + c * c;
+    J = mx * sqrt_1_3(s);
+    const double z = recip_for_quot(J);
+    n[0] = quot(-c0, J, z);
+    n[1] = quot(-c1, J, z);
+    n[2] = quot(-c2, J, z);
+  } else {
+    J = julia_hypot3(c0, c1, c2);
+    n[0] = -c0 / J;
+    n[1] = -c1 / J;
+    n[2] = -c2 / J;
+  }
+}
+
+// The surface of an element in the oracle's operation order without fused multiply-adds.  On
+// the elements around the source node n.d is rounding noise (a flat element contains its own
+// node) divided by r^3 at cells ~1e-6 of the element: only geometry that rounds as the CPU
+// restatement's does reproduces that noise.  Left out are additions of zero only (the leading
+// 0 + and the nodes whose derivative is zero).  On flat elements t_u, t_v, n and J do not
+// depend on the point: they are formed once.
+template <int NG>
+struct Surface {
+  double X[NG][3], n[3], J;
+  __device__ __forceinline__ void begin() {
+#pragma clang fp contract(off)
+    if constexpr (NG == 3) {  // -X1 + X2, -X1 + X3
+      const double u0 = X[1][0] - X[0][0], u1 = X[1][1] - X[0][1], u2 = X[1][2] - X[0][2];
+      const double v0 = X[2][0] - X[0][0], v1 = X[2][1] - X[0][1], v2 = X[2][2] - X[0][2];
+      sparse_normal(u1 * v2 - u2 * v1, u2 * v0 - u0 * v2, u0 * v1 - u1 * v0, n, J);
+    }
+  }
+  // y (and on curved elements n, J) at a point from the bases there
+  __device__ __forceinline__ void at(const double (&N)[NG], const double (&Du)[NG],
+                                     const double (&Dv)[NG], double (&y)[3]) {
+#pragma clang fp contract(off)
+    double tu[3], tv[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      double a = X[0][d] * N[0];
+#pragma unroll
+      for (int g = 1; g < NG; ++g) a = a + X[g][d] * N[g];
+      y[d] = a;
+      if constexpr (NG == 6) {  // Du[2] = Dv[1] = 0
+        double b = X[0][d] * Du[0], c = X[0][d] * Dv[0];
+        b = b + X[1][d] * Du[1];
+        c = c + X[2][d] * Dv[2];
+#pragma unroll
+        for (int g = 3; g < 6; ++g) {
+          b = b + X[g][d] * Du[g];
+          c = c + X[g][d] * Dv[g];
+        }
+        tu[d] = b;
+        tv[d] = c;
+      }
+    }
+    if constexpr (NG == 6)
+      sparse_normal(tu[1] * tv[2] - tu[2] * tv[1], tu[2] * tv[0] - tu[0] * tv[2],
+                    tu[0] * tv[1] - tu[1] * tv[0], n, J);
+  }
 };
 
-// d = y - x, the reference's normal n = -(t_u x t_v)/J and J at one rule point, in the
-// oracle's operation order without fused multiply-adds.  On the elements around the source
-// node n.d is rounding noise (a flat element contains its own node) divided by r^3 at
-// cells ~1e-6 of the element: only bit-identical geometry reproduces that noise, so this
-// part is evaluated exactly as the CPU restatement does.
-template <int NG>
-__device__ __forceinline__ SparseGeom sparse_geometry(const double (&X)[NG][3],
-                                                      const double (&N)[NG],
-                                                      const double (&Du)[NG],
-                                                      const double (&Dv)[NG], double x0,
-                                                      double x1, double x2) {
+// The kernels at one rule point for a source x: G = e^{ikr} J w / (4 pi r) and
+// F = e^{ikr} (ikr - 1) (n.d) J w / (4 pi r^3) (freens3d!, greens3d!, kernels.jl:13-37), d = y - x
+// and n.d in the oracle's order.
+template <bool CPLX, bool FAST>
+__device__ __forceinline__ void sparse_point_kernels(const double (&y)[3], const double (&n)[3],
+                                                     double J, const double (&x)[3], double wq,
+                                                     double kr, double ki, const Trig& tr,
+                                                     double& Fr, double& Fi, double& Gr,
+                                                     double& Gi) {
+  double dx, dy, dz, nd;
+  {
 #pragma clang fp contract(off)
-  double y[3], tu[3], tv[3];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    double a = 0.0, b = 0.0, c = 0.0;
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      a = a + X[g][d] * N[g];
-      b = b + X[g][d] * Du[g];
-      c = c + X[g][d] * Dv[g];
-    }
-    y[d] = a;
-    tu[d] = b;
-    tv[d] = c;
+    dx = y[0] - x[0];
+    dy = y[1] - x[1];
+    dz = y[2] - x[2];
+    nd = n[0] * dx + n[1] * dy + n[2] * dz;
   }
-  const double c0 = tu[1] * tv[2] - tu[2] * tv[1], c1 = tu[2] * tv[0] - tu[0] * tv[2],
-               c2 = tu[0] * tv[1] - tu[1] * tv[0];
-  SparseGeom sg;
-  sg.J = julia_hypot3(c0, c1, c2);
-  sg.dx = y[0] - x0;
-  sg.dy = y[1] - x1;
-  sg.dz = y[2] - x2;
-  sg.nd = (-c0 / sg.J) * sg.dx + (-c1 / sg.J) * sg.dy + (-c2 / sg.J) * sg.dz;
-  return sg;
-}
-
-// The surface at one rule point without the source: y, the reference's normal
-// n = -(t_u x t_v) / J and J, operation for operation as sparse_geometry.
-template <int NG>
-__device__ __forceinline__ void sparse_surface(const double (&X)[NG][3], const double (&N)[NG],
-                                               const double (&Du)[NG], const double (&Dv)[NG],
-                                               double (&y)[3], double (&n)[3], double& J) {
-#pragma clang fp contract(off)
-  double tu[3], tv[3];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    double a = 0.0, b = 0.0, c = 0.0;
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      a = a + X[g][d] * N[g];
-      b = b + X[g][d] * Du[g];
-      c = c + X[g][d] * Dv[g];
-    }
-    y[d] = a;
-    tu[d] = b;
-    tv[d] = c;
-  }
-  const double c0 = tu[1] * tv[2] - tu[2] * tv[1], c1 = tu[2] * tv[0] - tu[0] * tv[2],
-               c2 = tu[0] * tv[1] - tu[1] * tv[0];
-  J = julia_hypot3(c0, c1, c2);
-  n[0] = -c0 / J;
-  n[1] = -c1 / J;
-  n[2] = -c2 / J;
-}
-
-// d = y - x and n.d for one source, in sparse_geometry's order.
-__device__ __forceinline__ SparseGeom sparse_toward(const double (&y)[3], const double (&n)[3],
-                                                    double J, double x0, double x1,
-                                                    double x2) {
-#pragma clang fp contract(off)
-  SparseGeom sg;
-  sg.J = J;
-  sg.dx = y[0] - x0;
-  sg.dy = y[1] - x1;
-  sg.dz = y[2] - x2;
-  sg.nd = n[0] * sg.dx + n[1] * sg.dy + n[2] * sg.dz;
-  return sg;
-}
-
-// The kernels at one rule point: G = e^{ikr} J w / (4 pi r) and
-// F = e^{ikr} (ikr - 1) (n.d) J w / (4 pi r^3) (freens3d!, greens3d!, kernels.jl:13-37).
-template <bool CPLX>
-__device__ __forceinline__ void sparse_point_kernels(const SparseArgs& a, const SparseGeom& sg,
-                                                     double wq, const double2* tab, double& Fr,
-                                                     double& Fi, double& Gr, double& Gi) {
-  const double dx = sg.dx, dy = sg.dy, dz = sg.dz, J = sg.J, nd = sg.nd;
   const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
   const double rinv = rsqrt_nr(r2);
   const double r = r2 * rinv;
-  const double g = J * wq * kInv4PiS * rinv;         // J w / (4 pi r)
-  const double ak = nd * rinv * rinv * g;             // (n.d) J w / (4 pi r^3)
-  double sn, cs;
-  sincos_tab(a.kr * r, tab, &sn, &cs);
-  if (CPLX) {
-    const double ex = exp(-a.ki * r);
-    cs *= ex;
-    sn *= ex;
-    const double ar = fma(-a.ki, r, -1.0), ai = a.kr * r;   // i k r - 1
-    Fr = ak * fma(cs, ar, -sn * ai);
-    Fi = ak * fma(cs, ai, sn * ar);
-  } else {
-    const double krr = a.kr * r;
-    Fr = -ak * fma(krr, sn, cs);
-    Fi = ak * fma(krr, cs, -sn);
-  }
-  Gr = g * cs;
-  Gi = g * sn;
+  const double krr = kr * r, kir = CPLX ? ki * r : 0.0;
+  Phase<CPLX, FAST> e;
+  e.begin(krr, kir, tr);
+  const double g = J * wq * kInv4PiS * rinv;  // J w / (4 pi r)
+  kernels_end<CPLX, FAST>(e, g, nd * (rinv * rinv), krr, kir, tr, Fr, Fi, Gr, Gi);
 }
 
-// The block's copy of the trig table for sincos_tab (every thread of the block takes part,
-// before any leaves).
-__device__ __forceinline__ void load_trig(const SparseArgs& a, double2* s_trig) {
-  for (int j = threadIdx.x; j < kTrigN; j += blockDim.x) s_trig[j] = a.trig[j];
+// Lane = point (q, q + step, ...) of the rule at R0: the sums of B rows, where bit j of m says
+// that row j takes part.  The next point's record is always under way.
+template <int NG, int NP, int B, bool CPLX, bool FAST>
+__device__ __forceinline__ void sparse_rule(const SparseArgs& a, Surface<NG>& sf,
+                                            const double (&x)[B][3], unsigned m,
+                                            const double* R0, int q, int Q, int step,
+                                            const Trig& tr, double (&acc)[B][NP][4]) {
+  static_assert(kSparseRec == 4, "a record is two 16-byte loads");
+  const double2* rec = reinterpret_cast<const double2*>(R0) + 2 * (size_t)min(q, Q - 1);
+  double2 uv = rec[0], wp = rec[1];
+  for (; q < Q; q += step) {
+    const double u = uv.x, v = uv.y, wq = wp.x;
+    rec += q + step < Q ? 2 * (size_t)step : 0;
+    uv = rec[0];
+    wp = rec[1];
+    double Ng[NG], Du[NG], Dv[NG], Np[NP], y[3];
+    sparse_geom_basis<NG>(u, v, Ng, Du, Dv);
+    sf.at(Ng, Du, Dv, y);
+    if constexpr (NP == NG) {
+      if (a.disc) {
+        sparse_phys_basis<NP>(true, a.beta, u, v, Np);
+      } else {
+#pragma unroll
+        for (int s = 0; s < NP; ++s) Np[s] = Ng[s];
+      }
+    } else {
+      sparse_phys_basis<NP>(a.disc, a.beta, u, v, Np);
+    }
+    // (tested anew for every point: a loop for each of the sets would interleave its rows and
+    // take all registers)
+    unsigned now = __builtin_amdgcn_readfirstlane(m);
+    if (B > 1) asm volatile("" : "+s"(now));
+#pragma unroll
+    for (int j = 0; j < B; ++j) {
+      if (B > 1 && !((now >> j) & 1u)) continue;
+      double Fr, Fi, Gr, Gi;
+      sparse_point_kernels<CPLX, FAST>(y, sf.n, sf.J, x[j], wq, a.kr, a.ki, tr, Fr, Fi, Gr, Gi);
+#pragma unroll
+      for (int s = 0; s < NP; ++s) {
+        acc[j][s][0] = fma(Fr, Np[s], acc[j][s][0]);
+        acc[j][s][1] = fma(Fi, Np[s], acc[j][s][1]);
+        acc[j][s][2] = fma(Gr, Np[s], acc[j][s][2]);
+        acc[j][s][3] = fma(Gi, Np[s], acc[j][s][3]);
+      }
+    }
+  }
+}
+
+// The block's copy of the trig table (every thread of the block takes part, before any
+// leaves).
+__device__ __forceinline__ Trig load_trig(const SparseArgs& a, double* s_trig) {
+  for (int j = threadIdx.x; j < kTrigDoubles + kExpN; j += blockDim.x) s_trig[j] = a.trig[j];
   __syncthreads();
+  return make_trig(s_trig);
 }
 
 __device__ __forceinline__ double wave_sum_d(double v) {
@@ -262,146 +330,113 @@ __device__ __forceinline__ double wave_sum_d(double v) {
   return v;
 }
 
-template <int NG, int NP, bool CPLX>
-__global__ void __launch_bounds__(256) k_sparse_pairs(const SparseArgs a) {
-  const int64_t p = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  __shared__ double2 s_trig[kTrigN];
-  load_trig(a, s_trig);
-  if (p >= a.n_pairs) return;  // the whole wave leaves together
-  const int lane = threadIdx.x & 63;
-  const int2 pr = a.pairs[p];
-  const double x0 = a.src[3 * (size_t)pr.x], x1 = a.src[3 * (size_t)pr.x + 1],
-               x2 = a.src[3 * (size_t)pr.x + 2];
-  // no distance below Inf (non-finite coordinates) falls to the sixth rule, the
-  // reference's final else branch (assembly_collocation_losses.jl:390-395)
-  const int c = select_rule<NG>(x0, x1, x2, a.gsel + (size_t)pr.y * NG * 4, 6, a.hyp) - 1;
-  double X[NG][3];
+template <int NG>
+__device__ __forceinline__ void sparse_element(const SparseArgs& a, int e, Surface<NG>& sf) {
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
-    const int node = a.topo[(size_t)pr.y * NG + g];
+    const int node = a.topo[(size_t)e * NG + g];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) X[g][d] = a.coords[3 * (size_t)node + d];
+    for (int d = 0; d < 3; ++d) sf.X[g][d] = a.coords[3 * (size_t)node + d];
   }
-  double fr[NP], fi[NP], gr[NP], gi[NP];
-#pragma unroll
-  for (int s = 0; s < NP; ++s) fr[s] = fi[s] = gr[s] = gi[s] = 0.0;
-  const double* R0 = a.rules + (size_t)a.off[c] * kSparseRec;
-  const int Q = a.len[c];
-  for (int q = lane; q < Q; q += 64) {
-    const double2 uv = *reinterpret_cast<const double2*>(R0 + (size_t)q * kSparseRec);
-    const double wq = R0[(size_t)q * kSparseRec + 2];
-    double Ng[NG], Du[NG], Dv[NG], Np[NP];
-    sparse_geom_basis<NG>(uv.x, uv.y, Ng, Du, Dv);
-    sparse_phys_basis<NP>(a.disc, a.beta, uv.x, uv.y, Np);
-    const SparseGeom sg = sparse_geometry<NG>(X, Ng, Du, Dv, x0, x1, x2);
-    double Fr, Fi, Gr, Gi;
-    sparse_point_kernels<CPLX>(a, sg, wq, s_trig, Fr, Fi, Gr, Gi);
-#pragma unroll
-    for (int s = 0; s < NP; ++s) {
-      const double ph = Np[s];
-      fr[s] = fma(Fr, ph, fr[s]);
-      fi[s] = fma(Fi, ph, fi[s]);
-      gr[s] = fma(Gr, ph, gr[s]);
-      gi[s] = fma(Gi, ph, gi[s]);
-    }
-  }
+  sf.begin();
+}
+
+template <int NP, bool SUM>
+__device__ __forceinline__ void sparse_add(const SparseArgs& a, int64_t p, bool writes,
+                                           const double (&acc)[NP][4]) {
   const bool doF = (a.flags & BIE_F) != 0, doG = (a.flags & BIE_G) != 0;
 #pragma unroll
   for (int s = 0; s < NP; ++s) {
-    const double vfr = wave_sum_d(fr[s]), vfi = wave_sum_d(fi[s]);
-    const double vgr = wave_sum_d(gr[s]), vgi = wave_sum_d(gi[s]);
-    if (lane == 0) {
+    double v[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) v[t] = SUM ? wave_sum_d(acc[s][t]) : acc[s][t];
+    if (writes) {
       const size_t e = 2 * (size_t)a.pos[p * NP + s];
       if (doF) {
-        unsafeAtomicAdd(a.F + e, vfr);
-        unsafeAtomicAdd(a.F + e + 1, vfi);
+        unsafeAtomicAdd(a.F + e, v[0]);
+        unsafeAtomicAdd(a.F + e + 1, v[1]);
       }
       if (doG) {
-        unsafeAtomicAdd(a.G + e, vgr);
-        unsafeAtomicAdd(a.G + e + 1, vgi);
+        unsafeAtomicAdd(a.G + e, v[2]);
+        unsafeAtomicAdd(a.G + e + 1, v[3]);
       }
     }
   }
 }
 
+// One wave per pair.
+template <int NG, int NP, bool CPLX, bool FAST>
+__global__ void __launch_bounds__(256) k_sparse_pairs(const SparseArgs a) {
+  const int64_t p =
+      (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  __shared__ double s_trig[kTrigDoubles + kExpN];
+  const Trig tr = load_trig(a, s_trig);
+  if (p >= a.n_pairs) return;  // the whole wave leaves together
+  const int lane = threadIdx.x & 63;
+  const int2 pr = a.pairs[p];
+  double x[1][3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) x[0][d] = a.src[3 * (size_t)pr.x + d];
+  // no distance below Inf (non-finite coordinates) falls to the sixth rule, the
+  // reference's final else branch (assembly_collocation_losses.jl:390-395)
+  const int c = __builtin_amdgcn_readfirstlane(
+      select_rule<NG>(x[0][0], x[0][1], x[0][2], a.gsel + (size_t)pr.y * NG * 4, 6, a.hyp) - 1);
+  Surface<NG> sf;
+  sparse_element<NG>(a, pr.y, sf);
+  double acc[1][NP][4] = {};
+  const double* R0 = a.rules + (size_t)a.off[c] * kSparseRec;
+  if (a.len[c] > 0)
+    sparse_rule<NG, NP, 1, CPLX, FAST>(a, sf, x, 1u, R0, lane, a.len[c], 64, tr, acc);
+  sparse_add<NP, true>(a, p, lane == 0, acc[0]);
+}
+
 // Short rules (the partial near field's gauss_points_triangle(n), n <= 13): one thread per
 // pair instead of one wave, the same per-point evaluation; the thread adds its sums into
 // the entries with FP64 atomics.
-template <int NG, int NP, bool CPLX>
+template <int NG, int NP, bool CPLX, bool FAST>
 __global__ void __launch_bounds__(256) k_sparse_pairs_short(const SparseArgs a) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  __shared__ double2 s_trig[kTrigN];
-  load_trig(a, s_trig);
+  __shared__ double s_trig[kTrigDoubles + kExpN];
+  const Trig tr = load_trig(a, s_trig);
   if (p >= a.n_pairs) return;
   const int2 pr = a.pairs[p];
-  const double x0 = a.src[3 * (size_t)pr.x], x1 = a.src[3 * (size_t)pr.x + 1],
-               x2 = a.src[3 * (size_t)pr.x + 2];
-  const int c = select_rule<NG>(x0, x1, x2, a.gsel + (size_t)pr.y * NG * 4, 6, a.hyp) - 1;
-  double X[NG][3];
+  double x[1][3];
 #pragma unroll
-  for (int g = 0; g < NG; ++g) {
-    const int node = a.topo[(size_t)pr.y * NG + g];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) X[g][d] = a.coords[3 * (size_t)node + d];
-  }
-  double fr[NP], fi[NP], gr[NP], gi[NP];
-#pragma unroll
-  for (int s = 0; s < NP; ++s) fr[s] = fi[s] = gr[s] = gi[s] = 0.0;
+  for (int d = 0; d < 3; ++d) x[0][d] = a.src[3 * (size_t)pr.x + d];
+  const int c =
+      select_rule<NG>(x[0][0], x[0][1], x[0][2], a.gsel + (size_t)pr.y * NG * 4, 6, a.hyp) - 1;
+  Surface<NG> sf;
+  sparse_element<NG>(a, pr.y, sf);
+  double acc[1][NP][4] = {};
   const double* R0 = a.rules + (size_t)a.off[c] * kSparseRec;
-  const int Q = a.len[c];
-  for (int q = 0; q < Q; ++q) {
-    const double2 uv = *reinterpret_cast<const double2*>(R0 + (size_t)q * kSparseRec);
-    const double wq = R0[(size_t)q * kSparseRec + 2];
-    double Ng[NG], Du[NG], Dv[NG], Np[NP];
-    sparse_geom_basis<NG>(uv.x, uv.y, Ng, Du, Dv);
-    sparse_phys_basis<NP>(a.disc, a.beta, uv.x, uv.y, Np);
-    const SparseGeom sg = sparse_geometry<NG>(X, Ng, Du, Dv, x0, x1, x2);
-    double Fr, Fi, Gr, Gi;
-    sparse_point_kernels<CPLX>(a, sg, wq, s_trig, Fr, Fi, Gr, Gi);
-#pragma unroll
-    for (int s = 0; s < NP; ++s) {
-      fr[s] = fma(Fr, Np[s], fr[s]);
-      fi[s] = fma(Fi, Np[s], fi[s]);
-      gr[s] = fma(Gr, Np[s], gr[s]);
-      gi[s] = fma(Gi, Np[s], gi[s]);
-    }
-  }
-  const bool doF = (a.flags & BIE_F) != 0, doG = (a.flags & BIE_G) != 0;
-#pragma unroll
-  for (int s = 0; s < NP; ++s) {
-    const size_t e = 2 * (size_t)a.pos[p * NP + s];
-    if (doF) {
-      unsafeAtomicAdd(a.F + e, fr[s]);
-      unsafeAtomicAdd(a.F + e + 1, fi[s]);
-    }
-    if (doG) {
-      unsafeAtomicAdd(a.G + e, gr[s]);
-      unsafeAtomicAdd(a.G + e + 1, gi[s]);
-    }
-  }
+  if (a.len[c] > 0)
+    sparse_rule<NG, NP, 1, CPLX, FAST>(a, sf, x, 1u, R0, 0, a.len[c], 1, tr, acc);
+  sparse_add<NP, false>(a, p, true, acc[0]);
 }
+
+// Rows per batch: as many as 256 registers hold the sums of, so that two waves share a SIMD.
+// (Depth 2, two to four thousand nodes, us: three six-node rows spilled, 3078 against 2992 with
+// two, and in 512 registers took 3666; four three-node rows 2495 and 3181 on flat and curved
+// elements against 2386 and 1979 with three.)
+constexpr int batch_rows(int NP) { return NP == 1 ? 4 : NP == 3 ? 3 : 2; }
 
 // Batches of up to B pairs that share an element (built on the host, grouped by the rule
 // the mesh sources select): one wave per batch evaluates the surface at each point of a rule
 // once and the kernels for every row of the batch that selected that rule - the surface
 // (~2/3 of the per-point work) is shared.  Each row's rule is selected here exactly as in
 // k_sparse_pairs, so explicit sources stay correct (they only share less).
-template <int NG, int NP, int B, bool CPLX>
-__global__ void __launch_bounds__(256) k_sparse_batch(const SparseArgs a) {
-  const int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  __shared__ double2 s_trig[kTrigN];
-  load_trig(a, s_trig);
+template <int NG, int NP, int B, bool CPLX, bool FAST>
+__global__ void __launch_bounds__(256, 2) k_sparse_batch(const SparseArgs a) {
+  const int64_t b =
+      (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  __shared__ double s_trig[kTrigDoubles + kExpN];
+  const Trig tr = load_trig(a, s_trig);
   if (b >= a.n_batches) return;  // the whole wave leaves together
   const int lane = threadIdx.x & 63;
   const int* rec = a.batches + (size_t)b * 8;
   const int e = rec[0], cnt = rec[1];
-  double X[NG][3];
-#pragma unroll
-  for (int g = 0; g < NG; ++g) {
-    const int node = a.topo[(size_t)e * NG + g];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) X[g][d] = a.coords[3 * (size_t)node + d];
-  }
+  Surface<NG> sf;
+  sparse_element<NG>(a, e, sf);
   double xs[B][3];
   int cr[B], pj[B];
 #pragma unroll
@@ -417,12 +452,9 @@ __global__ void __launch_bounds__(256) k_sparse_batch(const SparseArgs a) {
       cr[j] = select_rule<NG>(xs[j][0], xs[j][1], xs[j][2], a.gsel + (size_t)e * NG * 4, 6,
                               a.hyp) - 1;
     }
+    cr[j] = __builtin_amdgcn_readfirstlane(cr[j]);
   }
-  double acc[B][NP][4];
-#pragma unroll
-  for (int j = 0; j < B; ++j)
-#pragma unroll
-    for (int s = 0; s < NP; ++s) acc[j][s][0] = acc[j][s][1] = acc[j][s][2] = acc[j][s][3] = 0.0;
+  double acc[B][NP][4] = {};
   unsigned done = 0u;
   for (int j0 = 0; j0 < B; ++j0) {
     if (cr[j0] < 0 || ((done >> j0) & 1u)) continue;
@@ -433,51 +465,12 @@ __global__ void __launch_bounds__(256) k_sparse_batch(const SparseArgs a) {
       if (cr[j] >= 0 && a.off[cr[j]] == a.off[c] && a.len[cr[j]] == a.len[c]) m |= 1u << j;
     done |= m;
     const double* R0 = a.rules + (size_t)a.off[c] * kSparseRec;
-    const int Q = a.len[c];
-    for (int q = lane; q < Q; q += 64) {
-      const double2 uv = *reinterpret_cast<const double2*>(R0 + (size_t)q * kSparseRec);
-      const double wq = R0[(size_t)q * kSparseRec + 2];
-      double Ng[NG], Du[NG], Dv[NG], Np[NP], y[3], n[3], J;
-      sparse_geom_basis<NG>(uv.x, uv.y, Ng, Du, Dv);
-      sparse_phys_basis<NP>(a.disc, a.beta, uv.x, uv.y, Np);
-      sparse_surface<NG>(X, Ng, Du, Dv, y, n, J);
-#pragma unroll
-      for (int j = 0; j < B; ++j) {
-        if (!((m >> j) & 1u)) continue;
-        const SparseGeom sg = sparse_toward(y, n, J, xs[j][0], xs[j][1], xs[j][2]);
-        double Fr, Fi, Gr, Gi;
-        sparse_point_kernels<CPLX>(a, sg, wq, s_trig, Fr, Fi, Gr, Gi);
-#pragma unroll
-        for (int s = 0; s < NP; ++s) {
-          acc[j][s][0] = fma(Fr, Np[s], acc[j][s][0]);
-          acc[j][s][1] = fma(Fi, Np[s], acc[j][s][1]);
-          acc[j][s][2] = fma(Gr, Np[s], acc[j][s][2]);
-          acc[j][s][3] = fma(Gi, Np[s], acc[j][s][3]);
-        }
-      }
-    }
+    if (a.len[c] > 0)
+      sparse_rule<NG, NP, B, CPLX, FAST>(a, sf, xs, m, R0, lane, a.len[c], 64, tr, acc);
   }
-  const bool doF = (a.flags & BIE_F) != 0, doG = (a.flags & BIE_G) != 0;
 #pragma unroll
-  for (int j = 0; j < B; ++j) {
-    if (pj[j] < 0) continue;
-#pragma unroll
-    for (int s = 0; s < NP; ++s) {
-      const double vfr = wave_sum_d(acc[j][s][0]), vfi = wave_sum_d(acc[j][s][1]);
-      const double vgr = wave_sum_d(acc[j][s][2]), vgi = wave_sum_d(acc[j][s][3]);
-      if (lane == 0) {
-        const size_t ent = 2 * (size_t)a.pos[(size_t)pj[j] * NP + s];
-        if (doF) {
-          unsafeAtomicAdd(a.F + ent, vfr);
-          unsafeAtomicAdd(a.F + ent + 1, vfi);
-        }
-        if (doG) {
-          unsafeAtomicAdd(a.G + ent, vgr);
-          unsafeAtomicAdd(a.G + ent + 1, vgi);
-        }
-      }
-    }
-  }
+  for (int j = 0; j < B; ++j)
+    if (pj[j] >= 0) sparse_add<NP, true>(a, pj[j], lane == 0, acc[j]);
 }
 
 }  // namespace
@@ -493,7 +486,7 @@ void launch_sparse_pairs(const SparseLaunch& L, hipStream_t s) {
   a.topo = L.topo;
   a.gsel = L.gsel;
   a.rules = L.rules;
-  a.trig = reinterpret_cast<const double2*>(L.trig);
+  a.trig = L.trig;
   for (int c = 0; c < 6; ++c) {
     a.off[c] = L.off[c];
     a.len[c] = L.len[c];
@@ -519,18 +512,19 @@ void launch_sparse_pairs(const SparseLaunch& L, hipStream_t s) {
   BIE_REQUIRE(blocks < 2147483647LL, BIE_EINVAL, "too many sparse pairs");
   const dim3 grid((unsigned)blocks);
   const bool cplx = L.ki != 0.0;
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a); };
+  auto run = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a); };
   // geometry nodes 3 or 6; physics nodes 1 (discontinuous constant), 3 or 6
   auto pick = [&](auto ng, auto np, auto cx) {
     constexpr int NG = decltype(ng)::value, NP = decltype(np)::value;
     constexpr bool C = decltype(cx)::value;
-    constexpr int B = NP == 1 ? 4 : 3;
+    constexpr int B = batch_rows(NP);
     if (shortr)
-      go(k_sparse_pairs_short<NG, NP, C>);
+      L.fast ? run(k_sparse_pairs_short<NG, NP, C, true>)
+             : run(k_sparse_pairs_short<NG, NP, C, false>);
     else if (batched)
-      go(k_sparse_batch<NG, NP, B, C>);
+      L.fast ? run(k_sparse_batch<NG, NP, B, C, true>) : run(k_sparse_batch<NG, NP, B, C, false>);
     else
-      go(k_sparse_pairs<NG, NP, C>);
+      L.fast ? run(k_sparse_pairs<NG, NP, C, true>) : run(k_sparse_pairs<NG, NP, C, false>);
   };
   auto by_cx = [&](auto ng, auto np) {
     cplx ? pick(ng, np, std::true_type()) : pick(ng, np, std::false_type());
@@ -554,6 +548,6 @@ void launch_sparse_pairs(const SparseLaunch& L, hipStream_t s) {
 
 int sparse_record_doubles() { return kSparseRec; }
 
-int sparse_batch_rows(int NP) { return NP == 1 ? 4 : 3; }
+int sparse_batch_rows(int NP) { return batch_rows(NP); }
 
 }  // namespace bie

@@ -167,3 +167,40 @@ def test_batched_k_derivative(kind, nm):
         ref = al[i][0] @ (D @ ps[i][0])
         scale = np.abs(al[i][0]) @ (np.abs(D) @ np.abs(ps[i][0]))
         assert abs(got[i] - ref) <= 1e-12 * scale, i
+
+
+@pytest.mark.parametrize("kind,physics", [("linear", "geometry"), ("quadratic", "geometry"),
+                                          ("quadratic", "linear")])
+@pytest.mark.parametrize("depth", [1, 2])
+def test_near_field_out_of_the_middle_of_the_range(kind, physics, depth):
+    """The near field of a mesh 2^200 times as large, at k / 2^200: a power of two commutes with
+    every rounding, so the normals formed by division (the Jacobian is beyond the range of the
+    reciprocal form) give the same F, and G 2^200 times as large, but for the order of the
+    additions to an entry."""
+    from bie_amd.assembly import sparse_assemble_parallel
+    kw = {} if physics == "geometry" else dict(physics=physics)
+    mesh = M.ellipsoid(2, axes=(1.2, 1.0, 0.7), order=kind, **kw)
+    s = 2.0 ** 200
+    big = M.Mesh3d(mesh.coordinates * s, mesh.topology, mesh.sources * s, mesh.physics_topology,
+                   mesh.geometry_kind, mesh.physics_kind)
+    F, G = sparse_assemble_parallel(mesh, 3.0, mesh.sources, depth=depth)
+    Fb, Gb = sparse_assemble_parallel(big, 3.0 / s, big.sources, depth=depth)
+    fs = max(np.max(np.abs(F.data)), np.max(np.abs(G.data)))
+    assert np.max(np.abs(F.data - Fb.data)) <= 1e-14 * fs
+    assert np.max(np.abs(G.data - Gb.data / s)) <= 1e-14 * fs
+
+
+def test_near_field_of_a_far_source():
+    """An explicit source whose |k| r leaves the range of the branch-free sincos, among others
+    (its wave takes the other one)."""
+    from bie_amd.assembly import sparse_assemble_parallel
+    mesh = M.icosphere(2, "quadratic")
+    pts = np.array(mesh.sources, order="F")
+    F, G = sparse_assemble_parallel(mesh, 3.0, pts, depth=1)
+    pts[:, 7] = (0.0, 0.0, 5e14)
+    F2, G2 = sparse_assemble_parallel(mesh, 3.0, pts, depth=1)
+    rows = np.repeat(np.arange(F.shape[0]), np.diff(F.indptr))
+    near = rows != 7
+    assert np.max(np.abs(G.data - G2.data)[near]) <= 1e-14 * np.max(np.abs(G.data))
+    assert np.max(np.abs(F.data - F2.data)[near]) <= 1e-14 * np.max(np.abs(G.data))
+    assert np.isfinite(F2.data).all() and 0 < np.max(np.abs(G2.data[~near])) < 1e-12

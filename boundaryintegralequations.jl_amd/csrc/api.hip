@@ -438,9 +438,8 @@ StreamPrep stream_prep(bie_dmesh* dm, const AssemblyArgs& a, const bie_dmesh::St
 
 // The sweep kernel's schedule: S slots and at least min_segments segments (0: as suits the
 // collocation rows).  It does not depend on a call's targets or matrices: a graph keeps it.
-bie_dmesh::Stream& ensure_sweep_stream(bie_dmesh* dm, int S, int64_t min_segments, int cus,
-                                       hipStream_t s) {
-  bie_dmesh::Stream& out = dm->sstream;
+bie_dmesh::Stream& ensure_sweep_stream(bie_dmesh* dm, bie_dmesh::Stream& out, int S,
+                                       int64_t min_segments, int cus, hipStream_t s) {
   const int64_t key = min_segments * 65536 + std::min(dm->rs.len[0], 65535);
   if (out.key == key && out.S == S && out.d_order) return out;
   int64_t want = std::max(min_segments, least_segments(dm));
@@ -623,16 +622,17 @@ void sweep_device_impl(bie_dmesh* dm, const double* d_k, int nk, const double* d
   BIE_REQUIRE(sizeof(double) * (size_t)dm->rs.R * dm->rs.Qmax * dm->pk <= 24 * 1024,
               BIE_EUNSUPPORTED, "sweep supports quadrature orders up to n*m' = 36");
   const int cus = device_cus(dm->device);
-  const StreamPlan plan = sweep_plan(dm->rs, flat_elements(dm), dm->sweep_slots);
+  const bool lean = taylor && flat_elements(dm) && (flags & BIE_G) == 0;
+  const StreamPlan plan = sweep_plan(dm->rs, flat_elements(dm), lean, dm->sweep_slots);
   const int64_t min_seg =
       dm->sweep_elems_per_tile
           ? std::max<int64_t>(1, (dm->E + dm->sweep_elems_per_tile - 1) / dm->sweep_elems_per_tile)
           : 0;
-  const bie_dmesh::Stream& sc = ensure_sweep_stream(dm, plan.S, min_seg, cus, s);
+  const bie_dmesh::Stream& sc = ensure_sweep_stream(dm, lean ? dm->lstream : dm->sstream, plan.S, min_seg, cus, s);
   // the wavenumbers of a sweep are on the device: its tiles decide there
   const bool fast = taylor && fast_trig_ok(dm, k_re, target_radius);
   const int64_t rowblocks = (M + 63) / 64;
-  const int KB = sweep_block_size(dm->pk, (flags & BIE_G) != 0);
+  const int KB = sweep_block_size(dm->pk, (flags & BIE_G) != 0, lean);
   ensure_lists(lists, plan.mids, M, dm->E, sc.segments,
                fast ? 0 : (int64_t)((nk + KB - 1) / KB) * rowblocks * sc.segments);
   AssemblyArgs a = make_args(dm, d_targets, M, 0.0, 0.0, flags, dF, dG, dC);
@@ -1049,6 +1049,7 @@ int bie_dmesh_destroy(bie_dmesh* dm) {
   free_stream(dm->stream);
   free_stream(dm->bstream);
   free_stream(dm->sstream);
+  free_stream(dm->lstream);
   free_lists(dm->lists);
   free_lists(dm->blists);
   free_lists(dm->slists);

@@ -220,9 +220,10 @@ struct SweepArgs {
   int nk;
   int taylor;                // 1: the nk matrices are d^q/dk^q, q = 0..nk-1, at k_re + i k_im
 };
-int sweep_block_size(int NP, bool gon);  // matrices per block of the kernel
+// lean: F alone of the k-derivatives on flat elements
+int sweep_block_size(int NP, bool gon, bool lean);  // matrices per block of the kernel
 // slots: at most so many LDS slots (0: as many as fit)
-StreamPlan sweep_plan(const RuleSet& rs, bool flat, int slots);
+StreamPlan sweep_plan(const RuleSet& rs, bool flat, bool lean, int slots);
 // prepare_only: sets the kernels' attributes, launches nothing
 void launch_sweep(const StreamInst& in, const SweepArgs& sw, const StreamPlan& pl,
                   const double* d_tab, unsigned* d_counters, int* d_slow, int cus, bool fast,
@@ -422,8 +423,9 @@ struct bie_dmesh {
     std::vector<int> h_seg_begin;  // (batch) host copy, for the tile list
   };
   double* d_eflat = nullptr;     // records of flat elements in element order (k-derivatives)
-  // of single-mesh calls, of batches, of sweeps and k-derivatives
-  Stream stream, bstream, sstream;
+  // of single-mesh calls, of batches, of sweeps and k-derivatives (F alone on flat elements:
+  // lstream, whose slots are smaller)
+  Stream stream, bstream, sstream, lstream;
   bie::StreamLists lists, blists, slists;
   double* d_stab = nullptr;      // its tables for the cached rule set (stream_tables)
   // tile shape of the frequency sweep (bie_sweep_tune): elements per tile (0: one segment per

@@ -20,6 +20,8 @@
 //     F_m = -(n.d) [k A_{m-1} + (m - 1) A_{m-2}], G_m = A_m:
 //     one sequence of sums (two products and six multiply-adds per point and order) gives
 //     both.
+// 16 wavenumbers on 4002 nodes, 16 points: 17.0 -> 11.5 ms (VALU busy 83 % of the time, 134
+// instructions per point and four wavenumbers); 26 orders of F, four points: 8.7 -> 5.0 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -31,13 +33,18 @@
 namespace bie {
 namespace {
 
-constexpr int kSweepWaves = 8;
-
-// Matrices of a block.
-__host__ __device__ constexpr int sweep_block(int NP, bool gon) {
-  return (NP == 6 ? 2 : 4) * (gon ? 1 : 2);
+// Shape of a kernel: matrices of a block, waves of a workgroup, doubles of a slot.  F alone of
+// the k-derivatives on flat elements (`lean`) keeps sums for one order more than its block
+// and no others: six orders fit 168 registers and so twelve waves, which its short rules need
+// (few points a pair: half of the time is the hand-over).  26 orders on 4002 nodes, four
+// points: 4.99 ms; eight orders and eight waves 5.69, four and sixteen 5.43.
+struct SweepShape {
+  int kb, waves, slot;
+};
+__host__ __device__ constexpr SweepShape sweep_shape(int NP, bool gon, bool lean) {
+  return lean ? SweepShape{6, 12, 6 * 128}
+              : SweepShape{(NP == 6 ? 2 : 4) * (gon ? 1 : 2), 8, (NP == 6 ? 2 : 4) * 256};
 }
-constexpr int sweep_slot_doubles(int NP) { return sweep_block(NP, true) * 256; }
 
 typedef const __attribute__((address_space(4))) SweepArgs* SweepPtr;
 
@@ -162,9 +169,8 @@ __device__ __forceinline__ void sweep_pair_flat(const double (&d0)[3], const dou
     sweep_point_flat<KB, K, GON, FAST, REC, false>(d0, a, b, n, tab += 4, kv, tr, v, c3);
 }
 
-// One point of a flat element for the derivative orders m0 .. m0 + K - 1 (m0 a multiple of
-// four): sums of N r^j e^{ikr} w / (4 pi r), j = m0 - 2 .., without the factors i^j.
-template <int NA, bool CPLX, bool FAST, bool FIRST>
+// One point of a flat element for the derivative orders m0 .. m0 + K - 1 (m0 even): sums of N r^j e^{ikr} w / (4 pi r), j = m0 - 2 .., without the factors i^j.
+template <int NA, bool CPLX, bool FAST>
 __device__ __forceinline__ void taylor_point_flat(const double (&d0)[3], const double (&a)[3],
                                                   const double (&b)[3], double (&n)[4],
                                                   const double* next, double kr, double ki,
@@ -185,7 +191,7 @@ __device__ __forceinline__ void taylor_point_flat(const double (&d0)[3], const d
   double q = m[3] * rinv;
   if (m0 == 0) {
     q *= rinv * rinv;
-    c3 = FIRST ? q : c3 + q;
+    c3 += q;
   } else {  // r^(m0 - 2): even, by binary powering
     double p = r2;
     for (int x = (m0 - 2) >> 1; x != 0; x >>= 1) {
@@ -205,29 +211,37 @@ __device__ __forceinline__ void taylor_point_flat(const double (&d0)[3], const d
     }
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
-      plus<FIRST>(ac[j][s], C, m[s]);
-      plus<FIRST>(as[j][s], S, m[s]);
+      ac[j][s] = fma(C, m[s], ac[j][s]);
+      as[j][s] = fma(S, m[s], as[j][s]);
     }
   }
 }
 
-template <int KB, int K, bool CPLX, bool GON, bool FAST>
+template <int KB, bool CPLX, bool GON, bool FAST>
 __device__ __forceinline__ void taylor_pair_flat(const double (&d0)[3], const double (&a)[3],
                                                  const double (&b)[3], const double* tab, int Q,
                                                  double kr, double ki, int m0, double nd,
                                                  double J, const Trig& tr,
                                                  Multi<3, KB, GON>& v, double& c3) {
-  constexpr int NA = K + (GON ? 2 : 1);
+  constexpr int NA = KB + (GON ? 2 : 1);
   double ac[NA][3], as[NA][3];
   double n[4] = {tab[0], tab[1], tab[2], tab[3]};
-  taylor_point_flat<NA, CPLX, FAST, true>(d0, a, b, n, tab += 4, kr, ki, m0, tr, ac, as, c3);
+#pragma unroll
+  for (int j = 0; j < NA; ++j)
+#pragma unroll
+    for (int s = 0; s < 3; ++s) ac[j][s] = as[j][s] = 0.0;
+  c3 = 0.0;
 #pragma unroll 1
-  for (int q = 1; q < Q; ++q)
-    taylor_point_flat<NA, CPLX, FAST, false>(d0, a, b, n, tab += 4, kr, ki, m0, tr, ac, as, c3);
+  for (int q = 0; q < Q; ++q)
+    taylor_point_flat<NA, CPLX, FAST>(d0, a, b, n, tab += 4, kr, ki, m0, tr, ac, as, c3);
   // F_m = (n.d) i^m [(m - 1) A'_{m-2} + i k A'_{m-1}], G_m = J i^m A'_m (A' without i^j)
+  if (m0 & 2) {
+    nd = -nd;
+    J = -J;
+  }
   const double kn = nd * kr, kin = CPLX ? nd * ki : 0.0;
 #pragma unroll
-  for (int q = 0; q < K; ++q) {
+  for (int q = 0; q < KB; ++q) {
     const double mn = nd * (double)(m0 + q - 1);
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
@@ -450,12 +464,13 @@ __device__ __forceinline__ void finish_multi(InstPtr in, SweepPtr sw, const int4
 template <int NP, bool FLAT, bool TAY, bool CPLX, bool GON, bool FAST>
 __device__ __forceinline__ void sweep_tile(InstPtr in, SweepPtr sw, int rb, int seg, int kb,
                                            int S, int tab_doubles, double* lds, int parity) {
-  constexpr int W = kSweepWaves, KB = sweep_block(NP, GON);
+  constexpr SweepShape kShape = sweep_shape(NP, GON, FLAT && TAY && !GON);
+  constexpr int W = kShape.waves, KB = kShape.kb;
   constexpr bool kMids = NP == 6;
   const int lane = threadIdx.x & 63;
   const int R = in->a.R;
   const int Q = in->a.len[0];
-  const Layout L = layout_of(S, sweep_slot_doubles(NP), tab_doubles, W, 0, kMids && R == 6);
+  const Layout L = layout_of(S, kShape.slot, tab_doubles, W, 0, kMids && R == 6);
   double* acc = lds;
   const double* tab = lds + L.tab;
   const Trig tr = make_trig(tab + tab_doubles);
@@ -512,12 +527,8 @@ __device__ __forceinline__ void sweep_tile(InstPtr in, SweepPtr sw, int rb, int 
       const double* tc = tab + c * tab_rule;
       double c3 = 0.0;
       if constexpr (TAY) {
-        if (KB > 4 && nb <= KB / 2)
-          taylor_pair_flat<KB, KB / 2, CPLX, GON, FAST>(d0, ea, eb, tc, Q, kv.k[0], ki, k0, nd,
-                                                        J, tr, v, c3);
-        else
-          taylor_pair_flat<KB, KB, CPLX, GON, FAST>(d0, ea, eb, tc, Q, kv.k[0], ki, k0, nd, J,
-                                                    tr, v, c3);
+        taylor_pair_flat<KB, CPLX, GON, FAST>(d0, ea, eb, tc, Q, kv.k[0], ki, k0, nd, J, tr, v,
+                                              c3);
       } else {
         if (!rec)
           sweep_pair_flat<KB, KB, GON, FAST, false>(d0, ea, eb, tc, Q, kv, tr, v, c3);
@@ -586,7 +597,7 @@ __device__ __forceinline__ void sweep_tile(InstPtr in, SweepPtr sw, int rb, int 
 }
 
 template <int NP, bool FLAT, bool TAY, bool CPLX, bool GON, bool FAST>
-__global__ void __launch_bounds__(64 * kSweepWaves)
+__global__ void __launch_bounds__(64 * sweep_shape(NP, GON, FLAT && TAY && !GON).waves)
 k_sweep(const StreamInst one, const SweepArgs args, int n_tiles, const StreamRun run) {
   extern __shared__ double lds[];
   const auto* base = (const __attribute__((address_space(4))) char*)
@@ -606,14 +617,15 @@ k_sweep(const StreamInst one, const SweepArgs args, int n_tiles, const StreamRun
     if constexpr (TAY) {
       return fabs(sw->k_re);
     } else {  // of the block's wavenumbers and of their spacing
-      constexpr int KB = sweep_block(NP, GON);
+      constexpr int KB = sweep_shape(NP, GON, false).kb;
       const int k0 = tile / per_kb * KB;
       double m = 0.0;
       for (int q = k0; q < min(k0 + KB, sw->nk); ++q) m = fmax(m, fabs(sload(sw->k + q)));
       return 2.0 * m;
     }
   };
-  stream_run<sweep_slot_doubles(NP), kSweepWaves, NP == 6, FAST>(
+  constexpr SweepShape kShape = sweep_shape(NP, GON, FLAT && TAY && !GON);
+  stream_run<kShape.slot, kShape.waves, NP == 6, FAST>(
       inst_of, kmax_of, [&](InstPtr, int tile) { return tile < per_kb; },
       [&](InstPtr p, int rb, int seg, int tile, int parity) {
         sweep_tile<NP, FLAT, TAY, CPLX, GON, FAST>(p, sw, rb, seg, tile / per_kb, run.S,
@@ -678,17 +690,17 @@ void with_sweep_kernel(int NP, bool flat, bool tay, bool cplx, bool gon, bool fa
 
 }  // namespace
 
-int sweep_block_size(int NP, bool gon) { return sweep_block(NP, gon); }
+int sweep_block_size(int NP, bool gon, bool lean) { return sweep_shape(NP, gon, lean).kb; }
 
-StreamPlan sweep_plan(const RuleSet& rs, bool flat, int slots) {
+StreamPlan sweep_plan(const RuleSet& rs, bool flat, bool lean, int slots) {
+  const SweepShape sh = sweep_shape(rs.pk, true, lean);
   StreamPlan pl;
   pl.flat = flat;
-  pl.waves = kSweepWaves;
+  pl.waves = sh.waves;
   pl.tab_doubles = stream_tab_doubles(rs, flat);
   pl.mids = uses_mid_rules(rs.R, rs.pk);
-  const int sd = sweep_slot_doubles(rs.pk);
   auto bytes = [&](int S) {
-    return layout_of(S, sd, pl.tab_doubles, kSweepWaves, 0, pl.mids).total * 8L;
+    return layout_of(S, sh.slot, pl.tab_doubles, pl.waves, 0, pl.mids).total * 8L;
   };
   while (pl.S < 120 && bytes(pl.S + 1) <= kLdsBytes) ++pl.S;
   if (slots > 0) pl.S = std::min(pl.S, slots);
@@ -700,7 +712,7 @@ void launch_sweep(const StreamInst& in, const SweepArgs& sw, const StreamPlan& p
                   const double* d_tab, unsigned* d_counters, int* d_slow, int cus, bool fast,
                   bool prepare_only, hipStream_t s) {
   const bool gon = (in.a.flags & BIE_G) != 0, tay = sw.taylor != 0, cplx = sw.k_im != 0.0;
-  const int KB = sweep_block(in.a.NP, gon);
+  const int KB = sweep_shape(in.a.NP, gon, pl.flat && tay && !gon).kb;
   const int64_t tiles =
       (int64_t)((sw.nk + KB - 1) / KB) * in.n_segments * (int64_t)in.n_rowblocks;
   BIE_REQUIRE(tiles > 0 && tiles < 2147483647LL, BIE_EINVAL, "too many sweep tiles");
@@ -714,7 +726,7 @@ void launch_sweep(const StreamInst& in, const SweepArgs& sw, const StreamPlan& p
                                         (int)pl.shmem));
       if (prepare_only) return;
       hipLaunchKernelGGL(kern, dim3((unsigned)std::min<int64_t>(tiles, cus)),
-                         dim3(64 * kSweepWaves), pl.shmem, s, in, sw, (int)tiles, run);
+                         dim3(64 * pl.waves), pl.shmem, s, in, sw, (int)tiles, run);
       if (pl.mids && pass == (fast ? 0 : 1))
         hipLaunchKernelGGL(mid, dim3(512, (unsigned)std::min(sw.nk, 1024)), dim3(256),
                            sizeof(double) *

@@ -280,24 +280,31 @@ void upload_stream(bie_dmesh* dm, bie_dmesh::Stream& out, const StreamSchedule& 
 // Segments cannot have more elements than a position within one has bits (24).
 int64_t least_segments(const bie_dmesh* dm) { return dm->E / (1 << 24) + 1; }
 
-// The schedule for S slots that suits single-mesh calls of rowblocks row blocks.
-bie_dmesh::Stream& ensure_stream(bie_dmesh* dm, int S, int64_t rowblocks, int cus,
-                                 hipStream_t s) {
-  bie_dmesh::Stream& out = dm->stream;
+// The schedule for S slots that suits single-mesh calls of rowblocks row blocks, in `out`.
+// Calls on the mesh's own rows and on others, with and without G (which has larger slots) have
+// one each, so that a program that alternates between them does not build them anew; other row
+// counts that want as many segments share one.
+bie_dmesh::Stream& ensure_stream(bie_dmesh* dm, bie_dmesh::Stream& out, int S,
+                                 int64_t rowblocks, int cus, hipStream_t s) {
   const int Q = dm->rs.len[0];
-  const int64_t key = rowblocks * 65536 + std::min(Q, 65535);
-  if (out.key == key && out.S == S && out.d_order) return out;
-  const std::vector<double> cent = element_centres(dm);
+  const bool same_call = out.rowblocks == rowblocks && out.Q == Q;
+  if (same_call && out.S == S && out.d_order) return out;
   const int64_t least = least_segments(dm);
   int want = choose_stream_segments(rowblocks, dm->E, Q, dm->pk, cus, least);
-  StreamSchedule sc = stream_schedule(dm, cent, S, want);
-  if (sc.n_segments != want) {  // the slots force more: fill the rounds of those
-    want = choose_stream_segments(rowblocks, dm->E, Q, dm->pk, cus, sc.n_segments);
-    StreamSchedule other = stream_schedule(dm, cent, S, want);
-    if (std::abs(other.n_segments - want) <= 1 || other.n_segments < sc.n_segments)
-      sc = std::move(other);
+  const int64_t key = want;
+  if (out.key != key || out.S != S || !out.d_order) {
+    const std::vector<double> cent = element_centres(dm);
+    StreamSchedule sc = stream_schedule(dm, cent, S, want);
+    if (sc.n_segments != want) {  // the slots force more: fill the rounds of those
+      want = choose_stream_segments(rowblocks, dm->E, Q, dm->pk, cus, sc.n_segments);
+      StreamSchedule other = stream_schedule(dm, cent, S, want);
+      if (std::abs(other.n_segments - want) <= 1 || other.n_segments < sc.n_segments)
+        sc = std::move(other);
+    }
+    upload_stream(dm, out, sc, S, key, s);
   }
-  upload_stream(dm, out, sc, S, key, s);
+  out.rowblocks = rowblocks;
+  out.Q = Q;
   return out;
 }
 
@@ -569,7 +576,9 @@ void assemble_device_impl(bie_dmesh* dm, double kr, double ki, const double* d_t
       const int64_t rowblocks = (M + 63) / 64;
       const bool fast = fast_trig_ok(dm, kr, target_radius);
       const int cus = device_cus(dm->device);
-      bie_dmesh::Stream& sc = ensure_stream(dm, plan.S, rowblocks, cus, s);
+      const bool own_rows = d_targets == dm->d_sources && M == dm->N;
+      bie_dmesh::Stream& sc = ensure_stream(
+          dm, dm->stream[own_rows ? 0 : 1][(flags & BIE_G) ? 1 : 0], plan.S, rowblocks, cus, s);
       StreamLists& l = dm->lists;
       ensure_lists(l, plan.mids, M, dm->E, sc.segments, fast ? 0 : rowblocks * sc.segments);
       launch_stream_prep(stream_prep(dm, a, sc, l, 1, 0), s);
@@ -1046,7 +1055,8 @@ int bie_dmesh_destroy(bie_dmesh* dm) {
   dfree(dm->d_elem);
   dfree(dm->d_stab);
   dfree(dm->d_eflat);
-  free_stream(dm->stream);
+  for (auto& by_g : dm->stream)
+    for (auto& sc : by_g) free_stream(sc);
   free_stream(dm->bstream);
   free_stream(dm->sstream);
   free_stream(dm->lstream);

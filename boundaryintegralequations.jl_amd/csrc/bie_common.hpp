@@ -413,6 +413,8 @@ struct bie_dmesh {
   struct Stream {
     int S = -1;                  // slots it was built for
     int64_t key = -1;            // and what the segments were chosen for
+    int64_t rowblocks = -1;      // (single-mesh calls) of the last call, and its rule length
+    int Q = -1;
     int segments = 0, zero_cols = 0;
     int* d_seg_begin = nullptr;
     int* d_order = nullptr;
@@ -423,9 +425,9 @@ struct bie_dmesh {
     std::vector<int> h_seg_begin;  // (batch) host copy, for the tile list
   };
   double* d_eflat = nullptr;     // records of flat elements in element order (k-derivatives)
-  // of single-mesh calls, of batches, of sweeps and k-derivatives (F alone on flat elements:
-  // lstream, whose slots are smaller)
-  Stream stream, bstream, sstream, lstream;
+  // of single-mesh calls (own rows or others, without or with G), of batches, of sweeps and
+  // k-derivatives (F alone on flat elements: lstream, whose slots are smaller)
+  Stream stream[2][2], bstream, sstream, lstream;
   bie::StreamLists lists, blists, slists;
   double* d_stab = nullptr;      // its tables for the cached rule set (stream_tables)
   // tile shape of the frequency sweep (bie_sweep_tune): elements per tile (0: one segment per

@@ -691,9 +691,8 @@ def main():
                      "quadrature_points": main_res["flops"]["points_dense"],
                      "pairs": main_res["flops"]["pairs"],
                      "fp64_unit": "VALU (MI355X FP64 vector peak = published FP64 peak)",
-                     "mid_edge_kernel": {"kernel": "k_mid_compute (on a side stream, while the "
-                                                   "dense kernel runs) + k_mid_scatter; pairs "
-                                                   "recorded at the first collocation call",
+                     "mid_edge_kernel": {"kernel": "k_stream_mid; pairs listed by the dense "
+                                                   "kernel",
                                          "ms_after_dense_kernel": main_res["mid_ms"],
                                          "flops_per_launch": main_res["flops"]["mid"]},
                      "assembly_pass_tflops": main_res["pass_tflops"]},

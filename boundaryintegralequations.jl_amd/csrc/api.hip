@@ -520,7 +520,7 @@ double radius_about(const double* c, const double* x, int64_t n) {
   return std::sqrt(r2);
 }
 
-// Whether every argument k r of the slot kernel's sincos stays below kTabFastMaxArg: r is
+// Whether every argument k r of the kernels' sincos stays below kTabFastMaxArg: r is
 // at most |x - c| + |y - c| for a target x and an element point y, and y = sum N_k X_k with
 // sum |N_k| <= 2 on linear and quadratic triangles, so |y - c| <= 2 coord_radius (taken
 // twice again for margin).  target_radius < 0: unknown (device targets), never fast.
@@ -583,9 +583,10 @@ void assemble_device_impl(bie_dmesh* dm, double kr, double ki, const double* d_t
       ensure_lists(l, plan.mids, M, dm->E, sc.segments, fast ? 0 : rowblocks * sc.segments);
       launch_stream_prep(stream_prep(dm, a, sc, l, 1, 0), s);
       if (timed) BIE_HIP_CHECK(hipEventRecord(ev[1], s));
-      launch_stream(stream_inst(dm, a, sc, l, rowblocks), plan, dm->d_stab, l.counters, l.slow,
-                    cus, fast, s);
+      const StreamInst in = stream_inst(dm, a, sc, l, rowblocks);
+      launch_stream(in, plan, dm->d_stab, l.counters, l.slow, cus, fast, s);
       if (timed) BIE_HIP_CHECK(hipEventRecord(ev[2], s));
+      launch_stream_mid(in, plan, dm->d_stab, fast, s);
     }
   } else if (timed) {
     BIE_HIP_CHECK(hipEventRecord(ev[1], s));
@@ -1290,8 +1291,7 @@ int bie_assemble(const bie_mesh* mesh, double k_re, double k_im, const double* t
   if (rc != BIE_OK) return rc;
   bie_dmesh* dm = handle.get();
   // targets equal to the mesh sources value for value are collocation (the reference's own
-  // call passes mesh.sources as in_sources): the collocation path then applies (recorded
-  // mid-edge pairs, no M x E pair queue)
+  // call passes mesh.sources as in_sources): no copy of them is uploaded
   if (targets && n_targets == mesh->n_sources &&
       (n_targets == 0 || std::memcmp(targets, mesh->sources, 24 * (size_t)n_targets) == 0))
     targets = nullptr;
@@ -1321,6 +1321,12 @@ int bie_assemble(const bie_mesh* mesh, double k_re, double k_im, const double* t
       copy_to_host(G, dG, fg * sizeof(double));
     }
     if (M) BIE_HIP_CHECK(hipMemcpy(C, dC, 16 * M, hipMemcpyDeviceToHost));
+    // the kept mesh holds no pair list between calls
+    std::lock_guard<std::mutex> lk(dm->mu);
+    if (dm->lists.mid_queue) {
+      BIE_HIP_CHECK(hipDeviceSynchronize());  // another thread's call may have been enqueued
+      free_lists(dm->lists);
+    }
   });
   dfree(dT);
   dfree(dF);
@@ -1848,7 +1854,7 @@ int bie_host_cache_info(int64_t* hits, int64_t* builds, int64_t* n_sources,
       *queue_entries = 0;
       if (c.dm) {
         std::lock_guard<std::mutex> dl(c.dm->mu);
-        *queue_entries = std::max(c.dm->lists.mid_cap, c.dm->slists.mid_cap);
+        *queue_entries = c.dm->lists.mid_cap;
       }
     }
   });
@@ -2403,18 +2409,19 @@ int bie_batch_tune(bie_batch* b, const double* k_re, const double* k_im, uint32_
     BIE_HIP_CHECK(hipEventCreate(&e1));
     struct Cand {
       int T, S, order;
+      bool fitted;
     };
-    std::vector<Cand> cands;
+    std::vector<Cand> cands{{64, 0, 0, true}};  // the batch's own choice (as if not configured)
     for (int T : {32, 64, 128})
       for (int S : {32, 0})
-        for (int o : {0, 1}) cands.push_back(Cand{T, S, o});
+        for (int o : {0, 1}) cands.push_back(Cand{T, S, o, false});
     double best = INFINITY;
     Cand pick = cands[0];
     try {
       for (const Cand& c : cands) {
         {
           std::lock_guard<std::mutex> bl(b->mu);
-          b->fitted = false;
+          b->fitted = c.fitted;
           b->elems_per_tile = c.T;
           b->slots = c.S;
           b->order = c.order;
@@ -2440,6 +2447,7 @@ int bie_batch_tune(bie_batch* b, const double* k_re, const double* k_im, uint32_
     (void)hipEventDestroy(e1);
     {
       std::lock_guard<std::mutex> bl(b->mu);
+      b->fitted = pick.fitted;
       b->elems_per_tile = pick.T;
       b->slots = pick.S;
       b->order = pick.order;

@@ -110,7 +110,10 @@ constexpr int kSlotWaves = 8;   // elements per step of the schedule check
 constexpr int kSlotCount = 64;  // LDS slots of the schedule check (64 rows x 4 doubles each)
 constexpr int kLdsBytes = 160 * 1024;  // LDS per CU (one workgroup of the slot kernels)
 
-constexpr int kStageMaxQ = 16;  // vertex rules up to this length are staged in LDS per wave
+// Vertex rules up to this length are staged in LDS per wave: three rules of 16 rows are three
+// 16-byte loads per lane, all that the registers hold beside a pair; longer ones are read from
+// memory in the point loop.
+constexpr int kStageMaxQ = 16;
 
 // Table of (cos, sin)(j pi / 64), j < kTrigN, for the table-driven sincos of the slot
 // kernels.
@@ -197,6 +200,9 @@ StreamPlan stream_plan(const RuleSet& rs, bool flat, bool gon, int slots = 0);
 void launch_stream_prep(const StreamPrep& p, hipStream_t s);
 void launch_stream(const StreamInst& in, const StreamPlan& pl, const double* d_tab,
                    unsigned* d_counters, int* d_slow, int cus, bool fast, hipStream_t s);
+// the mid-edge pairs it listed
+void launch_stream_mid(const StreamInst& in, const StreamPlan& pl, const double* d_tab,
+                       bool fast, hipStream_t s);
 
 // One instance of an uneven batch: its assembly and schedule, and the columns to zero.
 struct BatchInst {

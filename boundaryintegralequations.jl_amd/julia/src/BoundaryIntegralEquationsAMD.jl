@@ -119,7 +119,7 @@ function assemble_hip(mesh::BIE.Mesh3d, k::Number, in_sources::AbstractMatrix;
     srcs = Matrix{Float64}(mesh.sources)
     ptopo = Matrix{Int64}(mesh.physics_topology)
     # collocation (the sources themselves, or an equal array: the library also recognises
-    # value-identical targets) passes NULL, which selects the recorded mid-edge pairs
+    # value-identical targets) passes NULL (no copy of them is uploaded)
     collocation = in_sources === mesh.sources || in_sources == mesh.sources
     targets = collocation ? srcs : Matrix{Float64}(in_sources)
     M = size(targets, 2)

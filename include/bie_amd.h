@@ -110,7 +110,7 @@ int bie_version(void);
  * C: M complex, caller-allocated; disabled outputs are zero-filled (as :308-310).
  * Rule selection for any target reads mesh sources (defined behaviour; the reference
  * indexes the targets there, :325/:436, which is only valid for collocation).
- * The device form of the last mesh (upload, rule tables, schedule, recorded mid-edge pairs)
+ * The device form of the last mesh (upload, rule tables, schedule)
  * is kept for the next call: a call whose mesh matches it byte for byte skips that setup
  * (a frequency loop calling assemble_parallel! once per k); device memory it holds is
  * released when another mesh replaces it or the process ends.  Outputs of 256 MiB or more
@@ -122,9 +122,9 @@ int bie_assemble(const bie_mesh* mesh, double k_re, double k_im, const double* t
 
 /* State of the host-array entry point's kept mesh (no counterpart in the reference):
  * calls that reused it (hits), meshes uploaded (builds), its n_sources (-1: none kept) and
- * the entries of its mid-edge pair queue (0 when none is held; any pointer may be NULL).
- * Targets equal to the mesh sources value for value are collocation; the pair queue of
- * other targets is released when the call returns. */
+ * the entries of its mid-edge pair list (0 when none is held; any pointer may be NULL).
+ * Targets equal to the mesh sources value for value are collocation; the pair list is
+ * released when the call returns. */
 int bie_host_cache_info(int64_t* hits, int64_t* builds, int64_t* n_sources,
                         int64_t* queue_entries);
 /* Releases the kept mesh (its device memory is freed when no call is using it) and the
@@ -296,7 +296,7 @@ int bie_taylor_expand_device(int32_t n_terms, int64_t n, const double* dA, int64
  * Collocation assembly (targets = each mesh's sources) of many meshes of different sizes,
  * each with its own wavenumber, in one persistent kernel launch: every workgroup stages
  * the shared basis table once and takes (instance, 64-row block, element segment) tiles
- * from a device counter.  All meshes share geometry and physics kinds and the rule set
+ * from a device counter; unless configured, the segments suit the batch's work.  All meshes share geometry and physics kinds and the rule set
  * (n, m); each instance i writes its own F_i, G_i (N_i x N_i, column-major complex128) and
  * C_i (N_i), same values as bie_assemble_device on that mesh.  Arrays of per-instance
  * values (k_re, k_im, dF, dG, dC) live on the host; the pointers in dF / dG / dC are device
@@ -318,7 +318,8 @@ int bie_batch_info(bie_batch* b, int32_t* elems_per_tile, int32_t* slots, int32_
 int bie_batch_assemble(bie_batch* b, const double* k_re, const double* k_im, uint32_t flags,
                        double* const* dF, double* const* dG, double* const* dC, void* stream);
 /* Autotuner: times every schedule in {32, 64, 128} elements per tile x {32, 64} slots x
- * {longest-first, interleaved} on these inputs (synchronising), keeps the fastest and
+ * {longest-first, interleaved} and the one the batch chooses unconfigured (reported as 64
+ * elements, 0 slots, order 0) on these inputs (synchronising), keeps the fastest and
  * leaves its outputs in dF / dG / dC; *best_ms (may be NULL) receives its time. */
 int bie_batch_tune(bie_batch* b, const double* k_re, const double* k_im, uint32_t flags,
                    double* const* dF, double* const* dG, double* const* dC, void* stream,
@@ -336,7 +337,7 @@ int bie_batch_tune(bie_batch* b, const double* k_re, const double* k_im, uint32_
  * examples/2d_optimization.jl:184-216). */
 /* The batched assembly (bie_batch_assemble with these arguments) captured into a HIP graph:
  * kernels only (fill kernels for the zeroing, no memset nodes), with the graph's own copies of
- * the instance table, the tile list and the tile counter, and its own mid-edge pair queues
+ * the instance table, the tile list and the tile counter, and its own mid-edge pair lists
  * (quadratic physics); launching it replays the batch on any stream (bie_graph_launch),
  * destroying it frees those (bie_graph_destroy).  The graph keeps the output pointers and
  * the meshes' rule tables and schedules: replays must not overlap other work on the batch

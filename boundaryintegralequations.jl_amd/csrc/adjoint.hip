@@ -72,8 +72,17 @@ __device__ __forceinline__ void points_flat(const double* tab, int Q, Point poin
   }
 }
 
-template <int NG, int NP, bool CPLX>
-__global__ void __launch_bounds__(256) k_adjoint(const AdjointArgs a, int ech) {
+// Curved elements: one target per thread, the element the same for the whole wave (its nodes
+// and p in scalar registers, so that two waves fit a SIMD).  Bound by FP64 issue, some 220
+// instructions per point.  3242 quadratic nodes, 16 points: 2.72 -> 2.00 ms with the table
+// sincos and the second wave.
+template <int NG, int NP, bool CPLX, bool FAST>
+__global__ void __launch_bounds__(256, 2)
+k_adjoint(const AdjointArgs a, int ech, const double* trig) {
+  __shared__ double s_trig[kTrigDoubles + kExpN];
+  for (int t = threadIdx.x; t < kTrigDoubles + kExpN; t += 256) s_trig[t] = trig[t];
+  __syncthreads();
+  const Trig tr = make_trig(s_trig);
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   const bool active = i < a.M;
   const int64_t ic = active ? i : (a.M - 1);
@@ -90,16 +99,17 @@ __global__ void __launch_bounds__(256) k_adjoint(const AdjointArgs a, int ech) {
     double X[NG][3];
 #pragma unroll
     for (int q = 0; q < NG; ++q) {
-      const int node = a.topo[(size_t)e * NG + q];
+      const int node = sload(a.topo + (size_t)e * NG + q);
 #pragma unroll
-      for (int d = 0; d < 3; ++d) X[q][d] = a.coords[3 * (size_t)node + d];
+      for (int d = 0; d < 3; ++d) X[q][d] = sload(a.coords + 3 * (size_t)node + d);
     }
     double pr[NP], pim[NP];
 #pragma unroll
     for (int s = 0; s < NP; ++s) {
-      const double2 v = a.p[a.ptopo[(size_t)e * NP + s]];
-      pr[s] = v.x;
-      pim[s] = v.y;
+      const double* v =
+          reinterpret_cast<const double*>(a.p + sload(a.ptopo + (size_t)e * NP + s));
+      pr[s] = sload(v);
+      pim[s] = sload(v + 1);
     }
     double gX[NG][3];
 #pragma unroll
@@ -138,12 +148,13 @@ __global__ void __launch_bounds__(256) k_adjoint(const AdjointArgs a, int ech) {
       }
       const double A1r = w * (al.x * phr - al.y * phi_), A1i = w * (al.x * phi_ + al.y * phr);
       const double A2r = w * be.x;
-      double sn, cs;
-      sincos_f64(k * r, &sn, &cs);
+      double sn, cs, damp;
+      Phase<CPLX, FAST> ph;
+      ph.begin(k * r, CPLX ? ki * r : 0.0, tr);
+      ph.end(tr, sn, cs, damp);
       if (CPLX) {  // e^{ikr} = e^{-Im k r} e^{i Re k r}
-        const double ex = exp(-ki * r);
-        cs *= ex;
-        sn *= ex;
+        cs *= damp;
+        sn *= damp;
       }
       const double i4r = kInv4Pi * rinv;            // 1/(4 pi r)
       const double i4r3 = i4r * rinv * rinv;        // 1/(4 pi r^3)
@@ -644,11 +655,21 @@ void launch_adjoint(const AdjointArgs& a, int gk, int pk, bool flat, bool cplx, 
   const int ech = (int)((a.E + chunks - 1) / chunks);
   chunks = (a.E + ech - 1) / ech;
   const dim3 grid((unsigned)rowblocks, (unsigned)chunks);
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a, ech); };
-  if (gk == 6 && pk == 6)
-    cplx ? go(k_adjoint<6, 6, true>) : go(k_adjoint<6, 6, false>);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a, ech, d_tab + tab_doubles);
+  };
+  auto by_fast = [&](auto np, auto cx) {
+    constexpr int N = decltype(np)::value;
+    constexpr bool C = decltype(cx)::value;
+    fast ? go(k_adjoint<6, N, C, true>) : go(k_adjoint<6, N, C, false>);
+  };
+  auto by_np = [&](auto np) {
+    cplx ? by_fast(np, std::true_type{}) : by_fast(np, std::false_type{});
+  };
+  if (pk == 6)
+    by_np(std::integral_constant<int, 6>{});
   else
-    cplx ? go(k_adjoint<6, 3, true>) : go(k_adjoint<6, 3, false>);
+    by_np(std::integral_constant<int, 3>{});
   BIE_HIP_CHECK(hipGetLastError());
 }
 

@@ -363,7 +363,7 @@ constexpr int64_t kApplyScratchComplex = int64_t(1) << 20;
 void zgemm_device_noalloc(int64_t M, int64_t nrhs, int64_t K, const double* dA, int64_t lda,
                           const double* dX, int64_t ldx, double* dY, int64_t ldy,
                           hipStream_t s);
-// d_tab: stream_tables (flat elements); fast: every |k| r is below the fast sincos bound
+// d_tab: stream_tables; fast: every |k| r is below the fast sincos bound
 void launch_adjoint(const AdjointArgs& a, int gk, int pk, bool flat, bool cplx, bool fast,
                     const double* d_tab, int tab_doubles, int cus, hipStream_t s);
 // tiles: (64-row block, chunk of ech elements) of every instance, rows fastest; d_basis: flat

@@ -1128,7 +1128,7 @@ int bie_element_geometry(bie_dmesh* dm, int32_t rule, int32_t n, int32_t m, doub
 namespace {
 
 // The host-array entry point keeps the device form of the last mesh it was given (upload,
-// rule tables, slot schedule, recorded mid-edge pairs), so a caller that assembles one
+// rule tables, schedules), so a caller that assembles one
 // mesh at many wavenumbers - a frequency loop calling assemble_parallel! once per k - pays
 // that setup once.  A mesh is matched byte for byte against a copy of its fields and
 // arrays.  The cache is never destroyed (device memory is released with the process, not

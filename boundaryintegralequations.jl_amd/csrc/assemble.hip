@@ -202,13 +202,6 @@ k_assemble(const AssemblyArgs a, int ech) {
 
 }  // namespace
 
-__global__ void k_zero_u32(unsigned* p) { *p = 0u; }
-
-void launch_fill_zero_u32(unsigned* p, hipStream_t s) {
-  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, p);
-  BIE_HIP_CHECK(hipGetLastError());
-}
-
 void launch_fill_zero(double* p, int64_t n_doubles, hipStream_t s) {
   if (n_doubles <= 0) return;
   const int64_t n2 = n_doubles / 2;

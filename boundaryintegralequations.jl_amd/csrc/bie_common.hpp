@@ -33,7 +33,7 @@ struct Error {
 
 constexpr double kPi = 3.14159265358979323846;
 
-// Bound on |x| for the branch-free table sincos of the slot kernels (sincos_tab_fast): 2^46,
+// Bound on |x| for the branch-free table sincos (Phase with FAST, stream_device.hpp): 2^46,
 // so that 64 |x| / pi stays below 2^51 and its rounding by an added 1.5 * 2^52 is exact.
 // The host chooses that form only when |k| times a bound on every target-to-element-point
 // distance is below it.
@@ -340,7 +340,6 @@ void geometry_basis(int kind, double u, double v, double* N, double* du, double*
 
 // Launchers (assemble.hip)
 void launch_fill_zero(double* p, int64_t n_doubles, hipStream_t s);
-void launch_fill_zero_u32(unsigned* p, hipStream_t s);
 void launch_geometry(const double* coords, const int* topo, int gk, int E,
                      const double* d_pts, int Pe, double* elem, hipStream_t s);
 void launch_gather_selnodes(const double* sources, const int* ptopo, int NP, int E,

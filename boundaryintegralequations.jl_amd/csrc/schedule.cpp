@@ -293,6 +293,12 @@ struct StreamNodes {
         ++count[node];
       }
   }
+  // the most contributions to one node
+  int most() const {
+    int best = 0;
+    for (int node : touched) best = std::max(best, count[node]);
+    return best;
+  }
   // the largest number of slots held at once: a node holds one from its first position to
   // kStreamLag past its last; a node with a single contribution needs none
   int front(size_t n) const {
@@ -322,7 +328,7 @@ StreamSchedule build_stream_schedule(const int* ptopo, int NP, int E, int N, con
     std::iota(all.begin(), all.end(), 0);
     auto fits = [&](const std::vector<int>& idx) {
       nd.sweep(idx, ptopo, NP);
-      return nd.front(idx.size()) <= S;
+      return nd.front(idx.size()) <= S && nd.most() <= kStreamMost;
     };
     split(std::move(all), std::max(1, min_segments), cent, fits, segs);
   }
@@ -408,7 +414,7 @@ void validate_stream_schedule(const StreamSchedule& sc, const int* ptopo, int NP
           if (x.count != 1) fail("direct node with several contributions");
           continue;
         }
-        if (x.slot >= sc.S || x.count < 2) fail("slot out of range");
+        if (x.slot >= sc.S || x.count < 2 || x.count > kStreamMost) fail("slot out of range");
         Hold& h = hold[x.slot];
         if (h.node != node) {
           if (h.got != h.count) fail("slot handed on before its node is complete");

@@ -1,4 +1,4 @@
-// Slot schedule of the LDS-accumulator assembly kernel (built by schedule.cpp).
+// Schedules of the LDS-accumulator assembly kernels (built by schedule.cpp).
 #pragma once
 
 #include <cstdint>
@@ -53,6 +53,8 @@ struct StreamSchedule {
 // earliest (any positive distance is correct; a few positions keep the waves, which run
 // that far apart, from waiting for each other).
 constexpr int kStreamLag = 6;
+// A slot's claims and finished contributions are counted in 16 bits each.
+constexpr int kStreamMost = 0xffff;
 StreamSchedule build_stream_schedule(const int* ptopo, int NP, int E, int N, const double* cent,
                                      int S, int min_segments);
 void validate_stream_schedule(const StreamSchedule& sc, const int* ptopo, int NP, int E, int N);

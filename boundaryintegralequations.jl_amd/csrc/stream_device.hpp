@@ -86,8 +86,12 @@ __device__ __forceinline__ Trig make_trig(const double* t) {
 }
 
 // e^{ikr} in two stages, so that the table entries are under way while the caller reads what
-// it needs next: the argument reductions and table reads (sincos_tab_fast's), then the
-// polynomials.  The damping e^{x}, x = -Im k r: x = (64 i + j) ln 2 / 64 + d with |d| <=
+// it needs next: the argument reductions and table reads, then the polynomials.  FAST, for
+// |x| < kTabFastMaxArg: sincos_tab without its branch; n = rint(64 x / pi) is formed by adding
+// 1.5 * 2^52 to x * 64 / pi inside one fused multiply-add (the sum's unit in the last place is
+// 1, so it is rounded to an integer there), the reduction uses n = sum - 1.5 * 2^52 (exact), and
+// the table index n mod 128 is the low bits of the sum's mantissa (two's complement for negative
+// n).  NaN and infinite x give NaN (the index is masked into the table whatever the bits are).  The damping e^{x}, x = -Im k r: x = (64 i + j) ln 2 / 64 + d with |d| <=
 // ln 2 / 128, 2^(j/64) from the table, e^d by its Taylor polynomial to d^5 (truncation below
 // 4e-17), the exponent by ldexp; arguments beyond the range of a double are clamped there.
 template <bool CPLX, bool FAST>

@@ -164,7 +164,7 @@ struct StreamLists {
 struct StreamRun {
   const double* tab;        // stream_tables
   unsigned* counters;       // kStreamCounters
-  int* slow;                // tiles left to the second launch
+  int* slow;                // tiles left to the second launch, or NULL: there is none
   int tab_doubles, S, row_doubles, mids;
 };
 

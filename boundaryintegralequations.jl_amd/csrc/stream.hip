@@ -754,7 +754,8 @@ void launch_stream(const StreamInst& in, const StreamPlan& pl, const double* d_t
   const bool cplx = in.a.ki != 0.0, gon = (in.a.flags & BIE_G) != 0;
   const int grid = (int)std::min<int64_t>(tiles, cus);
   const int mode = pl.flat ? kFlat : (pl.row_doubles ? kStaged : kRead);
-  const StreamRun run{d_tab, d_counters, d_slow, pl.tab_doubles, pl.S, pl.row_doubles,
+  // (fast: no list, no tile is left out)
+  const StreamRun run{d_tab, d_counters, fast ? nullptr : d_slow, pl.tab_doubles, pl.S, pl.row_doubles,
                       pl.mids ? 1 : 0};
   // not known to be fast: the tiles that are not are left to a second launch
   for (int pass = 0; pass < (fast ? 1 : 2); ++pass) {
@@ -799,7 +800,8 @@ void launch_stream_batch(const BatchInst* d_inst, int n_inst, int64_t max_cols,
   BIE_REQUIRE(pl.S > 0 && pl.shmem <= (size_t)kLdsBytes, BIE_EINVAL,
               "internal: batch kernel without LDS slots");
   const int mode = pl.flat ? kFlat : (pl.row_doubles ? kStaged : kRead);
-  const StreamRun run{d_tab, d_counters, d_slow, pl.tab_doubles, pl.S, pl.row_doubles,
+  // (fast: no list, no tile is left out)
+  const StreamRun run{d_tab, d_counters, fast ? nullptr : d_slow, pl.tab_doubles, pl.S, pl.row_doubles,
                       pl.mids ? 1 : 0};
   for (int pass = 0; pass < (fast ? 1 : 2); ++pass) {
     with_stream_kernel<true>(NP, mode, cplx, gon, pass == 0, [&](auto kern) {

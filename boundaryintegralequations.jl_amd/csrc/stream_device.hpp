@@ -628,7 +628,7 @@ __device__ __forceinline__ void stream_run(InstOf inst_of, KmaxOf kmax_of, First
       const double* x = in->a.targets + 3 * min((int64_t)rb * 64 + lane, in->a.M - 1);
       const double cx = x[0] - in->center[0], cy = x[1] - in->center[1], cz = x[2] - in->center[2];
       const double far = kmax_of(in, tile) * (sqrt(fma(cx, cx, fma(cy, cy, cz * cz))) + in->reach);
-      skip = __any(!(far < 0.5 * kTabFastMaxArg));
+      skip = run.slow && __any(!(far < 0.5 * kTabFastMaxArg));
       if (skip && threadIdx.x == 0) run.slow[atomicAdd(run.counters + kSlowCount, 1u)] = tile;
     }
     if (!skip) body(in, rb, seg, tile, parity);

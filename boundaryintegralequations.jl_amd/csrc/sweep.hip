@@ -718,7 +718,8 @@ void launch_sweep(const StreamInst& in, const SweepArgs& sw, const StreamPlan& p
   BIE_REQUIRE(tiles > 0 && tiles < 2147483647LL, BIE_EINVAL, "too many sweep tiles");
   BIE_REQUIRE(pl.S > 0 && pl.shmem <= (size_t)kLdsBytes, BIE_EINVAL,
               "internal: sweep kernel without LDS slots");
-  const StreamRun run{d_tab, d_counters, d_slow, pl.tab_doubles, pl.S, 0, pl.mids ? 1 : 0};
+  const StreamRun run{d_tab, d_counters, fast ? nullptr : d_slow, pl.tab_doubles, pl.S, 0,
+                      pl.mids ? 1 : 0};
   for (int pass = 0; pass < (fast ? 1 : 2); ++pass)
     with_sweep_kernel(in.a.NP, pl.flat, tay, cplx, gon, pass == 0, [&](auto kern, auto mid) {
       BIE_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),

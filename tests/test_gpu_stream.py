@@ -204,3 +204,22 @@ def test_near_field_of_a_far_source():
     assert np.max(np.abs(G.data - G2.data)[near]) <= 1e-14 * np.max(np.abs(G.data))
     assert np.max(np.abs(F.data - F2.data)[near]) <= 1e-14 * np.max(np.abs(G.data))
     assert np.isfinite(F2.data).all() and 0 < np.max(np.abs(G2.data[~near])) < 1e-12
+
+
+@pytest.mark.parametrize("kind", ["linear", "quadratic"])
+def test_a_source_that_is_not_a_number(kind):
+    """Its row is NaN, its elements take the rules the reference's comparisons leave them; the
+    other rows are the oracle's.  (No bound on |k| r holds for its tile, and no second launch
+    exists to leave it to.)"""
+    mesh = M.icosphere(3 if kind == "linear" else 2, kind)
+    src = mesh.sources.copy()
+    src[:, 5] = np.nan
+    mesh = M.Mesh3d(mesh.coordinates, mesh.topology, src, mesh.physics_topology,
+                    mesh.geometry_kind, mesh.physics_kind)
+    rows = np.arange(mesh.n_sources) != 5
+    Fo, Go, Co = oracle.assemble(mesh, 3.0, n=3, m=3)
+    F, G, C = assemble_parallel(mesh, 3.0, n=3, m=3)
+    T = taylor_assemble(mesh, 3.0, M=0, n=3, m=3)
+    for X, Xo in ((F, Fo), (G, Go), (C, Co), (T[0][:, :, 0], Fo), (T[1][:, :, 0], Go)):
+        assert rel(X[rows], Xo[rows]) <= TOL
+        assert np.isnan(X[5]).any()

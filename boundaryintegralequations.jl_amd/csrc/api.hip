@@ -325,10 +325,24 @@ void ensure_flat(bie_dmesh* dm, hipStream_t s) {
 }
 
 // The schedule of dm in a batch: S slots, at least `segments` segments.  The records of flat
-// elements are written here, once (a single-mesh call writes its own each time).
-bie_dmesh::Stream& ensure_batch_stream(bie_dmesh* dm, int S, int64_t segments, hipStream_t s) {
-  bie_dmesh::Stream& out = dm->bstream;
-  if (out.key == segments && out.S == S && out.d_order) return out;
+// elements are written here, once (a single-mesh call writes its own each time).  The mesh
+// keeps the last few, so that a new batch finds them; a batch and its graphs hold theirs until
+// they let go of it, whatever other batches ask of the mesh meanwhile.
+std::shared_ptr<bie_dmesh::Stream> batch_stream(bie_dmesh* dm, int S, int64_t segments,
+                                                hipStream_t s) {
+  auto& kept = dm->bstreams;
+  for (size_t q = 0; q < kept.size(); ++q)
+    if (kept[q]->key == segments && kept[q]->S == S) {
+      std::rotate(kept.begin(), kept.begin() + q, kept.begin() + q + 1);
+      return kept[0];
+    }
+  const int device = dm->device;
+  std::shared_ptr<bie_dmesh::Stream> sp(new bie_dmesh::Stream, [device](bie_dmesh::Stream* x) {
+    (void)hipSetDevice(device);
+    free_stream(*x);
+    delete x;
+  });
+  bie_dmesh::Stream& out = *sp;
   upload_stream(dm, out,
                 stream_schedule(dm, element_centres(dm), S,
                                 std::max(segments, least_segments(dm))),
@@ -346,7 +360,9 @@ bie_dmesh::Stream& ensure_batch_stream(bie_dmesh* dm, int S, int64_t segments, h
     // another stream's batch may read them before an event of this one is recorded
     BIE_HIP_CHECK(hipStreamSynchronize(s));
   }
-  return out;
+  kept.insert(kept.begin(), sp);
+  if (kept.size() > bie_dmesh::kBatchStreams) kept.pop_back();
+  return sp;
 }
 
 void free_lists(StreamLists& l) {
@@ -704,13 +720,7 @@ void batch_configure(bie_batch* b, const StreamPlan& pl, int cus, hipStream_t s)
       b->fitted ? fitted_elems_per_tile(b->meshes, d0->rs.len[0], b->pk, cus) : b->elems_per_tile;
   const int64_t key = per_tile * 2 + b->order;
   const int S = pl.S;
-  bool current = b->configured_key == key && b->d_tiles != nullptr && b->slots_used == S;
-  // a mesh's batch schedule may have been rebuilt by another batch that shares it
-  for (size_t ii = 0; current && ii < b->meshes.size(); ++ii) {
-    const bie_dmesh::Stream& sc = b->meshes[ii]->bstream;
-    current = sc.d_order != nullptr && sc.S == S && sc.key == b->min_segments[ii];
-  }
-  if (current) return;
+  if (b->configured_key == key && b->d_tiles != nullptr && b->slots_used == S) return;
   struct Tile {
     int elems, inst, rb, seg;
     int64_t rank;
@@ -719,14 +729,14 @@ void batch_configure(bie_batch* b, const StreamPlan& pl, int cus, hipStream_t s)
   const int n_inst = (int)b->meshes.size();
   b->configured_key = -1;
   b->rowblocks.assign(n_inst, 0);
-  b->min_segments.assign(n_inst, 0);
+  std::vector<std::shared_ptr<bie_dmesh::Stream>> streams(n_inst);
   for (int ii = 0; ii < n_inst; ++ii) {
     bie_dmesh* dm = b->meshes[ii];
     const int64_t rbs = (dm->N + 63) / 64;
     b->rowblocks[ii] = rbs;
     const int64_t min_seg = std::max<int64_t>(1, (dm->E + per_tile - 1) / per_tile);
-    b->min_segments[ii] = min_seg;
-    const bie_dmesh::Stream& sc = ensure_batch_stream(dm, S, min_seg, s);
+    streams[ii] = batch_stream(dm, S, min_seg, s);
+    const bie_dmesh::Stream& sc = *streams[ii];
     if (dm->N == 0 || dm->E == 0) continue;
     int64_t rank = 0;
     for (int g = 0; g < sc.segments; ++g) {
@@ -753,6 +763,7 @@ void batch_configure(bie_batch* b, const StreamPlan& pl, int cus, hipStream_t s)
   b->d_slow = dalloc<int>(std::max<size_t>(h.size(), 1));
   b->d_tiles = upload_vec(h, s);
   BIE_HIP_CHECK(hipStreamSynchronize(s));
+  b->streams.swap(streams);  // (the former ones go once nothing holds them)
   b->n_tiles = (int)h.size();
   b->slots_used = S;
   b->configured_key = key;
@@ -816,7 +827,7 @@ BatchPlan batch_fill(bie_batch* b, const double* k_re, const double* k_im, uint3
     const double ki = k_im ? k_im[ii] : 0.0;
     plan.cplx = plan.cplx || ki != 0.0;
     plan.fast = plan.fast && fast_trig_ok(dm, k_re[ii], dm->source_radius);
-    bie_dmesh::Stream& sc = dm->bstream;
+    const bie_dmesh::Stream& sc = *b->streams[ii];
     ensure_lists(dm->blists, plan.pl.mids, dm->N, dm->E, sc.segments, 0);
     BatchInst& bi = b->h_inst[ii];
     bi.s = stream_inst(
@@ -1058,7 +1069,7 @@ int bie_dmesh_destroy(bie_dmesh* dm) {
   dfree(dm->d_eflat);
   for (auto& by_g : dm->stream)
     for (auto& sc : by_g) free_stream(sc);
-  free_stream(dm->bstream);
+  dm->bstreams.clear();
   free_stream(dm->sstream);
   free_stream(dm->lstream);
   free_lists(dm->lists);
@@ -2154,6 +2165,7 @@ struct bie_graph {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   std::vector<void*> owned;  // device buffers the captured kernels read (freed with the graph)
+  std::vector<std::shared_ptr<bie_dmesh::Stream>> streams;  // (batch) their schedules
 };
 
 int bie_sweep_graph_create(bie_dmesh* dm, const double* d_k, int32_t nk,
@@ -2214,6 +2226,7 @@ int bie_graph_destroy(bie_graph* g) {
   if (g->exec) (void)hipGraphExecDestroy(g->exec);
   if (g->graph) (void)hipGraphDestroy(g->graph);
   if (!g->owned.empty()) (void)hipDeviceSynchronize();  // a replay may still read them
+  g->streams.clear();
   for (void* p : g->owned) (void)hipFree(p);
   delete g;
   return BIE_OK;
@@ -2239,6 +2252,7 @@ int bie_batch_graph_create(bie_batch* b, const double* k_re, const double* k_im,
       // gets its own copies of the table, the tile list and the tile counter
       for (bie_dmesh* dm : b->meshes) order_after_previous(dm, cs);
       const BatchPlan plan = batch_fill(b, k_re, k_im, flags, dF, dG, dC, cs);
+      g->streams = b->streams;
       // quadratic instances list their mid-edge pairs: in lists of the graph's own (a mesh's
       // are emptied by every batch call)
       for (int ii = 0; ii < n_inst; ++ii) {

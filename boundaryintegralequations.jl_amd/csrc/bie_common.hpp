@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -430,9 +431,12 @@ struct bie_dmesh {
     std::vector<int> h_seg_begin;  // (batch) host copy, for the tile list
   };
   double* d_eflat = nullptr;     // records of flat elements in element order (k-derivatives)
-  // of single-mesh calls (own rows or others, without or with G), of batches, of sweeps and
-  // k-derivatives (F alone on flat elements: lstream, whose slots are smaller)
-  Stream stream[2][2], bstream, sstream, lstream;
+  // of single-mesh calls (own rows or others, without or with G), of sweeps and k-derivatives
+  // (F alone on flat elements: lstream, whose slots are smaller)
+  Stream stream[2][2], sstream, lstream;
+  // of batches: the last few that batches asked for, shared with the batches that use them
+  static constexpr size_t kBatchStreams = 4;
+  std::vector<std::shared_ptr<Stream>> bstreams;
   bie::StreamLists lists, blists, slists;
   double* d_stab = nullptr;      // its tables for the cached rule set (stream_tables)
   // tile shape of the frequency sweep (bie_sweep_tune): elements per tile (0: one segment per
@@ -471,6 +475,6 @@ struct bie_batch {
   int* d_slow = nullptr;             // tiles left to the launch for large arguments
   unsigned* d_counter = nullptr;
   std::vector<int64_t> rowblocks;
-  std::vector<int64_t> min_segments; // per instance: the schedule the tile list indexes
+  std::vector<std::shared_ptr<bie_dmesh::Stream>> streams;  // per instance: what it indexes
   std::mutex mu;
 };

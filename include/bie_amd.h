@@ -340,9 +340,10 @@ int bie_batch_tune(bie_batch* b, const double* k_re, const double* k_im, uint32_
  * the instance table, the tile list and the tile counter, and its own mid-edge pair lists
  * (quadratic physics); launching it replays the batch on any stream (bie_graph_launch),
  * destroying it frees those (bie_graph_destroy).  The graph keeps the output pointers and
- * the meshes' rule tables and schedules: replays must not overlap other work on the batch
- * or its meshes, and reconfiguring or tuning the batch, assembling its meshes with another
- * rule set (n, m), or destroying either invalidates it.
+ * the meshes' rule tables: replays must not overlap other work on the batch or its meshes,
+ * and assembling its meshes with another rule set (n, m) or destroying them invalidates it.
+ * Other batches on the same meshes, and reconfiguring, tuning or destroying this one, do not:
+ * the graph holds its schedules.
  * No counterpart in the reference (a persistent launch captured in a graph is the GPU form
  * of its per-mesh loop). */
 int bie_batch_graph_create(bie_batch* b, const double* k_re, const double* k_im,

@@ -1,0 +1,77 @@
+"""Schedules and lists that several users of one mesh hold side by side: what one of them asks
+for leaves the others' alone."""
+import numpy as np
+import pytest
+
+from bie_amd import mesh as M
+from bie_amd.assembly import Batch, DeviceMesh
+from gpu_helpers import DevBuf, rel, sync
+
+pytestmark = pytest.mark.gpu
+
+
+def outputs(meshes):
+    return [(DevBuf(16 * x.n_sources**2), DevBuf(16 * x.n_sources**2), DevBuf(16 * x.n_sources))
+            for x in meshes]
+
+
+def pointers(bufs):
+    return [[b[i].ptr for b in bufs] for i in range(3)]
+
+
+def values(bufs):
+    sync()
+    return [[x.download(np.empty(x.nbytes // 16, dtype=np.complex128)) for x in b] for b in bufs]
+
+
+def spoil(bufs):
+    for b in bufs:
+        for x in b:
+            x.upload(np.full(x.nbytes // 8, np.nan))
+
+
+@pytest.mark.parametrize("kind", ["linear", "quadratic"])
+def test_a_batch_graph_and_another_batch_on_its_mesh(kind):
+    """Unconfigured batches that share a mesh fit different segments to it.  A graph of one is
+    replayed between eager calls of the others, and every result stays the first one's."""
+    small, large = (8, 16) if kind == "linear" else (4, 8)
+    meshes = [M.icosphere(small, kind), M.ellipsoid(large, (1.0, 0.7, 1.3), kind)]
+    dms = [DeviceMesh(x) for x in meshes]
+    a, b, c = Batch(dms[:1], n=3, m=2), Batch(dms, n=3, m=2), Batch(dms[1:], n=3, m=2)
+    ka, kb = [2.0], [3.0, 1.5]
+    ba, bb, bc = outputs(meshes[:1]), outputs(meshes), outputs(meshes[1:])
+    a.assemble(ka, *pointers(ba))
+    ref_a = values(ba)
+    g = a.graph(ka, *pointers(ba))
+    b.assemble(kb, *pointers(bb))
+    ref_b = values(bb)
+    c.assemble(kb[1:], *pointers(bc))
+    # the case that is meant: the batches cut the shared meshes into different segments
+    assert a.info()["n_tiles"] + c.info()["n_tiles"] != b.info()["n_tiles"]
+    gb = b.graph(kb, *pointers(bb))
+    for _ in range(3):
+        spoil(ba), spoil(bb), spoil(bc)
+        sync()
+        g.launch()
+        gb.launch()
+        c.assemble(kb[1:], *pointers(bc))
+        for got, ref in zip(values(ba) + values(bb) + values(bc), ref_a + ref_b + ref_b[1:]):
+            for x, y in zip(got, ref):
+                assert rel(x, y) < 1e-14
+        b.assemble(kb, *pointers(bb))
+        a.assemble([4.0], *pointers(ba))
+    # schedules are let go of with the last that holds them
+    b.configure(32, 0, 0)
+    b.assemble(kb, *pointers(bb))
+    b.close()
+    spoil(ba), spoil(bb)
+    sync()
+    g.launch()
+    gb.launch()
+    for got, ref in zip(values(ba) + values(bb), ref_a + ref_b):
+        for x, y in zip(got, ref):
+            assert rel(x, y) < 1e-14
+    g.close()
+    gb.close()
+    a.close()
+    c.close()

@@ -15,6 +15,7 @@
 #include <mutex>
 #include <new>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "bie_common.hpp"
@@ -381,25 +382,21 @@ void ensure_lists(StreamLists& l, bool mids, int64_t M, int64_t E, int segments,
   const int64_t cap =
       std::min<int64_t>(std::min<int64_t>(pairs, pairs / 16 + (1 << 18)), 1LL << 30);
   const int64_t tiles = (M + 63) / 64 * segments;
-  if (mids && (l.mid_cap < cap || l.mid_tiles_cap < tiles)) {
-    if (l.mid_queue) (void)hipDeviceSynchronize();  // a launch may still use them
-    dfree(l.mid_queue);
-    dfree(l.mid_tiles);
-    l.mid_queue = l.mid_tiles = nullptr;
-    l.mid_cap = l.mid_tiles_cap = 0;
-    l.mid_queue = dalloc<int2>((size_t)cap);
-    l.mid_tiles = dalloc<int2>((size_t)tiles);
-    l.mid_cap = cap;
-    l.mid_tiles_cap = tiles;
+  // (each grows by itself: calls of many rows and few segments and of few and many take turns)
+  auto grow = [](auto*& x, int64_t& have, int64_t want) {
+    if (have >= want) return;
+    if (x) (void)hipDeviceSynchronize();  // a launch may still use it
+    dfree(x);
+    x = nullptr;
+    have = 0;
+    x = dalloc<std::remove_reference_t<decltype(*x)>>((size_t)want);
+    have = want;
+  };
+  if (mids) {
+    grow(l.mid_queue, l.mid_cap, cap);
+    grow(l.mid_tiles, l.mid_tiles_cap, tiles);
   }
-  if (l.slow_cap < slow_tiles) {
-    if (l.slow) (void)hipDeviceSynchronize();
-    dfree(l.slow);
-    l.slow = nullptr;
-    l.slow_cap = 0;
-    l.slow = dalloc<int>((size_t)slow_tiles);
-    l.slow_cap = slow_tiles;
-  }
+  grow(l.slow, l.slow_cap, slow_tiles);
 }
 
 StreamInst stream_inst(const bie_dmesh* dm, const AssemblyArgs& a, const bie_dmesh::Stream& sc,
@@ -593,9 +590,10 @@ void assemble_device_impl(bie_dmesh* dm, double kr, double ki, const double* d_t
       const bool fast = fast_trig_ok(dm, kr, target_radius);
       const int cus = device_cus(dm->device);
       const bool own_rows = d_targets == dm->d_sources && M == dm->N;
-      bie_dmesh::Stream& sc = ensure_stream(
-          dm, dm->stream[own_rows ? 0 : 1][(flags & BIE_G) ? 1 : 0], plan.S, rowblocks, cus, s);
-      StreamLists& l = dm->lists;
+      const int kind = own_rows ? 0 : 1, with_g = (flags & BIE_G) ? 1 : 0;
+      bie_dmesh::Stream& sc =
+          ensure_stream(dm, dm->stream[kind][with_g], plan.S, rowblocks, cus, s);
+      StreamLists& l = dm->lists[kind][with_g];
       ensure_lists(l, plan.mids, M, dm->E, sc.segments, fast ? 0 : rowblocks * sc.segments);
       launch_stream_prep(stream_prep(dm, a, sc, l, 1, 0), s);
       if (timed) BIE_HIP_CHECK(hipEventRecord(ev[1], s));
@@ -1072,7 +1070,8 @@ int bie_dmesh_destroy(bie_dmesh* dm) {
   dm->bstreams.clear();
   free_stream(dm->sstream);
   free_stream(dm->lstream);
-  free_lists(dm->lists);
+  for (auto& by_g : dm->lists)
+    for (auto& l : by_g) free_lists(l);
   free_lists(dm->blists);
   free_lists(dm->slists);
   delete dm;
@@ -1334,10 +1333,12 @@ int bie_assemble(const bie_mesh* mesh, double k_re, double k_im, const double* t
     if (M) BIE_HIP_CHECK(hipMemcpy(C, dC, 16 * M, hipMemcpyDeviceToHost));
     // the kept mesh holds no pair list between calls
     std::lock_guard<std::mutex> lk(dm->mu);
-    if (dm->lists.mid_queue) {
-      BIE_HIP_CHECK(hipDeviceSynchronize());  // another thread's call may have been enqueued
-      free_lists(dm->lists);
-    }
+    for (auto& by_g : dm->lists)
+      for (auto& l : by_g)
+        if (l.mid_queue) {
+          BIE_HIP_CHECK(hipDeviceSynchronize());  // another thread's call may have been enqueued
+          free_lists(l);
+        }
   });
   dfree(dT);
   dfree(dF);
@@ -1865,7 +1866,8 @@ int bie_host_cache_info(int64_t* hits, int64_t* builds, int64_t* n_sources,
       *queue_entries = 0;
       if (c.dm) {
         std::lock_guard<std::mutex> dl(c.dm->mu);
-        *queue_entries = c.dm->lists.mid_cap;
+        for (const auto& by_g : c.dm->lists)
+          for (const auto& l : by_g) *queue_entries += l.mid_cap;
       }
     }
   });

@@ -437,7 +437,7 @@ struct bie_dmesh {
   // of batches: the last few that batches asked for, shared with the batches that use them
   static constexpr size_t kBatchStreams = 4;
   std::vector<std::shared_ptr<Stream>> bstreams;
-  bie::StreamLists lists, blists, slists;
+  bie::StreamLists lists[2][2], blists, slists;  // (lists: as stream)
   double* d_stab = nullptr;      // its tables for the cached rule set (stream_tables)
   // tile shape of the frequency sweep (bie_sweep_tune): elements per tile (0: one segment per
   // row block) and LDS slots (0: as many as fit)

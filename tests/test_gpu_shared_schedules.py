@@ -75,3 +75,32 @@ def test_a_batch_graph_and_another_batch_on_its_mesh(kind):
     gb.close()
     a.close()
     c.close()
+
+
+def test_a_captured_assembly_and_calls_of_other_rows():
+    """A caller's own capture of the collocation assembly, replayed between calls with other
+    rows (some of them more than the mesh's) and without G, whose pair lists are larger: they
+    are not the captured call's."""
+    import torch
+    mesh = M.icosphere(4, "quadratic")
+    N, n, m, k = mesh.n_sources, 3, 2, 3.0
+    dm = DeviceMesh(mesh)
+    F, G, C = outputs([mesh])[0]
+    more = 6 * N
+    t = DevBuf(24 * more)
+    t.upload(1.5 * np.random.default_rng(1).standard_normal((more, 3)))
+    Ff, Gf, Cf = DevBuf(16 * more * N), DevBuf(16 * more * N), DevBuf(16 * more)
+    dm.assemble(k, F.ptr, G.ptr, C.ptr, n=n, m=m)
+    ref = values([(F, G, C)])[0]
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+        dm.assemble(k, F.ptr, G.ptr, C.ptr, n=n, m=m, stream=stream.cuda_stream)
+    for rows in (more, 70, N + 1):
+        dm.assemble(k, Ff.ptr, Gf.ptr, Cf.ptr, n=n, m=m, targets_ptr=t.ptr, n_targets=rows)
+        dm.assemble(k, Ff.ptr, Gf.ptr, Cf.ptr, n=n, m=m, gOn=False)
+        spoil([(F, G, C)])
+        sync()
+        graph.replay()
+        torch.cuda.synchronize()
+        for x, y in zip(values([(F, G, C)])[0], ref):
+            assert rel(x, y) < 1e-14

@@ -415,16 +415,18 @@ __device__ __forceinline__ double wave_total(double v) {
   return (at(0) + at(16)) + (at(32) + at(48));
 }
 
-template <bool CPLX, bool FAST>
+// LONG: the rules' points stay in memory (see launch_adjoint_flat).
+template <bool CPLX, bool FAST, bool LONG>
 __global__ void __launch_bounds__(256, 2)
 k_adjoint_flat(const AdjointArgs a, int rows, const double* tab_src, int tab_doubles,
                int check) {
   extern __shared__ double lds[];
-  double* gx = lds + tab_doubles + kTrigDoubles + kExpN;  // rows x 3
-  for (int t = threadIdx.x; t < tab_doubles + kTrigDoubles + kExpN; t += 256) lds[t] = tab_src[t];
+  const int skip = LONG ? tab_doubles : 0, n_lds = tab_doubles - skip + kTrigDoubles + kExpN;
+  double* gx = lds + n_lds;  // rows x 3
+  for (int t = threadIdx.x; t < n_lds; t += 256) lds[t] = tab_src[skip + t];
   for (int t = threadIdx.x; t < 3 * rows; t += 256) gx[t] = 0.0;
   __syncthreads();
-  const Trig tr = make_trig(lds + tab_doubles);
+  const Trig tr = make_trig(lds + tab_doubles - skip);
   const int lane = threadIdx.x & 63;
   const int e = blockIdx.x * 256 + threadIdx.x;
   const bool active = e < a.E;
@@ -478,7 +480,7 @@ k_adjoint_flat(const AdjointArgs a, int rows, const double* tab_src, int tab_dou
     }
     const double d0[3] = {X1[0] - x0, X1[1] - x1, X1[2] - x2};
     const double kap = fma(cv[0], d0[0], fma(cv[1], d0[1], cv[2] * d0[2]));
-    const double* tab = lds + c * (4 * Q + 2);
+    const double* tab = (LONG ? tab_src : lds) + c * (4 * Q + 2);
     double H0 = 0, H1 = 0, H2 = 0, T0 = 0, T1 = 0, T2 = 0, T11 = 0, T12 = 0, T22 = 0, Zr = 0,
            Zi = 0;
     points_flat(tab, Q, [&](const double (&b)[4]) {
@@ -622,7 +624,11 @@ static void launch_adjoint_flat(const AdjointArgs& a, bool cplx, bool fast, cons
   const int64_t chunks = std::max<int64_t>(1, rounds * at_once / eb);
   const int rows = (int)std::min<int64_t>(512, std::max<int64_t>(8, (a.M + chunks - 1) / chunks));
   const int64_t ny = (a.M + rows - 1) / rows;
-  const size_t shmem = sizeof(double) * (size_t)(tab_doubles + kTrigDoubles + kExpN + 3 * rows);
+  // Rules of up to 48 KB (510 points) come from LDS: with the rows' sums that is below the
+  // 64 KB of a plain launch, and two workgroups fit a CU.  Longer ones come from memory.
+  const bool in_lds = sizeof(double) * (size_t)tab_doubles <= 48 * 1024;
+  const size_t shmem =
+      sizeof(double) * (size_t)((in_lds ? tab_doubles : 0) + kTrigDoubles + kExpN + 3 * rows);
   for (int64_t y0 = 0; y0 < ny; y0 += 65535) {  // (the grid's second dimension ends there)
     AdjointArgs b = a;
     b.targets += 3 * y0 * rows;
@@ -636,8 +642,15 @@ static void launch_adjoint_flat(const AdjointArgs& a, bool cplx, bool fast, cons
       hipLaunchKernelGGL(kern, grid, dim3(256), shmem, s, b, rows, d_tab, tab_doubles,
                          fast ? 0 : 1);
     };
-    cplx ? go(k_adjoint_flat<true, true>) : go(k_adjoint_flat<false, true>);
-    if (!fast) cplx ? go(k_adjoint_flat<true, false>) : go(k_adjoint_flat<false, false>);
+    auto by = [&](auto cx, auto fs) {
+      constexpr bool C = decltype(cx)::value, S = decltype(fs)::value;
+      in_lds ? go(k_adjoint_flat<C, S, false>) : go(k_adjoint_flat<C, S, true>);
+    };
+    auto by_fast = [&](auto fs) {
+      cplx ? by(std::true_type{}, fs) : by(std::false_type{}, fs);
+    };
+    by_fast(std::true_type{});
+    if (!fast) by_fast(std::false_type{});
   }
   BIE_HIP_CHECK(hipGetLastError());
 }

@@ -223,3 +223,29 @@ def test_a_source_that_is_not_a_number(kind):
     for X, Xo in ((F, Fo), (G, Go), (C, Co), (T[0][:, :, 0], Fo), (T[1][:, :, 0], Go)):
         assert rel(X[rows], Xo[rows]) <= TOL
         assert np.isnan(X[5]).any()
+
+
+@pytest.mark.parametrize("nm", [(22, 23), (16, 32), (40, 41), (64, 64)])
+@pytest.mark.parametrize("k", [3.0, 2.0 + 0.3j])
+def test_flat_adjoint_of_long_rules(nm, k):
+    """Rules on both sides of what the kernel takes into LDS, and up to the longest there are.
+    (The oracle's n.d of a node's own elements is rounding noise, 1e-17, which its derivative
+    takes times 3 w / r^4: with Gauss points 3.5e-4 from the corner about 1e-11 of the
+    functional's terms; held to 1e-9 of their sum.)"""
+    from bie_amd.adjoint import assembly_vjp, source_nodes
+    from dual_oracle import assemble_F_C
+    mesh = M.perturb_radial(M.icosphere(1, "linear"), 0.01, 4)
+    n, m = nm
+    rng = np.random.default_rng(n)
+    N = mesh.n_sources
+    alpha, beta, p = (rng.standard_normal(N) + 1j * rng.standard_normal(N) for _ in range(3))
+    g, gk = assembly_vjp(DeviceMesh(mesh), k, alpha, p, beta=beta,
+                         target_node=source_nodes(mesh), n=n, m=m)
+    rules = oracle.select(mesh, None)
+    V = rng.standard_normal(mesh.coordinates.shape)
+    for dX, dk, got in ((V, 0.0, float(np.sum(g * V))),
+                        (np.zeros_like(V), 1.0, float(np.atleast_1d(gk)[0]))):
+        F, C = assemble_F_C(mesh, mesh.coordinates, dX, k, dk, rules, targets=None, n=n, m=m)
+        dd = np.real(alpha @ (F.d @ p) + beta @ C.d)
+        scale = np.abs(alpha) @ (np.abs(F.d) @ np.abs(p)) + np.abs(beta) @ np.abs(C.d)
+        assert abs(got - dd) <= 1e-9 * scale

@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "bie_common.hpp"
@@ -415,20 +416,23 @@ __device__ __forceinline__ double wave_total(double v) {
   return (at(0) + at(16)) + (at(32) + at(48));
 }
 
-// LONG: the rules' points stay in memory (see launch_adjoint_flat).
+// LONG: the rules' points stay in memory.  ew: waves that share 64 elements, each taking every
+// ew-th row (see launch_adjoint_flat).
 template <bool CPLX, bool FAST, bool LONG>
 __global__ void __launch_bounds__(256, 2)
-k_adjoint_flat(const AdjointArgs a, int rows, const double* tab_src, int tab_doubles,
+k_adjoint_flat(const AdjointArgs a, int rows, int ew, const double* tab_src, int tab_doubles,
                int check) {
   extern __shared__ double lds[];
   const int skip = LONG ? tab_doubles : 0, n_lds = tab_doubles - skip + kTrigDoubles + kExpN;
-  double* gx = lds + n_lds;  // rows x 3
+  double* gx = lds + n_lds;       // rows x 3
+  double* ge = gx + 3 * rows;     // (ew > 1) 9 x 64 node gradients of the elements
   for (int t = threadIdx.x; t < n_lds; t += 256) lds[t] = tab_src[skip + t];
-  for (int t = threadIdx.x; t < 3 * rows; t += 256) gx[t] = 0.0;
+  for (int t = threadIdx.x; t < 3 * rows + (ew > 1 ? 576 : 0); t += 256) gx[t] = 0.0;
   __syncthreads();
   const Trig tr = make_trig(lds + tab_doubles - skip);
   const int lane = threadIdx.x & 63;
-  const int e = blockIdx.x * 256 + threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int e = ew > 1 ? blockIdx.x * 64 + lane : blockIdx.x * 256 + threadIdx.x;
   const bool active = e < a.E;
   const int ec = active ? e : a.E - 1;
   double P[3][3], X1[3], ea[3], eb[3], pr[3], pi[3];
@@ -457,7 +461,7 @@ k_adjoint_flat(const AdjointArgs a, int rows, const double* tab_src, int tab_dou
   double D[3] = {0, 0, 0}, V[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, hn[3] = {0, 0, 0};
   double M1 = 0, M2 = 0, M11 = 0, M12 = 0, M22 = 0, gk = 0, gki = 0;
   const int64_t i0 = (int64_t)blockIdx.y * rows, i1 = min(a.M, i0 + rows);
-  for (int64_t i = i0; i < i1; ++i) {
+  for (int64_t i = i0 + (ew > 1 ? wave : 0); i < i1; i += ew) {
     const double x0 = sload(a.targets + 3 * i), x1 = sload(a.targets + 3 * i + 1),
                  x2 = sload(a.targets + 3 * i + 2);
     if (check) {  // rows whose |k| r may be large are the other launch's
@@ -563,9 +567,13 @@ k_adjoint_flat(const AdjointArgs a, int rows, const double* tab_src, int tab_dou
       const double w0 = fma(cv[d], hn[0], fma(ea[d], M1, fma(eb[d], M2, V[0][d])));
       const double w1 = fma(cv[d], hn[1], fma(ea[d], M11, fma(eb[d], M12, V[1][d])));
       const double w2 = fma(cv[d], hn[2], fma(ea[d], M12, fma(eb[d], M22, V[2][d])));
-      unsafeAtomicAdd(a.gradX + 3 * (size_t)node[0] + d, (w0 - w1 - w2) - (gtu[d] + gtv[d]));
-      unsafeAtomicAdd(a.gradX + 3 * (size_t)node[1] + d, w1 + gtu[d]);
-      unsafeAtomicAdd(a.gradX + 3 * (size_t)node[2] + d, w2 + gtv[d]);
+      const double g[3] = {(w0 - w1 - w2) - (gtu[d] + gtv[d]), w1 + gtu[d], w2 + gtv[d]};
+#pragma unroll
+      for (int s = 0; s < 3; ++s)
+        if (ew > 1)
+          atomicAdd(ge + (3 * s + d) * 64 + lane, g[s]);
+        else
+          unsafeAtomicAdd(a.gradX + 3 * (size_t)node[s] + d, g[s]);
     }
   }
   if (a.gradk) {
@@ -576,8 +584,13 @@ k_adjoint_flat(const AdjointArgs a, int rows, const double* tab_src, int tab_dou
       if (lane == 0) unsafeAtomicAdd(a.gradk + 1, t);
     }
   }
+  if (a.tvert || ew > 1) __syncthreads();
+  if (ew > 1 && active) {
+#pragma unroll
+    for (int q = 0; q < 9; ++q)
+      if (q % 4 == wave) unsafeAtomicAdd(a.gradX + 3 * (size_t)node[q / 3] + q % 3, ge[q * 64 + lane]);
+  }
   if (a.tvert) {
-    __syncthreads();
     for (int t = threadIdx.x; t < 3 * (int)(i1 - i0); t += 256) {
       const int v = a.tvert[i0 + t / 3];
       if (v >= 0) unsafeAtomicAdd(a.gradX + 3 * (size_t)v + t % 3, gx[t]);
@@ -616,19 +629,35 @@ void launch_dfdk_batch(const DfdkInst* d_inst, int n_inst, int n_tiles, int ech,
 }
 
 // Rows per workgroup (256 elements): whole rounds of about two workgroups a CU, of some 64
-// rows each (the lanes' atomics and element data are then a per cent of the work).
+// rows each (the lanes' atomics and element data are then a per cent of the work).  Meshes of
+// up to 2048 elements leave most of the chip idle that way, and a row's points are a serial
+// chain: there the four waves of a workgroup share 64 elements and divide the rows, as long as
+// the workgroups fit the chip at once.  Their rows grow as sqrt(M): every further workgroup
+// shortens the chain and adds atomics to the same nodes.  (16 points, one wave per element,
+// then four: 42 nodes 39 and 18 us, 162 nodes 47 and 28, 642 nodes 95 and 55; 200 field rows
+// on 720 elements 71 and 41; one row, or 5120 elements and 30 rows, are 5-10 % slower.)
 static void launch_adjoint_flat(const AdjointArgs& a, bool cplx, bool fast, const double* d_tab,
                                 int tab_doubles, int cus, hipStream_t s) {
-  const int64_t eb = (a.E + 255) / 256, at_once = 2 * (int64_t)cus;
+  int64_t eb = (a.E + 255) / 256;
+  const int64_t at_once = 2 * (int64_t)cus, eb64 = (a.E + 63) / 64;
   const int64_t rounds = std::max<int64_t>(1, (eb * a.M / 64 + at_once / 2) / at_once);
   const int64_t chunks = std::max<int64_t>(1, rounds * at_once / eb);
-  const int rows = (int)std::min<int64_t>(512, std::max<int64_t>(8, (a.M + chunks - 1) / chunks));
+  int rows = (int)std::min<int64_t>(512, std::max<int64_t>(8, (a.M + chunks - 1) / chunks));
+  const int shared_rows = 4 * (int)std::min(8.0, std::ceil(0.3 * std::sqrt((double)a.M)));
+  const int ew = a.M > 4 && eb64 <= 32 &&
+                         eb64 * ((a.M + shared_rows - 1) / shared_rows) <= at_once
+                     ? 4
+                     : 1;
+  if (ew > 1) {
+    eb = eb64;
+    rows = shared_rows;
+  }
   const int64_t ny = (a.M + rows - 1) / rows;
   // Rules of up to 48 KB (510 points) come from LDS: with the rows' sums that is below the
   // 64 KB of a plain launch, and two workgroups fit a CU.  Longer ones come from memory.
   const bool in_lds = sizeof(double) * (size_t)tab_doubles <= 48 * 1024;
-  const size_t shmem =
-      sizeof(double) * (size_t)((in_lds ? tab_doubles : 0) + kTrigDoubles + kExpN + 3 * rows);
+  const size_t shmem = sizeof(double) * (size_t)((in_lds ? tab_doubles : 0) + kTrigDoubles +
+                                                 kExpN + 3 * rows + (ew > 1 ? 576 : 0));
   for (int64_t y0 = 0; y0 < ny; y0 += 65535) {  // (the grid's second dimension ends there)
     AdjointArgs b = a;
     b.targets += 3 * y0 * rows;
@@ -639,7 +668,7 @@ static void launch_adjoint_flat(const AdjointArgs& a, bool cplx, bool fast, cons
     const dim3 grid((unsigned)eb, (unsigned)std::min<int64_t>(65535, ny - y0));
     b.M = std::min<int64_t>(b.M, (int64_t)grid.y * rows);
     auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, grid, dim3(256), shmem, s, b, rows, d_tab, tab_doubles,
+      hipLaunchKernelGGL(kern, grid, dim3(256), shmem, s, b, rows, ew, d_tab, tab_doubles,
                          fast ? 0 : 1);
     };
     auto by = [&](auto cx, auto fs) {

@@ -249,3 +249,27 @@ def test_flat_adjoint_of_long_rules(nm, k):
         dd = np.real(alpha @ (F.d @ p) + beta @ C.d)
         scale = np.abs(alpha) @ (np.abs(F.d) @ np.abs(p)) + np.abs(beta) @ np.abs(C.d)
         assert abs(got - dd) <= 1e-9 * scale
+
+
+@pytest.mark.parametrize("f,rows", [(1, None), (3, 3), (3, 5), (6, None), (10, 37), (11, 33)])
+def test_flat_adjoint_of_few_elements(f, rows):
+    """Waves that share their elements and divide the rows: elements short of a wave, rows short
+    of a workgroup's, both sides of the sizes (2048 elements, 4 rows) where it begins."""
+    from bie_amd.adjoint import assembly_vjp, source_nodes
+    from dual_oracle import assemble_F_C
+    mesh = M.perturb_radial(M.icosphere(f, "linear"), 0.01, 4)
+    rng = np.random.default_rng(f)
+    t = None if rows is None else np.asfortranarray(M.fibonacci_sphere(rows, 1.7))
+    N, Mt = mesh.n_sources, rows or mesh.n_sources
+    alpha, beta = (rng.standard_normal(Mt) + 1j * rng.standard_normal(Mt) for _ in range(2))
+    p = rng.standard_normal(N) + 1j * rng.standard_normal(N)
+    rules = oracle.select(mesh, t)
+    V = rng.standard_normal(mesh.coordinates.shape)
+    dm = DeviceMesh(mesh)
+    for k in (3.0, 2.0 + 0.3j):
+        g, _ = assembly_vjp(dm, k, alpha, p, beta=beta, targets=t, n=3, m=3,
+                            target_node=source_nodes(mesh) if t is None else None)
+        F, C = assemble_F_C(mesh, mesh.coordinates, V, k, 0.0, rules, targets=t, n=3, m=3)
+        dd = np.real(alpha @ (F.d @ p) + beta @ C.d)
+        scale = np.abs(alpha) @ (np.abs(F.d) @ np.abs(p)) + np.abs(beta) @ np.abs(C.d)
+        assert abs(float(np.sum(g * V)) - dd) <= 1e-10 * scale

@@ -1592,6 +1592,9 @@ void sparse_assemble_impl(bie_sparse* sp, double kr, double ki, const double* d_
   L.trig = sp->d_trig;
   // (the radius of explicit sources is not known here)
   L.fast = fast_trig_ok(dm, kr, d_sources ? -1.0 : dm->source_radius);
+  L.explicit_src = d_sources != nullptr;
+  for (int d = 0; d < 3; ++d) L.center[d] = dm->center[d];
+  L.reach = 4.0 * dm->coord_radius;
   L.batches = sp->d_batches;
   L.n_batches = sp->n_batches;
   for (int c = 0; c < 6; ++c) {

@@ -299,6 +299,8 @@ struct SparseLaunch {
   const double* rules;    // point records (u, v, w, 0), sparse_record_doubles() each (device)
   const double* trig;     // (cos, sin)(j pi / 64), interleaved, then 2^(j / 64) (device)
   bool fast;              // every |k| r is below the fast sincos bound
+  bool explicit_src = false;  // the caller's sources: not known here whether they are
+  double center[3], reach;    // every element point is within reach of the centre
   int off[6], len[6];     // per geometry node: first record and point count
   int NG, NP, hyp;
   const int* batches = nullptr;  // pair batches sharing an element (device; 8 ints each)

@@ -54,6 +54,8 @@ struct SparseArgs {
   int off[6], len[6];
   const int* batches;     // 8 ints per batch: element, count, up to 4 pair indices
   int64_t n_batches;
+  bool check;             // (batches) waves of near and far rows are a launch each
+  double center[3], reach; // every element point is within reach of the centre
   int hyp;
   bool disc;              // discontinuous physics, nodes at beta
   double beta;
@@ -425,7 +427,8 @@ constexpr int batch_rows(int NP) { return NP == 1 ? 4 : NP == 3 ? 3 : 2; }
 // once and the kernels for every row of the batch that selected that rule - the surface
 // (~2/3 of the per-point work) is shared.  Each row's rule is selected here exactly as in
 // k_sparse_pairs, so explicit sources stay correct (they only share less).
-template <int NG, int NP, int B, bool CPLX, bool FAST>
+// CHECK: compiled apart (in the loop's registers its few instructions cost 3 %).
+template <int NG, int NP, int B, bool CPLX, bool FAST, bool CHECK>
 __global__ void __launch_bounds__(256, 2) k_sparse_batch(const SparseArgs a) {
   const int64_t b =
       (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -435,6 +438,16 @@ __global__ void __launch_bounds__(256, 2) k_sparse_batch(const SparseArgs a) {
   const int lane = threadIdx.x & 63;
   const int* rec = a.batches + (size_t)b * 8;
   const int e = rec[0], cnt = rec[1];
+  if (CHECK && a.check) {  // whether the batch is this launch's (the whole wave leaves together)
+    bool near = true;
+    for (int j = 0; j < cnt; ++j) {
+      const double* x = a.src + 3 * (size_t)a.pairs[rec[2 + j]].x;
+      const double cx = x[0] - a.center[0], cy = x[1] - a.center[1], cz = x[2] - a.center[2];
+      const double far = fabs(a.kr) * (sqrt(fma(cx, cx, fma(cy, cy, cz * cz))) + a.reach);
+      near = near && far < 0.5 * kTabFastMaxArg;
+    }
+    if (__builtin_amdgcn_readfirstlane((int)near) != (FAST ? 1 : 0)) return;
+  }
   Surface<NG> sf;
   sparse_element<NG>(a, e, sf);
   double xs[B][3];
@@ -491,6 +504,8 @@ void launch_sparse_pairs(const SparseLaunch& L, hipStream_t s) {
     a.off[c] = L.off[c];
     a.len[c] = L.len[c];
   }
+  for (int d = 0; d < 3; ++d) a.center[d] = L.center[d];
+  a.reach = L.reach;
   a.hyp = L.hyp;
   a.batches = L.batches;
   a.n_batches = L.n_batches;
@@ -521,10 +536,20 @@ void launch_sparse_pairs(const SparseLaunch& L, hipStream_t s) {
     if (shortr)
       L.fast ? run(k_sparse_pairs_short<NG, NP, C, true>)
              : run(k_sparse_pairs_short<NG, NP, C, false>);
-    else if (batched)
-      L.fast ? run(k_sparse_batch<NG, NP, B, C, true>) : run(k_sparse_batch<NG, NP, B, C, false>);
-    else
+    else if (batched) {
+      // Explicit sources: the waves whose rows are near and the others are a launch each, the
+      // second as a rule empty (4 us).  The full reduction beside the sums of several rows
+      // takes more registers than there are: all waves with it, two launches, and sources known
+      // to be near (us, depth 2): 1962 linear nodes 606, 557, 515; complex k 931, 663, 638;
+      // 2562 quadratic nodes 2095, 1833, 1822; disctrilinear on 720 quadratic elements 935,
+      // 704, 690.
+      a.check = L.explicit_src && !L.fast;
+      if (L.fast) run(k_sparse_batch<NG, NP, B, C, true, false>);
+      if (a.check) run(k_sparse_batch<NG, NP, B, C, true, true>);
+      if (!L.fast) run(k_sparse_batch<NG, NP, B, C, false, true>);
+    } else {
       L.fast ? run(k_sparse_pairs<NG, NP, C, true>) : run(k_sparse_pairs<NG, NP, C, false>);
+    }
   };
   auto by_cx = [&](auto ng, auto np) {
     cplx ? pick(ng, np, std::true_type()) : pick(ng, np, std::false_type());

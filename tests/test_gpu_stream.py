@@ -273,3 +273,32 @@ def test_flat_adjoint_of_few_elements(f, rows):
         dd = np.real(alpha @ (F.d @ p) + beta @ C.d)
         scale = np.abs(alpha) @ (np.abs(F.d) @ np.abs(p)) + np.abs(beta) @ np.abs(C.d)
         assert abs(float(np.sum(g * V)) - dd) <= 1e-10 * scale
+
+
+@pytest.mark.parametrize("kind,physics", [("linear", "geometry"), ("quadratic", "geometry"),
+                                          ("quadratic", "disctrilinear"),
+                                          ("linear", "disctriconstant")])
+@pytest.mark.parametrize("k", [3.0, 2.0 + 0.3j])
+def test_near_field_batches_with_far_sources(kind, physics, k):
+    """Explicit sources of batches of pairs: those with a source beyond the range of the
+    branch-free sincos, or one that is not a number, are the other launch's; each pair is some
+    launch's, once."""
+    from bie_amd.assembly import sparse_assemble_parallel
+    mesh = M.ellipsoid(3 if kind == "linear" else 2, axes=(1.2, 1.0, 0.7), order=kind)
+    if physics != "geometry":
+        mesh = M.with_discontinuous_physics(mesh, physics)
+    pts = np.array(mesh.sources, order="F")
+    F0, G0 = sparse_assemble_parallel(mesh, k, depth=2)
+    F, G = sparse_assemble_parallel(mesh, k, pts, depth=2)
+    scale = max(np.max(np.abs(F0.data)), np.max(np.abs(G0.data)))
+    assert np.max(np.abs(F.data - F0.data)) <= 1e-14 * scale
+    assert np.max(np.abs(G.data - G0.data)) <= 1e-14 * scale
+    pts[:, 7] = (0.0, 0.0, 5e14)
+    pts[:, 20] = np.nan
+    F2, G2 = sparse_assemble_parallel(mesh, k, pts, depth=2)
+    rows = np.repeat(np.arange(F.shape[0]), np.diff(F.indptr))
+    others = (rows != 7) & (rows != 20)
+    assert np.max(np.abs(F2.data - F0.data)[others]) <= 1e-14 * scale
+    assert np.max(np.abs(G2.data - G0.data)[others]) <= 1e-14 * scale
+    assert np.isfinite(G2.data[rows == 7]).all() and np.max(np.abs(G2.data[rows == 7])) < 1e-12
+    assert np.isnan(G2.data[rows == 20]).all() and np.isnan(F2.data[rows == 20]).all()

@@ -552,10 +552,13 @@ __device__ __forceinline__ void flat_record(const StreamPrep& p, int t) {
   }
   const double c0 = a[1] * b[2] - a[2] * b[1], c1 = a[2] * b[0] - a[0] * b[2],
                c2 = a[0] * b[1] - a[1] * b[0];
-  o[18] = -c0;
-  o[19] = -c1;
-  o[20] = -c2;
-  o[21] = sqrt(c0 * c0 + c1 * c1 + c2 * c2);
+  const double J = sqrt(c0 * c0 + c1 * c1 + c2 * c2);
+  // n = -c / J is not a number, or times J not c, where J leaves the range: F and C are NaN
+  const bool normal = J > 0.0 && J < INFINITY;
+  o[18] = normal ? -c0 : NAN;
+  o[19] = normal ? -c1 : NAN;
+  o[20] = normal ? -c2 : NAN;
+  o[21] = J;
   o[22] = o[23] = 0.0;
 }
 

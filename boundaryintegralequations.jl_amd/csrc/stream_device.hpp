@@ -424,14 +424,16 @@ __device__ __forceinline__ void mid_pair_add(InstPtr in, const MidOut& o, int64_
     const double c0 = tu[2] * tv[1] - tu[1] * tv[2], c1 = tu[0] * tv[2] - tu[2] * tv[0],
                  c2 = tu[1] * tv[0] - tu[0] * tv[1];  // n J
     const double J2 = fma(c0, c0, fma(c1, c1, c2 * c2));
-    const double J = J2 * rsqrt_nr(J2);
+    // n = -c / J is not a number where J is 0 or infinite: F and C are NaN there
+    const bool normal = J2 > 0.0 && J2 < INFINITY;
+    const double J = normal ? J2 * rsqrt_nr(J2) : J2;
     const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
     const double rinv = rsqrt_nr(r2);
     const double r = r2 * rinv;
     const double krr = kr * r, kir = CPLX ? ki * r : 0.0;
     Phase<CPLX, FAST> ph;
     ph.begin(krr, kir, tr);
-    const double nd = fma(c0, dx, fma(c1, dy, c2 * dz));
+    const double nd = normal ? fma(c0, dx, fma(c1, dy, c2 * dz)) : NAN;
     const double g = w * rinv, t = rinv * rinv;
     csum = fma(-nd, t * g, csum);
     double Fr, Fi, Gr, Gi;

@@ -302,3 +302,58 @@ def test_near_field_batches_with_far_sources(kind, physics, k):
     assert np.max(np.abs(G2.data - G0.data)[others]) <= 1e-14 * scale
     assert np.isfinite(G2.data[rows == 7]).all() and np.max(np.abs(G2.data[rows == 7])) < 1e-12
     assert np.isnan(G2.data[rows == 20]).all() and np.isnan(F2.data[rows == 20]).all()
+
+
+def with_collapsed_element(kind):
+    """A sphere and one more element, of no area: its first two vertices are the origin.  (The
+    third is at powers of two: the tangent's terms then cancel whether they are rounded or
+    fused.)"""
+    mesh = M.icosphere(3 if kind == "linear" else 2, kind)
+    B = np.array([0.25, 0.5, -0.125])
+    extra = [0 * B, 0 * B, B] + ([0 * B, B / 2, B / 2] if kind == "quadratic" else [])
+    X = np.concatenate([mesh.coordinates, np.array(extra).T], axis=1)
+    T = np.concatenate([mesh.topology, mesh.n_coordinates + np.arange(len(extra))[:, None]], axis=1)
+    return M.Mesh3d(X, T, X.copy(), T.copy(), mesh.geometry_kind, mesh.physics_kind)
+
+
+@pytest.mark.parametrize("kind", ["linear", "quadratic"])
+def test_an_element_of_no_area(kind, monkeypatch):
+    """The reference divides by the Jacobian: F in its columns and C are not numbers, G is what
+    the other elements leave, on every path and for every rule (mid-edge ones among them).  (But
+    for the rows of its own mid-edge nodes, which lie on points of its rules: 0 / 0.)"""
+    from bie_amd.assembly import Batch
+    mesh = with_collapsed_element(kind)
+    N, k = mesh.n_sources, 3.0
+    Fo, Go, Co = oracle.assemble(mesh, k, n=3, m=2)
+    hole, some = np.isnan(Fo), np.isfinite(Go)
+    assert np.isnan(Co).all() and hole.any() and some[:-2].all()
+    rules = oracle.select(mesh, None)[:, -1]
+    assert kind == "linear" or (rules > 3).any()
+
+    def check(F, G, C):
+        assert (np.isnan(F) == hole).all() and np.isnan(C).all()
+        assert rel(F[~hole], Fo[~hole]) <= TOL
+        assert G is None or rel(G[some], Go[some]) <= TOL
+
+    check(*assemble_parallel(mesh, k, n=3, m=2))
+    F, _, C = assemble_parallel(mesh, k, n=3, m=2, gOn=False)
+    check(F, None, C)
+    F, G, C = sweep(mesh, [k, 4.0], mesh.sources, 3, 2)
+    check(F[0], G[0], C)
+    F, G, C = taylor_assemble(mesh, k, M=1, n=3, m=2)
+    check(F[:, :, 0], G[:, :, 0], C)
+    F, _, C = taylor_assemble(mesh, k, M=1, n=3, m=2, gOn=False)
+    check(F[:, :, 0], None, C)
+    monkeypatch.setenv("BIE_AMD_KERNEL", "atomic")
+    check(*assemble_parallel(mesh, k, n=3, m=2))
+    monkeypatch.delenv("BIE_AMD_KERNEL")
+    b = Batch([DeviceMesh(mesh)], n=3, m=2)
+    F, G, C, w = DevBuf(16 * N * N), DevBuf(16 * N * N), DevBuf(16 * N), DevBuf(16)
+    b.assemble([k], [F.ptr], [G.ptr], [C.ptr])
+    sync()
+    check(*[x.download(np.empty(s, dtype=np.complex128, order="F"))
+            for x, s in ((F, (N, N)), (G, (N, N)), (C, (N,)))])
+    one = DevBuf(16 * N)
+    one.upload(np.ones(N, dtype=np.complex128))
+    b.dfdk([k], [one.ptr], [one.ptr], w.ptr)
+    assert np.isnan(w.download(np.empty(1, dtype=np.complex128))).all()

@@ -466,7 +466,7 @@ k_adjoint_flat(const AdjointArgs a, int rows, int ew, const double* tab_src, int
                  x2 = sload(a.targets + 3 * i + 2);
     if (check) {  // rows whose |k| r may be large are the other launch's
       const double cx = x0 - a.center[0], cy = x1 - a.center[1], cz = x2 - a.center[2];
-      const double far = fabs(k) * (sqrt(fma(cx, cx, fma(cy, cy, cz * cz))) + a.reach);
+      const double far = fmax(fabs(k), kFastMinK) * (sqrt(fma(cx, cx, fma(cy, cy, cz * cz))) + a.reach);
       if (__builtin_amdgcn_readfirstlane((int)(far < 0.5 * kTabFastMaxArg)) != (FAST ? 1 : 0))
         continue;
     }
@@ -511,7 +511,9 @@ k_adjoint_flat(const AdjointArgs a, int rows, int ew, const double* tab_src, int
       const double u = CPLX ? fma(krr, zi, fma(kir, zr, zr)) : fma(krr, zi, zr);
       const double H = q3 * (be + u);
       const double kz = CPLX ? fma(k2r, zr, -(k2i * zi)) : k2r * zr;
-      const double T = fma(q3, kz, -3.0 * rinv2 * H);
+      // (FAST: without kappa, which is multiplied in below)
+      const double kr2 = FAST ? rinv2 : kap * rinv2;
+      const double T = FAST ? fma(q3, kz, -3.0 * rinv2 * H) : fma(kr2 * q1, kz, -3.0 * kr2 * H);
       Zr = fma(q1, zr, Zr);
       if (CPLX) Zi = fma(q1, zi, Zi);
       H0 += H;
@@ -525,17 +527,18 @@ k_adjoint_flat(const AdjointArgs a, int rows, int ew, const double* tab_src, int
       T12 = fma(t1, b[2], T12);
       T22 = fma(t2, b[2], T22);
     });
-    T0 *= kap;
-    T1 *= kap;
-    T2 *= kap;
+    const double kapt = FAST ? kap : 1.0;
+    T0 *= kapt;
+    T1 *= kapt;
+    T2 *= kapt;
     hn[0] += H0;
     hn[1] += H1;
     hn[2] += H2;
     M1 += T1;
     M2 += T2;
-    M11 = fma(kap, T11, M11);
-    M12 = fma(kap, T12, M12);
-    M22 = fma(kap, T22, M22);
+    M11 = fma(kapt, T11, M11);
+    M12 = fma(kapt, T12, M12);
+    M22 = fma(kapt, T22, M22);
     double gd[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {

@@ -114,11 +114,13 @@ __device__ __forceinline__ void pair_rows(double x0, double x1, double x2,
 
 // Pair on a flat three-node element with its own linear physics: tab holds {N1, N2, N3,
 // w / (4 pi)} per point; a, b are the edges from node 1, d0 = X1 - x.  The sums leave out
-// the constant factors J (of G) and n.d J (of F and C), which the caller multiplies in.
+// the constant factors J (of G) and n.d J (of F and C), which the caller multiplies in; where
+// lengths may be anywhere in the range (not FAST) 1 / r^3 is not formed by itself, and F and C
+// take n.d J here.
 template <bool CPLX, bool GON, bool FAST, bool FIRST>
 __device__ __forceinline__ void point_flat(const double (&d0)[3], const double (&a)[3],
                                            const double (&b)[3], double (&n)[4],
-                                           const double* next, double kr, double ki,
+                                           const double* next, double kr, double ki, double nd,
                                            const Trig& tr, Sums<3, GON>& v, double& c3) {
   const double m[4] = {n[0], n[1], n[2], n[3]};
 #pragma unroll
@@ -134,7 +136,7 @@ __device__ __forceinline__ void point_flat(const double (&d0)[3], const double (
   Phase<CPLX, FAST> e;
   e.begin(krr, kir, tr);
   const double g = m[3] * rinv;
-  const double t = rinv * rinv;
+  const double t = FAST ? rinv * rinv : (nd * rinv) * rinv;
   c3 = FIRST ? t * g : fma(t, g, c3);
   double Fr, Fi, Gr, Gi;
   kernels_end<CPLX, FAST>(e, g, t, krr, kir, tr, Fr, Fi, Gr, Gi);
@@ -146,19 +148,19 @@ __device__ __forceinline__ void point_flat(const double (&d0)[3], const double (
 template <bool CPLX, bool GON, bool FAST>
 __device__ __forceinline__ void pair_flat(const double (&d0)[3], const double (&a)[3],
                                           const double (&b)[3], const double* tab, int Q,
-                                          double kr, double ki, const Trig& tr,
+                                          double kr, double ki, double nd, const Trig& tr,
                                           Sums<3, GON>& v, double& c3) {
   double n[4] = {tab[0], tab[1], tab[2], tab[3]};
-  point_flat<CPLX, GON, FAST, true>(d0, a, b, n, tab += 4, kr, ki, tr, v, c3);
+  point_flat<CPLX, GON, FAST, true>(d0, a, b, n, tab += 4, kr, ki, nd, tr, v, c3);
   int q = 1;
   if (!(Q & 1)) {
-    point_flat<CPLX, GON, FAST, false>(d0, a, b, n, tab += 4, kr, ki, tr, v, c3);
+    point_flat<CPLX, GON, FAST, false>(d0, a, b, n, tab += 4, kr, ki, nd, tr, v, c3);
     q = 2;
   }
 #pragma unroll 1
   for (; q < Q; q += 2, tab += 8) {  // two points at a time
-    point_flat<CPLX, GON, FAST, false>(d0, a, b, n, tab + 4, kr, ki, tr, v, c3);
-    point_flat<CPLX, GON, FAST, false>(d0, a, b, n, tab + 8, kr, ki, tr, v, c3);
+    point_flat<CPLX, GON, FAST, false>(d0, a, b, n, tab + 4, kr, ki, nd, tr, v, c3);
+    point_flat<CPLX, GON, FAST, false>(d0, a, b, n, tab + 8, kr, ki, nd, tr, v, c3);
   }
 }
 
@@ -350,12 +352,14 @@ __device__ __forceinline__ void stream_tile(InstPtr in, int rb, int seg, int S,
       const double nd = fma(r2[2], d0[0], fma(r2[3], d0[1], r2[4] * d0[2]));  // n.d J
       const double J = r2[5];
       double c3 = 0.0;
-      pair_flat<CPLX, GON, FAST>(d0, ea, eb, tab + c * tab_rule, Q, kr, ki, tr, v, c3);
-      csum = fma(-nd, c3, csum);
+      pair_flat<CPLX, GON, FAST>(d0, ea, eb, tab + c * tab_rule, Q, kr, ki, nd, tr, v, c3);
+      csum = FAST ? fma(-nd, c3, csum) : csum - c3;
 #pragma unroll
       for (int s = 0; s < 3; ++s) {
-        v.fr[s] *= nd;
-        v.fi[s] *= nd;
+        if constexpr (FAST) {
+          v.fr[s] *= nd;
+          v.fi[s] *= nd;
+        }
         if constexpr (GON) {
           v.gr[s] *= J;
           v.gi[s] *= J;

@@ -434,8 +434,8 @@ __device__ __forceinline__ void mid_pair_add(InstPtr in, const MidOut& o, int64_
     Phase<CPLX, FAST> ph;
     ph.begin(krr, kir, tr);
     const double nd = normal ? fma(c0, dx, fma(c1, dy, c2 * dz)) : NAN;
-    const double g = w * rinv, t = rinv * rinv;
-    csum = fma(-nd, t * g, csum);
+    const double g = w * rinv, t = (nd * rinv) * rinv;
+    csum = fma(-t, g, csum);
     double Fr, Fi, Gr, Gi;
     if constexpr (TAY) {  // G = r^m g e^{ikr}, F = t (ikr - 1 + m) G, both times i^m below
       double sn, cs, damp, gm = g, rb = r;
@@ -453,8 +453,6 @@ __device__ __forceinline__ void mid_pair_add(InstPtr in, const MidOut& o, int64_
     } else {
       kernels_end<CPLX, FAST>(ph, g, t, krr, kir, tr, Fr, Fi, Gr, Gi);
     }
-    Fr *= nd;
-    Fi *= nd;
     Gr *= J;
     Gi *= J;
     if (!in->own_basis) {
@@ -629,7 +627,7 @@ __device__ __forceinline__ void stream_run(InstOf inst_of, KmaxOf kmax_of, First
     if constexpr (FAST) {
       const double* x = in->a.targets + 3 * min((int64_t)rb * 64 + lane, in->a.M - 1);
       const double cx = x[0] - in->center[0], cy = x[1] - in->center[1], cz = x[2] - in->center[2];
-      const double far = kmax_of(in, tile) * (sqrt(fma(cx, cx, fma(cy, cy, cz * cz))) + in->reach);
+      const double far = fmax(kmax_of(in, tile), kFastMinK) * (sqrt(fma(cx, cx, fma(cy, cy, cz * cz))) + in->reach);
       skip = run.slow && __any(!(far < 0.5 * kTabFastMaxArg));
       if (skip && threadIdx.x == 0) run.slow[atomicAdd(run.counters + kSlowCount, 1u)] = tile;
     }

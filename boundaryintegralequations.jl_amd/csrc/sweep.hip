@@ -97,12 +97,13 @@ struct Block {
 };
 
 // One point of a flat element: K <= KB wavenumbers; the sums leave out J (of G) and n.d J (of
-// F).  H = G / r^2 runs through the wavenumbers.
+// F).  H = G / r^2 runs through the wavenumbers; not FAST: H = G, and F takes n.d J / r^2 here
+// (as point_flat in stream.hip).
 template <int KB, int K, bool GON, bool FAST, bool REC, bool FIRST>
 __device__ __forceinline__ void sweep_point_flat(const double (&d0)[3], const double (&a)[3],
                                                  const double (&b)[3], double (&n)[4],
                                                  const double* next, const Block<KB>& kv,
-                                                 const Trig& tr, Multi<3, KB, GON>& v,
+                                                 double nd, const Trig& tr, Multi<3, KB, GON>& v,
                                                  double& c3) {
   const double m[4] = {n[0], n[1], n[2], n[3]};
 #pragma unroll
@@ -117,12 +118,16 @@ __device__ __forceinline__ void sweep_point_flat(const double (&d0)[3], const do
   Phase<false, FAST> e0, e1;
   e0.begin(kv.k[0] * r, 0.0, tr);
   if (REC) e1.begin(kv.dk * r, 0.0, tr);
-  const double h = (m[3] * rinv) * (rinv * rinv);
-  c3 = FIRST ? h : c3 + h;
+  const double h = FAST ? (m[3] * rinv) * (rinv * rinv) : m[3] * rinv;
+  const double t = FAST ? 1.0 : (nd * rinv) * rinv;
+  if constexpr (FAST)
+    c3 = FIRST ? h : c3 + h;
+  else
+    c3 = FIRST ? t * h : fma(t, h, c3);
   double w[3];
   if constexpr (GON) {
 #pragma unroll
-    for (int s = 0; s < 3; ++s) w[s] = m[s] * r2;
+    for (int s = 0; s < 3; ++s) w[s] = FAST ? m[s] * r2 : m[s];
   }
   double sn, cs, zs = 0.0, zc = 0.0, damp;
   e0.end(tr, sn, cs, damp);
@@ -144,7 +149,11 @@ __device__ __forceinline__ void sweep_point_flat(const double (&d0)[3], const do
       }
     }
     const double krr = kv.k[q] * r;
-    const double Fr = fma(-krr, Hi, -Hr), Fi = fma(krr, Hr, -Hi);
+    double Fr = fma(-krr, Hi, -Hr), Fi = fma(krr, Hr, -Hi);
+    if constexpr (!FAST) {
+      Fr *= t;
+      Fi *= t;
+    }
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
       plus<FIRST>(v.fr[q][s], Fr, m[s]);
@@ -160,20 +169,45 @@ __device__ __forceinline__ void sweep_point_flat(const double (&d0)[3], const do
 template <int KB, int K, bool GON, bool FAST, bool REC>
 __device__ __forceinline__ void sweep_pair_flat(const double (&d0)[3], const double (&a)[3],
                                                 const double (&b)[3], const double* tab, int Q,
-                                                const Block<KB>& kv, const Trig& tr,
+                                                const Block<KB>& kv, double nd, const Trig& tr,
                                                 Multi<3, KB, GON>& v, double& c3) {
   double n[4] = {tab[0], tab[1], tab[2], tab[3]};
-  sweep_point_flat<KB, K, GON, FAST, REC, true>(d0, a, b, n, tab += 4, kv, tr, v, c3);
+  sweep_point_flat<KB, K, GON, FAST, REC, true>(d0, a, b, n, tab += 4, kv, nd, tr, v, c3);
 #pragma unroll 1
   for (int q = 1; q < Q; ++q)
-    sweep_point_flat<KB, K, GON, FAST, REC, false>(d0, a, b, n, tab += 4, kv, tr, v, c3);
+    sweep_point_flat<KB, K, GON, FAST, REC, false>(d0, a, b, n, tab += 4, kv, nd, tr, v, c3);
+}
+
+// A pair on a flat element (d0 = X1 - x, edges a and b, n.d J, J) whose lengths may be anywhere
+// in the range, in units of a power of two s near the largest of them (exactly), so that the
+// derivatives' 1 / r^3 is formed near 1: k r is k s r then, n.d J w / r^3 and J w / r are what
+// they were, and r^m is in units of s^m.  The exponent of s.
+__device__ __forceinline__ int pair_unit(double (&d0)[3], double (&a)[3], double (&b)[3],
+                                         double& nd, double& J, double& s) {
+  double m = 0.0;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) m = fmax(m, fmax(fabs(d0[d]), fmax(fabs(a[d]), fabs(b[d]))));
+  int e = 0;
+  if (m > 0.0 && m < INFINITY) (void)frexp(m, &e);
+  e = max(-1000, min(1000, e));
+  s = ldexp(1.0, e);
+  const double u = ldexp(1.0, -e);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    d0[d] *= u;
+    a[d] *= u;
+    b[d] *= u;
+  }
+  nd = ((nd * u) * u) * u;
+  J *= u;
+  return e;
 }
 
 // One point of a flat element for the derivative orders m0 .. m0 + K - 1 (m0 even): sums of N r^j e^{ikr} w / (4 pi r), j = m0 - 2 .., without the factors i^j.
 template <int NA, bool CPLX, bool FAST>
 __device__ __forceinline__ void taylor_point_flat(const double (&d0)[3], const double (&a)[3],
                                                   const double (&b)[3], double (&n)[4],
-                                                  const double* next, double kr, double ki,
+                                                  const double* next, double kr, double ki, double unit,
                                                   int m0, const Trig& tr, double (&ac)[NA][3],
                                                   double (&as)[NA][3], double& c3) {
   const double m[4] = {n[0], n[1], n[2], n[3]};
@@ -186,8 +220,9 @@ __device__ __forceinline__ void taylor_point_flat(const double (&d0)[3], const d
   const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
   const double rinv = rsqrt_nr(r2);
   const double r = r2 * rinv;
+  const double ru = FAST ? r : r * unit;  // (see pair_unit)
   Phase<CPLX, FAST> e;
-  e.begin(kr * r, CPLX ? ki * r : 0.0, tr);
+  e.begin(kr * ru, CPLX ? ki * ru : 0.0, tr);
   double q = m[3] * rinv;
   if (m0 == 0) {
     q *= rinv * rinv;
@@ -221,7 +256,8 @@ template <int KB, bool CPLX, bool GON, bool FAST>
 __device__ __forceinline__ void taylor_pair_flat(const double (&d0)[3], const double (&a)[3],
                                                  const double (&b)[3], const double* tab, int Q,
                                                  double kr, double ki, int m0, double nd,
-                                                 double J, const Trig& tr,
+                                                 double J, double unit, int unit_exp,
+                                                 const Trig& tr,
                                                  Multi<3, KB, GON>& v, double& c3) {
   constexpr int NA = KB + (GON ? 2 : 1);
   double ac[NA][3], as[NA][3];
@@ -233,13 +269,13 @@ __device__ __forceinline__ void taylor_pair_flat(const double (&d0)[3], const do
   c3 = 0.0;
 #pragma unroll 1
   for (int q = 0; q < Q; ++q)
-    taylor_point_flat<NA, CPLX, FAST>(d0, a, b, n, tab += 4, kr, ki, m0, tr, ac, as, c3);
+    taylor_point_flat<NA, CPLX, FAST>(d0, a, b, n, tab += 4, kr, ki, unit, m0, tr, ac, as, c3);
   // F_m = (n.d) i^m [(m - 1) A'_{m-2} + i k A'_{m-1}], G_m = J i^m A'_m (A' without i^j)
   if (m0 & 2) {
     nd = -nd;
     J = -J;
   }
-  const double kn = nd * kr, kin = CPLX ? nd * ki : 0.0;
+  const double kn = nd * (FAST ? kr : kr * unit), kin = CPLX ? nd * (FAST ? ki : ki * unit) : 0.0;
 #pragma unroll
   for (int q = 0; q < KB; ++q) {
     const double mn = nd * (double)(m0 + q - 1);
@@ -252,11 +288,19 @@ __device__ __forceinline__ void taylor_pair_flat(const double (&d0)[3], const do
         im = fma(-kin, as[q + 1][s], im);
       }
       rotate(q, re, im);
+      if constexpr (!FAST) {  // r^m in units of s^m
+        re = ldexp(re, unit_exp * (m0 + q));
+        im = ldexp(im, unit_exp * (m0 + q));
+      }
       v.fr[q][s] = re;
       v.fi[q][s] = im;
       if constexpr (GON) {
         double gr = J * ac[q + 2][s], gi = J * as[q + 2][s];
         rotate(q, gr, gi);
+        if constexpr (!FAST) {
+          gr = ldexp(gr, unit_exp * (m0 + q));
+          gi = ldexp(gi, unit_exp * (m0 + q));
+        }
         v.gr[q][s] = gr;
         v.gi[q][s] = gi;
       }
@@ -519,36 +563,42 @@ __device__ __forceinline__ void sweep_tile(InstPtr in, SweepPtr sw, int rb, int 
       const d8 r0 = sload8(rec24), r1 = sload8(rec24 + 8), r2 = sload8(rec24 + 16);
       const double P[3][3] = {{r0[0], r0[1], r0[2]}, {r0[3], r0[4], r0[5]},
                               {r0[6], r0[7], r1[0]}};
-      const double ea[3] = {r1[4], r1[5], r1[6]}, eb[3] = {r1[7], r2[0], r2[1]};
+      double ea[3] = {r1[4], r1[5], r1[6]}, eb[3] = {r1[7], r2[0], r2[1]};
       const int c = select_rule_s<3>(x0, x1, x2, P, rec24, R, in) - 1;
-      const double d0[3] = {r1[1] - x0, r1[2] - x1, r1[3] - x2};
-      const double nd = fma(r2[2], d0[0], fma(r2[3], d0[1], r2[4] * d0[2]));  // n.d J
-      const double J = r2[5];
+      double d0[3] = {r1[1] - x0, r1[2] - x1, r1[3] - x2};
+      double nd = fma(r2[2], d0[0], fma(r2[3], d0[1], r2[4] * d0[2]));  // n.d J
+      double J = r2[5];
       const double* tc = tab + c * tab_rule;
       double c3 = 0.0;
       if constexpr (TAY) {
-        taylor_pair_flat<KB, CPLX, GON, FAST>(d0, ea, eb, tc, Q, kv.k[0], ki, k0, nd, J, tr, v,
-                                              c3);
+        double unit = 1.0;
+        int unit_exp = 0;
+        if constexpr (!FAST) unit_exp = pair_unit(d0, ea, eb, nd, J, unit);
+        taylor_pair_flat<KB, CPLX, GON, FAST>(d0, ea, eb, tc, Q, kv.k[0], ki, k0, nd, J, unit,
+                                              unit_exp, tr, v, c3);
+        csum = fma(-nd, c3, csum);
       } else {
         if (!rec)
-          sweep_pair_flat<KB, KB, GON, FAST, false>(d0, ea, eb, tc, Q, kv, tr, v, c3);
+          sweep_pair_flat<KB, KB, GON, FAST, false>(d0, ea, eb, tc, Q, kv, nd, tr, v, c3);
         else if (KB > 4 && nb <= KB / 2)
-          sweep_pair_flat<KB, KB / 2, GON, FAST, true>(d0, ea, eb, tc, Q, kv, tr, v, c3);
+          sweep_pair_flat<KB, KB / 2, GON, FAST, true>(d0, ea, eb, tc, Q, kv, nd, tr, v, c3);
         else
-          sweep_pair_flat<KB, KB, GON, FAST, true>(d0, ea, eb, tc, Q, kv, tr, v, c3);
+          sweep_pair_flat<KB, KB, GON, FAST, true>(d0, ea, eb, tc, Q, kv, nd, tr, v, c3);
+        csum = FAST ? fma(-nd, c3, csum) : csum - c3;
 #pragma unroll
         for (int q = 0; q < KB; ++q)
 #pragma unroll
           for (int s = 0; s < 3; ++s) {
-            v.fr[q][s] *= nd;
-            v.fi[q][s] *= nd;
+            if constexpr (FAST) {
+              v.fr[q][s] *= nd;
+              v.fi[q][s] *= nd;
+            }
             if constexpr (GON) {
               v.gr[q][s] *= J;
               v.gi[q][s] *= J;
             }
           }
       }
-      csum = fma(-nd, c3, csum);
     } else {
       int c = 0;
       if (R > 1) {

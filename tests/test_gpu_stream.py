@@ -357,3 +357,61 @@ def test_an_element_of_no_area(kind, monkeypatch):
     one.upload(np.ones(N, dtype=np.complex128))
     b.dfdk([k], [one.ptr], [one.ptr], w.ptr)
     assert np.isnan(w.download(np.empty(1, dtype=np.complex128))).all()
+
+
+@pytest.mark.parametrize("kind", ["linear", "quadratic"])
+@pytest.mark.parametrize("far,down", [(210, 110), (365, 220)])
+def test_targets_far_beyond_the_range_of_one_over_r_cubed(kind, far, down):
+    """Targets at 2^far times the body's size, others near: F and C are the same, G is 2^down
+    times as large, an order's derivative and the shape gradient in their units, as for the
+    body and targets 2^down times smaller (every rounding is the same there, so they agree but
+    for the order of operations: 1e-12.  C of a target outside a closed body is 0: it is held
+    to its terms, which are F's.  (The gradient forms 1 / r^4 by itself: up to 2^250.)"""
+    from bie_amd.adjoint import assembly_vjp
+    body = M.perturb_radial(M.icosphere(3 if kind == "linear" else 2, kind), 0.02, 4)
+    rng = np.random.default_rng(far)
+    t = 1.5 * rng.standard_normal((3, 70))
+    t[:, 3::5] *= 2.0 ** far
+    s = 2.0 ** -down
+    small = M.Mesh3d(body.coordinates * s, body.topology, body.sources * s, body.physics_topology,
+                     body.geometry_kind, body.physics_kind)
+    k = 2.0 ** (1 - far)
+    ks = [k, 1.5 * k, 1.75 * k, 3.0 * k, 4.0 * k]
+    alpha = rng.standard_normal(70) + 1j * rng.standard_normal(70)
+    p = rng.standard_normal(body.n_sources) + 1j * rng.standard_normal(body.n_sources)
+    far_rows = np.arange(70) % 5 == 3
+
+    def everything(mesh, u):
+        x = np.asfortranarray(t * u)
+        out = {}
+        for c, kk in (("", k / u), ("c", (k + 0.5j * k) / u)):
+            F, G, C = assemble_parallel(mesh, kk, x, n=3, m=2)
+            out.update({"F" + c: F, "G" + c: G / u, "C" + c: C})
+            F, G, _ = taylor_assemble(mesh, kk, x, M=2, n=3, m=2)
+            Fx = taylor_assemble(mesh, kk, x, M=2, n=3, m=2, gOn=False)[0]
+            for q in range(3):
+                v = u ** -q * (k if q else 1.0) ** q
+                out.update({f"TF{q}" + c: F[:, :, q] * v, f"TG{q}" + c: G[:, :, q] / u * v,
+                            f"TX{q}" + c: Fx[:, :, q] * v})
+            for rows, name in ((far_rows, "far"), (~far_rows, "near")) if far < 250 else ():
+                g, _ = assembly_vjp(DeviceMesh(mesh), kk, alpha[rows], p, targets=x[:, rows], n=3,
+                                    m=2)
+                out[f"V{name}{c}"] = g * u
+        F, G, C = sweep(mesh, np.array(ks) / u, x, 3, 2)
+        Fx = sweep(mesh, np.array(ks) / u, x, 3, 2, gOn=False)[0]
+        for q in range(len(ks)):
+            out.update({f"SF{q}": F[q], f"SG{q}": G[q] / u, f"SX{q}": Fx[q]})
+        out["SC"] = C
+        return out
+
+    big, ref = everything(body, 1.0), everything(small, s)
+    for name, x in big.items():
+        y = ref[name]
+        for rows in ([slice(None)] if name[0] == "V" else [far_rows, ~far_rows]):
+            a, b = x[rows], y[rows]
+            if name in ("C", "Cc", "SC"):
+                b = np.abs(ref["F"][rows]).sum(axis=1)
+                a = x[rows] - y[rows] + b
+            m = np.max(np.abs(b))
+            assert 0 < m < np.inf, name
+            assert np.linalg.norm(a / m - b / m) <= 1e-12 * np.linalg.norm(b / m), name

@@ -165,11 +165,14 @@ struct StreamLists {
   int64_t slow_cap = 0;
 };
 
+// 2^22, which no wait of a valid schedule comes near; BIE_AMD_POLLS sets another number (tests).
+int stream_polls();
 struct StreamRun {
   const double* tab;        // stream_tables
   unsigned* counters;       // kStreamCounters
   int* slow;                // tiles left to the second launch, or NULL: there is none
   int tab_doubles, S, row_doubles, mids;
+  int polls = stream_polls();  // of a wait for another wave, before it gives up
 };
 
 struct StreamPlan {

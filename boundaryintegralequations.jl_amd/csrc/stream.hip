@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdlib>
 #include <type_traits>
 
 #include "bie_common.hpp"
@@ -169,7 +170,8 @@ __device__ __forceinline__ void pair_flat(const double (&d0)[3], const double (&
 // First and middle contributions: into the slot.
 template <int NP, bool GON>
 __device__ __forceinline__ void give(const int4& en, const Roles& r, int lane, double* acc,
-                                     unsigned* claims, const Sums<NP, GON>& v, bool& ok) {
+                                     unsigned* claims, unsigned* ctr, const Sums<NP, GON>& v,
+                                     bool& ok) {
   constexpr int SD = GON ? 256 : 128;
   const bool mine_first = lane_of_mask(r.first), mine_more = lane_of_mask(r.more);
 #pragma unroll
@@ -188,7 +190,10 @@ __device__ __forceinline__ void give(const int4& en, const Roles& r, int lane, d
     if (mine_first) lds_count(claims + en.x, 0x10000u);
   }
   if (r.more) {
-    ok &= spin([&] { return !mine_more || (lds_peek(claims + en.x) >> 16) != 0; });
+    if (!spin(ctr, [&] { return !mine_more || (lds_peek(claims + en.x) >> 16) != 0; })) {
+      ok = false;
+      return;
+    }
 #pragma unroll
     for (int s = 0; s < NP; ++s)
       if ((r.more >> s) & 1) {
@@ -209,14 +214,14 @@ __device__ __forceinline__ void give(const int4& en, const Roles& r, int lane, d
 template <int NP, bool GON>
 __device__ __forceinline__ void finish(InstPtr in, const int4& en, const Roles& r,
                                        int lane, int64_t i0, bool active, const double* acc,
-                                       unsigned* claims, unsigned* turns,
-                                       const Sums<NP, GON>& v, bool& ok) {
+                                       unsigned* claims, unsigned* turns, unsigned* ctr,
+                                       const Sums<NP, GON>& v, bool ok) {
   constexpr int SD = GON ? 256 : 128;
   const bool mine = lane_of_mask(r.last);
   if (r.last)
-    ok &= spin([&] {
-      return !mine || (lds_peek(claims + en.x) >> 16) == (unsigned)en.y - 1u;
-    });
+    ok = spin(ctr, [&] {
+           return !mine || (lds_peek(claims + en.x) >> 16) == (unsigned)en.y - 1u;
+         }) && ok;
   const double bad = ok ? 0.0 : NAN;
   const InstPtr p = fresh(in);
   const bool doF = (p->a.flags & BIE_F) != 0;
@@ -248,7 +253,7 @@ __device__ __forceinline__ void finish(InstPtr in, const int4& en, const Roles& 
       if constexpr (GON) column_store(G + at, 16u * lane, shared, g0, g1);
     }
   }
-  if (mine) {  // after the slot's reads above (LDS operations of a wave are in order)
+  if (mine && ok) {  // after the slot's reads above (LDS operations of a wave are in order)
     lds_wait();
     lds_poke(claims + en.x, 0u);
     lds_poke(turns + en.x, (unsigned)en.z + 1u);
@@ -409,12 +414,13 @@ __device__ __forceinline__ void stream_tile(InstPtr in, int rb, int seg, int S,
     const int l = fresh_lane(lane);
     const int4 en = fresh(in)->ent[(size_t)pos * NP + min(l, NP - 1)];
     bool ok;
-    const Roles r = claim<NP>(en, l, claims, turns, ok);
-    give<NP, GON>(en, r, l, acc, claims, v, ok);
+    const Roles r = claim<NP>(en, l, claims, turns, ctr, ok);
+    give<NP, GON>(en, r, l, acc, claims, ctr, v, ok);
     // before the column stores: loads and stores retire in order, so waiting for the rows
     // behind them would wait for the stores
     if constexpr (STAGED) rows_store();
-    finish<NP, GON>(in, en, r, l, (int64_t)rb * 64, active, acc, claims, turns, v, ok);
+    finish<NP, GON>(in, en, r, l, (int64_t)rb * 64, active, acc, claims, turns, ctr, v,
+                    ok);
     pos = nxt;
   }
   if constexpr (FLAT) atomicAdd(lds + L.csum + lane, csum);
@@ -705,6 +711,11 @@ std::vector<double> stream_tables(const RuleSet& rs, bool flat) {
   }
   for (int j = 0; j < kExpN; ++j) *e++ = (double)exp2l((long double)j / kExpN);
   return t;
+}
+
+int stream_polls() {
+  const char* v = std::getenv("BIE_AMD_POLLS");
+  return v ? std::atoi(v) : 1 << 22;
 }
 
 int stream_tab_doubles(const RuleSet& rs, bool flat) {

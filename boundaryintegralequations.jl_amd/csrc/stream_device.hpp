@@ -16,8 +16,6 @@
 namespace bie {
 namespace {
 
-constexpr int kSpinLimit = 1 << 22;  // polls of a bounded wait (never reached by a valid schedule)
-
 typedef double d8 __attribute__((ext_vector_type(8), aligned(8)));
 
 // The instance is read through the scalar cache where it is needed: fresh(p) keeps the
@@ -287,7 +285,8 @@ __host__ __device__ inline Layout layout_of(int S, int slot_doubles, int tab_dou
 
 // How a pair finds its points: flat elements, rows staged in LDS, rows read from memory.
 enum { kFlat = 0, kStaged = 1, kRead = 2 };
-enum { kTicket = 0, kTile = 1, kMidN = 2 };  // after the slot words (kMidN: two)
+// after the slot words (kMidN: two; kFailed: a wait of the tile gave up; kPolls: when it does)
+enum { kTicket = 0, kTile = 1, kMidN = 2, kFailed = 4, kPolls = 5 };
 
 // Adds v to an LDS counter from one lane; the value before, in every lane.  (Written out: the
 // compiler makes a wave-aggregated atomic of it, with a count over the lanes.)
@@ -317,15 +316,25 @@ __device__ __forceinline__ void column_store(double* col, unsigned at, bool shar
   }
 }
 
-// Waits (bounded) until ready() holds in every lane.
+// Waits until ready() holds in every lane, at most so many polls (from ctr): then, or once another
+// wave of the tile has given up, false.  A wave that gave up neither claims, nor adds, nor frees a
+// slot any more for what it waited for: its nodes are then never complete, and whoever was to
+// write their columns, or this wave, writes NaN.
 template <class P>
-__device__ __forceinline__ bool spin(P ready) {
+__device__ __forceinline__ bool spin(unsigned* ctr, P ready) {
+  bool done = !__any(!ready());
+  if (!done) {
+    const unsigned polls = lds_peek(ctr + kPolls);
 #pragma unroll 1
-  for (int n = 0; n < kSpinLimit; ++n) {
-    if (!__any(!ready())) return true;
-    __builtin_amdgcn_s_sleep(1);
+    for (unsigned n = 0; n < polls && !done; ++n) {
+      if (lds_peek(ctr + kFailed) != 0) break;
+      __builtin_amdgcn_s_sleep(1);
+      done = !__any(!ready());
+    }
+    if (!done) lds_poke(ctr + kFailed, 1u);
   }
-  return false;
+  asm volatile("" ::: "memory");  // what follows is read after what was waited for
+  return done;
 }
 
 struct Roles {
@@ -338,7 +347,7 @@ struct Roles {
 // never waits for one that waits for a slot.
 template <int NP>
 __device__ __forceinline__ Roles claim(const int4& en, int lane, unsigned* claims,
-                                       const unsigned* turns, bool& ok) {
+                                       const unsigned* turns, unsigned* ctr, bool& ok) {
   const bool slotted = lane < NP && en.x >= 0;
   // A SIMD issues for its oldest wave first; left alone, some waves run far ahead and then
   // wait here for the others.  A wave that has to wait gives way, one that need not is behind.
@@ -346,14 +355,15 @@ __device__ __forceinline__ Roles claim(const int4& en, int lane, unsigned* claim
     __builtin_amdgcn_s_setprio(0);
   else
     __builtin_amdgcn_s_setprio(2);
-  ok = spin([&] { return !slotted || lds_peek(turns + en.x) == (unsigned)en.z; });
+  ok = spin(ctr, [&] { return !slotted || lds_peek(turns + en.x) == (unsigned)en.z; });
+  const bool mine = slotted && ok;
   unsigned old = 0;
-  if (slotted) old = lds_count(claims + en.x, 1u) & 0xffffu;
+  if (mine) old = lds_count(claims + en.x, 1u) & 0xffffu;
   Roles r;
-  r.first = __ballot(slotted && old == 0);
-  r.last = __ballot(slotted && old == (unsigned)en.y - 1u);
-  r.more = __ballot(slotted && old != 0 && old != (unsigned)en.y - 1u);
-  r.direct = __ballot(lane < NP && en.x < 0);
+  r.first = __ballot(mine && old == 0);
+  r.last = __ballot(mine && old == (unsigned)en.y - 1u);
+  r.more = __ballot(mine && old != 0 && old != (unsigned)en.y - 1u);
+  r.direct = __ballot(lane < NP && !mine);  // (not ok: NaN to all of them)
   return r;
 }
 
@@ -593,12 +603,14 @@ __device__ __forceinline__ void stream_run(InstOf inst_of, KmaxOf kmax_of, First
   const int ntab = run.tab_doubles + kTrigDoubles + kExpN;
   for (int t = threadIdx.x; t < ntab; t += 64 * W) lds[L.tab + t] = run.tab[t];
   if (threadIdx.x < 64) lds[L.csum + threadIdx.x] = 0.0;
+  if (threadIdx.x == 0) ctr[kPolls] = (unsigned)run.polls;
   int parity = 0, prev = -1;
   for (;;) {
     // between the barriers nobody works on a tile
     for (int t = threadIdx.x; t < 2 * S; t += 64 * W) words[t] = 0u;  // claims and turns
     if (threadIdx.x == 0) {
       ctr[kTicket] = 0u;
+      ctr[kFailed] = 0u;
       ctr[kMidN + parity] = 0u;
     }
     int rb, seg;

@@ -402,8 +402,8 @@ __device__ __forceinline__ void multi_pair_rows(double x0, double x1, double x2,
 // First and middle contributions of nb matrices: into the slot (see stream.hip's give).
 template <int NP, int KB, bool GON>
 __device__ __forceinline__ void give_multi(const int4& en, const Roles& r, int lane, double* acc,
-                                           unsigned* claims, const Multi<NP, KB, GON>& v, int nb,
-                                           bool& ok) {
+                                           unsigned* claims, unsigned* ctr,
+                                           const Multi<NP, KB, GON>& v, int nb, bool& ok) {
   constexpr int SK = GON ? 256 : 128, SD = KB * SK;
   const bool mine_first = lane_of_mask(r.first), mine_more = lane_of_mask(r.more);
 #pragma unroll
@@ -426,7 +426,10 @@ __device__ __forceinline__ void give_multi(const int4& en, const Roles& r, int l
     if (mine_first) lds_count(claims + en.x, 0x10000u);
   }
   if (r.more) {
-    ok &= spin([&] { return !mine_more || (lds_peek(claims + en.x) >> 16) != 0; });
+    if (!spin(ctr, [&] { return !mine_more || (lds_peek(claims + en.x) >> 16) != 0; })) {
+      ok = false;
+      return;
+    }
 #pragma unroll
     for (int s = 0; s < NP; ++s)
       if ((r.more >> s) & 1) {
@@ -452,14 +455,14 @@ template <int NP, int KB, bool GON>
 __device__ __forceinline__ void finish_multi(InstPtr in, SweepPtr sw, const int4& en,
                                              const Roles& r, int lane, int64_t i0, bool active,
                                              int k0, int nb, const double* acc, unsigned* claims,
-                                             unsigned* turns, const Multi<NP, KB, GON>& v,
-                                             bool& ok) {
+                                             unsigned* turns, unsigned* ctr,
+                                             const Multi<NP, KB, GON>& v, bool ok) {
   constexpr int SK = GON ? 256 : 128, SD = KB * SK;
   const bool mine = lane_of_mask(r.last);
   if (r.last)
-    ok &= spin([&] {
-      return !mine || (lds_peek(claims + en.x) >> 16) == (unsigned)en.y - 1u;
-    });
+    ok = spin(ctr, [&] {
+           return !mine || (lds_peek(claims + en.x) >> 16) == (unsigned)en.y - 1u;
+         }) && ok;
   const double bad = ok ? 0.0 : NAN;
   const InstPtr p = fresh(in);
   const bool doF = (p->a.flags & BIE_F) != 0;
@@ -497,7 +500,7 @@ __device__ __forceinline__ void finish_multi(InstPtr in, SweepPtr sw, const int4
       }
     }
   }
-  if (mine) {
+  if (mine && ok) {
     lds_wait();
     lds_poke(claims + en.x, 0u);
     lds_poke(turns + en.x, (unsigned)en.z + 1u);
@@ -507,7 +510,8 @@ __device__ __forceinline__ void finish_multi(InstPtr in, SweepPtr sw, const int4
 // Elements of the tile's segment, drawn by this wave, for the matrices k0 .. of a block.
 template <int NP, bool FLAT, bool TAY, bool CPLX, bool GON, bool FAST>
 __device__ __forceinline__ void sweep_tile(InstPtr in, SweepPtr sw, int rb, int seg, int kb,
-                                           int S, int tab_doubles, double* lds, int parity) {
+                                           int S, int tab_doubles, double* lds,
+                                           int parity) {
   constexpr SweepShape kShape = sweep_shape(NP, GON, FLAT && TAY && !GON);
   constexpr int W = kShape.waves, KB = kShape.kb;
   constexpr bool kMids = NP == 6;
@@ -637,10 +641,10 @@ __device__ __forceinline__ void sweep_tile(InstPtr in, SweepPtr sw, int rb, int 
       csum += cs_pair;
     }
     bool ok;
-    const Roles r = claim<NP>(en, l, claims, turns, ok);
-    give_multi<NP, KB, GON>(en, r, l, acc, claims, v, nb, ok);
+    const Roles r = claim<NP>(en, l, claims, turns, ctr, ok);
+    give_multi<NP, KB, GON>(en, r, l, acc, claims, ctr, v, nb, ok);
     finish_multi<NP, KB, GON>(in, sw, en, r, l, (int64_t)rb * 64, active, k0, nb, acc, claims,
-                              turns, v, ok);
+                              turns, ctr, v, ok);
     pos = nxt;
   }
   if (kb == 0) atomicAdd(lds + L.csum + lane, csum);

@@ -415,3 +415,50 @@ def test_targets_far_beyond_the_range_of_one_over_r_cubed(kind, far, down):
             m = np.max(np.abs(b))
             assert 0 < m < np.inf, name
             assert np.linalg.norm(a / m - b / m) <= 1e-12 * np.linalg.norm(b / m), name
+
+
+@pytest.mark.parametrize("kind", ["linear", "quadratic"])
+@pytest.mark.parametrize("polls", [0, 1, 2])
+def test_waits_that_give_up(kind, polls, monkeypatch):
+    """With so few polls that waves give up waiting for each other, an entry is not a number or
+    it is right (C, which no wave waits for, is right).  Sixteen waves at once always meet: with
+    no poll after the first look some entries are not numbers."""
+    from bie_amd.assembly import Batch
+    mesh = M.perturb_radial(M.icosphere(12 if kind == "linear" else 5, kind), 0.01, 2)
+    N, k, n, m = mesh.n_sources, 3.0, 2, 2
+    dms = [DeviceMesh(mesh), DeviceMesh(M.icosphere(3, kind))]
+    bufs = [[DevBuf(16 * s) for s in (d.n_sources**2, d.n_sources**2, d.n_sources)] for d in dms]
+
+    def batch():
+        b = Batch(dms, n=n, m=m)
+        b.assemble([k, k], *[[x[q].ptr for x in bufs] for q in range(3)])
+        sync()
+        return [x.download(np.empty(s, dtype=np.complex128, order="F"))
+                for x, s in zip(bufs[0], ((N, N), (N, N), (N,)))]
+
+    def sweeps(gOn):
+        F, G, C = sweep(mesh, [k, 4.0, 5.0], mesh.sources, n, m, gOn=gOn)
+        return F[2], (G[2] if gOn else None), C
+
+    def orders(gOn):
+        F, G, C = taylor_assemble(mesh, k, M=2, n=n, m=m, gOn=gOn)
+        return F[:, :, 2], (G[:, :, 2] if gOn else None), C
+
+    calls = [lambda: assemble_parallel(mesh, k, n=n, m=m),
+             lambda: assemble_parallel(mesh, k + 0.2j, n=n, m=m), batch,
+             lambda: sweeps(True), lambda: sweeps(False), lambda: orders(True),
+             lambda: orders(False)]
+    given_up = 0
+    for number, call in enumerate(calls):
+        monkeypatch.delenv("BIE_AMD_POLLS", raising=False)
+        ref = call()
+        monkeypatch.setenv("BIE_AMD_POLLS", str(polls))
+        for x, y in zip(call(), ref):
+            if y is None:
+                continue
+            bad = np.isnan(x)
+            assert np.max(np.abs(x - y)[~bad], initial=0.0) <= 1e-12 * np.max(np.abs(y)), number
+            assert y.ndim == 2 or not bad.any(), number
+            given_up += int(bad.sum())
+    print(f"  {given_up} entries given up", flush=True)
+    assert polls > 0 or given_up > 0

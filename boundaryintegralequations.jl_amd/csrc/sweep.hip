@@ -612,7 +612,9 @@ __device__ __forceinline__ void sweep_tile(InstPtr in, SweepPtr sw, int rb, int 
         for (int s = 0; s < NP; ++s)
 #pragma unroll
           for (int d = 0; d < 3; ++d) P[s][d] = sload(ps + 3 * s + d);
-        c = select_rule_s<NP>(x0, x1, x2, P, ps, R, in) - 1;
+        // (no distance below Inf falls to the last rule, a mid-edge one on quadratic geometry:
+        // without six nodes to queue it for, such a row, which is NaN, runs along on the third)
+        c = select_rule_s<NP>(x0, x1, x2, P, ps, kMids ? R : min(R, 3), in) - 1;
       }
       const bool mid = kMids && c >= 3;
       const int cr = mid ? 0 : c;

@@ -462,3 +462,23 @@ def test_waits_that_give_up(kind, polls, monkeypatch):
             given_up += int(bad.sum())
     print(f"  {given_up} entries given up", flush=True)
     assert polls > 0 or given_up > 0
+
+
+@pytest.mark.parametrize("physics", ["linear", "disctriconstant", "disctrilinear"])
+@pytest.mark.parametrize("nm", [(3, 2), (5, 5)])
+def test_targets_that_are_not_numbers_on_quadratic_geometry(physics, nm):
+    """Such a row falls to the last of six rules, of which fewer than six nodes have three: it is
+    NaN, and the other rows are those of a call without it (rules staged, and read from
+    memory).  C, 0 outside a closed body, is held to the solid angles it cancels from."""
+    n, m = nm
+    mesh = (M.icosphere(3, "quadratic", physics="linear") if physics == "linear"
+            else M.with_discontinuous_physics(M.icosphere(3, "quadratic"), physics))
+    t = np.asfortranarray(M.fibonacci_sphere(130, 1.6))
+    t[:, 70], t[1, 5] = np.nan, np.inf
+    rows = np.isfinite(t).all(axis=0)
+    Fo, Go, Co = assemble_parallel(mesh, 3.0, t[:, rows], n=n, m=m)
+    F, G, C = assemble_parallel(mesh, 3.0, t, n=n, m=m)
+    Fs, Gs, Cs = sweep(mesh, [3.0, 4.0], t, n, m)
+    for X, Xo in ((F, Fo), (G, Go), (C, Co), (Fs[0], Fo), (Gs[0], Go), (Cs, Co)):
+        assert (np.max(np.abs(X[rows] - Xo)) if X.ndim == 1 else rel(X[rows], Xo)) <= TOL
+        assert np.isnan(X[~rows]).all()

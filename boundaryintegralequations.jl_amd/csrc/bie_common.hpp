@@ -134,6 +134,10 @@ constexpr int kFlatDoubles = 24;  // record of a flat element
 // Waves of its workgroup (one per CU): four per SIMD with 128 VGPRs each; eight- and nine-node
 // physics keep 32 and 36 sums per lane and take two per SIMD.
 constexpr int stream_waves(int NP) { return NP >= 8 ? 8 : 16; }
+// and of the kernels for large arguments with six-node physics or complex k, whose reduction
+// does not fit 128 VGPRs beside a pair (2562 quadratic nodes 1210 us with sixteen waves, 466 with
+// eight; 4002 linear nodes, real k, 1163 and 1248)
+constexpr int kSlowWaves = 8;
 
 struct StreamInst {
   AssemblyArgs a;

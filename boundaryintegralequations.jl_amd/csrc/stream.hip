@@ -620,10 +620,12 @@ void with_stream_kernel(int NP, int mode, bool cplx, bool gon, bool fast, Fn&& f
     constexpr int MD = decltype(md)::value;
     constexpr bool CX = decltype(cx)::value, G = decltype(g)::value;
     auto by_fast = [&](auto f) {
+      constexpr bool FS = decltype(f)::value;
+      constexpr int WV = FS || (N < 6 && !CX) ? W : kSlowWaves;
       if constexpr (BATCH)
-        fn(k_stream_batch<N, MD, CX, G, W, decltype(f)::value>);
+        fn(k_stream_batch<N, MD, CX, G, WV, FS>, WV);
       else
-        fn(k_stream<N, MD, CX, G, W, decltype(f)::value>);
+        fn(k_stream<N, MD, CX, G, WV, FS>, WV);
     };
     fast ? by_fast(std::true_type{}) : by_fast(std::false_type{});
   };
@@ -779,11 +781,11 @@ void launch_stream(const StreamInst& in, const StreamPlan& pl, const double* d_t
                       pl.mids ? 1 : 0};
   // not known to be fast: the tiles that are not are left to a second launch
   for (int pass = 0; pass < (fast ? 1 : 2); ++pass) {
-    with_stream_kernel<false>(in.a.NP, mode, cplx, gon, pass == 0, [&](auto kern) {
+    with_stream_kernel<false>(in.a.NP, mode, cplx, gon, pass == 0, [&](auto kern, int waves) {
       BIE_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                         hipFuncAttributeMaxDynamicSharedMemorySize,
                                         (int)pl.shmem));
-      hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * pl.waves), pl.shmem, s, in,
+      hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * waves), pl.shmem, s, in,
                          (int)tiles, run);
     });
   }
@@ -824,11 +826,11 @@ void launch_stream_batch(const BatchInst* d_inst, int n_inst, int64_t max_cols,
   const StreamRun run{d_tab, d_counters, fast ? nullptr : d_slow, pl.tab_doubles, pl.S, pl.row_doubles,
                       pl.mids ? 1 : 0};
   for (int pass = 0; pass < (fast ? 1 : 2); ++pass) {
-    with_stream_kernel<true>(NP, mode, cplx, gon, pass == 0, [&](auto kern) {
+    with_stream_kernel<true>(NP, mode, cplx, gon, pass == 0, [&](auto kern, int waves) {
       BIE_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                         hipFuncAttributeMaxDynamicSharedMemorySize,
                                         (int)pl.shmem));
-      hipLaunchKernelGGL(kern, dim3((unsigned)std::min(n_tiles, cus)), dim3(64 * pl.waves),
+      hipLaunchKernelGGL(kern, dim3((unsigned)std::min(n_tiles, cus)), dim3(64 * waves),
                          pl.shmem, s, d_inst, d_tiles, n_tiles, run);
     });
   }

@@ -41,8 +41,9 @@ namespace {
 struct SweepShape {
   int kb, waves, slot;
 };
-__host__ __device__ constexpr SweepShape sweep_shape(int NP, bool gon, bool lean) {
-  return lean ? SweepShape{6, 12, 6 * 128}
+__host__ __device__ constexpr SweepShape sweep_shape(int NP, bool gon, bool lean,
+                                                     bool fast = true) {
+  return lean ? SweepShape{6, fast ? 12 : kSlowWaves, 6 * 128}
               : SweepShape{(NP == 6 ? 2 : 4) * (gon ? 1 : 2), 8, (NP == 6 ? 2 : 4) * 256};
 }
 
@@ -512,7 +513,7 @@ template <int NP, bool FLAT, bool TAY, bool CPLX, bool GON, bool FAST>
 __device__ __forceinline__ void sweep_tile(InstPtr in, SweepPtr sw, int rb, int seg, int kb,
                                            int S, int tab_doubles, double* lds,
                                            int parity) {
-  constexpr SweepShape kShape = sweep_shape(NP, GON, FLAT && TAY && !GON);
+  constexpr SweepShape kShape = sweep_shape(NP, GON, FLAT && TAY && !GON, FAST);
   constexpr int W = kShape.waves, KB = kShape.kb;
   constexpr bool kMids = NP == 6;
   const int lane = threadIdx.x & 63;
@@ -653,7 +654,7 @@ __device__ __forceinline__ void sweep_tile(InstPtr in, SweepPtr sw, int rb, int 
 }
 
 template <int NP, bool FLAT, bool TAY, bool CPLX, bool GON, bool FAST>
-__global__ void __launch_bounds__(64 * sweep_shape(NP, GON, FLAT && TAY && !GON).waves)
+__global__ void __launch_bounds__(64 * sweep_shape(NP, GON, FLAT && TAY && !GON, FAST).waves)
 k_sweep(const StreamInst one, const SweepArgs args, int n_tiles, const StreamRun run) {
   extern __shared__ double lds[];
   const auto* base = (const __attribute__((address_space(4))) char*)
@@ -680,7 +681,7 @@ k_sweep(const StreamInst one, const SweepArgs args, int n_tiles, const StreamRun
       return 2.0 * m;
     }
   };
-  constexpr SweepShape kShape = sweep_shape(NP, GON, FLAT && TAY && !GON);
+  constexpr SweepShape kShape = sweep_shape(NP, GON, FLAT && TAY && !GON, FAST);
   stream_run<kShape.slot, kShape.waves, NP == 6, FAST>(
       inst_of, kmax_of, [&](InstPtr, int tile) { return tile < per_kb; },
       [&](InstPtr p, int rb, int seg, int tile, int parity) {
@@ -768,7 +769,8 @@ void launch_sweep(const StreamInst& in, const SweepArgs& sw, const StreamPlan& p
                   const double* d_tab, unsigned* d_counters, int* d_slow, int cus, bool fast,
                   bool prepare_only, hipStream_t s) {
   const bool gon = (in.a.flags & BIE_G) != 0, tay = sw.taylor != 0, cplx = sw.k_im != 0.0;
-  const int KB = sweep_shape(in.a.NP, gon, pl.flat && tay && !gon).kb;
+  const bool lean = pl.flat && tay && !gon;
+  const int KB = sweep_shape(in.a.NP, gon, lean).kb;
   const int64_t tiles =
       (int64_t)((sw.nk + KB - 1) / KB) * in.n_segments * (int64_t)in.n_rowblocks;
   BIE_REQUIRE(tiles > 0 && tiles < 2147483647LL, BIE_EINVAL, "too many sweep tiles");
@@ -783,7 +785,8 @@ void launch_sweep(const StreamInst& in, const SweepArgs& sw, const StreamPlan& p
                                         (int)pl.shmem));
       if (prepare_only) return;
       hipLaunchKernelGGL(kern, dim3((unsigned)std::min<int64_t>(tiles, cus)),
-                         dim3(64 * pl.waves), pl.shmem, s, in, sw, (int)tiles, run);
+                         dim3(64 * sweep_shape(in.a.NP, gon, lean, pass == 0).waves), pl.shmem, s,
+                         in, sw, (int)tiles, run);
       if (pl.mids && pass == (fast ? 0 : 1))
         hipLaunchKernelGGL(mid, dim3(512, (unsigned)std::min(sw.nk, 1024)), dim3(256),
                            sizeof(double) *

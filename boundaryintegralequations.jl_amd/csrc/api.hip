@@ -533,15 +533,15 @@ double radius_about(const double* c, const double* x, int64_t n) {
   return std::sqrt(r2);
 }
 
-// Whether every argument k r of the kernels' sincos stays below kTabFastMaxArg: r is
+// Whether every argument k r of the kernels' sincos stays below kTabFastMaxArg (and r below
+// kFastMaxDist): r is
 // at most |x - c| + |y - c| for a target x and an element point y, and y = sum N_k X_k with
 // sum |N_k| <= 2 on linear and quadratic triangles, so |y - c| <= 2 coord_radius (taken
-// twice again for margin).  target_radius < 0: unknown (device targets), never fast.  See also
-// kFastMinK.
+// twice again for margin).  target_radius < 0: unknown (device targets), never fast.
 bool fast_trig_ok(const bie_dmesh* dm, double kr, double target_radius) {
   if (!(target_radius >= 0.0)) return false;
   const double reach = target_radius + 4.0 * dm->coord_radius;
-  return std::isfinite(reach) && std::max(std::fabs(kr), kFastMinK) * reach < 0.5 * kTabFastMaxArg;
+  return reach < kFastMaxDist && std::fabs(kr) * reach < 0.5 * kTabFastMaxArg;
 }
 
 void assemble_device_impl(bie_dmesh* dm, double kr, double ki, const double* d_targets,

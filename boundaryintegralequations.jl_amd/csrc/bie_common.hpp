@@ -39,9 +39,9 @@ constexpr double kPi = 3.14159265358979323846;
 // The host chooses that form only when |k| times a bound on every target-to-element-point
 // distance is below it.
 constexpr double kTabFastMaxArg = 70368744177664.0;
-// The kernels of that form divide by up to r^5 at once: it is taken up to distances of 1e50
-// (and so as if |k| were at least this); the other form stays in range as far as r^2 does.
-constexpr double kFastMinK = 0.5 * kTabFastMaxArg / 1e50;
+// The kernels of that form divide by up to r^5 at once: it is taken up to these distances; the
+// other form stays in range as far as r^2 does.
+constexpr double kFastMaxDist = 1e50;
 
 // Point record of the concatenated rule set: u, v, w, then N, dN/du, dN/dv of the
 // geometry basis (6 slots each, unused slots zero).

@@ -443,8 +443,8 @@ __global__ void __launch_bounds__(256, 2) k_sparse_batch(const SparseArgs a) {
     for (int j = 0; j < cnt; ++j) {
       const double* x = a.src + 3 * (size_t)a.pairs[rec[2 + j]].x;
       const double cx = x[0] - a.center[0], cy = x[1] - a.center[1], cz = x[2] - a.center[2];
-      const double far = fmax(fabs(a.kr), kFastMinK) * (sqrt(fma(cx, cx, fma(cy, cy, cz * cz))) + a.reach);
-      near = near && far < 0.5 * kTabFastMaxArg;
+      const double dist = sqrt(fma(cx, cx, fma(cy, cy, cz * cz))) + a.reach;
+      near = near && fabs(a.kr) * dist < 0.5 * kTabFastMaxArg && dist < kFastMaxDist;
     }
     if (__builtin_amdgcn_readfirstlane((int)near) != (FAST ? 1 : 0)) return;
   }

@@ -643,7 +643,10 @@ __device__ __forceinline__ void stream_run(InstOf inst_of, KmaxOf kmax_of, First
     if constexpr (FAST) {
       const double* x = in->a.targets + 3 * min((int64_t)rb * 64 + lane, in->a.M - 1);
       const double cx = x[0] - in->center[0], cy = x[1] - in->center[1], cz = x[2] - in->center[2];
-      const double far = fmax(kmax_of(in, tile), kFastMinK) * (sqrt(fma(cx, cx, fma(cy, cy, cz * cz))) + in->reach);
+      const double dist = sqrt(fma(cx, cx, fma(cy, cy, cz * cz))) + in->reach;
+      // (both bounds at once, as a sum)
+      constexpr double kPerDist = 0.5 * kTabFastMaxArg / kFastMaxDist;
+      const double far = fma(kmax_of(in, tile), dist, kPerDist * dist);
       skip = run.slow && __any(!(far < 0.5 * kTabFastMaxArg));
       if (skip && threadIdx.x == 0) run.slow[atomicAdd(run.counters + kSlowCount, 1u)] = tile;
     }

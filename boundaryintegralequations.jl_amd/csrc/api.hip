@@ -325,13 +325,14 @@ void ensure_flat(bie_dmesh* dm, hipStream_t s) {
   dm->d_eflat = rec;
 }
 
-// The schedule of dm in a batch: S slots, at least `segments` segments.  The records of flat
-// elements are written here, once (a single-mesh call writes its own each time).  The mesh
-// keeps the last few, so that a new batch finds them; a batch and its graphs hold theirs until
-// they let go of it, whatever other batches ask of the mesh meanwhile.
-std::shared_ptr<bie_dmesh::Stream> batch_stream(bie_dmesh* dm, int S, int64_t segments,
-                                                hipStream_t s) {
-  auto& kept = dm->bstreams;
+// The schedule of dm for S slots and at least `segments` segments from `kept`, where the mesh keeps
+// the last ones (at most `most`), so that a new batch or a sweep of as many matrices finds them;
+// batches and graphs hold theirs until they let go of it, whatever else is asked of the mesh
+// meanwhile.  records: the records of flat elements are written here, once (other calls write
+// their own each time).
+std::shared_ptr<bie_dmesh::Stream> kept_stream(
+    bie_dmesh* dm, std::vector<std::shared_ptr<bie_dmesh::Stream>>& kept, size_t most, int S,
+    int64_t segments, bool records, hipStream_t s) {
   for (size_t q = 0; q < kept.size(); ++q)
     if (kept[q]->key == segments && kept[q]->S == S) {
       std::rotate(kept.begin(), kept.begin() + q, kept.begin() + q + 1);
@@ -348,7 +349,7 @@ std::shared_ptr<bie_dmesh::Stream> batch_stream(bie_dmesh* dm, int S, int64_t se
                 stream_schedule(dm, element_centres(dm), S,
                                 std::max(segments, least_segments(dm))),
                 S, segments, s);
-  if (out.d_flat) {
+  if (records && out.d_flat) {
     StreamPrep p{};
     p.E = (int)dm->E;
     p.coords = dm->d_coords;
@@ -362,7 +363,7 @@ std::shared_ptr<bie_dmesh::Stream> batch_stream(bie_dmesh* dm, int S, int64_t se
     BIE_HIP_CHECK(hipStreamSynchronize(s));
   }
   kept.insert(kept.begin(), sp);
-  if (kept.size() > bie_dmesh::kBatchStreams) kept.pop_back();
+  if (kept.size() > most) kept.pop_back();
   return sp;
 }
 
@@ -454,20 +455,6 @@ StreamPrep stream_prep(bie_dmesh* dm, const AssemblyArgs& a, const bie_dmesh::St
   p.flat = sc.d_flat;
   p.elem = sc.d_flat ? nullptr : dm->d_elem;
   return p;
-}
-
-// The sweep kernel's schedule: S slots and at least min_segments segments (0: as suits the
-// collocation rows).  It does not depend on a call's targets or matrices: a graph keeps it.
-bie_dmesh::Stream& ensure_sweep_stream(bie_dmesh* dm, bie_dmesh::Stream& out, int S,
-                                       int64_t min_segments, int cus, hipStream_t s) {
-  const int64_t key = min_segments * 65536 + std::min(dm->rs.len[0], 65535);
-  if (out.key == key && out.S == S && out.d_order) return out;
-  int64_t want = std::max(min_segments, least_segments(dm));
-  if (min_segments == 0)
-    want = choose_stream_segments((dm->N + 63) / 64, dm->E, dm->rs.len[0], dm->pk, cus,
-                                  least_segments(dm));
-  upload_stream(dm, out, stream_schedule(dm, element_centres(dm), S, want), S, key, s);
-  return out;
 }
 
 AssemblyArgs make_args(bie_dmesh* dm, const double* d_targets, int64_t M, double kr,
@@ -618,12 +605,13 @@ void assemble_device_impl(bie_dmesh* dm, double kr, double ki, const double* d_t
 // Batched sweep over nk real wavenumbers (d_k on the device), or with taylor the k
 // derivatives of orders 0..nk-1 at k_re + i k_im (d_k unused).  prepare_only builds every
 // cache (rules, schedule, lists) without launching, so that a later call can be captured
-// into a graph; lists are the graph's own then.
+// into a graph; lists are the graph's own then, and it keeps the schedule (keep).
 void sweep_device_impl(bie_dmesh* dm, const double* d_k, int nk, const double* d_targets,
                        int64_t M, int n, int m, uint32_t flags, double* dF, double* dG,
                        int64_t stride, double* dC, hipStream_t s, StreamLists& lists,
                        bool prepare_only, bool taylor = false, double k_re = 0.0,
-                       double k_im = 0.0) {
+                       double k_im = 0.0,
+                       std::shared_ptr<bie_dmesh::Stream>* keep = nullptr) {
   BIE_REQUIRE(dm != nullptr, BIE_EINVAL, "dmesh is NULL");
   BIE_REQUIRE(!kind_is_quad(dm->gkind), BIE_EUNSUPPORTED,
               "sweeps and k-derivatives: triangular meshes only");
@@ -649,15 +637,32 @@ void sweep_device_impl(bie_dmesh* dm, const double* d_k, int nk, const double* d
   const int cus = device_cus(dm->device);
   const bool lean = taylor && flat_elements(dm) && (flags & BIE_G) == 0;
   const StreamPlan plan = sweep_plan(dm->rs, flat_elements(dm), lean, dm->sweep_slots);
-  const int64_t min_seg =
+  const int KB = sweep_block_size(dm->pk, (flags & BIE_G) != 0, lean);
+  // Segments that were configured, or as suit the collocation rows.  A small mesh needs many, and
+  // so small tiles, to fill the chip with one block of matrices; eight blocks and more fill it by
+  // themselves (362 nodes, 9 points, 40 wavenumbers: 422 us with the segments of one block, 190
+  // with those of all).
+  const int64_t rows = (dm->N + 63) / 64, blocks = (nk + KB - 1) / KB;
+  const bool many = blocks >= 8 && 16 * rows <= cus && (M + 63) / 64 == rows;
+  auto& choice = dm->sweep_choice[many ? 1 : 0];
+  const int64_t tiles = many ? rows * blocks : rows;
+  if (choice.Q != dm->rs.len[0] || choice.tiles != tiles) {
+    choice.Q = dm->rs.len[0];
+    choice.tiles = tiles;
+    choice.segments =
+        choose_stream_segments(tiles, dm->E, choice.Q, dm->pk, cus, least_segments(dm));
+  }
+  const int64_t segments =
       dm->sweep_elems_per_tile
           ? std::max<int64_t>(1, (dm->E + dm->sweep_elems_per_tile - 1) / dm->sweep_elems_per_tile)
-          : 0;
-  const bie_dmesh::Stream& sc = ensure_sweep_stream(dm, lean ? dm->lstream : dm->sstream, plan.S, min_seg, cus, s);
+          : choice.segments;
+  const std::shared_ptr<bie_dmesh::Stream> held =
+      kept_stream(dm, dm->sstreams, bie_dmesh::kSweepStreams, plan.S, segments, false, s);
+  const bie_dmesh::Stream& sc = *held;
+  if (keep) *keep = held;
   // the wavenumbers of a sweep are on the device: its tiles decide there
   const bool fast = taylor && fast_trig_ok(dm, k_re, target_radius);
   const int64_t rowblocks = (M + 63) / 64;
-  const int KB = sweep_block_size(dm->pk, (flags & BIE_G) != 0, lean);
   ensure_lists(lists, plan.mids, M, dm->E, sc.segments,
                fast ? 0 : (int64_t)((nk + KB - 1) / KB) * rowblocks * sc.segments);
   AssemblyArgs a = make_args(dm, d_targets, M, 0.0, 0.0, flags, dF, dG, dC);
@@ -734,7 +739,7 @@ void batch_configure(bie_batch* b, const StreamPlan& pl, int cus, hipStream_t s)
     const int64_t rbs = (dm->N + 63) / 64;
     b->rowblocks[ii] = rbs;
     const int64_t min_seg = std::max<int64_t>(1, (dm->E + per_tile - 1) / per_tile);
-    streams[ii] = batch_stream(dm, S, min_seg, s);
+    streams[ii] = kept_stream(dm, dm->bstreams, bie_dmesh::kBatchStreams, S, min_seg, true, s);
     const bie_dmesh::Stream& sc = *streams[ii];
     if (dm->N == 0 || dm->E == 0) continue;
     int64_t rank = 0;
@@ -1069,8 +1074,7 @@ int bie_dmesh_destroy(bie_dmesh* dm) {
   for (auto& by_g : dm->stream)
     for (auto& sc : by_g) free_stream(sc);
   dm->bstreams.clear();
-  free_stream(dm->sstream);
-  free_stream(dm->lstream);
+  dm->sstreams.clear();
   for (auto& by_g : dm->lists)
     for (auto& l : by_g) free_lists(l);
   free_lists(dm->blists);
@@ -2171,7 +2175,7 @@ struct bie_graph {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   std::vector<void*> owned;  // device buffers the captured kernels read (freed with the graph)
-  std::vector<std::shared_ptr<bie_dmesh::Stream>> streams;  // (batch) their schedules
+  std::vector<std::shared_ptr<bie_dmesh::Stream>> streams;  // their schedules
 };
 
 int bie_sweep_graph_create(bie_dmesh* dm, const double* d_k, int32_t nk,
@@ -2191,7 +2195,7 @@ int bie_sweep_graph_create(bie_dmesh* dm, const double* d_k, int32_t nk,
     try {
       // build every cache and set kernel attributes outside the capture
       sweep_device_impl(dm, d_k, nk, d_targets, n_targets, n, m, flags, dF, dG, stride, dC, cs,
-                        lists, true);
+                        lists, true, false, 0.0, 0.0, &g->streams.emplace_back());
       BIE_HIP_CHECK(hipStreamSynchronize(cs));
       BIE_HIP_CHECK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
       try {

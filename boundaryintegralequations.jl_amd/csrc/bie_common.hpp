@@ -443,12 +443,15 @@ struct bie_dmesh {
     std::vector<int> h_seg_begin;  // (batch) host copy, for the tile list
   };
   double* d_eflat = nullptr;     // records of flat elements in element order (k-derivatives)
-  // of single-mesh calls (own rows or others, without or with G), of sweeps and k-derivatives
-  // (F alone on flat elements: lstream, whose slots are smaller)
-  Stream stream[2][2], sstream, lstream;
-  // of batches: the last few that batches asked for, shared with the batches that use them
-  static constexpr size_t kBatchStreams = 4;
-  std::vector<std::shared_ptr<Stream>> bstreams;
+  Stream stream[2][2];  // of single-mesh calls (own rows or others, without or with G)
+  // of batches, and of sweeps and k-derivatives: the last few that were asked for, shared with
+  // the batches and graphs that use them
+  static constexpr size_t kBatchStreams = 4, kSweepStreams = 8;
+  std::vector<std::shared_ptr<Stream>> bstreams, sstreams;
+  struct {
+    int Q = -1, segments = 0;
+    int64_t tiles = -1;
+  } sweep_choice[2];             // the last choice of segments, for few and for many matrices
   bie::StreamLists lists[2][2], blists, slists;  // (lists: as stream)
   double* d_stab = nullptr;      // its tables for the cached rule set (stream_tables)
   // tile shape of the frequency sweep (bie_sweep_tune): elements per tile (0: one segment per

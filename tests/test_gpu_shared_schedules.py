@@ -104,3 +104,41 @@ def test_a_captured_assembly_and_calls_of_other_rows():
         torch.cuda.synchronize()
         for x, y in zip(values([(F, G, C)])[0], ref):
             assert rel(x, y) < 1e-14
+
+
+@pytest.mark.parametrize("kind", ["linear", "quadratic"])
+def test_a_sweep_graph_and_sweeps_of_other_lengths(kind):
+    """Sweeps of few and of many wavenumbers cut a small mesh into different segments, more kinds
+    of them than a mesh keeps: a graph's replays stay right beside them, and so do they."""
+    import oracle
+    mesh = M.icosphere(4 if kind == "linear" else 2, kind)
+    N, n, m, most = mesh.n_sources, 3, 2, 44
+    dm = DeviceMesh(mesh)
+    ks = np.linspace(0.5, 6.0, most)
+    kb = DevBuf(8 * most)
+    kb.upload(ks)
+    F, G, C = DevBuf(16 * N * N * most), DevBuf(16 * N * N * most), DevBuf(16 * N)
+    Fg, Gg, Cg = DevBuf(16 * N * N * 40), DevBuf(16 * N * N * 40), DevBuf(16 * N)
+    g = dm.sweep_graph(kb.ptr, 40, Fg.ptr, Gg.ptr, N * N, Cg.ptr, n=n, m=m)
+    ref = {q: oracle.assemble(mesh, ks[q], n=n, m=m) for q in (0, 2, 33, 39)}
+
+    def check(bufs, nk):
+        for q, (Fo, Go, Co) in ref.items():
+            if q < nk:
+                for x, y in zip(bufs[:2], (Fo, Go)):
+                    v = x.download(np.empty(nk * N * N, dtype=np.complex128)).reshape(nk, N, N)
+                    assert rel(v[q].T, y) < 1e-12
+        assert rel(bufs[2].download(np.empty(N, dtype=np.complex128)), ref[0][2]) < 1e-12
+
+    for nk in (1, 3, 34, 35, 36, 37, 38, 39, 41, 42, 43, 44):
+        for gOn in (False, True):
+            dm.assemble_sweep(kb.ptr, nk, F.ptr, G.ptr, N * N, C.ptr, n=n, m=m, gOn=gOn)
+        sync()
+        check((F, G, C), nk)
+        if nk in (3, 38, 44):
+            spoil([(Fg, Gg, Cg)])
+            sync()
+            g.launch()
+            sync()
+            check((Fg, Gg, Cg), 40)
+    g.close()

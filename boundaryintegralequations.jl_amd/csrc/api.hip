@@ -1929,8 +1929,9 @@ int bie_schedule_check(const bie_mesh* mesh, int32_t min_segments, int64_t* stat
                                           (int)mesh->n_sources, cent.data(), kSlotWaves,
                                           kSlotCount, min_segments);
     validate_slot_schedule(sc, ptopo.data(), np, (int)E, (int)mesh->n_sources);
-    // the schedules of the kernels as well: few slots and many
-    for (int S : {17, 34, kSlotCount}) {
+    // the schedules of the kernels as well: with as few slots as they have (17: four matrices of F
+    // and G) and as many (120: one of F)
+    for (int S : {17, 34, kSlotCount, 120}) {
       if (S < 2 * np) continue;
       const StreamSchedule st = build_stream_schedule(ptopo.data(), np, (int)E,
                                                       (int)mesh->n_sources, cent.data(), S,

@@ -1,21 +1,22 @@
-// Host scheduler for the LDS-accumulator assembly kernel.
+// Host schedules of the assembly kernels.
 //
 // The dense assembly writes F[i, j] = sum over elements e incident to node j of that
-// element's contribution for target i.  A workgroup owns 64 target rows and one
-// *segment* of elements; it sweeps the segment in steps of W elements (one per wave) and
-// accumulates node contributions in LDS *slots*.  A node occupies a slot from the step
-// of its first incident element in the segment to the step of its last; the kernel
-// flushes it to F and G during the following step (overlapped with that step's
-// quadrature, one barrier per step), so the slot becomes free for a new node one step
-// after that: a node whose last step is t holds its slot through step t + 1 and the slot
-// is reused at step t + 2 at the earliest.  Nodes whose elements all lie in one segment
-// ("owned") are written once with a plain store; nodes touched by several segments
-// ("shared") are added atomically into columns zeroed beforehand.
+// element's contribution for target i.  A workgroup owns 64 target rows and one *segment* of
+// elements, an ordered list that its waves draw from one element at a time; a node's
+// contributions meet in an LDS *slot*, which it occupies from its first element in the segment
+// to a few positions past its last (build_stream_schedule; stream.hip has the hand-over).
+// Nodes whose elements all lie in one segment ("owned") are written once with a plain store;
+// nodes touched by several segments ("shared") are added atomically into columns zeroed
+// beforehand.
 //
 // Segments come from recursive coordinate splitting of the element centroids into the
 // requested number of parts; each is swept along its longest axis, which keeps the number
 // of occupied slots (the sweep front) near the segment's width.  Segments are split
 // further until their front fits the slot budget.
+//
+// build_slot_schedule is the same for waves that meet at a barrier after every step of W
+// elements: a node is flushed during the step after its last element, and its slot is free one
+// step later.  No kernel runs by it: bie_schedule_check reports its statistics.
 #include <algorithm>
 #include <cmath>
 #include <deque>

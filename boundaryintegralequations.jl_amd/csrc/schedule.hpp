@@ -1,4 +1,4 @@
-// Schedules of the LDS-accumulator assembly kernels (built by schedule.cpp).
+// Schedules of the assembly kernels' LDS slots (built by schedule.cpp).
 #pragma once
 
 #include <cstdint>
@@ -11,6 +11,7 @@ namespace bie {
 
 constexpr int kSharedBit = 1 << 30;
 
+// Slot schedule in steps of W elements (bie_schedule_check's statistics; no kernel runs by it).
 struct SlotSchedule {
   int W = 0;            // elements per step (waves per workgroup)
   int S = 0;            // LDS slots available

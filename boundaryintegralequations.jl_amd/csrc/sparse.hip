@@ -16,11 +16,11 @@
 // One wave per (row, element) pair or per batch of pairs that share an element: lanes take the
 // rule's points (a few thousand), the partial sums are reduced across the wave and added into
 // the entries with FP64 atomics (a row's entries receive several elements' contributions).
-// Bound by instruction issue (VALU busy 85 % of the time): curved elements cost 290 per point
-// and pair, of which the surface with its exactly rounded normal is 200; flat ones 80.  Before
-// and after the cheaper exact divisions, the normal of flat elements taken out of the loop and
-// the branch-free sincos, 40-point rules (us): 10242 nodes, depth 1: 2350 -> 1737; depth 2,
-// quadratic 4002 nodes 5359 -> 2992, linear 1962 nodes 712 -> 622.
+// Bound by instruction issue (VALU busy 94 % of the time, 10242 quadratic nodes, depth 1): curved
+// elements cost 290 per point and pair, of which the surface with its exactly rounded normal is
+// 200; flat ones 80.  Before and after the cheaper exact divisions, the normal of flat elements
+// taken out of the loop and the branch-free sincos (us): 10242 nodes, depth 1: 2350 -> 1686;
+// depth 2, quadratic 2562 nodes 3400 -> 1822, linear 1962 nodes 642 -> 515.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -156,7 +156,8 @@ __device__ __forceinline__ double quot(double a, double b, double y) {
   const double q = a * y;
   return fma(fma(-b, q, a), y, q);
 }
-// sqrt(s), correctly rounded, for s in [1, 3].
+// sqrt(s), correctly rounded, for s in [1, 3]: Goldschmidt's coupled iteration for sqrt(s) and
+// 1 / (2 sqrt(s)), then two corrections by the exact residual s - g^2.
 __device__ __forceinline__ double sqrt_1_3(double s) {
   const double y = __builtin_amdgcn_rsq(s);
   double g = s * y, h = 0.5 * y;
@@ -416,10 +417,13 @@ __global__ void __launch_bounds__(256) k_sparse_pairs_short(const SparseArgs a) 
   sparse_add<NP, false>(a, p, true, acc[0]);
 }
 
-// Rows per batch: as many as 256 registers hold the sums of, so that two waves share a SIMD.
-// (Depth 2, two to four thousand nodes, us: three six-node rows spilled, 3078 against 2992 with
-// two, and in 512 registers took 3666; four three-node rows 2495 and 3181 on flat and curved
-// elements against 2386 and 1979 with three.)
+// Rows per batch, at two waves a SIMD (256 registers): the most that paid.  One- and three-node
+// physics on flat elements fit; with curved elements or six nodes some registers spill (the
+// branch-free kernels: 10-14 with three rows of three nodes on curved elements, with two of six
+// nodes 35-41 on flat and 121-125 on curved ones).  (Depth 2, two to four
+// thousand nodes, us: three six-node rows 3078 against 2992 with two, and in 512 registers 3666;
+// four three-node rows 2495 and 3181 on flat and curved elements against 2386 and 1979 with
+// three.)
 constexpr int batch_rows(int NP) { return NP == 1 ? 4 : NP == 3 ? 3 : 2; }
 
 // Batches of up to B pairs that share an element (built on the host, grouped by the rule

@@ -9,9 +9,10 @@
 // What does not depend on the matrix is formed once per pair or point: rule selection, y - x,
 // 1/r, the C integrand (first block only).  Four matrices of F and G (eight of F alone, two
 // and four with six-node physics) are 96 registers of sums; eight waves per CU (two per SIMD,
-// 256 VGPRs) hold them (with twelve, 168 VGPRs, they spilled: 11.9 ms and 10.9 ms where eight
-// take 11.8 and 5.7 for 16 wavenumbers and 26 orders on 4002 nodes).  A slot of 8 KB leaves 17
-// of them, which the surface's segments have to fit (44 for 8000 elements).
+// 256 VGPRs) hold them (eight of F alone on flat elements spill 20 registers; with twelve waves,
+// 168 VGPRs, all spilled: 11.9 ms and 10.9 ms where eight take 11.8 and 5.7 for 16 wavenumbers
+// and 26 orders on 4002 nodes).  A slot of 8 KB leaves 17 of them, which the surface's segments
+// have to fit (44 for 8000 elements).
 //   * Uniformly spaced k: e^{i k_b r} = e^{i k_0 r} (e^{i dk r})^b, two sincos per point and
 //     one complex product per further k; other blocks form each e^{i k_b r}.  The kernel
 //     finds out for every block, so any list of k is exact.
@@ -21,7 +22,7 @@
 //     one sequence of sums (two products and six multiply-adds per point and order) gives
 //     both.
 // 16 wavenumbers on 4002 nodes, 16 points: 17.0 -> 11.5 ms (VALU busy 83 % of the time, 134
-// instructions per point and four wavenumbers); 26 orders of F, four points: 8.7 -> 5.0 ms.
+// instructions per point and four wavenumbers); 26 orders of F, four points: 8.7 -> 4.9 ms (75 %).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -34,10 +35,11 @@ namespace bie {
 namespace {
 
 // Shape of a kernel: matrices of a block, waves of a workgroup, doubles of a slot.  F alone of
-// the k-derivatives on flat elements (`lean`) keeps sums for one order more than its block
-// and no others: six orders fit 168 registers and so twelve waves, which its short rules need
-// (few points a pair: half of the time is the hand-over).  26 orders on 4002 nodes, four
-// points: 4.99 ms; eight orders and eight waves 5.69, four and sixteen 5.43.
+// the k-derivatives on flat elements (`lean`) keeps sums for one order more than its block and no
+// others: twelve waves of 168 registers take six orders (14 registers spill, 25 with complex k),
+// and its short rules need the waves (few points a pair: half of the time is the hand-over).  26
+// orders on 4002 nodes, four points: 4.99 ms; eight orders and eight waves 5.69, four and sixteen
+// 5.43.
 struct SweepShape {
   int kb, waves, slot;
 };

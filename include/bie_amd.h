@@ -227,11 +227,12 @@ int bie_select_rules_device(bie_dmesh* dm, const double* d_targets, int64_t n_ta
 int bie_element_geometry(bie_dmesh* dm, int32_t rule, int32_t n, int32_t m, double* y,
                          double* normals, double* jw);
 
-/* Builds the LDS-slot schedule of the assembly kernel for a host mesh and replays it,
- * checking every invariant the kernel relies on (no counterpart in the reference; the
- * reference's threads own whole rows, assembly_collocation.jl:314), for steps of one and of
- * two elements per wave.  stats (6 values, one element per wave): segments, steps, max
- * live slots, shared nodes, zeroed columns, flush entries. */
+/* Builds the LDS-slot schedules of the assembly kernels for a host mesh, for the fewest to the
+ * most slots that they have, and replays them, checking every invariant the kernels rely on (no
+ * counterpart in the reference; the reference's threads own whole rows,
+ * assembly_collocation.jl:314).  stats (6 values) describe the schedule of the same segments in
+ * steps of eight elements over 64 slots: segments, steps, max live slots, shared nodes, zeroed
+ * columns, flush entries. */
 int bie_schedule_check(const bie_mesh* mesh, int32_t min_segments, int64_t* stats);
 
 /* ---- Batched frequency sweep ------------------------------------------------------------
@@ -259,7 +260,8 @@ int bie_sweep_tune(bie_dmesh* dm, const double* d_k, int32_t nk, const double* d
                    double* dG, int64_t stride, double* dC, void* stream,
                    int32_t* elems_per_tile, int32_t* slots, double* best_ms);
 /* The same sweep captured once into a HIP graph (kernels only, no memset nodes); launching
- * the graph replays it on any stream.  The graph keeps the pointers it was built with. */
+ * the graph replays it on any stream.  The graph keeps the pointers it was built with, lists
+ * and the schedule of its own; calls on this mesh with another rule set (n, m) invalidate it. */
 int bie_sweep_graph_create(bie_dmesh* dm, const double* d_k, int32_t nk,
                            const double* d_targets, int64_t n_targets, int32_t n, int32_t m,
                            uint32_t flags, double* dF, double* dG, int64_t stride, double* dC,

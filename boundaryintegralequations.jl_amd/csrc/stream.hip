@@ -719,7 +719,7 @@ std::vector<double> stream_tables(const RuleSet& rs, bool flat) {
 
 int stream_polls() {
   const char* v = std::getenv("BIE_AMD_POLLS");
-  return v ? std::atoi(v) : 1 << 22;
+  return v ? std::max(0, std::atoi(v)) : 1 << 22;
 }
 
 int stream_tab_doubles(const RuleSet& rs, bool flat) {
